@@ -1,84 +1,17 @@
-// Direct convolution over NHWC: the general path (any kernel size, stride,
-// padding, dilation, group count and channel count).  The MFMA implicit-GEMM
-// kernel takes the shapes it is eligible for; everything else lands here:
-// small input-channel counts (the RGB stem), channel counts that are not a
-// multiple of 4, grouped convolutions with 1 < group < C.
+// Direct convolution over NHWC: everything the MFMA implicit-GEMM kernels do not take (channel
+// counts that fill no 16-byte vector, grouped convolutions, the RGB stem).  Three kernels:
+// conv_stem_* (K = k*k*C <= 32, group 1), conv_patch_mfma (input patch and filter staged in
+// LDS, contracted on the MFMA units) and conv_direct_general (one thread per output, for what
+// neither takes: patches that do not fit LDS, groups too small for an MFMA block).
 //
-// Semantics follow conv2d.glsl:29-92 / conv2d_grp.glsl:30-123: accumulator
-// starts at the bias, taps outside the image are skipped, then the fused
-// activation.  Accumulation order is ky, kx, input channel ascending.
+// Semantics follow conv2d.glsl:29-92 / conv2d_grp.glsl:30-123: bias, taps outside the image
+// contribute nothing, then the fused activation.
 #include <algorithm>
 #include <type_traits>
 #include "common.h"
 
 namespace ogle {
 namespace {
-
-// Small-K kernel (the RGB stem): one thread produces OPT consecutive output
-// channels of one pixel.  Filter taps [O][K] (K = k*k*C, OHWI order) are staged
-// through LDS transposed to [K][O]; a wave then reads the OPT weights of one
-// (tap, channel) as 16-byte broadcasts, and each input value is loaded once per
-// thread.  O must be a multiple of OPT.
-template <typename T, int OPT>
-__global__ __launch_bounds__(256) void conv_direct_small_k(
-    const T* __restrict__ x, const T* __restrict__ w, const float* __restrict__ bias,
-    T* __restrict__ y, int n, int h, int wd, int c, int oh, int ow, int o, int k, int stride,
-    int pad, int dil, Epilogue ep, int ktot) {
-  extern __shared__ __attribute__((aligned(16))) float lds_w[];  // [ktot][o]
-  for (int i = threadIdx.x; i < ktot * o; i += blockDim.x) {
-    int oc = i / ktot, kk = i - oc * ktot;
-    lds_w[kk * o + oc] = to_f32(w[i]);
-  }
-  __syncthreads();
-  const int groups_per_pixel = o / OPT;
-  const long total = (long)n * oh * ow * groups_per_pixel;
-  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-       idx += (long)gridDim.x * blockDim.x) {
-    const int og = (int)(idx % groups_per_pixel);
-    long pix = idx / groups_per_pixel;
-    const int ox = (int)(pix % ow);
-    pix /= ow;
-    const int oy = (int)(pix % oh);
-    const int b = (int)(pix / oh);
-    const int oc0 = og * OPT;
-    float acc[OPT];
-#pragma unroll
-    for (int j = 0; j < OPT; ++j) acc[j] = bias != nullptr ? bias[oc0 + j] : 0.f;
-    for (int r = 0; r < k; ++r) {
-      const int iy = oy * stride - pad + r * dil;
-      if (iy < 0 || iy >= h) continue;
-      for (int s = 0; s < k; ++s) {
-        const int ix = ox * stride - pad + s * dil;
-        if (ix < 0 || ix >= wd) continue;
-        const T* xp = x + (((long)b * h + iy) * wd + ix) * c;
-        const float* wp = lds_w + (long)((r * k + s) * c) * o + oc0;
-        for (int ci = 0; ci < c; ++ci) {
-          const float xv = to_f32(xp[ci]);
-          const float4* w4 = reinterpret_cast<const float4*>(wp + ci * o);
-#pragma unroll
-          for (int j = 0; j < OPT / 4; ++j) {
-            const float4 wv = w4[j];
-            acc[4 * j + 0] += xv * wv.x;
-            acc[4 * j + 1] += xv * wv.y;
-            acc[4 * j + 2] += xv * wv.z;
-            acc[4 * j + 3] += xv * wv.w;
-          }
-        }
-      }
-    }
-    T* yp = y + (((long)b * oh + oy) * ow + ox) * o + oc0;
-    if constexpr (sizeof(T) == 4) {
-#pragma unroll
-      for (int j = 0; j < OPT / 4; ++j)
-        reinterpret_cast<float4*>(yp)[j] =
-            make_float4(apply_epilogue(acc[4 * j], ep), apply_epilogue(acc[4 * j + 1], ep),
-                        apply_epilogue(acc[4 * j + 2], ep), apply_epilogue(acc[4 * j + 3], ep));
-    } else {
-#pragma unroll
-      for (int j = 0; j < OPT; ++j) yp[j] = from_f32<T>(apply_epilogue(acc[j], ep));
-    }
-  }
-}
 
 // Stem kernel: few input channels, K = k*k*C <= 32 (the RGB stem has K = 27), on
 // the MFMA units.  A wave owns 32 output pixels x 32 output channels at a time and
@@ -290,40 +223,473 @@ __global__ __launch_bounds__(256) void conv_stem_rgb_mfma(
   }
 }
 
-// Fully general kernel: one thread per output element, output channel
-// fastest.  Filter OHWI with I = c/groups.
+struct DirectGeom {
+  int n, h, w, c, oh, ow, o, k, stride, pad, dil, groups;
+};
+
+DirectGeom direct_geom(const OgleConvArgs& a) {
+  return DirectGeom{a.n,      a.in_h,        a.in_w,   a.in_c,    a.out_h,    a.out_w,
+                    a.out_c,  a.kernel_size, a.stride, a.padding, a.dilation, a.group};
+}
+
+// One output element: bias first, then ky, kx, input channel ascending; taps outside the image
+// are skipped.  Filter OHWI with I = c/groups.
+template <typename T>
+__device__ __forceinline__ float direct_output(const T* __restrict__ x, const T* __restrict__ w,
+                                               const float* __restrict__ bias, const DirectGeom& q, int b,
+                                               int oy, int ox, int oc) {
+  const int cpg = q.c / q.groups;
+  const int g = oc / (q.o / q.groups);
+  float acc = bias != nullptr ? bias[oc] : 0.f;
+  const T* wf = w + (long)oc * q.k * q.k * cpg;
+  for (int r = 0; r < q.k; ++r) {
+    const int iy = oy * q.stride - q.pad + r * q.dil;
+    if (iy < 0 || iy >= q.h) continue;
+    for (int s = 0; s < q.k; ++s) {
+      const int ix = ox * q.stride - q.pad + s * q.dil;
+      if (ix < 0 || ix >= q.w) continue;
+      const T* xp = x + (((long)b * q.h + iy) * q.w + ix) * q.c + g * cpg;
+      const T* wp = wf + (r * q.k + s) * cpg;
+      for (int ci = 0; ci < cpg; ++ci) acc += to_f32(xp[ci]) * to_f32(wp[ci]);
+    }
+  }
+  return acc;
+}
+
+// Fully general kernel: one thread per output element, output channel fastest.
 template <typename T>
 __global__ __launch_bounds__(256) void conv_direct_general(
     const T* __restrict__ x, const T* __restrict__ w, const float* __restrict__ bias,
-    T* __restrict__ y, int n, int h, int wd, int c, int oh, int ow, int o, int k, int stride,
-    int pad, int dil, int groups, Epilogue ep) {
-  const int cpg = c / groups;
-  const int opg = o / groups;
-  const long total = (long)n * oh * ow * o;
+    T* __restrict__ y, DirectGeom q, Epilogue ep) {
+  const long total = (long)q.n * q.oh * q.ow * q.o;
   for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
        idx += (long)gridDim.x * blockDim.x) {
-    const int oc = (int)(idx % o);
-    long pix = idx / o;
-    const int ox = (int)(pix % ow);
-    pix /= ow;
-    const int oy = (int)(pix % oh);
-    const int b = (int)(pix / oh);
-    const int g = oc / opg;
-    float acc = bias != nullptr ? bias[oc] : 0.f;
-    const T* wf = w + (long)oc * k * k * cpg;
-    for (int r = 0; r < k; ++r) {
-      const int iy = oy * stride - pad + r * dil;
-      if (iy < 0 || iy >= h) continue;
-      for (int s = 0; s < k; ++s) {
-        const int ix = ox * stride - pad + s * dil;
-        if (ix < 0 || ix >= wd) continue;
-        const T* xp = x + (((long)b * h + iy) * wd + ix) * c + g * cpg;
-        const T* wp = wf + (r * k + s) * cpg;
-        for (int ci = 0; ci < cpg; ++ci) acc += to_f32(xp[ci]) * to_f32(wp[ci]);
+    const int oc = (int)(idx % q.o);
+    long pix = idx / q.o;
+    const int ox = (int)(pix % q.ow);
+    pix /= q.ow;
+    const int oy = (int)(pix % q.oh);
+    const int b = (int)(pix / q.oh);
+    y[idx] = from_f32<T>(apply_epilogue(direct_output(x, w, bias, q, b, oy, ox, oc), ep));
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Patch kernel: any kernel size, stride, dilation, group count and channel count, on the MFMA
+// units.  A workgroup owns 128 output pixels (a box of tb images x th rows x tw columns, powers
+// of two) and `gp` groups x COLS output channels.  It stages the input patch those pixels read
+// and the filter values of the channels in LDS as fp32 and contracts out of LDS: both are read
+// from memory once per workgroup, whatever their alignment, and the gather is an LDS address
+// (pixel base + tap offset).  A wave owns 32 of the pixels.  Bound by the fp32 MFMA rate with
+// its padding (COLS 16 / 32 / 64 against the channels a group has, K steps of 2 or 4), and for
+// small groups by staging and launch latency.
+//
+// K is walked in runs: consecutive values both in the patch and in a filter row.  A run is one
+// tap's channels; with an odd channel count, dilation 1 and all channels staged it is a whole
+// filter row of taps (7x7x3: seven runs of 21 instead of 49 of 3).  LDS pitches are odd, so
+// lanes on neighbouring pixels hit different banks.  Channels that do not fit LDS at once are
+// staged `cc` at a time.
+//
+// Taps outside the image are staged as zeros.  0 * w is 0 only for a finite w, so a workgroup
+// that meets an infinite or NaN filter value recomputes its outputs one by one, skipping taps.
+struct FastDiv {   // n / d for n, d < 2^16: with mul = ceil(2^32 / d) the error n * (mul * d - 2^32) stays below 2^32
+  unsigned mul;
+  int d;
+};
+__host__ __device__ __forceinline__ FastDiv fast_div(int d) {
+  return FastDiv{0xffffffffu / (unsigned)d + 1u, d};   // ceil(2^32 / d); d == 1 is not looked up
+}
+__device__ __forceinline__ int div_fast(int n, const FastDiv& f) {
+  return f.d == 1 ? n : (int)__umulhi((unsigned)n, f.mul);
+}
+
+struct PatchPlan {
+  int th_log, tw_log;             // box of output pixels of a workgroup (128 >> both images)
+  int tiles_b, tiles_y, tiles_x;  // boxes along images, rows, columns
+  int ph, pw, pitch;              // patch rows, columns, floats per patch pixel
+  int in_step, box_step;          // input pixels per patch pixel, patch pixels per output pixel
+  int cc;                         // input channels per group staged at once
+  int gp, gblocks;                // groups per workgroup; ceil(groups / gp)
+  int cols, col_blocks;           // output channels per workgroup and group
+  int runs_x;                     // K runs per filter row: one per tap, or one in all
+  int tile_blocks;                // workgroups along the boxes (each walks several when channels fit at once)
+  int vec_x, vec_w;               // patch / filter read four values at a time
+  int patch_floats, lds_floats;
+  FastDiv d_cs, d_pw, d_ph, d_runk, d_col;
+};
+
+constexpr int kPatchPixels = 128;
+// Scalar loads a thread has in flight while it stages.  More make longer code that is fetched
+// cold by every launch, and 16 spilled registers (12 groups of 8 -> 12 channels, 3x3: 33 us).
+constexpr int kPatchBatch = 8;
+
+// V consecutive values (V 4: from a 4-element boundary) as fp32; zeros unless `on`, when `src`
+// is some readable address all the same.
+template <typename T, int V>
+__device__ __forceinline__ void load_some(const T* src, bool on, float (&v)[V]) {
+  struct __attribute__((aligned(sizeof(T) * V))) Pack { T e[V]; };
+  const Pack q = *reinterpret_cast<const Pack*>(src);
+#pragma unroll
+  for (int e = 0; e < V; ++e) v[e] = on ? to_f32(q.e[e]) : 0.f;
+}
+
+template <typename T, int COLS>
+__global__ __launch_bounds__(256) void conv_patch_mfma(const T* __restrict__ x, const T* __restrict__ w,
+                                                       const float* __restrict__ bias, T* __restrict__ y,
+                                                       DirectGeom q, PatchPlan p, Epilogue ep) {
+  extern __shared__ __attribute__((aligned(16))) float patch_lds[];
+  constexpr int MB = COLS == 16 ? 16 : 32;            // MFMA block
+  constexpr int FR = 32 / MB;                         // blocks along a wave's 32 pixels
+  constexpr int NB = COLS / MB;                       // blocks along the columns
+  constexpr int KQ = 64 / MB;                         // k values of one MFMA
+  constexpr int WP = COLS + 1;                        // filter row pitch in LDS
+  constexpr int REGS = MB == 32 ? 16 : 4;
+  typedef float acc32_t __attribute__((ext_vector_type(16)));
+  typedef float acc16_t __attribute__((ext_vector_type(4)));
+  typedef typename std::conditional<MB == 32, acc32_t, acc16_t>::type Acc;
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lrow = lane % MB, lq = lane / MB;
+  float* const patch = patch_lds;
+  float* const wl = patch_lds + p.patch_floats;
+  const int cpg = q.c / q.groups, opg = q.o / q.groups;
+  const int ktot = q.k * q.k * cpg;
+
+  // column blocks fastest, then groups: the workgroups that read one patch are neighbours, on
+  // one XCD's L2
+  int id = xcd_swizzle((int)blockIdx.x, (int)gridDim.x);
+  const int cb = id % p.col_blocks;
+  id /= p.col_blocks;
+  const int g0 = (id % p.gblocks) * p.gp;
+  const int tblock = id / p.gblocks;
+  const int groups_here = min(p.gp, q.groups - g0);
+  const int col0 = cb * COLS;
+  const int cols_here = min(COLS, opg - col0);
+  const int tiles = p.tiles_b * p.tiles_y * p.tiles_x;
+  const int box_w = 1 << p.tw_log, box_h = 1 << p.th_log;
+  const int row_pitch = p.pw * p.pitch, img_pitch = p.ph * row_pitch;
+
+  // patch offset of this lane's pixel in each of its MFMA blocks
+  int pix_off[FR];
+#pragma unroll
+  for (int f = 0; f < FR; ++f) {
+    const int pix = wave * 32 + f * MB + lrow;
+    const int tx = pix & (box_w - 1), ty = (pix >> p.tw_log) & (box_h - 1), tb = pix >> (p.tw_log + p.th_log);
+    pix_off[f] = tb * img_pitch + (ty * row_pitch + tx * p.pitch) * p.box_step;
+  }
+
+  bool bad = false;   // an infinite or NaN filter value has been staged
+  for (int tile = tblock; tile < tiles; tile += p.tile_blocks) {
+    const int bx = tile % p.tiles_x;
+    const int rest = tile / p.tiles_x;
+    const int by = rest % p.tiles_y, bb = rest / p.tiles_y;
+    const int ox0 = bx << p.tw_log, oy0 = by << p.th_log, b0 = bb * (kPatchPixels >> (p.tw_log + p.th_log));
+    const int iy0 = oy0 * q.stride - q.pad, ix0 = ox0 * q.stride - q.pad;
+
+    // where this lane's results go: register r is pixel 8*(r/4) + 4*(lane/32) + r%4 (32x32) or
+    // 4*(lane/16) + r (16x16) of the block, column lane % MB
+    constexpr unsigned kNoPixel = 0xffffffffu;
+    unsigned y_off[FR][REGS];
+#pragma unroll
+    for (int f = 0; f < FR; ++f)
+#pragma unroll
+      for (int r = 0; r < REGS; ++r) {
+        const int pix = wave * 32 + f * MB + (MB == 32 ? (r >> 2) * 8 + lq * 4 + (r & 3) : lq * 4 + r);
+        const int ox = ox0 + (pix & (box_w - 1)), oy = oy0 + ((pix >> p.tw_log) & (box_h - 1));
+        const int b = b0 + (pix >> (p.tw_log + p.th_log));
+        y_off[f][r] = ox < q.ow && oy < q.oh && b < q.n ? (unsigned)(((b * q.oh + oy) * q.ow + ox) * q.o) : kNoPixel;
+      }
+
+    // with gp > 1 all channels are staged at once: only one of the two loops below has more
+    // than one turn, and one set of accumulators serves both
+    Acc acc[FR][NB];
+    for (int c0 = 0; c0 < cpg; c0 += p.cc) {
+      const int cc = min(p.cc, cpg - c0);
+      const int cs = p.gp > 1 ? groups_here * cpg : cc;   // channels per patch pixel this time
+      // the last chunk and the last group block are narrower than the divisors the host prepared
+      const bool full = cc == p.cc && groups_here == p.gp;
+      const FastDiv d_cs = full ? p.d_cs : fast_div(cs), d_runk = full ? p.d_runk : fast_div(q.k * q.k * cc);
+      __syncthreads();   // the previous contraction has read its operands
+      // input patch: [image][row][column][channel], zeros outside the image
+      {
+        const T* src = x + g0 * cpg + c0;
+        const int total = (kPatchPixels >> (p.tw_log + p.th_log)) * p.ph * p.pw * cs;
+        auto stage = [&](auto vec) {
+          constexpr int V = decltype(vec)::value, U = V == 1 ? kPatchBatch : 2;
+          for (int i0 = tid * V; i0 < total; i0 += 256 * V * U) {
+            float v[U][V];
+            int at[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {   // every load of the batch before the first LDS write
+              const int i = i0 + u * 256 * V;
+              const int px_all = div_fast(i, d_cs);
+              const int ch = i - px_all * cs;
+              const int prow = div_fast(px_all, p.d_pw);
+              const int px = px_all - prow * p.pw;
+              const int b = div_fast(prow, p.d_ph);
+              const int iy = iy0 + (prow - b * p.ph) * p.in_step, ix = ix0 + px * p.in_step;
+              const bool in = i < total && b0 + b < q.n && (unsigned)iy < (unsigned)q.h && (unsigned)ix < (unsigned)q.w;
+              at[u] = i < total ? px_all * p.pitch + ch : -1;
+              load_some<T, V>(src + (in ? (unsigned)((((b0 + b) * q.h + iy) * q.w + ix) * q.c + ch) : 0u), in, v[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (at[u] >= 0)
+#pragma unroll
+                for (int e = 0; e < V; ++e) patch[at[u] + e] = v[u][e];
+          }
+        };
+        // four channels at a time where every pixel's share starts on a vector boundary
+        if (p.vec_x && (cs & 3) == 0) stage(std::integral_constant<int, 4>());
+        else stage(std::integral_constant<int, 1>());
+      }
+      // filter values: [group][run][k in run][column]; they stay when all channels fit at once
+      if (tile == tblock || p.cc < cpg) {
+        const int kk_total = q.k * q.k * cc;
+        const int total = groups_here * cols_here * kk_total;
+        auto stage = [&](auto vec) {
+          constexpr int V = decltype(vec)::value, U = V == 1 ? kPatchBatch : 2;
+          for (int i0 = tid * V; i0 < total; i0 += 256 * V * U) {
+            float v[U][V];
+            int at[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              // kk fastest: a filter row is read contiguously (all channels staged) or run by run
+              const int i = i0 + u * 256 * V;
+              const int row = div_fast(i, d_runk);
+              const int kk = i - row * kk_total;
+              const int gi = cols_here == COLS ? row / COLS : div_fast(row, p.d_col);
+              const int col = row - gi * cols_here;
+              long from = ((long)(g0 + gi) * opg + col0 + col) * ktot;
+              if (cc == cpg) {
+                from += kk;
+              } else {
+                const int tap = div_fast(kk, d_cs);   // gp == 1: cs is cc
+                from += tap * cpg + c0 + (kk - tap * cc);
+              }
+              at[u] = i < total ? (gi * kk_total + kk) * WP + col : -1;
+              load_some<T, V>(w + (i < total ? from : 0), i < total, v[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (at[u] >= 0)
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                  bad = bad || !(fabsf(v[u][e]) <= 3.402823466e38f);
+                  wl[at[u] + e * WP] = v[u][e];
+                }
+          }
+        };
+        if (p.vec_w) stage(std::integral_constant<int, 4>());
+        else stage(std::integral_constant<int, 1>());
+      }
+      __syncthreads();
+
+      const int len = p.runs_x == 1 ? q.k * cc : cc;    // values per run
+      for (int gi = 0; gi < groups_here; ++gi) {
+        if (c0 == 0) {
+#pragma unroll
+          for (int f = 0; f < FR; ++f)
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+              for (int r = 0; r < REGS; ++r) acc[f][n][r] = 0.f;
+        }
+        int wrow = gi * q.k * q.k * cc;
+        for (int ky = 0; ky < q.k; ++ky) {
+          for (int kx = 0; kx < p.runs_x; ++kx, wrow += len) {
+            const float* pa = patch + ky * q.dil * row_pitch + kx * q.dil * p.pitch + gi * cpg + lq;
+            const float* pb = wl + (wrow + lq) * WP + lrow;
+            auto multiply = [&](const float (&av)[FR], const float (&bv)[NB]) {
+#pragma unroll
+              for (int f = 0; f < FR; ++f)
+#pragma unroll
+                for (int n = 0; n < NB; ++n) {
+                  if constexpr (MB == 32)
+                    acc[f][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[f], bv[n], acc[f][n], 0, 0, 0);
+                  else
+                    acc[f][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[f], bv[n], acc[f][n], 0, 0, 0);
+                }
+            };
+            int j = 0;
+            for (; j + 4 * KQ <= len; j += 4 * KQ) {   // four steps of operands read ahead
+              float av[4][FR], bv[4][NB];
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+#pragma unroll
+                for (int f = 0; f < FR; ++f) av[u][f] = pa[pix_off[f] + j + u * KQ];
+#pragma unroll
+                for (int n = 0; n < NB; ++n) bv[u][n] = pb[(j + u * KQ) * WP + n * MB];
+              }
+#pragma unroll
+              for (int u = 0; u < 4; ++u) multiply(av[u], bv[u]);
+            }
+            for (; j + KQ <= len; j += KQ) {
+              float av[FR], bv[NB];
+#pragma unroll
+              for (int f = 0; f < FR; ++f) av[f] = pa[pix_off[f] + j];
+#pragma unroll
+              for (int n = 0; n < NB; ++n) bv[n] = pb[j * WP + n * MB];
+              multiply(av, bv);
+            }
+            if (j < len) {   // the run's last values: lanes past its end contribute 0 * 0
+              const bool on = lq < len - j;
+              const int back = on ? 0 : lq;
+              float av[FR], bv[NB];
+#pragma unroll
+              for (int f = 0; f < FR; ++f) av[f] = on ? pa[pix_off[f] + j - back] : 0.f;
+#pragma unroll
+              for (int n = 0; n < NB; ++n) bv[n] = on ? pb[(j - back) * WP + n * MB] : 0.f;
+              multiply(av, bv);
+            }
+          }
+        }
+        if (c0 + p.cc < cpg) continue;   // more channels of this group to come (gp == 1)
+        const int obase = (g0 + gi) * opg + col0;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+          const int col = n * MB + lrow;
+          if (col >= cols_here) continue;
+          const float bv = bias != nullptr ? bias[obase + col] : 0.f;
+#pragma unroll
+          for (int f = 0; f < FR; ++f)
+#pragma unroll
+            for (int r = 0; r < REGS; ++r)
+              if (y_off[f][r] != kNoPixel)
+                y[y_off[f][r] + (unsigned)(obase + col)] = from_f32<T>(apply_epilogue(acc[f][n][r] + bv, ep));
+        }
       }
     }
-    y[idx] = from_f32<T>(apply_epilogue(acc, ep));
+
+    if (tile == tblock) bad = __syncthreads_or(bad) != 0;   // (in chunks: one box per workgroup)
+    if (bad) {
+      const int per_pixel = groups_here * cols_here;
+      for (int i = tid; i < kPatchPixels * per_pixel; i += 256) {
+        const int pix = i / per_pixel, rest2 = i - pix * per_pixel;
+        const int gi = rest2 / cols_here, col = rest2 - gi * cols_here;
+        const int ox = ox0 + (pix & (box_w - 1)), oy = oy0 + ((pix >> p.tw_log) & (box_h - 1));
+        const int b = b0 + (pix >> (p.tw_log + p.th_log));
+        const int oc = (g0 + gi) * opg + col0 + col;
+        if (ox < q.ow && oy < q.oh && b < q.n)
+          y[(unsigned)(((b * q.oh + oy) * q.ow + ox) * q.o + oc)] =
+              from_f32<T>(apply_epilogue(direct_output(x, w, bias, q, b, oy, ox, oc), ep));
+      }
+    }
   }
+}
+
+// The patch kernel's box, chunk and grid for a convolution; false if it does not take it.
+bool plan_patch(const OgleConvArgs& a, PatchPlan* out) {
+  const int cpg = a.in_c / a.group, opg = a.out_c / a.group, k = a.kernel_size;
+  const long lim = 0x7fffffffL;
+  if ((long)a.n * a.in_h * a.in_w * a.in_c > lim || (long)a.n * a.out_h * a.out_w * a.out_c > lim) return false;
+  if ((long)a.n + kPatchPixels > lim || (long)a.in_h + a.padding > lim / 2 || (long)a.in_w + a.padding > lim / 2)
+    return false;
+  // Under 64 products per pixel and group most of an MFMA block is padding and one thread per
+  // output is faster.  Measured at 4 x 48 x 48, us with one thread per output / with this kernel,
+  // groups x (channels in -> out): 64 x (2 -> 2) 3x3 25 / 44, 32 x (4 -> 8) 1x1 15.3 / 17.9;
+  // from 64 on 32 x (8 -> 8) 1x1 38 / 19, 16 x (4 -> 4) 3x3 27 / 17, 32 x (32 -> 32) 3x3 9905 / 122
+  if ((long)k * k * cpg * opg < 64) return false;
+  // A few thousand short sums are over before the patch is staged (one image 14 x 14, 32 x
+  // (8 -> 8) 1x1: 6.3 / 7.6; 9 x 9, 35 -> 75 1x1: 6.3 / 12.1; 4 x 28 x 28, 181 -> 9 1x1, whose
+  // patch is staged in three chunks: 20.8 / 31; but 3x3 with K = 72: 11.6 / 8.6, K = 891: 104 / 50).
+  if ((long)a.n * a.out_h * a.out_w * a.out_c <= 65536 && k * k * cpg <= (k == 1 ? 192 : 48)) return false;
+  const long span = (long)(k - 1) * a.dilation + 1;
+  if (span > 1024 || a.stride > 64) return false;   // no such patch fits LDS
+  PatchPlan p{};
+  // one tap: the pixels that a stride skips are not staged
+  p.in_step = k == 1 ? a.stride : 1;
+  p.box_step = k == 1 ? 1 : a.stride;
+  p.cols = opg <= 16 ? 16 : (opg <= 32 || (((opg + 31) / 32) % 2 == 1 && opg < 160)) ? 32 : 64;
+  // the box: fewest boxes, then the smallest patch
+  double best = 0;
+  for (int tw = 0; tw <= 7; ++tw) {
+    for (int th = 0; tw + th <= 7; ++th) {
+      const int box_b = kPatchPixels >> (tw + th);
+      if ((1 << tw) >= 2 * a.out_w || (1 << th) >= 2 * a.out_h) continue;
+      const long ph = ((1L << th) - 1) * p.box_step + span, pw = ((1L << tw) - 1) * p.box_step + span;
+      const double boxes = (double)((a.n + box_b - 1) / box_b) * ((a.out_h + (1 << th) - 1) >> th) *
+                           ((a.out_w + (1 << tw) - 1) >> tw);
+      const double cost = boxes * ((double)(ph * pw * box_b) + 2.0 * kPatchPixels);
+      if (best != 0 && cost >= best) continue;
+      best = cost;
+      p.tw_log = tw;
+      p.th_log = th;
+      p.ph = (int)ph;
+      p.pw = (int)pw;
+    }
+  }
+  const int box_b = kPatchPixels >> (p.tw_log + p.th_log);
+  p.tiles_b = (a.n + box_b - 1) / box_b;
+  p.tiles_y = (a.out_h + (1 << p.th_log) - 1) >> p.th_log;
+  p.tiles_x = (a.out_w + (1 << p.tw_log) - 1) >> p.tw_log;
+  const long tiles = (long)p.tiles_b * p.tiles_y * p.tiles_x;
+  // a grid that leaves compute units empty is cut finer along the channels instead: the time of
+  // such a launch is one workgroup's staging and serial contraction
+  while (p.cols > 16 && tiles * a.group * ((opg + p.cols - 1) / p.cols) < 256) p.cols /= 2;
+  p.col_blocks = (opg + p.cols - 1) / p.cols;
+  const long pixels = (long)box_b * p.ph * p.pw;
+  const long wp = p.cols + 1;
+  if (pixels > 0xffff) return false;
+  // channels staged at once: all of them, or the most that leave three workgroups per unit
+  // (48 KB of LDS each); 64 KB, the launch limit, where the grid gives a unit no third one
+  // anyway (fewer, longer chunks: each costs a round trip to memory) or nothing less will do
+  const bool roomy = tiles * a.group * p.col_blocks <= 512;
+  auto floats = [&](long cc, long gp) { return pixels * ((cc * gp) | 1) + gp * k * k * cc * wp; };
+  long cc = 0;
+  for (const long budget : {roomy ? 16384L : 12288L, 16384L}) {
+    if (floats(cpg, 1) <= budget) cc = cpg;
+    else
+      for (long t : {64L, 32L, 16L, 8L, 4L, 2L})
+        if (cc == 0 && t < cpg && floats(t, 1) <= budget) cc = t;
+    if (cc != 0) break;
+  }
+  if (cc == 0) return false;
+  p.cc = (int)cc;
+  // several groups per workgroup share a patch's cache lines, as long as the grid still has
+  // about two workgroups per compute unit
+  p.gp = 1;
+  if (cc == cpg && p.col_blocks == 1)
+    while (p.gp < a.group && floats(cpg, p.gp + 1) <= 8192 &&
+           tiles * ((a.group + p.gp) / (p.gp + 1)) >= 512)
+      ++p.gp;
+  p.gblocks = (a.group + p.gp - 1) / p.gp;
+  const bool merge = a.dilation == 1 && cc == cpg && p.gp == 1 && cpg % 2 == 1 && k > 1;
+  p.runs_x = merge ? 1 : k;
+  p.pitch = (int)(cc * p.gp) | 1;
+  p.patch_floats = (int)(pixels * p.pitch);
+  p.lds_floats = (int)floats(cc, p.gp);
+  const long per_tile = (long)p.gblocks * p.col_blocks;
+  // with all channels staged at once the filter stays in LDS while a workgroup walks boxes
+  const long most = cc == cpg ? std::max(1L, (768 + per_tile - 1) / per_tile) : tiles;
+  p.tile_blocks = (int)std::min(tiles, most);
+  if (per_tile * p.tile_blocks > lim || pixels * cc * p.gp > 0xffff ||
+      (long)p.gp * p.cols * k * k * cc > 0xffff)
+    return false;
+  const uintptr_t vec = 4 * (a.dtype == OGLE_F16 ? 2 : 4);
+  p.vec_x = a.in_c % 4 == 0 && cpg % 4 == 0 && cc % 4 == 0 && reinterpret_cast<uintptr_t>(a.input_dev) % vec == 0;
+  p.vec_w = cc == cpg && (k * k * cpg) % 4 == 0 && reinterpret_cast<uintptr_t>(a.filter_dev) % vec == 0;
+  p.d_cs = fast_div((int)(cc * p.gp));
+  p.d_pw = fast_div(p.pw);
+  p.d_ph = fast_div(p.ph);
+  p.d_runk = fast_div((int)(k * k * cc));
+  p.d_col = fast_div(std::min(p.cols, opg % p.cols == 0 ? p.cols : opg % p.cols));
+  *out = p;
+  return true;
+}
+
+template <typename T>
+int32_t launch_patch(const OgleConvArgs& a, const PatchPlan& p, const Epilogue& ep, hipStream_t s) {
+  const T* x = static_cast<const T*>(a.input_dev);
+  const T* w = static_cast<const T*>(a.filter_dev);
+  T* y = static_cast<T*>(a.output_dev);
+  const dim3 grid((unsigned)(p.tile_blocks * p.gblocks * p.col_blocks)), block(256);
+  const size_t lds = sizeof(float) * (size_t)p.lds_floats;
+  const DirectGeom q = direct_geom(a);
+  if (p.cols == 16) launch((conv_patch_mfma<T, 16>), grid, block, lds, s, x, w, a.bias_dev, y, q, p, ep);
+  else if (p.cols == 32) launch((conv_patch_mfma<T, 32>), grid, block, lds, s, x, w, a.bias_dev, y, q, p, ep);
+  else launch((conv_patch_mfma<T, 64>), grid, block, lds, s, x, w, a.bias_dev, y, q, p, ep);
+  return check_launch("conv_patch_mfma");
 }
 
 template <typename T>
@@ -333,7 +699,6 @@ int32_t run_direct(const OgleConvArgs& a, hipStream_t s) {
   const T* w = static_cast<const T*>(a.filter_dev);
   T* y = static_cast<T*>(a.output_dev);
   const int ktot = a.kernel_size * a.kernel_size * a.in_c;
-  const size_t lds = sizeof(float) * (size_t)ktot * a.out_c;
   const long pixels_all = (long)a.n * a.out_h * a.out_w;
   const long esz = (long)sizeof(T);
   const long x_bytes = (long)a.n * a.in_h * a.in_w * a.in_c * esz;
@@ -377,33 +742,14 @@ int32_t run_direct(const OgleConvArgs& a, hipStream_t s) {
 #undef OGLE_STEM_CASE
     return check_launch("conv_stem_mfma");
   }
-  if (a.group == 1 && lds <= 48 * 1024 && a.out_c % 4 == 0) {
-    // 16 channels per thread when that still leaves enough threads to fill the chip
-    const long pixels = (long)a.n * a.out_h * a.out_w;
-    const bool wide = a.out_c % 16 == 0 && pixels * (a.out_c / 16) >= 256L * 256 * 4;
-    const int opt = wide ? 16 : 4;
-    const long total = pixels * (a.out_c / opt);
-    int blocks = ceil_div(total, 256);
-    if (blocks > 256 * 32) blocks = 256 * 32;
-    if (blocks < 1) blocks = 1;
-    if (wide) {
-      launch((conv_direct_small_k<T, 16>), dim3(blocks), dim3(256), lds, s, x, w,
-                         a.bias_dev, y, a.n, a.in_h, a.in_w, a.in_c, a.out_h, a.out_w, a.out_c,
-                         a.kernel_size, a.stride, a.padding, a.dilation, ep, ktot);
-    } else {
-      launch((conv_direct_small_k<T, 4>), dim3(blocks), dim3(256), lds, s, x, w,
-                         a.bias_dev, y, a.n, a.in_h, a.in_w, a.in_c, a.out_h, a.out_w, a.out_c,
-                         a.kernel_size, a.stride, a.padding, a.dilation, ep, ktot);
-    }
-    return check_launch("conv_direct_small_k");
-  }
+  PatchPlan plan;
+  if (plan_patch(a, &plan)) return launch_patch<T>(a, plan, ep, s);
   const long total = (long)a.n * a.out_h * a.out_w * a.out_c;
   int blocks = ceil_div(total, 256);
   if (blocks > 256 * 64) blocks = 256 * 64;
   if (blocks < 1) blocks = 1;
-  launch((conv_direct_general<T>), dim3(blocks), dim3(256), 0, s, x, w, a.bias_dev,
-                     y, a.n, a.in_h, a.in_w, a.in_c, a.out_h, a.out_w, a.out_c, a.kernel_size,
-                     a.stride, a.padding, a.dilation, a.group, ep);
+  launch((conv_direct_general<T>), dim3(blocks), dim3(256), 0, s, x, w, a.bias_dev, y,
+         direct_geom(a), ep);
   return check_launch("conv_direct_general");
 }
 

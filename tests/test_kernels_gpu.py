@@ -136,6 +136,55 @@ def test_conv_stem_kernel(case, dtype):
     check_conv(x, wt, b, s, p, d, 1, act=H.ACT_CLIP, maxv=6.0, dtype=dtype, what=str(case))
 
 
+PATCH_CASES = [
+    # n, h, w, c, o, k, s, p, d, g   what only the direct kernels take: the LDS patch kernel
+    (4, 57, 43, 96, 144, 3, 1, 1, 1, 12),   # several groups per workgroup, vector staging, ragged box
+    (2, 23, 19, 80, 80, 3, 1, 1, 1, 5),     # 16 channels per group: exactly one 16-wide block
+    (2, 23, 19, 34, 34, 3, 1, 1, 1, 2),     # 17 per group: one past it, odd channel count (merged runs)
+    (1, 31, 33, 64, 99, 3, 2, 1, 1, 1),     # fp32 only the ragged N of the MFMA path; fp16: stays there
+    (1, 29, 31, 33, 64, 3, 2, 1, 1, 1),     # chunks of channels with a ragged last one, 64 columns
+    (1, 40, 41, 131, 65, 3, 1, 1, 1, 1),    # many chunks, one channel past a 64-wide block
+    (3, 21, 22, 77, 45, 1, 2, 0, 1, 1),     # one tap, stride 2: skipped pixels are not staged
+    (2, 40, 38, 3, 64, 7, 2, 3, 1, 1),      # 7x7 RGB stem: whole filter rows as runs, 4 column blocks
+    (9, 2, 3, 30, 42, 3, 1, 1, 1, 3),       # maps smaller than a box: several images per workgroup
+    (2, 24, 20, 21, 24, 3, 1, 2, 2, 3),     # dilation 2, seven channels per group
+    (1, 50, 50, 25, 40, 5, 3, 2, 1, 5),     # 5x5, stride 3
+    (1, 20, 20, 64, 64, 11, 1, 5, 1, 2),    # 11x11: a few channels at a time
+]
+
+
+@pytest.mark.parametrize("case", PATCH_CASES)
+@pytest.mark.parametrize("dtype", [H.F32, H.F16])
+def test_conv_patch_kernel(case, dtype):
+    n, h, w, c, o, k, s, p, d, g = case
+    r = rng(2900 + PATCH_CASES.index(case))
+    x = r.uniform(-1, 1, (n, h, w, c)).astype(np.float32)
+    wt = r.normal(0, 0.5, (o, c // g, k, k)).astype(np.float32)
+    b = r.uniform(-0.1, 0.1, o).astype(np.float32)
+    if dtype == H.F16:
+        x = x.astype(np.float16).astype(np.float32)
+        wt = wt.astype(np.float16).astype(np.float32)
+    check_conv(x, wt, b, s, p, d, g, act=H.ACT_CLIP, maxv=6.0, dtype=dtype, entry="ogle_hip_conv2d",
+               variant=H.VARIANT_ANY4 if g > 1 else H.VARIANT_NHWC4, what=str(case))
+
+
+def test_conv_patch_kernel_infinite_filter_values_meet_no_padding():
+    """Taps outside the image are skipped, not multiplied by zero: an infinite or NaN filter value
+    reaches exactly the outputs it reaches in the oracle, in chunked and whole staging alike."""
+    for n, h, w, c, o, k, g in ((2, 20, 18, 24, 36, 3, 3), (1, 17, 16, 130, 20, 3, 1)):
+        r = rng(2950 + c)
+        x = r.uniform(0.5, 1, (n, h, w, c)).astype(np.float32)
+        wt = r.normal(0, 0.5, (o, c // g, k, k)).astype(np.float32)
+        wt[3, 5, 0, 0] = np.inf
+        wt[o - 1, 1, 2, 1] = -np.inf
+        wt[7, 2, 1, 0] = np.nan
+        ref = O.conv2d(x, wt, None, 1, 1, 1, g, O.ACT_NONE, 0.0, 0.0, O.VARIANT_NHWC4)
+        got = gpu_conv(x, wt, None, 1, 1, 1, g, H.ACT_NONE, entry="ogle_hip_conv2d")
+        assert np.isfinite(ref[:, 0, 0, 3]).all()    # its only infinite tap lies in the padding
+        np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
+        np.testing.assert_array_equal(got[~np.isfinite(ref)], ref[~np.isfinite(ref)])
+
+
 WAVE_CASES = [
     # n, h, w, c, o, k, s, p, d   small problems with a long enough K: the wave-split kernel
     (1, 19, 19, 512, 512, 1, 1, 0, 1),    # 32x32 tiles, pointwise (a batch-1 MobileNet layer)
