@@ -123,16 +123,48 @@ struct WaveMma<__half, 16> {
   }
 };
 
+// fp32 operands as three bf16 pieces each: x = h + m + l exactly (24 significand bits in three
+// times 8; each piece is the rounded rest of the one before, every rest is exact in fp32), so
+// x * w = hh + hm + mh + hl + lh + mm plus terms below 2^-26 of the product, and a 32x32x16 step
+// is six bf16 MFMAs of 32 cycles where fp32 takes eight of 64.
+// Measured on MI355X, M = 11552, K = 512, N = 1024: 103 -> 72 us (168 TFLOP/s) with 128x128 tiles;
+// error against 64-bit sums 4.0e-7 -> 1.2e-7.  Bound by power: over long K the loop runs at 178
+// TFLOP/s (six times that in bf16) and 1.6 GHz, the library's bf16 GEMM of 8192 cubed reaches
+// 1145 / 6 = 191.  Hence nothing gained by residuals by v_dot2_f32_bf16, loads pinned to the top of a
+// slab, or MFMAs and splitting interleaved by hand (equal to 8 % behind).
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float floatx2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split_bf16(const u32x4& v, uint2 (&piece)[3]) {
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    floatx2_t x = {__uint_as_float(v[2 * e]), __uint_as_float(v[2 * e + 1])};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const bf16x2_t h = __builtin_convertvector(x, bf16x2_t);
+      (e == 0 ? piece[q].x : piece[q].y) = __builtin_bit_cast(unsigned, h);
+      if (q < 2) {
+        const unsigned b = __builtin_bit_cast(unsigned, h);
+        x[0] -= __uint_as_float(b << 16);
+        x[1] -= __uint_as_float(b & 0xffff0000u);
+      }
+    }
+  }
+}
+
 // One workgroup's share of one convolution: output tile / K range number `bid` of
 // the problem.  Shared by the single-problem kernel and the grouped kernel.
 // LDS bytes of one workgroup: two K-slab buffers of BM + BN padded rows.
-template <int BM, int BN, int ROWB>
+template <int BM, int BN, int ROWB, bool SPLIT = false>
 constexpr int igemm_lds_bytes() {
-  return 2 * (BM + BN) * (ROWB + 16);
+  return 2 * (BM + BN) * (SPLIT ? 96 : ROWB + 16);
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int ROWB, bool PW>
-__device__ __forceinline__ void igemm_tile(
+// SPLIT (fp32 only): the operands are contracted as bf16 pieces.  Returns false, before anything
+// is stored, if a sum is not finite: an operand was infinite, NaN or so large that a piece
+// overflowed, and the caller contracts the tile in fp32 instead.
+template <typename T, int BM, int BN, int WM, int WN, int ROWB, bool PW, bool SPLIT = false>
+__device__ __forceinline__ bool igemm_tile(
     unsigned char* __restrict__ lds, const ConvGeom& g, const T* __restrict__ x, const T* __restrict__ w,
     const float* __restrict__ bias, T* __restrict__ y, T* __restrict__ y2, int o1,
     const Epilogue& ep, int tiles_n, int tiles, float* __restrict__ partial,
@@ -171,9 +203,14 @@ __device__ __forceinline__ void igemm_tile(
   constexpr int CHUNKB = (64 / MB) * 16;  // bytes of a row one MFMA step consumes (64 / MB lane groups x 16)
   constexpr int CHUNKS = ROWB / CHUNKB;
   static_assert(CHUNKS >= 1, "a K slab holds at least one MFMA step");
-  constexpr int STAGE = (BM + BN) * (ROWB + 16);  // one buffer: A rows then B rows
-
-  static_assert(2 * STAGE == igemm_lds_bytes<BM, BN, ROWB>(), "LDS size");
+  constexpr int STAGE = igemm_lds_bytes<BM, BN, ROWB, SPLIT>() / 2;  // one buffer: A rows then B rows
+  // SPLIT: three planes (pieces) of rows of 16 bf16.  Eight rows fill a 256-byte window; in the
+  // windows of rows 16-31 of a block the two 16-byte groups of a row change places: the 16 rows
+  // an operand read serves in one cycle (0-3, 12-15, 20-23, 24-27 or the others) then fall into
+  // 16 different columns.
+  constexpr int PLANE = (BM + BN) * 32;
+  static_assert(!SPLIT || (sizeof(T) == 4 && ROWB == 64 && MB == 32), "split form");
+  auto window_perm = [](int row) { return (row >> 4) & 1; };
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -198,7 +235,7 @@ __device__ __forceinline__ void igemm_tile(
     const int rem = j % per_row;
     pid = r * tiles_n + rem / splits;
     split = rem % splits;
-    if (pid >= tiles) return;
+    if (pid >= tiles) return true;
   } else {
     const int xcd = bid & 7, j = bid >> 3;
     if (splits == 1) {
@@ -219,7 +256,7 @@ __device__ __forceinline__ void igemm_tile(
       pid = bid / splits;
       split = bid - pid * splits;
     }
-    if (pid >= tiles) return;
+    if (pid >= tiles) return true;
   }
   const int tile_n = pid % tiles_n;
   const int tile_m = pid / tiles_n;
@@ -307,14 +344,27 @@ __device__ __forceinline__ void igemm_tile(
   // Writes ra / rb into LDS buffer `buf`.
 #define OGLE_STORE_SLAB(buf, SET)                                                            \
   {                                                                                          \
-    unsigned char* base_ = lds + (buf) * STAGE + vrow * LROW +                               \
-                           (SWZ ? (vcol ^ row_perm(vrow)) : vcol) * 16;                      \
-    _Pragma("unroll") for (int p = 0; p < AP; ++p)                                           \
-      if (!A_PART || p * RPP + vrow < BM)                                                    \
-        *reinterpret_cast<u32x4*>(base_ + p * RPP * LROW) = ra[SET][p];                      \
-    _Pragma("unroll") for (int p = 0; p < BP; ++p)                                           \
-      if (!B_PART || p * RPP + vrow < BN)                                                    \
-        *reinterpret_cast<u32x4*>(base_ + (BM + p * RPP) * LROW) = rb[SET][p];               \
+    if constexpr (SPLIT) {                                                                   \
+      unsigned char* base_ = lds + (buf) * STAGE + (vrow >> 3) * 256 + (vcol & 1) * 8 +      \
+                             ((((vrow & 7) * 2 + (vcol >> 1)) ^ window_perm(vrow)) * 16);    \
+      _Pragma("unroll") for (int p = 0; p < AP + BP; ++p) {                                  \
+        const int row_ = p < AP ? p * RPP : BM + (p - AP) * RPP;                             \
+        if (p < AP ? (A_PART && row_ + vrow >= BM) : (B_PART && row_ + vrow >= BM + BN)) continue; \
+        uint2 piece_[3];                                                                     \
+        split_bf16(p < AP ? ra[SET][p < AP ? p : 0] : rb[SET][p < AP ? 0 : p - AP], piece_); \
+        _Pragma("unroll") for (int q = 0; q < 3; ++q)                                        \
+          *reinterpret_cast<uint2*>(base_ + q * PLANE + row_ * 32) = piece_[q];              \
+      }                                                                                      \
+    } else {                                                                                 \
+      unsigned char* base_ = lds + (buf) * STAGE + vrow * LROW +                             \
+                             (SWZ ? (vcol ^ row_perm(vrow)) : vcol) * 16;                    \
+      _Pragma("unroll") for (int p = 0; p < AP; ++p)                                         \
+        if (!A_PART || p * RPP + vrow < BM)                                                  \
+          *reinterpret_cast<u32x4*>(base_ + p * RPP * LROW) = ra[SET][p];                    \
+      _Pragma("unroll") for (int p = 0; p < BP; ++p)                                         \
+        if (!B_PART || p * RPP + vrow < BN)                                                  \
+          *reinterpret_cast<u32x4*>(base_ + (BM + p * RPP) * LROW) = rb[SET][p];             \
+    }                                                                                        \
   }
 
   Acc acc[TM][TN];
@@ -324,6 +374,19 @@ __device__ __forceinline__ void igemm_tile(
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < REGS; ++r) acc[i][j][r] = 0.f;
+
+  // SPLIT: the five products below h * h have sums of their own, a few hundredths of the main
+  // ones: their roundings vanish and the main sums are rounded once per 16 products (K = 4608:
+  // 5.3e-7 from the 64-bit sums with one set of accumulators; fp32 MFMAs 6.1e-7).
+  Acc rest[SPLIT ? TM : 1][SPLIT ? TN : 1];
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < REGS; ++r) rest[i][j][r] = 0.f;
+  }
 
   const int l32 = lane & 31;
   const int lh = lane >> 5;
@@ -335,9 +398,30 @@ __device__ __forceinline__ void igemm_tile(
   const int kt_begin = split * slabs_per_split;
   const int kt_end = min(g.ktiles, kt_begin + slabs_per_split);
 
+#define OGLE_SPLIT_PRODUCT(ACC, QA, QB)                                                      \
+  _Pragma("unroll") for (int i = 0; i < TM; ++i)                                             \
+    _Pragma("unroll") for (int j = 0; j < TN; ++j)                                           \
+      ACC[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[QA][i], bv[QB][j], ACC[i][j], 0, 0, 0);
+
   // One K slab from LDS buffer `buf` into the accumulators.
 #define OGLE_COMPUTE_SLAB(buf)                                                               \
-  {                                                                                          \
+  if constexpr (SPLIT) {                                                                     \
+    const unsigned char* pr_ = lds + (buf) * STAGE + (lrow >> 3) * 256 +                     \
+                               ((((lrow & 7) * 2 + lq) ^ window_perm(lrow)) * 16);           \
+    bf16x8_t av[3][TM], bv[3][TN];                                                           \
+    _Pragma("unroll") for (int q = 0; q < 3; ++q) {                                          \
+      _Pragma("unroll") for (int i = 0; i < TM; ++i)                                         \
+        av[q][i] = *reinterpret_cast<const bf16x8_t*>(pr_ + q * PLANE + (wave_m * WTM + i * 32) * 32); \
+      _Pragma("unroll") for (int j = 0; j < TN; ++j)                                         \
+        bv[q][j] = *reinterpret_cast<const bf16x8_t*>(pr_ + q * PLANE + (BM + wave_n * WTN + j * 32) * 32); \
+    }                                                                                        \
+    OGLE_SPLIT_PRODUCT(rest, 1, 1)                                                           \
+    OGLE_SPLIT_PRODUCT(acc, 0, 0)                                                            \
+    OGLE_SPLIT_PRODUCT(rest, 0, 2)                                                           \
+    OGLE_SPLIT_PRODUCT(rest, 2, 0)                                                           \
+    OGLE_SPLIT_PRODUCT(rest, 0, 1)                                                           \
+    OGLE_SPLIT_PRODUCT(rest, 1, 0)                                                           \
+  } else {                                                                                   \
     const unsigned char* pa = lds + (buf) * STAGE + (wave_m * WTM + lrow) * LROW;            \
     const unsigned char* pb = lds + (buf) * STAGE + (BM + wave_n * WTN + lrow) * LROW;       \
     _Pragma("unroll") for (int ch = 0; ch < CHUNKS; ++ch) {                                  \
@@ -389,8 +473,23 @@ __device__ __forceinline__ void igemm_tile(
     __syncthreads();
   }
 #undef OGLE_COMPUTE_SLAB
+#undef OGLE_SPLIT_PRODUCT
 #undef OGLE_LOAD_SLAB
 #undef OGLE_STORE_SLAB
+
+  if constexpr (SPLIT) {
+    float probe = 0.f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < REGS; ++r) {
+          acc[i][j][r] += rest[i][j][r];
+          probe = fmaf(acc[i][j][r], 0.f, probe);
+        }
+    if (__syncthreads_or(probe != 0.f || probe != probe)) return false;
+  }
 
   // Epilogue.  Destinations: split-K partial sums go to `partial` (rows of opitch floats,
   // the channel count rounded up to 4 so that rows stay 16-byte aligned); finished outputs
@@ -429,7 +528,7 @@ __device__ __forceinline__ void igemm_tile(
         }
       }
     }
-    return;
+    return true;
   } else {
   // The staging region (reused K-loop LDS) takes JC 32-column blocks of a wave's tile at a
   // time: as many as fit, so that a row segment a wave stores is as long as possible.
@@ -480,7 +579,7 @@ __device__ __forceinline__ void igemm_tile(
         }
       }
     }
-    return;
+    return true;
   }
   if constexpr (sizeof(T) == 2) {
     if ((g.o & 7) == 0 && y2 == nullptr && (g.oimg & 7) == 0) {
@@ -528,7 +627,7 @@ __device__ __forceinline__ void igemm_tile(
           }
         }
       }
-      return;
+      return true;
     }
   }
 #pragma unroll
@@ -555,6 +654,7 @@ __device__ __forceinline__ void igemm_tile(
     }
   }
   }  // MB == 32
+  return true;
 }
 
 // Everything one convolution's workgroups need, as plain data (a kernel argument).
@@ -570,8 +670,25 @@ struct IgemmProblem {
   int tiles_n, tiles;
   float* partial;
   int slabs_per_split, splits;
-  int variant;  // mixed-group kernel only: 2 * (tile is 128x32) + (pointwise); 4..7: wave-split 32 / 16; 8, 9: 128x16 tile
+  int variant;  // mixed-group kernel only: 2 * (tile is 128x32) + (pointwise); 4..7: wave-split 32 / 16; 8, 9: 128x16 tile; + 16: as bf16 pieces
 };
+
+template <int BM, int BN, int WM, int WN, bool PW>
+__device__ __forceinline__ void igemm_tile_split(unsigned char* lds, const IgemmProblem& p, int bid) {
+#define OGLE_TILE(SPLIT)                                                                             \
+  igemm_tile<float, BM, BN, WM, WN, 64, PW, SPLIT>(                                                   \
+      lds, p.g, static_cast<const float*>(p.x), static_cast<const float*>(p.w), p.bias,               \
+      static_cast<float*>(p.y), static_cast<float*>(p.y2), p.o1, p.ep, p.tiles_n, p.tiles, p.partial, \
+      p.slabs_per_split, p.splits, bid)
+  if (!OGLE_TILE(true)) OGLE_TILE(false);
+#undef OGLE_TILE
+}
+
+template <int BM, int BN, int WM, int WN, bool PW>
+__global__ __launch_bounds__(256, 2) void conv_igemm_split_kernel(IgemmProblem p) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[igemm_lds_bytes<BM, BN, 64, true>()];
+  igemm_tile_split<BM, BN, WM, WN, PW>(lds, p, (int)blockIdx.x);
+}
 
 template <typename T, int BM, int BN, int WM, int WN, int ROWB, bool PW>
 __global__ __launch_bounds__(256) void conv_igemm_kernel(IgemmProblem p) {
@@ -606,6 +723,14 @@ struct IgemmGroup {
   IgemmProblem p[kMaxGroup];
 };
 
+template <int BM, int BN, int WM, int WN, bool PW>
+__global__ __launch_bounds__(256, 2) void conv_igemm_group_split_kernel(IgemmGroup grp) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[igemm_lds_bytes<BM, BN, 64, true>()];
+  int i = 0;
+  while (i + 1 < grp.count && (int)blockIdx.x >= grp.first[i + 1]) ++i;
+  igemm_tile_split<BM, BN, WM, WN, PW>(lds, grp.p[i], (int)blockIdx.x - grp.first[i]);
+}
+
 template <typename T, int BM, int BN, int WM, int WN, int ROWB, bool PW>
 __global__ __launch_bounds__(256) void conv_igemm_group_kernel(IgemmGroup grp) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[igemm_lds_bytes<BM, BN, ROWB>()];
@@ -630,23 +755,36 @@ __device__ __forceinline__ void igemm_wave_tile(
 // uniform over the workgroup; all four paths keep 16 accumulator registers per
 // lane, so the register budget is that of the largest one.
 template <typename T, int ROWB>
-__global__ __launch_bounds__(256) void conv_igemm_mixed_kernel(IgemmGroup grp) {
-  constexpr int kLds = igemm_lds_bytes<128, 32, ROWB>();  // the largest of the tiles below
-  static_assert(kLds >= igemm_lds_bytes<128, 16, ROWB>() && kLds >= igemm_lds_bytes<64, 64, ROWB>(), "LDS size");
+__global__ __launch_bounds__(256, 3) void conv_igemm_mixed_kernel(IgemmGroup grp) {
+  constexpr bool kSplit = sizeof(T) == 4;
+  constexpr int kLds = igemm_lds_bytes<128, 32, ROWB, kSplit>();  // the largest of the tiles below
+  static_assert(kLds >= igemm_lds_bytes<128, 16, ROWB>() && kLds >= igemm_lds_bytes<64, 64, ROWB, kSplit>(), "LDS size");
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
   int i = 0;
   while (i + 1 < grp.count && (int)blockIdx.x >= grp.first[i + 1]) ++i;
-  const IgemmProblem& p = grp.p[i];
+  // a copy: with a use of the argument per path, the compiler keeps the whole group in scratch
+  const IgemmProblem p = grp.p[i];
   const int bid = (int)blockIdx.x - grp.first[i];
+#define OGLE_MIXED_TILE(SPLIT, BM, BN, WM, WN, PW)                                              \
+  igemm_tile<T, BM, BN, WM, WN, ROWB, PW, SPLIT>(                                               \
+      lds, p.g, static_cast<const T*>(p.x), static_cast<const T*>(p.w), p.bias,                 \
+      static_cast<T*>(p.y), static_cast<T*>(p.y2), p.o1, p.ep, p.tiles_n, p.tiles,              \
+      p.partial, p.slabs_per_split, p.splits, bid)
 #define OGLE_MIXED_CASE(V, BM, BN, WM, WN, PW)                                                  \
   case V:                                                                                       \
-    igemm_tile<T, BM, BN, WM, WN, ROWB, PW>(lds, p.g, static_cast<const T*>(p.x),               \
-                                            static_cast<const T*>(p.w), p.bias,                 \
-                                            static_cast<T*>(p.y), static_cast<T*>(p.y2), p.o1,  \
-                                            p.ep, p.tiles_n, p.tiles,                           \
-                                            p.partial, p.slabs_per_split, p.splits, bid);       \
+    OGLE_MIXED_TILE(false, BM, BN, WM, WN, PW);                                                 \
     break;
-  switch (p.variant) {
+  if constexpr (kSplit) {
+    bool done = false;
+    switch (p.variant) {
+      case 16: done = OGLE_MIXED_TILE(true, 64, 64, 2, 2, false); break;
+      case 17: done = OGLE_MIXED_TILE(true, 64, 64, 2, 2, true); break;
+      case 18: done = OGLE_MIXED_TILE(true, 128, 32, 4, 1, false); break;
+      case 19: done = OGLE_MIXED_TILE(true, 128, 32, 4, 1, true); break;
+    }
+    if (done) return;
+  }
+  switch (p.variant & 15) {
     OGLE_MIXED_CASE(0, 64, 64, 2, 2, false)
     OGLE_MIXED_CASE(1, 64, 64, 2, 2, true)
     OGLE_MIXED_CASE(2, 128, 32, 4, 1, false)
@@ -668,6 +806,7 @@ __global__ __launch_bounds__(256) void conv_igemm_mixed_kernel(IgemmGroup grp) {
 #undef OGLE_MIXED_WAVE
   }
 #undef OGLE_MIXED_CASE
+#undef OGLE_MIXED_TILE
 }
 
 // ---------------------------------------------------------------------------
@@ -968,13 +1107,13 @@ __global__ __launch_bounds__(256) void splitk_reduce_group_kernel(ReduceGroup gr
 
 // Tile configurations (BM, BN, waves along M, waves along N).
 enum TileCfg {
-  CFG_128x128 = 0, CFG_128x64 = 1, CFG_64x64 = 2, CFG_128x32 = 3, CFG_WAVE32 = 4, CFG_WAVE16 = 5,
-  CFG_128x96 = 6, CFG_128x160 = 7,  // all output channels of a narrow, long-K problem in one tile
-  CFG_128x256 = 8,                   // fp16 storage: 64x128 per wave, 64-byte K slabs
-  CFG_128x16 = 9                     // at most 16 output channels: 16x16 MFMA blocks
+  CFG_128x128 = 0, CFG_64x64 = 1, CFG_128x32 = 2, CFG_WAVE32 = 3, CFG_WAVE16 = 4,
+  CFG_128x96 = 5, CFG_128x160 = 6,  // all output channels of a narrow, long-K problem in one tile
+  CFG_128x256 = 7,                   // fp16 storage: 64x128 per wave, 64-byte K slabs
+  CFG_128x16 = 8                     // at most 16 output channels: 16x16 MFMA blocks
 };
-constexpr int kCfgBM[] = {128, 128, 64, 128, 32, 16, 128, 128, 128, 128};
-constexpr int kCfgBN[] = {128, 64, 64, 32, 32, 16, 96, 160, 256, 16};
+constexpr int kCfgBM[] = {128, 64, 128, 32, 16, 128, 128, 128, 128};
+constexpr int kCfgBN[] = {128, 64, 32, 32, 16, 96, 160, 256, 16};
 constexpr int kRowBytesF16Wide = 64;  // K bytes per tile row per slab of CFG_128x256
 
 struct IgemmPlan {
@@ -985,6 +1124,7 @@ struct IgemmPlan {
   int ktiles;
   int cchunks;
   size_t workspace_bytes;  // splits * M * N floats when splits > 1
+  bool pieces;             // fp32 contracted as bf16 pieces
 };
 
 constexpr long kComputeUnits = 256;
@@ -1006,14 +1146,20 @@ IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
   auto tiles = [&](int cfg) {
     return ((m + kCfgBM[cfg] - 1) / kCfgBM[cfg]) * ((a.out_c + kCfgBN[cfg] - 1) / kCfgBN[cfg]);
   };
-  // Measured on MI355X: 64x64 tiles (eight waves per SIMD resident) match or beat
-  // the larger tiles on every layer of the network because they quantise better
-  // over 256 CUs and hide latency with occupancy; 128x128 only pays off once there
-  // are enough tiles for several rounds.
+  // fp32 as bf16 pieces: a 128x128 tile splits and reads its operands from LDS half as often per
+  // product, a 64x64 tile quantises better over 256 units.  Measured on MI355X, us with 64x64 /
+  // 128x128 tiles: M = 11552, K = 512, N = 1024 (728 large tiles) 87 / 74, 6400 x 1024 x 1024
+  // (400) 103 / 85, 11552 x 256 x 512 (364) 26.6 / 26.4, 5776 x 512 x 512 (184) 26.5 / 28.2;
+  // with K = 128 even 704 large tiles are behind (28.8 / 30.3), 2813 are not (K = 64: 76 / 72).
+  // A last tile column that is mostly padding costs more than that.
   // fp16 storage: an MFMA does sixteen times the work per operand byte, so the
   // 64x64 tile is bound by LDS traffic and instruction issue; 128x128 pays off as soon
   // as its tiles cover the compute units.
-  const long big_tiles_wanted = a.dtype == OGLE_F16 ? kComputeUnits : 4 * kComputeUnits;
+  const long k_all = (long)a.kernel_size * a.kernel_size * a.in_c;
+  const long big_tiles_wanted = a.dtype == OGLE_F16 ? kComputeUnits
+                                : k_all >= 256      ? 3 * kComputeUnits / 2
+                                                    : 8 * kComputeUnits;
+  const bool big_columns_full = a.dtype == OGLE_F16 || ((a.out_c + 127) / 128) * 128 * 10 <= ((a.out_c + 63) / 64) * 64 * 11;
   // Narrow outputs with a long contraction (the SSD heads, box and class head of a feature
   // map fused: 75 or 150 channels, K = 2304 ... 9216): one tile column holds every output
   // channel, so the input is gathered once instead of once per 64-channel tile column, and
@@ -1038,7 +1184,7 @@ IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
     p.cfg = CFG_128x16;
   } else if (a.out_c <= 32) {
     p.cfg = CFG_128x32;
-  } else if (a.out_c > 64 && tiles(CFG_128x128) >= big_tiles_wanted) {
+  } else if (a.out_c > 64 && big_columns_full && tiles(CFG_128x128) >= big_tiles_wanted) {
     p.cfg = CFG_128x128;
   } else {
     p.cfg = CFG_64x64;
@@ -1124,6 +1270,13 @@ IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
   // partial sums are kept in rows of the channel count rounded up to four
   p.workspace_bytes =
       p.splits > 1 ? (size_t)p.splits * (size_t)m * ((a.out_c + 3) & ~3) * sizeof(float) : 0;
+  // Tiles of 32x32 MFMA blocks are contracted as bf16 pieces (but for the single-column tiles of
+  // the two-destination form) once they give a compute unit more than one workgroup.  A lone
+  // workgroup has nothing to cover the splitting with: 112x112x32 -> 64 3x3 (196 tiles) 11.1 us
+  // with fp32 MFMAs, 11.9 with pieces; 3703 x 88 x 168 (174) 6.3 / 6.9; 1600 x 512 x 1024 (400)
+  // 22.8 / 20.4.
+  p.pieces = a.dtype == OGLE_F32 && (p.cfg == CFG_128x128 || p.cfg == CFG_64x64 || p.cfg == CFG_128x32) &&
+             tiles(p.cfg) * p.splits > kComputeUnits;
   // Which operand an XCD's L2 should keep to itself: with K ranges pinned to XCDs the input is
   // fetched by all eight L2s and the filter by one, with tile rows pinned it is the other way
   // round (the rocprofv3 FETCH_SIZE of the 19x19x512 class head fell from 8.5x its input to
@@ -1217,7 +1370,7 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p) {
   out.prob.splits = p.rows_on_xcd ? -p.splits : p.splits;
   out.prob.variant = (p.cfg == CFG_WAVE32 ? 4 : p.cfg == CFG_WAVE16 ? 6 : p.cfg == CFG_128x32 ? 2 :
                       p.cfg == CFG_128x16 ? 8 : 0) +
-                     (is_pointwise(a) ? 1 : 0);
+                     (is_pointwise(a) ? 1 : 0) + (p.pieces ? 16 : 0);
   if (is_wave(p.cfg)) {
     out.grid = (unsigned)(tiles_m * tiles_n);
     return out;
@@ -1238,53 +1391,73 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p) {
   return out;
 }
 
-// Instantiates kernel `K<T, BM, BN, WM, WN, ROWB, PW>` for a runtime (dtype, cfg, pw).
-#define OGLE_IGEMM_DISPATCH(K, dtype, cfg, pw, ...)                                          \
-  do {                                                                                       \
-    if ((dtype) == OGLE_F16) {                                                               \
-      OGLE_IGEMM_DISPATCH_T(K, __half, 128, cfg, pw, __VA_ARGS__);                           \
-    } else {                                                                                 \
-      OGLE_IGEMM_DISPATCH_T(K, float, kRowBytesF32, cfg, pw, __VA_ARGS__);                   \
-    }                                                                                        \
-  } while (0)
-#define OGLE_IGEMM_DISPATCH_T(K, T, ROWB, cfg, pw, ...)                                      \
+// Instantiates kernel `K<BM, BN, WM, WN, PW>` for a runtime (cfg, pw).
+#define OGLE_SPLIT_DISPATCH(K, cfg, pw, grid, s, arg)                                        \
   do {                                                                                       \
     if (pw) {                                                                                \
-      OGLE_IGEMM_DISPATCH_C(K, T, ROWB, true, cfg, __VA_ARGS__);                             \
+      OGLE_SPLIT_DISPATCH_C(K, true, cfg, grid, s, arg)                                      \
     } else {                                                                                 \
-      OGLE_IGEMM_DISPATCH_C(K, T, ROWB, false, cfg, __VA_ARGS__);                            \
+      OGLE_SPLIT_DISPATCH_C(K, false, cfg, grid, s, arg)                                     \
     }                                                                                        \
   } while (0)
-#define OGLE_IGEMM_DISPATCH_C(K, T, ROWB, PW, cfg, grid, s, arg)                             \
+#define OGLE_SPLIT_DISPATCH_C(K, PW, cfg, grid, s, arg)                                      \
   switch (cfg) {                                                                             \
     case CFG_128x128:                                                                        \
-      launch((K<T, 128, 128, 2, 2, ROWB, PW>), dim3(grid), dim3(256), 0, s, arg); \
-      break;                                                                                 \
-    case CFG_128x64:                                                                         \
-      launch((K<T, 128, 64, 2, 2, ROWB, PW>), dim3(grid), dim3(256), 0, s, arg);  \
+      launch((K<128, 128, 2, 2, PW>), dim3(grid), dim3(256), 0, s, arg);                     \
       break;                                                                                 \
     case CFG_64x64:                                                                          \
-      launch((K<T, 64, 64, 2, 2, ROWB, PW>), dim3(grid), dim3(256), 0, s, arg);   \
-      break;                                                                                 \
-    case CFG_128x96:                                                                         \
-      launch((K<T, 128, 96, 4, 1, ROWB, PW>), dim3(grid), dim3(256), 0, s, arg);  \
-      break;                                                                                 \
-    case CFG_128x160:                                                                        \
-      launch((K<T, 128, 160, 4, 1, ROWB, PW>), dim3(grid), dim3(256), 0, s, arg); \
-      break;                                                                                 \
-    case CFG_128x16:                                                                         \
-      launch((K<T, 128, 16, 4, 1, ROWB, PW>), dim3(grid), dim3(256), 0, s, arg);  \
+      launch((K<64, 64, 2, 2, PW>), dim3(grid), dim3(256), 0, s, arg);                       \
       break;                                                                                 \
     default:                                                                                 \
-      launch((K<T, 128, 32, 4, 1, ROWB, PW>), dim3(grid), dim3(256), 0, s, arg);  \
+      launch((K<128, 32, 4, 1, PW>), dim3(grid), dim3(256), 0, s, arg);                      \
       break;                                                                                 \
   }
 
+// Instantiates kernel `K<T, BM, BN, WM, WN, ROWB, PW>` for a runtime (dtype, cfg, pw).
+#define OGLE_IGEMM_DISPATCH(K, dtype, cfg, pw, grid, s, arg)                                 \
+  do {                                                                                       \
+    if ((dtype) == OGLE_F16) {                                                               \
+      if (pw) {                                                                              \
+        OGLE_IGEMM_DISPATCH_F16(K, true, cfg, grid, s, arg)                                  \
+      } else {                                                                               \
+        OGLE_IGEMM_DISPATCH_F16(K, false, cfg, grid, s, arg)                                 \
+      }                                                                                      \
+    } else {                                                                                 \
+      if (pw) {                                                                              \
+        OGLE_IGEMM_DISPATCH_C(K, float, kRowBytesF32, true, cfg, grid, s, arg)               \
+      } else {                                                                               \
+        OGLE_IGEMM_DISPATCH_C(K, float, kRowBytesF32, false, cfg, grid, s, arg)              \
+      }                                                                                      \
+    }                                                                                        \
+  } while (0)
+#define OGLE_IGEMM_CASE(K, T, BM, BN, WM, WN, ROWB, PW, grid, s, arg)                        \
+  launch((K<T, BM, BN, WM, WN, ROWB, PW>), dim3(grid), dim3(256), 0, s, arg);                \
+  break;
+#define OGLE_IGEMM_DISPATCH_C(K, T, ROWB, PW, cfg, grid, s, arg)                             \
+  switch (cfg) {                                                                             \
+    case CFG_128x96: OGLE_IGEMM_CASE(K, T, 128, 96, 4, 1, ROWB, PW, grid, s, arg)            \
+    case CFG_128x160: OGLE_IGEMM_CASE(K, T, 128, 160, 4, 1, ROWB, PW, grid, s, arg)          \
+    case CFG_64x64: OGLE_IGEMM_CASE(K, T, 64, 64, 2, 2, ROWB, PW, grid, s, arg)              \
+    case CFG_128x32: OGLE_IGEMM_CASE(K, T, 128, 32, 4, 1, ROWB, PW, grid, s, arg)            \
+    default: OGLE_IGEMM_CASE(K, T, 128, 16, 4, 1, ROWB, PW, grid, s, arg)                    \
+  }
+#define OGLE_IGEMM_DISPATCH_F16(K, PW, cfg, grid, s, arg)                                    \
+  switch (cfg) {                                                                             \
+    case CFG_128x128: OGLE_IGEMM_CASE(K, __half, 128, 128, 2, 2, 128, PW, grid, s, arg)      \
+    case CFG_64x64: OGLE_IGEMM_CASE(K, __half, 64, 64, 2, 2, 128, PW, grid, s, arg)          \
+    case CFG_128x32: OGLE_IGEMM_CASE(K, __half, 128, 32, 4, 1, 128, PW, grid, s, arg)        \
+    default: OGLE_IGEMM_CASE(K, __half, 128, 16, 4, 1, 128, PW, grid, s, arg)                \
+  }
+
 // One problem, one grid of the LDS-tiled kernel.
-void launch_single(int dtype, int cfg, bool pw, unsigned grid, hipStream_t s, const IgemmProblem& prob) {
+void launch_single(int dtype, int cfg, bool pieces, bool pw, unsigned grid, hipStream_t s, const IgemmProblem& prob) {
   if (cfg == CFG_128x256) {  // fp16 storage only (plan_igemm)
     if (pw) launch(conv_igemm_wide_f16_kernel<true>, dim3(grid), dim3(256), 0, s, prob);
     else launch(conv_igemm_wide_f16_kernel<false>, dim3(grid), dim3(256), 0, s, prob);
+    return;
+  }
+  if (pieces) {
+    OGLE_SPLIT_DISPATCH(conv_igemm_split_kernel, cfg, pw, grid, s, prob);
     return;
   }
   OGLE_IGEMM_DISPATCH(conv_igemm_kernel, dtype, cfg, pw, grid, s, prob);
@@ -1345,7 +1518,7 @@ int32_t launch_conv_igemm(const OgleConvArgs& a, hipStream_t s) {
     launch_wave(a.dtype, pw, p.cfg, pr, s);
     return check_launch("conv_igemm_wave");
   }
-  launch_single(a.dtype, p.cfg, pw, pr.grid, s, pr.prob);
+  launch_single(a.dtype, p.cfg, p.pieces, pw, pr.grid, s, pr.prob);
   int32_t st = check_launch("conv_igemm");
   if (st != OGLE_OK || p.splits == 1) return st;
   if (a.dtype == OGLE_F16) launch_reduce_single<__half>(pr, s);
@@ -1364,7 +1537,7 @@ int32_t launch_conv_batch(const OgleConvArgs* args, int count, hipStream_t s,
                           int32_t* reduce_pending) {
   struct Item {
     int dtype, cfg;
-    bool pw;
+    bool pieces, pw;
     Prepared pr;
   };
   std::vector<Item> items;
@@ -1382,7 +1555,7 @@ int32_t launch_conv_batch(const OgleConvArgs* args, int count, hipStream_t s,
       continue;
     }
     const IgemmPlan p = final_plan(args[i], m);
-    items.push_back(Item{args[i].dtype, p.cfg, is_pointwise(args[i]), prepare(args[i], m, p)});
+    items.push_back(Item{args[i].dtype, p.cfg, p.pieces, is_pointwise(args[i]), prepare(args[i], m, p)});
     if (reduce_pending != nullptr && p.splits > 1) reduce_pending[i] = 1;
   }
   auto mixable = [](const Item& it) {
@@ -1398,7 +1571,7 @@ int32_t launch_conv_batch(const OgleConvArgs* args, int count, hipStream_t s,
     for (size_t b0 = a0; b0 < items.size() && grp.count < kMaxGroup; ++b0) {
       const Item& it = items[b0];
       if (done[b0] || it.dtype != head.dtype) continue;
-      const bool same = it.cfg == head.cfg && it.pw == head.pw && it.cfg != CFG_128x256;
+      const bool same = it.cfg == head.cfg && it.pw == head.pw && it.pieces == head.pieces && it.cfg != CFG_128x256;
       if (b0 != a0 && (it.cfg == CFG_128x256 || head.cfg == CFG_128x256)) continue;  // fills the chip alone
       if (!same && !(mixable(head) && mixable(it))) continue;
       uniform = uniform && same;
@@ -1415,7 +1588,9 @@ int32_t launch_conv_batch(const OgleConvArgs* args, int count, hipStream_t s,
     if (grp.count == 1 && is_wave(head.cfg)) {
       launch_wave(head.dtype, head.pw, head.cfg, head.pr, s);
     } else if (grp.count == 1) {
-      launch_single(head.dtype, head.cfg, head.pw, grid, s, grp.p[0]);
+      launch_single(head.dtype, head.cfg, head.pieces, head.pw, grid, s, grp.p[0]);
+    } else if (uniform && head.pieces) {
+      OGLE_SPLIT_DISPATCH(conv_igemm_group_split_kernel, head.cfg, head.pw, grid, s, grp);
     } else if (uniform && !is_wave(head.cfg)) {
       OGLE_IGEMM_DISPATCH(conv_igemm_group_kernel, head.dtype, head.cfg, head.pw, grid, s, grp);
     } else if (head.dtype == OGLE_F16) {

@@ -185,6 +185,66 @@ def test_conv_patch_kernel_infinite_filter_values_meet_no_padding():
         np.testing.assert_array_equal(got[~np.isfinite(ref)], ref[~np.isfinite(ref)])
 
 
+PIECES_CASES = [
+    # n, h, w, c, o, k, s, p   fp32 as bf16 pieces: more workgroups than compute units
+    (1, 96, 174, 64, 40, 1, 1, 0),      # 64x64 tiles, pointwise, ragged N; 261 workgroups
+    (1, 96, 168, 64, 40, 1, 1, 0),      # 252 workgroups: the fp32 tile, next to the line
+    (16, 19, 19, 512, 512, 1, 1, 0),    # 64x64 tiles, 728 workgroups
+    (1, 223, 221, 256, 128, 1, 1, 0),   # 128x128 tiles, 386 of them, last one ragged
+    (1, 217, 221, 260, 124, 1, 1, 0),   # 375 large tiles: 64x64; K tail inside a slab, ragged N
+    (2, 75, 73, 36, 32, 3, 1, 1),       # 128x32 tile, 3x3, 86 workgroups: fp32
+    (5, 84, 84, 36, 31, 3, 1, 1),       # 128x32 tile, 3x3, 276 workgroups, odd N
+    (3, 75, 73, 44, 70, 3, 2, 1),       # 64x64, stride 2: split-K partials or one tile column and a bit
+    (2, 19, 19, 512, 63, 3, 1, 1),      # split-K partials, odd N, K = 4608
+]
+
+
+def _pieces_reference(x, wt, k, s, p):
+    torch = pytest.importorskip("torch")
+    t = torch.nn.functional.conv2d(torch.from_numpy(x).double().permute(0, 3, 1, 2), torch.from_numpy(wt).double(),
+                                   None, s, p)
+    return t.permute(0, 2, 3, 1).numpy()
+
+
+@pytest.mark.parametrize("case", PIECES_CASES)
+def test_conv_fp32_as_bf16_pieces(case):
+    """The three pieces of a value add up to it exactly and the products left out are below 2^-26 of
+    a product, so what is left is the fp32 rounding of the running sums: one per 16 products (two
+    allowed for) plus a few at the end, relative to the sum of the products' magnitudes."""
+    n, h, w, c, o, k, s, p = case
+    r = rng(3100 + PIECES_CASES.index(case))
+    x = (r.uniform(-1, 1, (n, h, w, c)) * 2.0 ** r.integers(-12, 12, (n, h, w, c))).astype(np.float32)
+    wt = (r.normal(0, 0.2, (o, c, k, k)) * 2.0 ** r.integers(-8, 8, (o, c, k, k))).astype(np.float32)
+    ref = _pieces_reference(x, wt, k, s, p)
+    scale = _pieces_reference(np.abs(x), np.abs(wt), k, s, p)
+    for ws in (True, False):
+        got = gpu_conv(x, wt, None, s, p, workspace=ws, entry="ogle_hip_conv2d")
+        bound = (k * k * c / 8 + 16) * 2.0 ** -24
+        assert np.max(np.abs(got - ref) / scale) <= bound, (case, ws)
+
+
+@pytest.mark.parametrize("case", [(16, 19, 19, 512, 512, 1, 0), (1, 223, 221, 256, 128, 1, 0), (2, 75, 75, 64, 63, 3, 1)])
+def test_conv_fp32_as_bf16_pieces_not_finite(case):
+    """Infinite, NaN and very large operands, whose pieces are no numbers, give what fp32 gives."""
+    n, h, w, c, o, k, p = case
+    r = rng(3150 + o)
+    x = r.uniform(0.5, 1, (n, h, w, c)).astype(np.float32)
+    wt = r.uniform(0.001, 0.002, (o, c, k, k)).astype(np.float32)
+    x[0, 3, 4, 5] = np.inf
+    x[0, 9, 9, 7] = np.nan
+    x[n - 1, h - 2, w - 3, 1] = -np.inf
+    x[n - 1, 5, 6, 2] = 3.4e38       # rounds to infinity as bf16; times a filter value it is finite
+    wt[o - 1, 3, 0, 0] = 3.4e38
+    with np.errstate(over="ignore", invalid="ignore"):
+        ref = _pieces_reference(x, wt, k, 1, p).astype(np.float32)
+    got = gpu_conv(x, wt, None, 1, p, entry="ogle_hip_conv2d")
+    ok = np.isfinite(ref)
+    assert 0.9 < ok.mean() < 1
+    np.testing.assert_array_equal(np.isfinite(got), ok)
+    np.testing.assert_array_equal(got[~ok], ref[~ok])
+    np.testing.assert_allclose(got[ok], ref[ok], rtol=1e-4)
+
+
 WAVE_CASES = [
     # n, h, w, c, o, k, s, p, d   small problems with a long enough K: the wave-split kernel
     (1, 19, 19, 512, 512, 1, 1, 0, 1),    # 32x32 tiles, pointwise (a batch-1 MobileNet layer)
