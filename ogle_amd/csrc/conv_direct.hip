@@ -290,6 +290,14 @@ __global__ __launch_bounds__(256) void conv_direct_general(
 // lanes on neighbouring pixels hit different banks.  Channels that do not fit LDS at once are
 // staged `cc` at a time.
 //
+// Measured on MI355X, us before (one thread per output; for the 7x7 stem a vector kernel with the
+// filter broadcast from LDS) / with this kernel: 4 x 57 x 43, 12 groups of 8 -> 12 183 / 16;
+// 4 x 48 x 48, 32 groups of 32 -> 32 9909 / 117; 4 x 56 x 56, 99 -> 99 3x3 2995 / 96; 16 x 224 x 224,
+// 3 -> 64 7x7 stride 2 168 / 99 (the products alone: 24 at the fp32 MFMA rate).  Waits for staging
+// are what is left, so residency counts: registers are capped for three workgroups per unit (64
+// columns: 103 -> 99, 32 groups of 32: 142 -> 117).  Staging by whole rows, without index
+// arithmetic, was 15 % slower on the stem and its extra code cost the other shapes 8 %.
+//
 // Taps outside the image are staged as zeros.  0 * w is 0 only for a finite w, so a workgroup
 // that meets an infinite or NaN filter value recomputes its outputs one by one, skipping taps.
 struct FastDiv {   // n / d for n, d < 2^16: with mul = ceil(2^32 / d) the error n * (mul * d - 2^32) stays below 2^32
@@ -334,7 +342,7 @@ __device__ __forceinline__ void load_some(const T* src, bool on, float (&v)[V]) 
 }
 
 template <typename T, int COLS>
-__global__ __launch_bounds__(256) void conv_patch_mfma(const T* __restrict__ x, const T* __restrict__ w,
+__global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const T* __restrict__ x, const T* __restrict__ w,
                                                        const float* __restrict__ bias, T* __restrict__ y,
                                                        DirectGeom q, PatchPlan p, Epilogue ep) {
   extern __shared__ __attribute__((aligned(16))) float patch_lds[];
@@ -385,20 +393,6 @@ __global__ __launch_bounds__(256) void conv_patch_mfma(const T* __restrict__ x, 
     const int by = rest % p.tiles_y, bb = rest / p.tiles_y;
     const int ox0 = bx << p.tw_log, oy0 = by << p.th_log, b0 = bb * (kPatchPixels >> (p.tw_log + p.th_log));
     const int iy0 = oy0 * q.stride - q.pad, ix0 = ox0 * q.stride - q.pad;
-
-    // where this lane's results go: register r is pixel 8*(r/4) + 4*(lane/32) + r%4 (32x32) or
-    // 4*(lane/16) + r (16x16) of the block, column lane % MB
-    constexpr unsigned kNoPixel = 0xffffffffu;
-    unsigned y_off[FR][REGS];
-#pragma unroll
-    for (int f = 0; f < FR; ++f)
-#pragma unroll
-      for (int r = 0; r < REGS; ++r) {
-        const int pix = wave * 32 + f * MB + (MB == 32 ? (r >> 2) * 8 + lq * 4 + (r & 3) : lq * 4 + r);
-        const int ox = ox0 + (pix & (box_w - 1)), oy = oy0 + ((pix >> p.tw_log) & (box_h - 1));
-        const int b = b0 + (pix >> (p.tw_log + p.th_log));
-        y_off[f][r] = ox < q.ow && oy < q.oh && b < q.n ? (unsigned)(((b * q.oh + oy) * q.ow + ox) * q.o) : kNoPixel;
-      }
 
     // with gp > 1 all channels are staged at once: only one of the two loops below has more
     // than one turn, and one set of accumulators serves both
@@ -545,6 +539,19 @@ __global__ __launch_bounds__(256) void conv_patch_mfma(const T* __restrict__ x, 
           }
         }
         if (c0 + p.cc < cpg) continue;   // more channels of this group to come (gp == 1)
+        // where this lane's results go: register r is pixel 8*(r/4) + 4*(lane/32) + r%4 (32x32)
+        // or 4*(lane/16) + r (16x16) of the block, column lane % MB
+        constexpr unsigned kNoPixel = 0xffffffffu;
+        unsigned y_off[FR][REGS];
+#pragma unroll
+        for (int f = 0; f < FR; ++f)
+#pragma unroll
+          for (int r = 0; r < REGS; ++r) {
+            const int pix = wave * 32 + f * MB + (MB == 32 ? (r >> 2) * 8 + lq * 4 + (r & 3) : lq * 4 + r);
+            const int ox = ox0 + (pix & (box_w - 1)), oy = oy0 + ((pix >> p.tw_log) & (box_h - 1));
+            const int b = b0 + (pix >> (p.tw_log + p.th_log));
+            y_off[f][r] = ox < q.ow && oy < q.oh && b < q.n ? (unsigned)(((b * q.oh + oy) * q.ow + ox) * q.o) : kNoPixel;
+          }
         const int obase = (g0 + gi) * opg + col0;
 #pragma unroll
         for (int n = 0; n < NB; ++n) {
@@ -661,8 +668,10 @@ bool plan_patch(const OgleConvArgs& a, PatchPlan* out) {
   p.lds_floats = (int)floats(cc, p.gp);
   const long per_tile = (long)p.gblocks * p.col_blocks;
   // with all channels staged at once the filter stays in LDS while a workgroup walks boxes
-  const long most = cc == cpg ? std::max(1L, (768 + per_tile - 1) / per_tile) : tiles;
-  p.tile_blocks = (int)std::min(tiles, most);
+  // (no more workgroups than their LDS lets be resident, each with as many boxes as any other)
+  const long resident = 256 * (40L * 1024 / p.lds_floats);
+  const long turns = cc == cpg ? (tiles * per_tile + resident - 1) / resident : 1;
+  p.tile_blocks = (int)((tiles + turns - 1) / turns);
   if (per_tile * p.tile_blocks > lim || pixels * cc * p.gp > 0xffff ||
       (long)p.gp * p.cols * k * k * cc > 0xffff)
     return false;
