@@ -1151,7 +1151,6 @@ IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
   // 128x128 tiles: M = 11552, K = 512, N = 1024 (728 large tiles) 87 / 74, 6400 x 1024 x 1024
   // (400) 103 / 85, 11552 x 256 x 512 (364) 26.6 / 26.4, 5776 x 512 x 512 (184) 26.5 / 28.2;
   // with K = 128 even 704 large tiles are behind (28.8 / 30.3), 2813 are not (K = 64: 76 / 72).
-  // A last tile column that is mostly padding costs more than that.
   // fp16 storage: an MFMA does sixteen times the work per operand byte, so the
   // 64x64 tile is bound by LDS traffic and instruction issue; 128x128 pays off as soon
   // as its tiles cover the compute units.
@@ -1159,7 +1158,11 @@ IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
   const long big_tiles_wanted = a.dtype == OGLE_F16 ? kComputeUnits
                                 : k_all >= 256      ? 3 * kComputeUnits / 2
                                                     : 8 * kComputeUnits;
-  const bool big_columns_full = a.dtype == OGLE_F16 || ((a.out_c + 127) / 128) * 128 * 10 <= ((a.out_c + 63) / 64) * 64 * 11;
+  // A last tile column that is mostly padding costs more than that, in fp16 while K is short
+  // (12 x 57 x 57, 88 -> 168: 128x128 tiles 16.3 us, 64x64 11.2; 256 -> 168 19.0 / 14.1; 8 x 40 x 40,
+  // 88 -> 300 17.2 / 8.8; K = 792 17.2 / 17.4).
+  const bool big_columns_full = (a.dtype == OGLE_F16 && k_all > 512) ||
+                                ((a.out_c + 127) / 128) * 128 * 10 <= ((a.out_c + 63) / 64) * 64 * 11;
   // Narrow outputs with a long contraction (the SSD heads, box and class head of a feature
   // map fused: 75 or 150 channels, K = 2304 ... 9216): one tile column holds every output
   // channel, so the input is gathered once instead of once per 64-channel tile column, and

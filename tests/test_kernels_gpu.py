@@ -185,6 +185,17 @@ def test_conv_patch_kernel_infinite_filter_values_meet_no_padding():
         np.testing.assert_array_equal(got[~np.isfinite(ref)], ref[~np.isfinite(ref)])
 
 
+@pytest.mark.parametrize("o,c", [(168, 88), (192, 64), (193, 40), (300, 72), (168, 520)])
+def test_fp16_tiles_by_filled_columns(o, c):
+    """fp16 storage, enough rows for 128x128 tiles: the tile depends on how much of the last tile
+    column is padding and on K (520: past the line)."""
+    r = rng(3000 + o + c)
+    x = r.uniform(-1, 1, (3, 75, 75, c)).astype(np.float16).astype(np.float32)
+    wt = r.normal(0, 0.3, (o, c, 1, 1)).astype(np.float16).astype(np.float32)
+    b = r.uniform(-0.1, 0.1, o).astype(np.float32)
+    check_conv(x, wt, b, act=H.ACT_CLIP, maxv=6.0, variant=H.VARIANT_PW, dtype=H.F16, what="%d %d" % (o, c))
+
+
 PIECES_CASES = [
     # n, h, w, c, o, k, s, p   fp32 as bf16 pieces: more workgroups than compute units
     (1, 96, 174, 64, 40, 1, 1, 0),      # 64x64 tiles, pointwise, ragged N; 261 workgroups
