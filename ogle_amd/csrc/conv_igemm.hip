@@ -1163,6 +1163,15 @@ IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
   // 88 -> 300 17.2 / 8.8; K = 792 17.2 / 17.4).
   const bool big_columns_full = (a.dtype == OGLE_F16 && k_all > 512) ||
                                 ((a.out_c + 127) / 128) * 128 * 10 <= ((a.out_c + 63) / 64) * 64 * 11;
+  // A contraction of 128 slabs or more is cut along K below 2048 tiles (further down), which takes
+  // scratch memory.  Large tiles neither bring that on nor avoid it where the scratch a caller
+  // has to bring would differ: from 1024 of them on they are cut as well, with fewer they are taken
+  // only where the small tiles would not be cut.
+  const bool long_f32 = a.dtype == OGLE_F32 && p.ktiles >= 128;
+  const bool big_tiles = long_f32 ? tiles(CFG_128x128) >= 4 * kComputeUnits ||
+                                        (big_columns_full && tiles(CFG_128x128) >= big_tiles_wanted &&
+                                         tiles(CFG_64x64) >= 8 * kComputeUnits)
+                                  : big_columns_full && tiles(CFG_128x128) >= big_tiles_wanted;
   // Narrow outputs with a long contraction (the SSD heads, box and class head of a feature
   // map fused: 75 or 150 channels, K = 2304 ... 9216): one tile column holds every output
   // channel, so the input is gathered once instead of once per 64-channel tile column, and
@@ -1187,7 +1196,7 @@ IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
     p.cfg = CFG_128x16;
   } else if (a.out_c <= 32) {
     p.cfg = CFG_128x32;
-  } else if (a.out_c > 64 && big_columns_full && tiles(CFG_128x128) >= big_tiles_wanted) {
+  } else if (a.out_c > 64 && big_tiles) {
     p.cfg = CFG_128x128;
   } else {
     p.cfg = CFG_64x64;
@@ -1218,7 +1227,8 @@ IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
     const long want = (3 * kComputeUnits + t - 1) / t;
     const long most = p.ktiles / 4;
     sp = want < most ? want : most;
-  } else if (allow_split && t < 8 * kComputeUnits && p.ktiles >= 128) {
+  } else if (allow_split && t < 8 * kComputeUnits && p.ktiles >= 128 &&
+             !(long_f32 && p.cfg == CFG_128x128 && t < 4 * kComputeUnits)) {
     // a few long workgroups per unit quantise badly (one unit gets two, its
     // neighbour one) and leave one wave per SIMD: cut the long contraction so that
     // about eight shorter workgroups land on every unit, 32 slabs or more each

@@ -79,3 +79,20 @@ def test_pool_concat_decode_argument_errors():
     assert lib.ogle_hip_packed_filter_elems(H.FILTER_HWC, 8, 2, 3, 3) == -1
     assert lib.ogle_hip_packed_filter_elems(H.FILTER_OHWI, 8, 2, 3, 3) == 144
     assert H.lib().ogle_hip_status_string(H.ERR_UNSUPPORTED) == b"unsupported"
+
+
+@pytest.mark.parametrize("shape,need", [
+    # n, h, w, c, o, k: the tile a convolution runs on does not change the scratch it asks for
+    ((64, 19, 19, 512, 512, 3), 0),             # 2888 small tiles, 724 large ones: not cut along K
+    ((32, 19, 19, 512, 512, 3), 47316992),      # 1448 small tiles: two K ranges
+    ((64, 19, 19, 512, 168, 3), 31051776),      # a last 128-wide column that is mostly padding
+    ((100, 38, 38, 256, 128, 3), 147865600),    # 1129 large tiles: cut
+    ((16, 128, 128, 256, 168, 3), 0),           # 4096 large tiles: not cut
+    ((64, 19, 19, 512, 63, 3), 23658496),
+    ((16, 19, 19, 512, 512, 1), 0),
+])
+def test_conv_workspace_of_long_contractions(shape, need):
+    n, h, w, c, o, k = shape
+    a = H.conv_args(4096, 4096, None, 4096, n, h, w, c, o, k, 1, k // 2, 1, 1, H.ACT_NONE, 0.0, 0.0,
+                    H.VARIANT_NHWC4, H.F32)
+    assert H.lib().ogle_hip_conv_workspace_bytes(ctypes.byref(a)) == need
