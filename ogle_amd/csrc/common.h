@@ -98,20 +98,20 @@ __device__ __forceinline__ __half from_f32<__half>(float v) { return __float2hal
 // of the network are 7 % faster this way, the fp16 GEMM of 12 GFLOP 13 %, a whole batch-16
 // pass 1.5 %.  (Non-temporal stores were slower than plain ones.)
 // The hardware reads a store's data registers while it issues, and for stores wider than 64
-// bits the slot right behind one may not overwrite them (the wide-store hazard the compiler
+// bits the two slots right behind one may not overwrite them (the wide-store hazard the compiler
 // pads its own stores for; it does not look into inline assembly).  So the 16-byte forms end
-// in a wait state of their own: without it a GEMM epilogue whose next instruction happened to
+// in two wait states of their own: without them a GEMM epilogue whose next instruction happened to
 // write the data registers stored a few wrong values in a hundred thousand.
 constexpr int kResultStoreAux = 17;   // raw buffer stores: sc0 | sc1
 __device__ __forceinline__ void store_result16(void* dst, float4 v) {
   typedef float f32x4_t __attribute__((ext_vector_type(4)));
   const f32x4_t t = {v.x, v.y, v.z, v.w};
-  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(dst), "v"(t) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(dst), "v"(t) : "memory");
 }
 __device__ __forceinline__ void store_result16(void* dst, uint4 v) {
   typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
   const u32x4_t t = {v.x, v.y, v.z, v.w};
-  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(dst), "v"(t) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(dst), "v"(t) : "memory");
 }
 __device__ __forceinline__ void store_result8(void* dst, uint2 v) {
   typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
