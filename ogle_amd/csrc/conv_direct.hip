@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <type_traits>
 #include "common.h"
+#include "conv_plan.h"
 
 namespace ogle {
 namespace {
@@ -300,33 +301,11 @@ __global__ __launch_bounds__(256) void conv_direct_general(
 //
 // Taps outside the image are staged as zeros.  0 * w is 0 only for a finite w, so a workgroup
 // that meets an infinite or NaN filter value recomputes its outputs one by one, skipping taps.
-struct FastDiv {   // n / d for n, d < 2^16: with mul = ceil(2^32 / d) the error n * (mul * d - 2^32) stays below 2^32
-  unsigned mul;
-  int d;
-};
-__host__ __device__ __forceinline__ FastDiv fast_div(int d) {
-  return FastDiv{0xffffffffu / (unsigned)d + 1u, d};   // ceil(2^32 / d); d == 1 is not looked up
-}
+
 __device__ __forceinline__ int div_fast(int n, const FastDiv& f) {
   return f.d == 1 ? n : (int)__umulhi((unsigned)n, f.mul);
 }
 
-struct PatchPlan {
-  int th_log, tw_log;             // box of output pixels of a workgroup (128 >> both images)
-  int tiles_b, tiles_y, tiles_x;  // boxes along images, rows, columns
-  int ph, pw, pitch;              // patch rows, columns, floats per patch pixel
-  int in_step, box_step;          // input pixels per patch pixel, patch pixels per output pixel
-  int cc;                         // input channels per group staged at once
-  int gp, gblocks;                // groups per workgroup; ceil(groups / gp)
-  int cols, col_blocks;           // output channels per workgroup and group
-  int runs_x;                     // K runs per filter row: one per tap, or one in all
-  int tile_blocks;                // workgroups along the boxes (each walks several when channels fit at once)
-  int vec_x, vec_w;               // patch / filter read four values at a time
-  int patch_floats, lds_floats;
-  FastDiv d_cs, d_pw, d_ph, d_runk, d_col;
-};
-
-constexpr int kPatchPixels = 128;
 // Scalar loads a thread has in flight while it stages.  More make longer code that is fetched
 // cold by every launch, and 16 spilled registers (12 groups of 8 -> 12 channels, 3x3: 33 us).
 constexpr int kPatchBatch = 8;
@@ -583,108 +562,6 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
       }
     }
   }
-}
-
-// The patch kernel's box, chunk and grid for a convolution; false if it does not take it.
-bool plan_patch(const OgleConvArgs& a, PatchPlan* out) {
-  const int cpg = a.in_c / a.group, opg = a.out_c / a.group, k = a.kernel_size;
-  const long lim = 0x7fffffffL;
-  if ((long)a.n * a.in_h * a.in_w * a.in_c > lim || (long)a.n * a.out_h * a.out_w * a.out_c > lim) return false;
-  if ((long)a.n + kPatchPixels > lim || (long)a.in_h + a.padding > lim / 2 || (long)a.in_w + a.padding > lim / 2)
-    return false;
-  // Under 64 products per pixel and group most of an MFMA block is padding and one thread per
-  // output is faster.  Measured at 4 x 48 x 48, us with one thread per output / with this kernel,
-  // groups x (channels in -> out): 64 x (2 -> 2) 3x3 25 / 44, 32 x (4 -> 8) 1x1 15.3 / 17.9;
-  // from 64 on 32 x (8 -> 8) 1x1 38 / 19, 16 x (4 -> 4) 3x3 27 / 17, 32 x (32 -> 32) 3x3 9905 / 122
-  if ((long)k * k * cpg * opg < 64) return false;
-  // A few thousand short sums are over before the patch is staged (one image 14 x 14, 32 x
-  // (8 -> 8) 1x1: 6.3 / 7.6; 9 x 9, 35 -> 75 1x1: 6.3 / 12.1; 4 x 28 x 28, 181 -> 9 1x1, whose
-  // patch is staged in three chunks: 20.8 / 31; but 3x3 with K = 72: 11.6 / 8.6, K = 891: 104 / 50).
-  if ((long)a.n * a.out_h * a.out_w * a.out_c <= 65536 && k * k * cpg <= (k == 1 ? 192 : 48)) return false;
-  const long span = (long)(k - 1) * a.dilation + 1;
-  if (span > 1024 || a.stride > 64) return false;   // no such patch fits LDS
-  PatchPlan p{};
-  // one tap: the pixels that a stride skips are not staged
-  p.in_step = k == 1 ? a.stride : 1;
-  p.box_step = k == 1 ? 1 : a.stride;
-  p.cols = opg <= 16 ? 16 : (opg <= 32 || (((opg + 31) / 32) % 2 == 1 && opg < 160)) ? 32 : 64;
-  // the box: fewest boxes, then the smallest patch
-  double best = 0;
-  for (int tw = 0; tw <= 7; ++tw) {
-    for (int th = 0; tw + th <= 7; ++th) {
-      const int box_b = kPatchPixels >> (tw + th);
-      if ((1 << tw) >= 2 * a.out_w || (1 << th) >= 2 * a.out_h) continue;
-      const long ph = ((1L << th) - 1) * p.box_step + span, pw = ((1L << tw) - 1) * p.box_step + span;
-      const double boxes = (double)((a.n + box_b - 1) / box_b) * ((a.out_h + (1 << th) - 1) >> th) *
-                           ((a.out_w + (1 << tw) - 1) >> tw);
-      const double cost = boxes * ((double)(ph * pw * box_b) + 2.0 * kPatchPixels);
-      if (best != 0 && cost >= best) continue;
-      best = cost;
-      p.tw_log = tw;
-      p.th_log = th;
-      p.ph = (int)ph;
-      p.pw = (int)pw;
-    }
-  }
-  const int box_b = kPatchPixels >> (p.tw_log + p.th_log);
-  p.tiles_b = (a.n + box_b - 1) / box_b;
-  p.tiles_y = (a.out_h + (1 << p.th_log) - 1) >> p.th_log;
-  p.tiles_x = (a.out_w + (1 << p.tw_log) - 1) >> p.tw_log;
-  const long tiles = (long)p.tiles_b * p.tiles_y * p.tiles_x;
-  // a grid that leaves compute units empty is cut finer along the channels instead: the time of
-  // such a launch is one workgroup's staging and serial contraction
-  while (p.cols > 16 && tiles * a.group * ((opg + p.cols - 1) / p.cols) < 256) p.cols /= 2;
-  p.col_blocks = (opg + p.cols - 1) / p.cols;
-  const long pixels = (long)box_b * p.ph * p.pw;
-  const long wp = p.cols + 1;
-  if (pixels > 0xffff) return false;
-  // channels staged at once: all of them, or the most that leave three workgroups per unit
-  // (48 KB of LDS each); 64 KB, the launch limit, where the grid gives a unit no third one
-  // anyway (fewer, longer chunks: each costs a round trip to memory) or nothing less will do
-  const bool roomy = tiles * a.group * p.col_blocks <= 512;
-  auto floats = [&](long cc, long gp) { return pixels * ((cc * gp) | 1) + gp * k * k * cc * wp; };
-  long cc = 0;
-  for (const long budget : {roomy ? 16384L : 12288L, 16384L}) {
-    if (floats(cpg, 1) <= budget) cc = cpg;
-    else
-      for (long t : {64L, 32L, 16L, 8L, 4L, 2L})
-        if (cc == 0 && t < cpg && floats(t, 1) <= budget) cc = t;
-    if (cc != 0) break;
-  }
-  if (cc == 0) return false;
-  p.cc = (int)cc;
-  // several groups per workgroup share a patch's cache lines, as long as the grid still has
-  // about two workgroups per compute unit
-  p.gp = 1;
-  if (cc == cpg && p.col_blocks == 1)
-    while (p.gp < a.group && floats(cpg, p.gp + 1) <= 8192 &&
-           tiles * ((a.group + p.gp) / (p.gp + 1)) >= 512)
-      ++p.gp;
-  p.gblocks = (a.group + p.gp - 1) / p.gp;
-  const bool merge = a.dilation == 1 && cc == cpg && p.gp == 1 && cpg % 2 == 1 && k > 1;
-  p.runs_x = merge ? 1 : k;
-  p.pitch = (int)(cc * p.gp) | 1;
-  p.patch_floats = (int)(pixels * p.pitch);
-  p.lds_floats = (int)floats(cc, p.gp);
-  const long per_tile = (long)p.gblocks * p.col_blocks;
-  // with all channels staged at once the filter stays in LDS while a workgroup walks boxes
-  // (no more workgroups than their LDS lets be resident, each with as many boxes as any other)
-  const long resident = 256 * (40L * 1024 / p.lds_floats);
-  const long turns = cc == cpg ? (tiles * per_tile + resident - 1) / resident : 1;
-  p.tile_blocks = (int)((tiles + turns - 1) / turns);
-  if (per_tile * p.tile_blocks > lim || pixels * cc * p.gp > 0xffff ||
-      (long)p.gp * p.cols * k * k * cc > 0xffff)
-    return false;
-  const uintptr_t vec = 4 * (a.dtype == OGLE_F16 ? 2 : 4);
-  p.vec_x = a.in_c % 4 == 0 && cpg % 4 == 0 && cc % 4 == 0 && reinterpret_cast<uintptr_t>(a.input_dev) % vec == 0;
-  p.vec_w = cc == cpg && (k * k * cpg) % 4 == 0 && reinterpret_cast<uintptr_t>(a.filter_dev) % vec == 0;
-  p.d_cs = fast_div((int)(cc * p.gp));
-  p.d_pw = fast_div(p.pw);
-  p.d_ph = fast_div(p.ph);
-  p.d_runk = fast_div((int)(k * k * cc));
-  p.d_col = fast_div(std::min(p.cols, opg % p.cols == 0 ? p.cols : opg % p.cols));
-  *out = p;
-  return true;
 }
 
 template <typename T>

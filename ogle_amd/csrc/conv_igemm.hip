@@ -35,6 +35,7 @@
 #include <vector>
 
 #include "common.h"
+#include "conv_plan.h"
 
 namespace ogle {
 namespace {
@@ -1105,210 +1106,6 @@ __global__ __launch_bounds__(256) void splitk_reduce_group_kernel(ReduceGroup gr
   }
 }
 
-// Tile configurations (BM, BN, waves along M, waves along N).
-enum TileCfg {
-  CFG_128x128 = 0, CFG_64x64 = 1, CFG_128x32 = 2, CFG_WAVE32 = 3, CFG_WAVE16 = 4,
-  CFG_128x96 = 5, CFG_128x160 = 6,  // all output channels of a narrow, long-K problem in one tile
-  CFG_128x256 = 7,                   // fp16 storage: 64x128 per wave, 64-byte K slabs
-  CFG_128x16 = 8                     // at most 16 output channels: 16x16 MFMA blocks
-};
-constexpr int kCfgBM[] = {128, 64, 128, 32, 16, 128, 128, 128, 128};
-constexpr int kCfgBN[] = {128, 64, 32, 32, 16, 96, 160, 256, 16};
-constexpr int kRowBytesF16Wide = 64;  // K bytes per tile row per slab of CFG_128x256
-
-struct IgemmPlan {
-  int cfg;
-  int splits;
-  bool rows_on_xcd;  // split-K work layout: tile rows, not K ranges, pinned to an XCD
-  int slabs_per_split;
-  int ktiles;
-  int cchunks;
-  size_t workspace_bytes;  // splits * M * N floats when splits > 1
-  bool pieces;             // fp32 contracted as bf16 pieces
-};
-
-constexpr long kComputeUnits = 256;
-constexpr int kRowBytesF32 = 64;   // bytes of K per tile row per slab, fp32
-
-bool is_pointwise(const OgleConvArgs& a);
-bool is_wave(int cfg);
-
-// Picks the output tile and the K split.  Problems with few output
-// tiles but a long contraction (the SSD heads, the small feature maps) are split
-// along K until the grid fills the chip, provided a workspace was supplied.
-IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
-  IgemmPlan p{};
-  const int esz = a.dtype == OGLE_F16 ? 2 : 4;
-  const int rowb = a.dtype == OGLE_F16 ? 128 : kRowBytesF32;
-  const int epr = rowb / esz;
-  p.cchunks = (a.in_c + epr - 1) / epr;
-  p.ktiles = a.kernel_size * a.kernel_size * p.cchunks;
-  auto tiles = [&](int cfg) {
-    return ((m + kCfgBM[cfg] - 1) / kCfgBM[cfg]) * ((a.out_c + kCfgBN[cfg] - 1) / kCfgBN[cfg]);
-  };
-  // fp32 as bf16 pieces: a 128x128 tile splits and reads its operands from LDS half as often per
-  // product, a 64x64 tile quantises better over 256 units.  Measured on MI355X, us with 64x64 /
-  // 128x128 tiles: M = 11552, K = 512, N = 1024 (728 large tiles) 87 / 74, 6400 x 1024 x 1024
-  // (400) 103 / 85, 11552 x 256 x 512 (364) 26.6 / 26.4, 5776 x 512 x 512 (184) 26.5 / 28.2;
-  // with K = 128 even 704 large tiles are behind (28.8 / 30.3), 2813 are not (K = 64: 76 / 72).
-  // fp16 storage: an MFMA does sixteen times the work per operand byte, so the
-  // 64x64 tile is bound by LDS traffic and instruction issue; 128x128 pays off as soon
-  // as its tiles cover the compute units.
-  const long k_all = (long)a.kernel_size * a.kernel_size * a.in_c;
-  const long big_tiles_wanted = a.dtype == OGLE_F16 ? kComputeUnits
-                                : k_all >= 256      ? 3 * kComputeUnits / 2
-                                                    : 8 * kComputeUnits;
-  // A last tile column that is mostly padding costs more than that, in fp16 while K is short
-  // (12 x 57 x 57, 88 -> 168: 128x128 tiles 16.3 us, 64x64 11.2; 256 -> 168 19.0 / 14.1; 8 x 40 x 40,
-  // 88 -> 300 17.2 / 8.8; K = 792 17.2 / 17.4).
-  const bool big_columns_full = (a.dtype == OGLE_F16 && k_all > 512) ||
-                                ((a.out_c + 127) / 128) * 128 * 10 <= ((a.out_c + 63) / 64) * 64 * 11;
-  // A contraction of 128 slabs or more is cut along K below 2048 tiles (further down), which takes
-  // scratch memory.  Large tiles neither bring that on nor avoid it where the scratch a caller
-  // has to bring would differ: from 1024 of them on they are cut as well, with fewer they are taken
-  // only where the small tiles would not be cut.
-  const bool long_f32 = a.dtype == OGLE_F32 && p.ktiles >= 128;
-  const bool big_tiles = long_f32 ? tiles(CFG_128x128) >= 4 * kComputeUnits ||
-                                        (big_columns_full && tiles(CFG_128x128) >= big_tiles_wanted &&
-                                         tiles(CFG_64x64) >= 8 * kComputeUnits)
-                                  : big_columns_full && tiles(CFG_128x128) >= big_tiles_wanted;
-  // Narrow outputs with a long contraction (the SSD heads, box and class head of a feature
-  // map fused: 75 or 150 channels, K = 2304 ... 9216): one tile column holds every output
-  // channel, so the input is gathered once instead of once per 64-channel tile column, and
-  // 96 / 160 columns waste far less of the MFMA work than two or three 64-wide tiles.
-  const bool narrow_long = a.dtype == OGLE_F32 && p.ktiles >= 32 &&
-                           ((a.out_c > 64 && a.out_c <= 96) || (a.out_c > 128 && a.out_c <= 160));
-  if (narrow_long) {
-    p.cfg = a.out_c <= 96 ? CFG_128x96 : CFG_128x160;
-  } else if (a.dtype == OGLE_F16 && a.out_c >= 256 && tiles(CFG_128x256) >= 2 * kComputeUnits) {
-    // fp16 storage: one MFMA does sixteen times the work per operand byte, and a wave that
-    // owns 64x64 outputs reads its operands from LDS as fast as the MFMA pipe consumes them.
-    // A wave with 64x128 outputs reads a third less per MFMA and the tile pulls a quarter
-    // less from L2; 64-byte slabs keep two such workgroups per compute unit.  Measured on
-    // MI355X: M = 46208, K = N = 1024 gains 8 % (610 -> 662 TFLOP/s), but with fewer than two
-    // tiles per compute unit (M = 11552, N = 1024: 364 tiles) the second round is mostly
-    // empty and the 128x128 tile stays ahead (480 against 448 TFLOP/s).
-    p.cfg = CFG_128x256;
-    const int epr2 = kRowBytesF16Wide / esz;
-    p.cchunks = (a.in_c + epr2 - 1) / epr2;
-    p.ktiles = a.kernel_size * a.kernel_size * p.cchunks;
-  } else if (a.out_c <= 16) {
-    p.cfg = CFG_128x16;
-  } else if (a.out_c <= 32) {
-    p.cfg = CFG_128x32;
-  } else if (a.out_c > 64 && big_tiles) {
-    p.cfg = CFG_128x128;
-  } else {
-    p.cfg = CFG_64x64;
-  }
-  p.splits = 1;
-  const long t = tiles(p.cfg);
-  long sp = 1;
-  bool exact_split = false;  // sp was chosen by the search below: any count is fine
-  if (allow_split && narrow_long && t < 2 * kComputeUnits) {
-    // One tile column, few tile rows, a long K: the K split decides how evenly the chip is
-    // filled.  Workgroups are (tile, K range) pairs dealt to 256 compute units, each doing
-    // ceil(ktiles / s) slabs plus a fixed cost (first loads, epilogue: about `fixed` slabs);
-    // take the s with the shortest estimated time, partial-sum traffic as the tie break.
-    const double fixed = p.cfg == CFG_128x96 ? 6.0 : 4.0;
-    double best = 1e30;
-    for (long s = 1; s <= 64 && p.ktiles / s >= 8; ++s) {
-      const long rounds = (t * s + kComputeUnits - 1) / kComputeUnits;
-      const double cost = (double)rounds * ((double)((p.ktiles + s - 1) / s) + fixed) + 0.25 * (double)s;
-      if (cost < best - 1e-9) {
-        best = cost;
-        sp = s;
-      }
-    }
-    exact_split = true;
-  } else if (allow_split && 2 * t <= kComputeUnits && p.ktiles >= 8) {
-    // too few tiles to occupy every compute unit: about three workgroups per unit,
-    // at least four slabs per split
-    const long want = (3 * kComputeUnits + t - 1) / t;
-    const long most = p.ktiles / 4;
-    sp = want < most ? want : most;
-  } else if (allow_split && t < 8 * kComputeUnits && p.ktiles >= 128 &&
-             !(long_f32 && p.cfg == CFG_128x128 && t < 4 * kComputeUnits)) {
-    // a few long workgroups per unit quantise badly (one unit gets two, its
-    // neighbour one) and leave one wave per SIMD: cut the long contraction so that
-    // about eight shorter workgroups land on every unit, 32 slabs or more each
-    const long want = (8 * kComputeUnits + t - 1) / t;
-    const long most = p.ktiles / 32;
-    sp = want < most ? want : most;
-  }
-  if (sp > 64) sp = 64;
-  // the kernel's XCD-aware work layout wants a divisor or a multiple of 8
-  if (exact_split) {}
-  else if (sp >= 8) sp -= sp % 8;
-  else if (sp >= 4) sp = 4;
-  else if (sp >= 2) sp = 2;
-  if (sp >= 2) p.splits = (int)sp;
-  // A small contraction that would be split across workgroups goes to the wave-split
-  // kernel instead (the split stays inside the workgroup: no workspace, no second
-  // launch), whether or not a workspace was offered.  Measured on MI355X against
-  // split-K + reduce: the 32x32 form wins once its tiles cover half the chip, for
-  // K <= 1024 pointwise and K <= 512 otherwise; the 16x16 form wins for pointwise
-  // K <= 1024 while its tiles stay under two per compute unit, and for K <= 1536 while they
-  // stay under one per unit (3x3x256 <- 5x5x128 at batch 16: 7.0 against 9.5 us); a longer K
-  // per wave is a serial chain of MFMAs and loses to the split across workgroups.
-  {
-    const long k_total = (long)a.kernel_size * a.kernel_size * a.in_c;
-    const bool pw = is_pointwise(a);
-    const bool would_split = (2 * t <= kComputeUnits && p.ktiles >= 8) ||
-                             (t < 8 * kComputeUnits && p.ktiles >= 128);
-    const long t32 = tiles(CFG_WAVE32), t16 = tiles(CFG_WAVE16);
-    const bool small16 = (pw && k_total <= 1024 && t16 <= 2 * kComputeUnits) ||
-                         (k_total <= 1536 && t16 <= kComputeUnits);
-    // other than pointwise: K <= 512, or up to 2304 while every 32x32 tile has a compute unit
-    // to itself (5x5x512 <- 10x10x256, 3x3 stride 2, at batch 16: 19.8 against 21.6 us)
-    const long k32cap = t32 <= kComputeUnits ? 2304 : 512;
-    if (narrow_long) {
-      // stays on the wide tile
-    } else if (would_split && !small16 && k_total <= (pw ? 1024 : k32cap) && t32 >= kComputeUnits / 2 &&
-        t32 <= 4 * kComputeUnits) {
-      p.cfg = CFG_WAVE32;
-      p.splits = 1;
-    } else if (would_split && small16) {
-      p.cfg = CFG_WAVE16;
-      p.splits = 1;
-    }
-  }
-  p.slabs_per_split = (p.ktiles + p.splits - 1) / p.splits;
-  if (p.splits > 1) {
-    p.slabs_per_split += p.slabs_per_split & 1;  // the K loop runs slab pairs
-    p.splits = (p.ktiles + p.slabs_per_split - 1) / p.slabs_per_split;  // no empty ranges
-  }
-  // (a split past the end of K would only add zeros; rounding splits down keeps the
-  // divisor-or-multiple-of-8 shape, so empty splits are simply avoided by the cap above)
-  // partial sums are kept in rows of the channel count rounded up to four
-  p.workspace_bytes =
-      p.splits > 1 ? (size_t)p.splits * (size_t)m * ((a.out_c + 3) & ~3) * sizeof(float) : 0;
-  // Tiles of 32x32 MFMA blocks are contracted as bf16 pieces (but for the single-column tiles of
-  // the two-destination form) once they give a compute unit more than one workgroup.  A lone
-  // workgroup has nothing to cover the splitting with: 112x112x32 -> 64 3x3 (196 tiles) 11.1 us
-  // with fp32 MFMAs, 11.9 with pieces; 3703 x 88 x 168 (174) 6.3 / 6.9; 1600 x 512 x 1024 (400)
-  // 22.8 / 20.4.
-  p.pieces = a.dtype == OGLE_F32 && (p.cfg == CFG_128x128 || p.cfg == CFG_64x64 || p.cfg == CFG_128x32) &&
-             tiles(p.cfg) * p.splits > kComputeUnits;
-  // Which operand an XCD's L2 should keep to itself: with K ranges pinned to XCDs the input is
-  // fetched by all eight L2s and the filter by one, with tile rows pinned it is the other way
-  // round (the rocprofv3 FETCH_SIZE of the 19x19x512 class head fell from 8.5x its input to
-  // about the input plus eight filters).
-  {
-    const long x_bytes = (long)a.n * a.in_h * a.in_w * a.in_c * esz;
-    const long w_bytes = (long)a.out_c * a.kernel_size * a.kernel_size * a.in_c * esz;
-    // whole tile rows per XCD: only when they spread evenly (within a tenth) over the eight
-    const long tiles_m = (m + kCfgBM[p.cfg] - 1) / kCfgBM[p.cfg];
-    const bool even = ((tiles_m + 7) / 8) * 8 * 10 <= tiles_m * 11;
-    p.rows_on_xcd = p.splits > 1 && !is_wave(p.cfg) && x_bytes > w_bytes && even;
-  }
-  return p;
-}
-
-bool is_wave(int cfg) { return cfg == CFG_WAVE32 || cfg == CFG_WAVE16; }
-int tile_bm(int cfg) { return kCfgBM[cfg]; }
-int tile_bn(int cfg) { return kCfgBN[cfg]; }
-
 // Grid size of one problem under the kernel's XCD-aware work layout.
 unsigned grid_blocks(const IgemmPlan& p, int tiles_m, int tiles_n) {
   const int tiles = tiles_m * tiles_n;
@@ -1317,33 +1114,6 @@ unsigned grid_blocks(const IgemmPlan& p, int tiles_m, int tiles_n) {
   if (p.splits != 2 && p.splits != 4) return (unsigned)tiles * (unsigned)p.splits;
   const int xpz = 8 / p.splits;
   return 8u * (unsigned)((tiles + xpz - 1) / xpz);
-}
-
-bool igemm_eligible(const OgleConvArgs& a, long* m_out) {
-  if (a.group != 1) return false;
-  const int ve = a.dtype == OGLE_F16 ? 8 : 4;
-  if (a.in_c % ve != 0) return false;
-  if ((long)a.kernel_size * a.kernel_size * a.in_c < 32) return false;
-  const long m = (long)a.n * a.out_h * a.out_w;
-  if (m <= 0 || m > 0x7fffffffL) return false;
-  // operands are addressed with 32-bit byte offsets through buffer loads
-  const long esz = a.dtype == OGLE_F16 ? 2 : 4;
-  const long lim = 0x7fffffffL;
-  if ((long)a.n * a.in_h * a.in_w * a.in_c * esz > lim) return false;
-  if ((long)a.out_c * a.kernel_size * a.kernel_size * a.in_c * esz > lim) return false;
-  *m_out = m;
-  return true;
-}
-
-bool is_pointwise(const OgleConvArgs& a) {
-  return a.kernel_size == 1 && a.stride == 1 && a.padding == 0;
-}
-
-// The plan the launch will use: split-K only with a workspace that is large enough.
-IgemmPlan final_plan(const OgleConvArgs& a, long m) {
-  IgemmPlan p = plan_igemm(a, m, a.workspace_dev != nullptr);
-  if (p.workspace_bytes > a.workspace_bytes) p = plan_igemm(a, m, false);
-  return p;
 }
 
 struct Prepared {
