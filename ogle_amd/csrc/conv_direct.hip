@@ -325,6 +325,7 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
                                                        const float* __restrict__ bias, T* __restrict__ y,
                                                        DirectGeom q, PatchPlan p, Epilogue ep) {
   extern __shared__ __attribute__((aligned(16))) float patch_lds[];
+  __shared__ int filter_not_finite;
   constexpr int MB = COLS == 16 ? 16 : 32;            // MFMA block
   constexpr int FR = 32 / MB;                         // blocks along a wave's 32 pixels
   constexpr int NB = COLS / MB;                       // blocks along the columns
@@ -365,7 +366,11 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
     pix_off[f] = tb * img_pitch + (ty * row_pitch + tx * p.pitch) * p.box_step;
   }
 
-  bool bad = false;   // an infinite or NaN filter value has been staged
+  // `bad`: this thread has staged an infinite or NaN filter value; `repair`: some thread of the
+  // workgroup has, known to all of them before the first output is stored, so that every output
+  // is stored once, either contracted or, below, one by one (by whichever wave its index falls to)
+  bool bad = false, repair = false;
+  if (tid == 0) filter_not_finite = 0;
   for (int tile = tblock; tile < tiles; tile += p.tile_blocks) {
     const int bx = tile % p.tiles_x;
     const int rest = tile / p.tiles_x;
@@ -376,7 +381,7 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
     // with gp > 1 all channels are staged at once: only one of the two loops below has more
     // than one turn, and one set of accumulators serves both
     Acc acc[FR][NB];
-    for (int c0 = 0; c0 < cpg; c0 += p.cc) {
+    for (int c0 = repair ? cpg : 0; c0 < cpg; c0 += p.cc) {
       const int cc = min(p.cc, cpg - c0);
       const int cs = p.gp > 1 ? groups_here * cpg : cc;   // channels per patch pixel this time
       // the last chunk and the last group block are narrower than the divisors the host prepared
@@ -455,8 +460,13 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
         };
         if (p.vec_w) stage(std::integral_constant<int, 4>());
         else stage(std::integral_constant<int, 1>());
+        if (bad) filter_not_finite = 1;
       }
       __syncthreads();
+      if (c0 + p.cc >= cpg && filter_not_finite != 0) {   // the whole filter has been seen
+        repair = true;
+        break;
+      }
 
       const int len = p.runs_x == 1 ? q.k * cc : cc;    // values per run
       for (int gi = 0; gi < groups_here; ++gi) {
@@ -547,8 +557,7 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
       }
     }
 
-    if (tile == tblock) bad = __syncthreads_or(bad) != 0;   // (in chunks: one box per workgroup)
-    if (bad) {
+    if (repair) {
       const int per_pixel = groups_here * cols_here;
       for (int i = tid; i < kPatchPixels * per_pixel; i += 256) {
         const int pix = i / per_pixel, rest2 = i - pix * per_pixel;

@@ -1,0 +1,35 @@
+// The convolution dispatch rules, for test_conv_plan_cpu.py: compiled on the spot by the host
+// compiler, loaded with ctypes.
+#include "conv_plan.h"
+
+using namespace ogle;
+
+extern "C" {
+
+// 1 if the patch kernel takes the convolution (once the implicit GEMM and the stem kernels have
+// not), then out = columns, groups and channels staged at once, K runs per filter row, boxes,
+// workgroups along the boxes, workgroups in all, vector staging of patch and filter, LDS floats.
+int probe_patch(const OgleConvArgs* a, int64_t* out) {
+  PatchPlan p;
+  long m = 0;
+  if (igemm_eligible(*a, &m) || !plan_patch(*a, &p)) return 0;
+  const int64_t boxes = (int64_t)p.tiles_b * p.tiles_y * p.tiles_x;
+  const int64_t v[] = {p.cols, p.gp, p.cc, p.runs_x, boxes, p.tile_blocks,
+                       (int64_t)p.tile_blocks * p.gblocks * p.col_blocks, p.vec_x, p.vec_w, p.lds_floats};
+  for (int i = 0; i < 10; ++i) out[i] = v[i];
+  return 1;
+}
+
+// 1 if the implicit GEMM takes the convolution, then out = rows and columns of the tile, tiles,
+// K ranges, whether fp32 is contracted as bf16 pieces, workspace bytes.
+int probe_igemm(const OgleConvArgs* a, int scratch, int64_t* out) {
+  long m = 0;
+  if (!igemm_eligible(*a, &m)) return 0;
+  const IgemmPlan p = plan_igemm(*a, m, scratch != 0);
+  const int bm = tile_bm(p.cfg), bn = tile_bn(p.cfg);
+  const int64_t v[] = {bm, bn, (int64_t)((m + bm - 1) / bm) * ((a->out_c + bn - 1) / bn),
+                       p.splits, p.pieces, (int64_t)p.workspace_bytes};
+  for (int i = 0; i < 6; ++i) out[i] = v[i];
+  return 1;
+}
+}

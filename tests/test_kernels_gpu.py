@@ -168,21 +168,34 @@ def test_conv_patch_kernel(case, dtype):
                variant=H.VARIANT_ANY4 if g > 1 else H.VARIANT_NHWC4, what=str(case))
 
 
-def test_conv_patch_kernel_infinite_filter_values_meet_no_padding():
+INFINITE_FILTER_CASES = [
+    # n, h, w, c, o, k, s, p, g
+    (2, 20, 18, 24, 36, 3, 1, 1, 3),        # one box per workgroup, all channels staged at once
+    (1, 17, 16, 130, 20, 3, 1, 1, 1),       # channels in chunks
+    (16, 57, 43, 96, 144, 3, 1, 1, 12),     # several groups and several boxes per workgroup
+    (8, 224, 222, 3, 64, 7, 2, 3, 1),       # several boxes, merged runs, 64 columns
+]
+
+
+@pytest.mark.parametrize("case", INFINITE_FILTER_CASES)
+def test_conv_patch_kernel_infinite_filter_values_meet_no_padding(case):
     """Taps outside the image are skipped, not multiplied by zero: an infinite or NaN filter value
-    reaches exactly the outputs it reaches in the oracle, in chunked and whole staging alike."""
-    for n, h, w, c, o, k, g in ((2, 20, 18, 24, 36, 3, 3), (1, 17, 16, 130, 20, 3, 1)):
-        r = rng(2950 + c)
-        x = r.uniform(0.5, 1, (n, h, w, c)).astype(np.float32)
-        wt = r.normal(0, 0.5, (o, c // g, k, k)).astype(np.float32)
-        wt[3, 5, 0, 0] = np.inf
-        wt[o - 1, 1, 2, 1] = -np.inf
-        wt[7, 2, 1, 0] = np.nan
-        ref = O.conv2d(x, wt, None, 1, 1, 1, g, O.ACT_NONE, 0.0, 0.0, O.VARIANT_NHWC4)
-        got = gpu_conv(x, wt, None, 1, 1, 1, g, H.ACT_NONE, entry="ogle_hip_conv2d")
-        assert np.isfinite(ref[:, 0, 0, 3]).all()    # its only infinite tap lies in the padding
-        np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
-        np.testing.assert_array_equal(got[~np.isfinite(ref)], ref[~np.isfinite(ref)])
+    reaches exactly the outputs it reaches in the oracle, in every box of a workgroup."""
+    n, h, w, c, o, k, s, p, g = case
+    r = rng(2950 + c)
+    x = r.uniform(0.5, 1, (n, h, w, c)).astype(np.float32)
+    wt = r.normal(0, 0.5, (o, c // g, k, k)).astype(np.float32)
+    wt[3, 2, 0, 0] = np.inf
+    wt[o - 1, 1, 2, 1] = -np.inf
+    wt[7, 2, 1, 0] = np.nan
+    ref = O.conv2d(x, wt, None, s, p, 1, g, O.ACT_NONE, 0.0, 0.0, O.VARIANT_NHWC4)
+    got = gpu_conv(x, wt, None, s, p, 1, g, H.ACT_NONE, entry="ogle_hip_conv2d")
+    assert np.isfinite(ref[:, 0, 0, 3]).all()    # its only infinite tap lies in the padding
+    np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
+    np.testing.assert_array_equal(got[~np.isfinite(ref)], ref[~np.isfinite(ref)])
+    scale = O.conv2d_abs(x, np.where(np.isfinite(wt), wt, 0), None, s, p, 1, g)
+    ok = np.isfinite(ref)
+    assert np.max(np.abs(got[ok] - ref[ok]) / scale[ok]) <= FP32_RTOL
 
 
 @pytest.mark.parametrize("o,c", [(168, 88), (192, 64), (193, 40), (300, 72), (168, 520)])
