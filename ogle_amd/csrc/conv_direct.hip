@@ -326,6 +326,7 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
                                                        DirectGeom q, PatchPlan p, Epilogue ep) {
   extern __shared__ __attribute__((aligned(16))) float patch_lds[];
   __shared__ int filter_not_finite;
+  static_assert(sizeof(filter_not_finite) <= kPatchStaticLds, "the plan leaves room for it");
   constexpr int MB = COLS == 16 ? 16 : 32;            // MFMA block
   constexpr int FR = 32 / MB;                         // blocks along a wave's 32 pixels
   constexpr int NB = COLS / MB;                       // blocks along the columns

@@ -266,6 +266,7 @@ struct PatchPlan {
 };
 
 constexpr int kPatchPixels = 128;
+constexpr int kPatchStaticLds = 16;   // bytes of LDS the kernel has beside the plan's lds_floats
 
 // The patch kernel's box, chunk and grid for a convolution; false if it does not take it.
 inline bool plan_patch(const OgleConvArgs& a, PatchPlan* out) {
@@ -321,12 +322,14 @@ inline bool plan_patch(const OgleConvArgs& a, PatchPlan* out) {
   const long wp = p.cols + 1;
   if (pixels > 0xffff) return false;
   // channels staged at once: all of them, or the most that leave three workgroups per unit
-  // (48 KB of LDS each); 64 KB, the launch limit, where the grid gives a unit no third one
-  // anyway (fewer, longer chunks: each costs a round trip to memory) or nothing less will do
+  // (48 KB of LDS each); 64 KB, what a launch may ask for, static part included, where the grid
+  // gives a unit no third one anyway (fewer, longer chunks: each costs a round trip to memory) or
+  // nothing less will do
   const bool roomy = tiles * a.group * p.col_blocks <= 512;
   auto floats = [&](long cc, long gp) { return pixels * ((cc * gp) | 1) + gp * k * k * cc * wp; };
+  const long most = (64L * 1024 - kPatchStaticLds) / 4;
   long cc = 0;
-  for (const long budget : {roomy ? 16384L : 12288L, 16384L}) {
+  for (const long budget : {roomy ? most : 12288L, most}) {
     if (floats(cpg, 1) <= budget) cc = cpg;
     else
       for (long t : {64L, 32L, 16L, 8L, 4L, 2L})
@@ -351,7 +354,7 @@ inline bool plan_patch(const OgleConvArgs& a, PatchPlan* out) {
   const long per_tile = (long)p.gblocks * p.col_blocks;
   // with all channels staged at once the filter stays in LDS while a workgroup walks boxes
   // (no more workgroups than their LDS lets be resident, each with as many boxes as any other)
-  const long resident = 256 * (40L * 1024 / p.lds_floats);
+  const long resident = 256 * (160L * 1024 / (4 * p.lds_floats + kPatchStaticLds));
   const long turns = cc == cpg ? (tiles * per_tile + resident - 1) / resident : 1;
   p.tile_blocks = (int)((tiles + turns - 1) / turns);
   if (per_tile * p.tile_blocks > lim || pixels * cc * p.gp > 0xffff ||

@@ -2,7 +2,9 @@
 the host: the plans stay inside what the kernels and a launch can hold, and the cases of the GPU
 tests run the code they name."""
 import ctypes
+import math
 import os
+import random
 import subprocess
 
 import pytest
@@ -46,3 +48,31 @@ def test_infinite_filter_cases_walk_several_boxes(probe):
     assert plans[1]["cc"] < 130
     assert plans[2]["gp"] > 1
     assert plans[3]["runs"] == 1 and plans[3]["cols"] == 64
+
+
+def random_direct(r):
+    """A convolution as the direct kernels may meet it, of any form; None if it has no output."""
+    g = r.choice([1, 1, 2, 3, 5, 8, 12, 32])
+    k, d, s = r.choice([1, 1, 3, 3, 5, 7, 11]), r.choice([1, 1, 1, 2, 3]), r.choice([1, 1, 2, 3, 4])
+    log = lambda lo, hi: int(round(math.exp(r.uniform(math.log(lo), math.log(hi)))))    # noqa: E731
+    h, w, p = log(1, 300), log(1, 300), r.choice([0, k // 2, k // 2, k])
+    if h + 2 * p < (k - 1) * d + 1 or w + 2 * p < (k - 1) * d + 1:
+        return None
+    return (log(1, 100), h, w, g * log(1, 200), g * log(1, 200), k, s, p, d, g)
+
+
+def test_patch_plan_stays_within_lds(probe):
+    """A workgroup's dynamic LDS and the kernel's own 16 bytes are at most the 64 KB that a launch
+    may ask for; the two pinned shapes fill them but for a few words."""
+    for n, h, w, c, o, k, st, p, d, g in K.FULL_LDS_CASES:
+        plan = patch_plan(probe, n, h, w, c, o, k, st, p, d, g)
+        assert plan is not None and 4 * plan["lds_floats"] + 16 <= 65536
+    r, taken, largest = random.Random(5), 0, 0
+    for _ in range(20000):
+        shape = random_direct(r)
+        plan = shape and patch_plan(probe, *shape, dtype=r.choice([H.F32, H.F16]))
+        if plan:
+            taken += 1
+            largest = max(largest, plan["lds_floats"])
+            assert 4 * plan["lds_floats"] + 16 <= 65536, shape
+    assert taken > 5000 and largest > 16000

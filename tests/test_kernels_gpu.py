@@ -152,12 +152,18 @@ PATCH_CASES = [
     (1, 20, 20, 64, 64, 11, 1, 5, 1, 2),    # 11x11: a few channels at a time
 ]
 
+FULL_LDS_CASES = [
+    # n, h, w, c, o, k, s, p, d, g   as much LDS as a launch may ask for
+    (8, 74, 74, 54, 96, 3, 2, 1, 1, 3),     # 18 channels of a group at once: 65,312 bytes
+    (4, 55, 42, 72, 180, 3, 1, 1, 3, 4),    # all 18 would be 65,528, and the kernel's own do not fit beside
+]
 
-@pytest.mark.parametrize("case", PATCH_CASES)
+
+@pytest.mark.parametrize("case", PATCH_CASES + FULL_LDS_CASES)
 @pytest.mark.parametrize("dtype", [H.F32, H.F16])
 def test_conv_patch_kernel(case, dtype):
     n, h, w, c, o, k, s, p, d, g = case
-    r = rng(2900 + PATCH_CASES.index(case))
+    r = rng(2900 + (PATCH_CASES + FULL_LDS_CASES).index(case))
     x = r.uniform(-1, 1, (n, h, w, c)).astype(np.float32)
     wt = r.normal(0, 0.5, (o, c // g, k, k)).astype(np.float32)
     b = r.uniform(-0.1, 0.1, o).astype(np.float32)
