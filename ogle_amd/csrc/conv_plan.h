@@ -357,7 +357,8 @@ inline bool plan_patch(const OgleConvArgs& a, PatchPlan* out) {
   const long resident = 256 * (160L * 1024 / (4 * p.lds_floats + kPatchStaticLds));
   const long turns = cc == cpg ? (tiles * per_tile + resident - 1) / resident : 1;
   p.tile_blocks = (int)((tiles + turns - 1) / turns);
-  if (per_tile * p.tile_blocks > lim || pixels * cc * p.gp > 0xffff ||
+  // (a launch holds fewer than 2^32 threads: a one-channel output of 8 GB in 128-pixel boxes does not fit)
+  if (per_tile * p.tile_blocks * 256 > 0xffffffffL || pixels * cc * p.gp > 0xffff ||
       (long)p.gp * p.cols * k * k * cc > 0xffff)
     return false;
   const uintptr_t vec = 4 * (a.dtype == OGLE_F16 ? 2 : 4);

@@ -76,3 +76,11 @@ def test_patch_plan_stays_within_lds(probe):
             largest = max(largest, plan["lds_floats"])
             assert 4 * plan["lds_floats"] + 16 <= 65536, shape
     assert taken > 5000 and largest > 16000
+
+
+def test_patch_plan_stays_within_a_launch(probe):
+    """Fewer than 2^32 threads.  The pinned shape, a 1x1 convolution of a padded map whose channels are
+    staged in chunks, has one box per workgroup and more of them than that."""
+    assert patch_plan(probe, 1, 1000, 1000, 511, 1, 1, 1, 22669) is None
+    plan = patch_plan(probe, 1, 1000, 1000, 511, 1, 1, 1, 2000)
+    assert plan["cc"] < 511 and plan["boxes"] == plan["blocks"] and plan["blocks"] * 256 < 2 ** 32
