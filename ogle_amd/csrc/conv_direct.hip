@@ -639,7 +639,7 @@ int32_t run_direct(const OgleConvArgs& a, hipStream_t s) {
     return check_launch("conv_stem_mfma");
   }
   PatchPlan plan;
-  if (plan_patch(a, &plan)) return launch_patch<T>(a, plan, ep, s);
+  if (plan_direct(a, &plan) == DIRECT_PATCH) return launch_patch<T>(a, plan, ep, s);
   const long total = (long)a.n * a.out_h * a.out_w * a.out_c;
   int blocks = ceil_div(total, 256);
   if (blocks > 256 * 64) blocks = 256 * 64;

@@ -373,6 +373,31 @@ inline bool plan_patch(const OgleConvArgs& a, PatchPlan* out) {
   return true;
 }
 
+// Whether a planned patch is worth it.  One thread per output is bound by its chain of products
+// while threads are few and by their number when they are many; the patch kernel by staging patch
+// and filter.  Both lines are fits of 1523 shapes (1 to 32 groups, 1x1 and 3x3, up to 100,000
+// pixels; the faster of the two each time would be 0.7 % faster on average).  Us with one thread per
+// output / with the patch kernel, 3x3 except as noted: 1 x 1, 17 -> 33 3.9 / 29.7; 4 x 4, 12 groups
+// of 16 -> 16 19.7 / 8.8; 14 x 14, 7 -> 33 8.7 / 9.4, 17 -> 33 18.7 / 13.0, 33 -> 33 35 / 18, with
+// stride 2 35 / 35; 56 x 56, 1x1 35 -> 33 7.4 / 11.4, 35 -> 75 12.1 / 11.6, 131 -> 33 23.8 / 26,
+// 131 -> 75 43 / 26; 4 x 56 x 56, 1x1, 4 groups of 8 -> 12 11.9 / 8.0.
+inline bool patch_pays(const OgleConvArgs& a, const PatchPlan& p) {
+  const int cpg = a.in_c / a.group, k = a.kernel_size;
+  // products of an output, without taps that can only lie in the padding of a small map
+  const double chain = (double)cpg * std::min(k, (a.in_h - 1) / a.dilation + 1) *
+                       std::min(k, (a.in_w - 1) / a.dilation + 1);
+  const double staged = (double)p.lds_floats * ((cpg + p.cc - 1) / p.cc);   // values, all chunks
+  const double staging = p.vec_x ? 1000 + staged / 2 : 9000 + staged;
+  const double outputs = (double)a.n * a.out_h * a.out_w * a.out_c;
+  return chain >= 0.006 * staging || outputs * chain > (p.vec_x ? 4.5e6 : 6e6);
+}
+
+// The kernel for a convolution that neither the implicit GEMM nor the stem kernels take.
+enum DirectKernel { DIRECT_GENERAL, DIRECT_PATCH };
+inline DirectKernel plan_direct(const OgleConvArgs& a, PatchPlan* plan) {
+  return plan_patch(a, plan) && patch_pays(a, *plan) ? DIRECT_PATCH : DIRECT_GENERAL;
+}
+
 }  // namespace ogle
 
 #endif  // OGLE_CSRC_CONV_PLAN_H_

@@ -12,7 +12,7 @@ extern "C" {
 int probe_patch(const OgleConvArgs* a, int64_t* out) {
   PatchPlan p;
   long m = 0;
-  if (igemm_eligible(*a, &m) || !plan_patch(*a, &p)) return 0;
+  if (igemm_eligible(*a, &m) || plan_direct(*a, &p) != DIRECT_PATCH) return 0;
   const int64_t boxes = (int64_t)p.tiles_b * p.tiles_y * p.tiles_x;
   const int64_t v[] = {p.cols, p.gp, p.cc, p.runs_x, boxes, p.tile_blocks,
                        (int64_t)p.tile_blocks * p.gblocks * p.col_blocks, p.vec_x, p.vec_w, p.lds_floats};

@@ -84,3 +84,19 @@ def test_patch_plan_stays_within_a_launch(probe):
     assert patch_plan(probe, 1, 1000, 1000, 511, 1, 1, 1, 22669) is None
     plan = patch_plan(probe, 1, 1000, 1000, 511, 1, 1, 1, 2000)
     assert plan["cc"] < 511 and plan["boxes"] == plan["blocks"] and plan["blocks"] * 256 < 2 ** 32
+
+
+@pytest.mark.parametrize("shape,patch", [
+    # n, h, w, c, o, k, s, p, d, g: next to the line on both sides, as measured (conv_plan.h)
+    ((1, 1, 1, 17, 33, 3, 1, 1), False),            # eight of nine taps lie in the padding
+    ((1, 4, 4, 192, 192, 3, 1, 1, 1, 12), True),
+    ((1, 14, 14, 7, 33, 3, 1, 1), False),
+    ((1, 14, 14, 17, 33, 3, 1, 1), True),
+    ((1, 56, 56, 35, 33, 1), False),
+    ((1, 56, 56, 35, 75, 1), True),
+    ((1, 28, 28, 131, 33, 1), False),
+    ((4, 56, 56, 32, 48, 1, 1, 0, 1, 4), True),
+    ((4, 57, 43, 96, 144, 3, 1, 1, 1, 12), True),
+])
+def test_patch_kernel_where_it_is_faster(probe, shape, patch):
+    assert (patch_plan(probe, *shape) is not None) == patch
