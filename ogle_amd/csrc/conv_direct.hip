@@ -1,8 +1,9 @@
 // Direct convolution over NHWC: everything the MFMA implicit-GEMM kernels do not take (channel
-// counts that fill no 16-byte vector, grouped convolutions, the RGB stem).  Three kernels:
+// counts that fill no 16-byte vector, grouped convolutions, the RGB stem).  Four kernels:
 // conv_stem_* (K = k*k*C <= 32, group 1), conv_patch_mfma (input patch and filter staged in
-// LDS, contracted on the MFMA units) and conv_direct_general (one thread per output, for what
-// neither takes: patches that do not fit LDS, groups too small for an MFMA block).
+// LDS, contracted on the MFMA units), conv_direct_small_k (group 1, the filter in LDS, one thread
+// per 4 or 16 channels of a pixel) and conv_direct_general (one thread per output).  plan_direct
+// chooses among the last three.
 //
 // Semantics follow conv2d.glsl:29-92 / conv2d_grp.glsl:30-123: bias, taps outside the image
 // contribute nothing, then the fused activation.
@@ -13,6 +14,72 @@
 
 namespace ogle {
 namespace {
+
+// Small-K kernel: one thread produces OPT consecutive output channels of one pixel.  Filter taps
+// [O][K] (K = k*k*C, OHWI order) are staged through LDS transposed to [K][O]; a wave then reads
+// the OPT weights of one (tap, channel) as 16-byte broadcasts, and each input value is loaded once
+// per thread.  O must be a multiple of OPT.  Bound by its chain of K products (about 0.08 us each)
+// while threads are few; plan_direct says which shapes it is for, and what they measured.
+template <typename T, int OPT>
+__global__ __launch_bounds__(256) void conv_direct_small_k(
+    const T* __restrict__ x, const T* __restrict__ w, const float* __restrict__ bias,
+    T* __restrict__ y, int n, int h, int wd, int c, int oh, int ow, int o, int k, int stride,
+    int pad, int dil, Epilogue ep, int ktot) {
+  extern __shared__ __attribute__((aligned(16))) float lds_w[];  // [ktot][o]
+  for (int i = threadIdx.x; i < ktot * o; i += blockDim.x) {
+    int oc = i / ktot, kk = i - oc * ktot;
+    lds_w[kk * o + oc] = to_f32(w[i]);
+  }
+  __syncthreads();
+  const int groups_per_pixel = o / OPT;
+  const long total = (long)n * oh * ow * groups_per_pixel;
+  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
+       idx += (long)gridDim.x * blockDim.x) {
+    const int og = (int)(idx % groups_per_pixel);
+    long pix = idx / groups_per_pixel;
+    const int ox = (int)(pix % ow);
+    pix /= ow;
+    const int oy = (int)(pix % oh);
+    const int b = (int)(pix / oh);
+    const int oc0 = og * OPT;
+    float acc[OPT];
+#pragma unroll
+    for (int j = 0; j < OPT; ++j) acc[j] = bias != nullptr ? bias[oc0 + j] : 0.f;
+    for (int r = 0; r < k; ++r) {
+      const int iy = oy * stride - pad + r * dil;
+      if (iy < 0 || iy >= h) continue;
+      for (int s = 0; s < k; ++s) {
+        const int ix = ox * stride - pad + s * dil;
+        if (ix < 0 || ix >= wd) continue;
+        const T* xp = x + (((long)b * h + iy) * wd + ix) * c;
+        const float* wp = lds_w + (long)((r * k + s) * c) * o + oc0;
+        for (int ci = 0; ci < c; ++ci) {
+          const float xv = to_f32(xp[ci]);
+          const float4* w4 = reinterpret_cast<const float4*>(wp + ci * o);
+#pragma unroll
+          for (int j = 0; j < OPT / 4; ++j) {
+            const float4 wv = w4[j];
+            acc[4 * j + 0] += xv * wv.x;
+            acc[4 * j + 1] += xv * wv.y;
+            acc[4 * j + 2] += xv * wv.z;
+            acc[4 * j + 3] += xv * wv.w;
+          }
+        }
+      }
+    }
+    T* yp = y + (((long)b * oh + oy) * ow + ox) * o + oc0;
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int j = 0; j < OPT / 4; ++j)
+        reinterpret_cast<float4*>(yp)[j] =
+            make_float4(apply_epilogue(acc[4 * j], ep), apply_epilogue(acc[4 * j + 1], ep),
+                        apply_epilogue(acc[4 * j + 2], ep), apply_epilogue(acc[4 * j + 3], ep));
+    } else {
+#pragma unroll
+      for (int j = 0; j < OPT; ++j) yp[j] = from_f32<T>(apply_epilogue(acc[j], ep));
+    }
+  }
+}
 
 // Stem kernel: few input channels, K = k*k*C <= 32 (the RGB stem has K = 27), on
 // the MFMA units.  A wave owns 32 output pixels x 32 output channels at a time and
@@ -639,7 +706,26 @@ int32_t run_direct(const OgleConvArgs& a, hipStream_t s) {
     return check_launch("conv_stem_mfma");
   }
   PatchPlan plan;
-  if (plan_direct(a, &plan) == DIRECT_PATCH) return launch_patch<T>(a, plan, ep, s);
+  const DirectKernel kernel = plan_direct(a, &plan);
+  if (kernel == DIRECT_PATCH) return launch_patch<T>(a, plan, ep, s);
+  if (kernel == DIRECT_SMALL_K) {
+    const bool wide = small_k_is_wide(a);
+    const size_t lds = sizeof(float) * (size_t)ktot * a.out_c;
+    const long total = pixels_all * (a.out_c / (wide ? 16 : 4));
+    int blocks = ceil_div(total, 256);
+    if (blocks > 256 * 32) blocks = 256 * 32;
+    if (blocks < 1) blocks = 1;
+    if (wide) {
+      launch((conv_direct_small_k<T, 16>), dim3(blocks), dim3(256), lds, s, x, w, a.bias_dev, y,
+             a.n, a.in_h, a.in_w, a.in_c, a.out_h, a.out_w, a.out_c, a.kernel_size, a.stride,
+             a.padding, a.dilation, ep, ktot);
+    } else {
+      launch((conv_direct_small_k<T, 4>), dim3(blocks), dim3(256), lds, s, x, w, a.bias_dev, y,
+             a.n, a.in_h, a.in_w, a.in_c, a.out_h, a.out_w, a.out_c, a.kernel_size, a.stride,
+             a.padding, a.dilation, ep, ktot);
+    }
+    return check_launch("conv_direct_small_k");
+  }
   const long total = (long)a.n * a.out_h * a.out_w * a.out_c;
   int blocks = ceil_div(total, 256);
   if (blocks > 256 * 64) blocks = 256 * 64;

@@ -373,6 +373,19 @@ inline bool plan_patch(const OgleConvArgs& a, PatchPlan* out) {
   return true;
 }
 
+// Products of an output that follow each other, without taps that can only lie in the padding of a
+// small map.
+inline double direct_chain(const OgleConvArgs& a) {
+  const int k = a.kernel_size;
+  return (double)(a.in_c / a.group) * std::min(k, (a.in_h - 1) / a.dilation + 1) *
+         std::min(k, (a.in_w - 1) / a.dilation + 1);
+}
+// Values a workgroup of the patch kernel stages, all chunks of channels.
+inline double patch_staged(const OgleConvArgs& a, const PatchPlan& p) {
+  const int cpg = a.in_c / a.group;
+  return (double)p.lds_floats * ((cpg + p.cc - 1) / p.cc);
+}
+
 // Whether a planned patch is worth it.  One thread per output is bound by its chain of products
 // while threads are few and by their number when they are many; the patch kernel by staging patch
 // and filter.  Both lines are fits of 1523 shapes (1 to 32 groups, 1x1 and 3x3, up to 100,000
@@ -382,20 +395,56 @@ inline bool plan_patch(const OgleConvArgs& a, PatchPlan* out) {
 // stride 2 35 / 35; 56 x 56, 1x1 35 -> 33 7.4 / 11.4, 35 -> 75 12.1 / 11.6, 131 -> 33 23.8 / 26,
 // 131 -> 75 43 / 26; 4 x 56 x 56, 1x1, 4 groups of 8 -> 12 11.9 / 8.0.
 inline bool patch_pays(const OgleConvArgs& a, const PatchPlan& p) {
-  const int cpg = a.in_c / a.group, k = a.kernel_size;
-  // products of an output, without taps that can only lie in the padding of a small map
-  const double chain = (double)cpg * std::min(k, (a.in_h - 1) / a.dilation + 1) *
-                       std::min(k, (a.in_w - 1) / a.dilation + 1);
-  const double staged = (double)p.lds_floats * ((cpg + p.cc - 1) / p.cc);   // values, all chunks
-  const double staging = p.vec_x ? 1000 + staged / 2 : 9000 + staged;
+  const double staging = p.vec_x ? 1000 + patch_staged(a, p) / 2 : 9000 + patch_staged(a, p);
   const double outputs = (double)a.n * a.out_h * a.out_w * a.out_c;
-  return chain >= 0.006 * staging || outputs * chain > (p.vec_x ? 4.5e6 : 6e6);
+  return direct_chain(a) >= 0.006 * staging || outputs * direct_chain(a) > (p.vec_x ? 4.5e6 : 6e6);
+}
+
+// The kernel with the filter in LDS, one thread per four channels of a pixel, or per sixteen (wide)
+// where that still leaves enough threads to fill the chip.
+inline bool small_k_fits(const OgleConvArgs& a) {
+  return a.group == 1 && a.out_c % 4 == 0 && 4L * a.kernel_size * a.kernel_size * a.in_c * a.out_c <= 48 * 1024;
+}
+inline bool small_k_is_wide(const OgleConvArgs& a) {
+  return a.out_c % 16 == 0 && (long)a.n * a.out_h * a.out_w * (a.out_c / 16) >= 256L * 256 * 4;
+}
+
+// The patch kernel against that one: the chain of products against staging again; many products
+// (a wide thread's cost a quarter; every workgroup stages the whole filter, which counts with the
+// channels); inputs beyond the L2s, of which a wave reads a cache line per pixel and value.  Fits of
+// 1426 shapes (the faster each time would be 1.1 % faster on average); us with that kernel / with the
+// patch kernel, 3x3 except as noted: 1 x 1, 33 -> 16 6.3 / 51; 14 x 14, 7 -> 16 7.5 / 9.3, 17 -> 16
+// 13.6 / 12.9, stride 2 14.0 / 16.7, 33 -> 16 24 / 18, stride 2 25 / 35; 56 x 56, 1x1 35 -> 64
+// 5.7 / 11.4, 131 -> 64 15.6 / 26; 4 x 56 x 56, 5 -> 128 23 / 15, 1x1 35 -> 256 50 / 23; 8 x 112 x 112,
+// 1x1 131 -> 16 68 / 44, 7x7 stride 2 3 -> 64 56 / 23.
+inline bool patch_beats_small_k(const OgleConvArgs& a, const PatchPlan& p) {
+  const double staging = p.vec_x ? 6000 + patch_staged(a, p) / 2 : 10000 + patch_staged(a, p);
+  const double products = (double)a.n * a.out_h * a.out_w * a.out_c * a.kernel_size * a.kernel_size * a.in_c;
+  const double x_bytes = (double)a.n * a.in_h * a.in_w * a.in_c * (a.dtype == OGLE_F16 ? 2 : 4);
+  const bool wide = small_k_is_wide(a);
+  return direct_chain(a) >= 0.007 * staging || products * (wide ? 0.25 : 1) * (1 + a.out_c / 32.0) > 2.3e8 ||
+         (x_bytes > 24e6 && !wide);
+}
+
+// Short sums of a small output, where one thread per output is as good or better (256 channels of
+// 14 x 14, K = 28: 7.1 us with the filter in LDS, 5.7 with one thread per output), but for the
+// pointwise ones that share many input values (28 x 28, 131 -> 64 15.3 / 16.4, 16 -> 16 3.6 / 4.3).
+inline bool general_beats_small_k(const OgleConvArgs& a) {
+  const int k = a.kernel_size, ktot = k * k * a.in_c;
+  if ((long)a.n * a.out_h * a.out_w * a.out_c > 65536 || ktot > (k == 1 ? 192 : 48)) return false;
+  return !(k == 1 && (long)a.n * a.out_h * a.out_w >= 16 &&
+           ((ktot > 96 && a.out_c >= 32) || (a.in_c % 4 == 0 && a.out_c >= 16 && a.out_c <= 64)));
 }
 
 // The kernel for a convolution that neither the implicit GEMM nor the stem kernels take.
-enum DirectKernel { DIRECT_GENERAL, DIRECT_PATCH };
+enum DirectKernel { DIRECT_GENERAL, DIRECT_PATCH, DIRECT_SMALL_K };
 inline DirectKernel plan_direct(const OgleConvArgs& a, PatchPlan* plan) {
-  return plan_patch(a, plan) && patch_pays(a, *plan) ? DIRECT_PATCH : DIRECT_GENERAL;
+  const bool patch = plan_patch(a, plan);
+  if (small_k_fits(a)) {
+    if (patch && patch_beats_small_k(a, *plan)) return DIRECT_PATCH;
+    return general_beats_small_k(a) ? DIRECT_GENERAL : DIRECT_SMALL_K;
+  }
+  return patch && patch_pays(a, *plan) ? DIRECT_PATCH : DIRECT_GENERAL;
 }
 
 }  // namespace ogle

@@ -20,6 +20,13 @@ int probe_patch(const OgleConvArgs* a, int64_t* out) {
   return 1;
 }
 
+// Which of the direct kernels takes the convolution (DirectKernel); -1 if the implicit GEMM does.
+int probe_direct(const OgleConvArgs* a) {
+  PatchPlan p;
+  long m = 0;
+  return igemm_eligible(*a, &m) ? -1 : (int)plan_direct(*a, &p);
+}
+
 // 1 if the implicit GEMM takes the convolution, then out = rows and columns of the tile, tiles,
 // K ranges, whether fp32 is contracted as bf16 pieces, workspace bytes.
 int probe_igemm(const OgleConvArgs* a, int scratch, int64_t* out) {

@@ -100,3 +100,32 @@ def test_patch_plan_stays_within_a_launch(probe):
 ])
 def test_patch_kernel_where_it_is_faster(probe, shape, patch):
     assert (patch_plan(probe, *shape) is not None) == patch
+
+
+GENERAL, PATCH, SMALL_K = 0, 1, 2   # DirectKernel
+
+
+@pytest.mark.parametrize("shape,dtype,kernel", [
+    ((1, 1, 1, 33, 16, 3, 1, 1), H.F32, SMALL_K),       # eight of nine taps lie in the padding
+    ((1, 14, 14, 7, 16, 3, 1, 1), H.F32, SMALL_K),
+    ((1, 14, 14, 17, 16, 3, 1, 1), H.F32, PATCH),
+    ((1, 28, 28, 33, 16, 3, 2, 1), H.F16, SMALL_K),     # stride 2: three chunks of channels to stage
+    ((1, 56, 56, 35, 64, 1), H.F32, SMALL_K),
+    ((1, 56, 56, 36, 64, 1), H.F16, SMALL_K),
+    ((4, 56, 56, 35, 256, 1), H.F32, PATCH),            # many products
+    ((8, 112, 112, 131, 16, 1), H.F32, PATCH),          # an input of 53 MB
+    ((8, 112, 112, 3, 64, 7, 2, 3), H.F32, PATCH),
+    ((1, 14, 14, 28, 256, 1), H.F32, GENERAL),          # short sums of a small output
+    ((1, 28, 28, 131, 64, 1), H.F32, SMALL_K),
+    ((1, 28, 28, 12, 16, 3, 1, 1), H.F16, PATCH),
+])
+def test_direct_kernel_with_the_filter_in_lds(probe, shape, dtype, kernel):
+    assert probe.probe_direct(ctypes.byref(conv(*shape, dtype=dtype))) == kernel
+
+
+@pytest.mark.parametrize("dtype", [H.F32, H.F16])
+def test_small_k_cases_run_that_kernel(probe, dtype):
+    for case in K.SMALL_K_CASES:
+        assert probe.probe_direct(ctypes.byref(conv(*case, dtype=dtype))) == SMALL_K, case
+    n, h, w, _, o = K.SMALL_K_CASES[-1][:5]
+    assert n * h * w * (o // 16) >= 256 * 256 * 4 > max(a[0] * a[1] * a[2] * (a[4] // 16) for a in K.SMALL_K_CASES[:-1])

@@ -174,6 +174,30 @@ def test_conv_patch_kernel(case, dtype):
                variant=H.VARIANT_ANY4 if g > 1 else H.VARIANT_NHWC4, what=str(case))
 
 
+SMALL_K_CASES = [
+    # n, h, w, c, o, k, s, p, d   the filter in LDS, one thread per 4 or 16 channels of a pixel
+    (1, 14, 13, 7, 16, 3, 1, 1, 1),      # four channels per thread, ragged last workgroup
+    (2, 1, 1, 33, 12, 3, 1, 1, 1),       # a map of one pixel: all taps but one in the padding
+    (3, 9, 7, 11, 20, 3, 2, 2, 2),       # stride 2, dilation 2
+    (1, 56, 55, 35, 64, 1, 1, 0, 1),     # pointwise, odd channel count
+    (8, 111, 112, 35, 64, 1, 1, 0, 1),   # sixteen channels per thread
+]
+
+
+@pytest.mark.parametrize("case", SMALL_K_CASES)
+@pytest.mark.parametrize("dtype", [H.F32, H.F16])
+def test_conv_small_k_kernel(case, dtype):
+    n, h, w, c, o, k, s, p, d = case
+    r = rng(2940 + SMALL_K_CASES.index(case))
+    x = r.uniform(-1, 1, (n, h, w, c)).astype(np.float32)
+    wt = r.normal(0, 0.5, (o, c, k, k)).astype(np.float32)
+    b = r.uniform(-0.1, 0.1, o).astype(np.float32)
+    if dtype == H.F16:
+        x = x.astype(np.float16).astype(np.float32)
+        wt = wt.astype(np.float16).astype(np.float32)
+    check_conv(x, wt, b, s, p, d, 1, act=H.ACT_CLIP, maxv=6.0, dtype=dtype, entry="ogle_hip_conv2d", what=str(case))
+
+
 INFINITE_FILTER_CASES = [
     # n, h, w, c, o, k, s, p, g
     (2, 20, 18, 24, 36, 3, 1, 1, 3),        # one box per workgroup, all channels staged at once
