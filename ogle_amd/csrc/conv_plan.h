@@ -409,20 +409,20 @@ inline bool small_k_is_wide(const OgleConvArgs& a) {
   return a.out_c % 16 == 0 && (long)a.n * a.out_h * a.out_w * (a.out_c / 16) >= 256L * 256 * 4;
 }
 
-// The patch kernel against that one: the chain of products against staging again; many products
-// (a wide thread's cost a quarter; every workgroup stages the whole filter, which counts with the
-// channels); inputs beyond the L2s, of which a wave reads a cache line per pixel and value.  Fits of
-// 1426 shapes (the faster each time would be 1.1 % faster on average); us with that kernel / with the
+// The patch kernel against that one: the chain of products against staging again; many products,
+// times the channels, since every workgroup stages the whole filter (a wide thread's cost a quarter);
+// inputs beyond the L2s, of which a wave reads a cache line per pixel and value.  Fits of 1426
+// shapes (the faster each time would be 0.9 % faster on average).  Us with that kernel / with the
 // patch kernel, 3x3 except as noted: 1 x 1, 33 -> 16 6.3 / 51; 14 x 14, 7 -> 16 7.5 / 9.3, 17 -> 16
 // 13.6 / 12.9, stride 2 14.0 / 16.7, 33 -> 16 24 / 18, stride 2 25 / 35; 56 x 56, 1x1 35 -> 64
-// 5.7 / 11.4, 131 -> 64 15.6 / 26; 4 x 56 x 56, 5 -> 128 23 / 15, 1x1 35 -> 256 50 / 23; 8 x 112 x 112,
-// 1x1 131 -> 16 68 / 44, 7x7 stride 2 3 -> 64 56 / 23.
+// 5.7 / 11.4, 131 -> 64 15.6 / 26; 4 x 56 x 56, 5 -> 128 23 / 15, 1x1 35 -> 256 50 / 23;
+// 8 x 112 x 112, 1x1 35 -> 32 17 / 28, 131 -> 16 68 / 44, 7x7 stride 2 3 -> 64 56 / 23.
 inline bool patch_beats_small_k(const OgleConvArgs& a, const PatchPlan& p) {
   const double staging = p.vec_x ? 6000 + patch_staged(a, p) / 2 : 10000 + patch_staged(a, p);
   const double products = (double)a.n * a.out_h * a.out_w * a.out_c * a.kernel_size * a.kernel_size * a.in_c;
   const double x_bytes = (double)a.n * a.in_h * a.in_w * a.in_c * (a.dtype == OGLE_F16 ? 2 : 4);
   const bool wide = small_k_is_wide(a);
-  return direct_chain(a) >= 0.007 * staging || products * (wide ? 0.25 : 1) * (1 + a.out_c / 32.0) > 2.3e8 ||
+  return direct_chain(a) >= 0.007 * staging || products * (wide ? 0.25 : 1) * a.out_c > 4e9 ||
          (x_bytes > 24e6 && !wide);
 }
 
