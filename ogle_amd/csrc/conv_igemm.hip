@@ -124,10 +124,19 @@ struct WaveMma<__half, 16> {
   }
 };
 
-// fp32 operands as three bf16 pieces each: x = h + m + l exactly (24 significand bits in three
-// times 8; each piece is the rounded rest of the one before, every rest is exact in fp32), so
+// fp32 operands as three bf16 pieces each: x = h + m + l (24 significand bits in three times 8;
+// each piece is the rounded rest of the one before, every rest is exact in fp32), so
 // x * w = hh + hm + mh + hl + lh + mm plus terms below 2^-26 of the product, and a 32x32x16 step
 // is six bf16 MFMAs of 32 cycles where fp32 takes eight of 64.
+// The three terms left out cost a product at most 0.43 ulp beside its rounding of half an ulp: a
+// sum that one product dominates may be 0.93 ulp off (fp32 MFMAs: 0.5), longer ones are nearer than
+// fp32 MFMAs bring them (figures below).
+// The pieces are exact for |x| from 2^-110 up to where h overflows.  Below, bf16's smallest
+// subnormal cuts them off at 2^-134, which shows in a sum only if its products are tiny too.  So a
+// tile with a sum that is not finite, or neither zero nor at least 2^-60, or with none but zeros,
+// is contracted by fp32 MFMAs.  What is left are operands below 2^-110 that meet others above 2^50
+// in one sum, and sums of operands below 2^-134 in a tile with larger sums: these are zero.  (Splitting operands scaled by 2^24
+// would be exact for those as well and cost 4 % of every tile, 7 % with 3x3.)
 // Measured on MI355X, M = 11552, K = 512, N = 1024: 103 -> 72 us (168 TFLOP/s) with 128x128 tiles;
 // error against 64-bit sums 4.0e-7 -> 1.2e-7.  Bound by power: over long K the loop runs at 178
 // TFLOP/s (six times that in bf16) and 1.6 GHz, the library's bf16 GEMM of 8192 cubed reaches
@@ -162,8 +171,9 @@ constexpr int igemm_lds_bytes() {
 }
 
 // SPLIT (fp32 only): the operands are contracted as bf16 pieces.  Returns false, before anything
-// is stored, if a sum is not finite: an operand was infinite, NaN or so large that a piece
-// overflowed, and the caller contracts the tile in fp32 instead.
+// is stored, if a sum is not finite (an operand was infinite, NaN or so large that a piece
+// overflowed) or so small that pieces may have been cut off, and the caller contracts the tile in
+// fp32 instead.
 template <typename T, int BM, int BN, int WM, int WN, int ROWB, bool PW, bool SPLIT = false>
 __device__ __forceinline__ bool igemm_tile(
     unsigned char* __restrict__ lds, const ConvGeom& g, const T* __restrict__ x, const T* __restrict__ w,
@@ -480,6 +490,7 @@ __device__ __forceinline__ bool igemm_tile(
 
   if constexpr (SPLIT) {
     float probe = 0.f;
+    unsigned low = 0xffffffffu;   // least magnitude of the sums that are not zero, as bits
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -488,8 +499,16 @@ __device__ __forceinline__ bool igemm_tile(
         for (int r = 0; r < REGS; ++r) {
           acc[i][j][r] += rest[i][j][r];
           probe = fmaf(acc[i][j][r], 0.f, probe);
+          low = min(low, (__float_as_uint(acc[i][j][r]) << 1) - 1u);
         }
-    if (__syncthreads_or(probe != 0.f || probe != probe)) return false;
+    // bit 0: a sum that is not zero, bit 1: one that the pieces may have got wrong
+    constexpr unsigned kLeast = (127u - 60u) << 24;   // 2^-60
+    __shared__ int verdict[4];
+    const bool wrong = probe != 0.f || probe != probe || low < kLeast - 1u;
+    const int mine = (__any(low != 0xffffffffu) ? 1 : 0) | (__any(wrong) ? 2 : 0);
+    if (lane == 0) verdict[wave] = mine;
+    __syncthreads();
+    if ((verdict[0] | verdict[1] | verdict[2] | verdict[3]) != 1) return false;
   }
 
   // Epilogue.  Destinations: split-K partial sums go to `partial` (rows of opitch floats,

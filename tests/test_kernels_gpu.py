@@ -299,6 +299,22 @@ def test_conv_fp32_as_bf16_pieces_not_finite(case):
     np.testing.assert_allclose(got[ok], ref[ok], rtol=1e-4)
 
 
+@pytest.mark.parametrize("case", [(16, 19, 19, 512, 512, 1, 0), (1, 223, 221, 256, 128, 1, 0), (8, 75, 75, 64, 32, 3, 1)])
+@pytest.mark.parametrize("low,high,wlow", [(-126, -123, 0), (-137, -130, 20), (-146, -140, 30), (-110, -100, 48)])
+def test_conv_fp32_as_bf16_pieces_of_tiny_operands(case, low, high, wlow):
+    """Operands whose pieces fall below bf16's smallest subnormal (2^-133): their sums are contracted
+    in fp32.  From 2^-110 on the pieces are exact, whatever the other operands.  Bound: every product
+    and every running sum rounded once in fp32, subnormal ones by half of 2^-149."""
+    n, h, w, c, o, k, p = case
+    r = rng(3170 + o - low)
+    x = (r.uniform(1, 2, (n, h, w, c)) * 2.0 ** r.integers(low, high, (n, h, w, c))).astype(np.float32)
+    wt = (r.uniform(1, 2, (o, c, k, k)) * 2.0 ** r.integers(wlow, wlow + 4, (o, c, k, k))).astype(np.float32)
+    ref = _pieces_reference(x, wt, k, 1, p)    # all positive: the reference is its own scale
+    got = gpu_conv(x, wt, None, 1, p, entry="ogle_hip_conv2d")
+    kt = k * k * c
+    assert np.max(np.abs(got - ref) - kt * 2.0 ** -149 - (kt + 16) * 2.0 ** -24 * ref) <= 0
+
+
 WAVE_CASES = [
     # n, h, w, c, o, k, s, p, d   small problems with a long enough K: the wave-split kernel
     (1, 19, 19, 512, 512, 1, 1, 0, 1),    # 32x32 tiles, pointwise (a batch-1 MobileNet layer)
