@@ -133,9 +133,10 @@ struct WaveMma<__half, 16> {
 // fp32 MFMAs bring them (figures below).
 // The pieces are exact for |x| from 2^-110 up to where h overflows.  Below, bf16's smallest
 // subnormal cuts them off at 2^-134, which shows in a sum only if its products are tiny too.  So a
-// tile with a sum that is not finite, or neither zero nor at least 2^-60, or with none but zeros,
-// is contracted by fp32 MFMAs.  What is left are operands below 2^-110 that meet others above 2^50
-// in one sum, and sums of operands below 2^-134 in a tile with larger sums: these are zero.  (Splitting operands scaled by 2^24
+// tile with a sum that is not finite, or neither zero nor at least 2^-60, or (whole sums: a range of
+// K can lie in the padding) with none but zeros, is contracted by fp32 MFMAs.  What is left are
+// operands below 2^-110 that meet others above 2^50 in one sum, and sums of operands below 2^-134
+// in a tile with larger sums or in a range of K: these are zero.  (Splitting operands scaled by 2^24
 // would be exact for those as well and cost 4 % of every tile, 7 % with 3x3.)
 // Measured on MI355X, M = 11552, K = 512, N = 1024: 103 -> 72 us (168 TFLOP/s) with 128x128 tiles;
 // error against 64-bit sums 4.0e-7 -> 1.2e-7.  Bound by power: over long K the loop runs at 178
@@ -508,7 +509,8 @@ __device__ __forceinline__ bool igemm_tile(
     const int mine = (__any(low != 0xffffffffu) ? 1 : 0) | (__any(wrong) ? 2 : 0);
     if (lane == 0) verdict[wave] = mine;
     __syncthreads();
-    if ((verdict[0] | verdict[1] | verdict[2] | verdict[3]) != 1) return false;
+    const int all = verdict[0] | verdict[1] | verdict[2] | verdict[3];
+    if ((all & 2) != 0 || (all == 0 && partial == nullptr)) return false;
   }
 
   // Epilogue.  Destinations: split-K partial sums go to `partial` (rows of opitch floats,
