@@ -36,6 +36,7 @@ struct IgemmPlan {
 
 constexpr long kComputeUnits = 256;
 constexpr int kRowBytesF32 = 64;   // bytes of K per tile row per slab, fp32
+constexpr int kPiecesSlabs = 3;    // least slabs of a contraction as bf16 pieces
 
 inline bool is_pointwise(const OgleConvArgs& a) {
   return a.kernel_size == 1 && a.stride == 1 && a.padding == 0;
@@ -80,10 +81,12 @@ inline IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
   // has to bring would differ: from 1024 of them on they are cut as well, with fewer they are taken
   // only where the small tiles would not be cut.
   const bool long_f32 = a.dtype == OGLE_F32 && p.ktiles >= 128;
+  // (fp32 128x128 tiles exist as pieces only: not for two slabs, see there)
   const bool big_tiles = long_f32 ? tiles(CFG_128x128) >= 4 * kComputeUnits ||
                                         (big_columns_full && tiles(CFG_128x128) >= big_tiles_wanted &&
                                          tiles(CFG_64x64) >= 8 * kComputeUnits)
-                                  : big_columns_full && tiles(CFG_128x128) >= big_tiles_wanted;
+                                  : big_columns_full && tiles(CFG_128x128) >= big_tiles_wanted &&
+                                        (a.dtype == OGLE_F16 || p.ktiles >= kPiecesSlabs);
   // Narrow outputs with a long contraction (the SSD heads, box and class head of a feature
   // map fused: 75 or 150 channels, K = 2304 ... 9216): one tile column holds every output
   // channel, so the input is gathered once instead of once per 64-channel tile column, and
@@ -195,13 +198,27 @@ inline IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
   // partial sums are kept in rows of the channel count rounded up to four
   p.workspace_bytes =
       p.splits > 1 ? (size_t)p.splits * (size_t)m * ((a.out_c + 3) & ~3) * sizeof(float) : 0;
-  // Tiles of 32x32 MFMA blocks are contracted as bf16 pieces (but for the single-column tiles of
-  // the two-destination form) once they give a compute unit more than one workgroup.  A lone
-  // workgroup has nothing to cover the splitting with: 112x112x32 -> 64 3x3 (196 tiles) 11.1 us
-  // with fp32 MFMAs, 11.9 with pieces; 3703 x 88 x 168 (174) 6.3 / 6.9; 1600 x 512 x 1024 (400)
-  // 22.8 / 20.4.
+  // fp32 tiles of 32x32 MFMA blocks are contracted as bf16 pieces (the 96 and 160 columns wide ones
+  // are not built as such) where a compute unit has more than one workgroup and more than 16 slabs:
+  // a lone workgroup has nothing to cover the splitting with, and a short sum is over before the faster
+  // unit has made up for it.  Not for two slabs at all, nor for pointwise convolutions to at most 32
+  // channels: both are bound by their bytes.  Time with pieces over time with fp32 MFMAs, 64x64 tiles:
+  //   slabs  workgroups to 384   512   768  1024  1536  2560  5000
+  //     2         1.20  1.23  1.13  1.12  1.09  1.12  1.07
+  //     3         1.12  1.13  1.07  1.03  0.99  0.98  0.90
+  //     4         1.12  1.15  1.07  1.03  0.98  0.99  0.91
+  //     6         1.02  1.05  0.99  0.95  0.93  0.95  0.87
+  //     9         0.97  0.96  0.92  0.87  0.84  0.86  0.84
+  //    16         0.97  0.98  0.90  0.93  0.88  0.89
+  //    36         0.87  0.90  0.88  0.90  0.85  0.89
+  //    72         0.84  0.90  0.88  0.89  0.86  0.86
+  // 128x32 tiles 0.83 to 0.98 from 9 slabs on with 3x3, 0.97 to 1.04 pointwise.  150x150x32 -> 64 at batch
+  // 16 26.4 us instead of 27.5, at batch 1 4.8 instead of 5.8.
+  const long workgroups = tiles(p.cfg) * p.splits;
   p.pieces = a.dtype == OGLE_F32 && (p.cfg == CFG_128x128 || p.cfg == CFG_64x64 || p.cfg == CFG_128x32) &&
-             tiles(p.cfg) * p.splits > kComputeUnits;
+             workgroups > kComputeUnits && p.slabs_per_split >= kPiecesSlabs &&
+             workgroups * p.slabs_per_split > 16 * kComputeUnits &&
+             !(p.cfg == CFG_128x32 && is_pointwise(a));
   // Which operand an XCD's L2 should keep to itself: with K ranges pinned to XCDs the input is
   // fetched by all eight L2s and the filter by one, with tile rows pinned it is the other way
   // round (the rocprofv3 FETCH_SIZE of the 19x19x512 class head fell from 8.5x its input to

@@ -129,3 +129,45 @@ def test_small_k_cases_run_that_kernel(probe, dtype):
         assert probe.probe_direct(ctypes.byref(conv(*case, dtype=dtype))) == SMALL_K, case
     n, h, w, _, o = K.SMALL_K_CASES[-1][:5]
     assert n * h * w * (o // 16) >= 256 * 256 * 4 > max(a[0] * a[1] * a[2] * (a[4] // 16) for a in K.SMALL_K_CASES[:-1])
+
+
+IGEMM_FIELDS = ("bm", "bn", "tiles", "splits", "pieces", "workspace")
+
+
+def igemm_plan(probe, *shape, scratch=True, **kw):
+    out = (ctypes.c_int64 * len(IGEMM_FIELDS))()
+    if not probe.probe_igemm(ctypes.byref(conv(*shape, **kw)), int(scratch), out):
+        return None
+    return dict(zip(IGEMM_FIELDS, out))
+
+
+@pytest.mark.parametrize("shape,pieces", [
+    # n, h, w, c, o, k, s, p   fp32 as bf16 pieces: next to the lines (conv_plan.h)
+    ((16, 150, 150, 32, 64, 1), False),             # two slabs, 5625 tiles
+    ((16, 150, 150, 36, 64, 1), True),              # three
+    ((1, 150, 150, 32, 64, 1), False),
+    ((1, 128, 128, 128, 128, 1), False),            # 512 workgroups of 8 slabs
+    ((1, 128, 128, 144, 128, 1), True),             # of 9
+    ((1, 19, 19, 512, 63, 3, 1, 1), False),         # class head of one image: 288 workgroups of 6 slabs
+    ((8, 19, 19, 512, 63, 3, 1, 1), True),
+    ((1, 189, 189, 512, 24, 1), False),             # pointwise to 24 channels
+    ((1, 189, 189, 64, 24, 3, 1, 1), True),
+    ((16, 19, 19, 512, 512, 1), True),
+])
+def test_pieces_where_they_are_faster(probe, shape, pieces):
+    assert igemm_plan(probe, *shape)["pieces"] == pieces
+
+
+def test_large_fp32_tiles_are_pieces(probe):
+    """128x128 tiles of fp32 are built as pieces only."""
+    r, large = random.Random(7), 0
+    for _ in range(40000):
+        k = r.choice([1, 1, 3])
+        h = int(math.exp(r.uniform(1, 6.5)))
+        shape = (r.choice([1, 2, 16, 64]), h, h, 4 * r.choice([2, 3, 4, 8, 9, 12, 16, 64, 128, 256]),
+                 r.choice([65, 100, 128, 168, 256, 512, 1024]), k, r.choice([1, 2]), k // 2)
+        plan = igemm_plan(probe, *shape, scratch=r.random() < 0.5)
+        if plan and (plan["bm"], plan["bn"]) == (128, 128):
+            large += 1
+            assert plan["pieces"], shape
+    assert large > 300
