@@ -32,6 +32,7 @@
 // groups take k 0..3, 4..7, 8..11, 12..15 of a 16-wide group and issue four MFMAs)
 // or v_mfma_f32_16x16x32_f16; register r of lane l is row 4*(l/16) + r, column l%16.
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -776,19 +777,20 @@ __device__ __forceinline__ void igemm_wave_tile(
 // pointwise: each workgroup takes the code path of its own problem.  The branch is
 // uniform over the workgroup; all four paths keep 16 accumulator registers per
 // lane, so the register budget is that of the largest one.
-template <typename T, int ROWB>
-__global__ __launch_bounds__(256, 3) void conv_igemm_mixed_kernel(IgemmGroup grp) {
-  constexpr bool kSplit = sizeof(T) == 4;
-  constexpr int kLds = igemm_lds_bytes<128, 32, ROWB, kSplit>();  // the largest of the tiles below
-  static_assert(kLds >= igemm_lds_bytes<128, 16, ROWB>() && kLds >= igemm_lds_bytes<64, 64, ROWB, kSplit>(), "LDS size");
+// SPLIT: some problem of the group is contracted as bf16 pieces.  Its tiles need more registers, LDS
+// and code than the others': a group without (the heads of one image) does without them as well.
+template <typename T, int ROWB, bool SPLIT>
+__global__ __launch_bounds__(256, SPLIT ? 3 : 1) void conv_igemm_mixed_kernel(IgemmGroup grp) {
+  constexpr int kLds = igemm_lds_bytes<128, 32, ROWB, SPLIT>();  // the largest of the tiles below
+  static_assert(kLds >= igemm_lds_bytes<128, 16, ROWB>() && kLds >= igemm_lds_bytes<64, 64, ROWB, SPLIT>(), "LDS size");
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
   int i = 0;
   while (i + 1 < grp.count && (int)blockIdx.x >= grp.first[i + 1]) ++i;
   // a copy: with a use of the argument per path, the compiler keeps the whole group in scratch
-  const IgemmProblem p = grp.p[i];
+  typename std::conditional<SPLIT, const IgemmProblem, const IgemmProblem&>::type p = grp.p[i];
   const int bid = (int)blockIdx.x - grp.first[i];
-#define OGLE_MIXED_TILE(SPLIT, BM, BN, WM, WN, PW)                                              \
-  igemm_tile<T, BM, BN, WM, WN, ROWB, PW, SPLIT>(                                               \
+#define OGLE_MIXED_TILE(PIECES, BM, BN, WM, WN, PW)                                             \
+  igemm_tile<T, BM, BN, WM, WN, ROWB, PW, PIECES>(                                              \
       lds, p.g, static_cast<const T*>(p.x), static_cast<const T*>(p.w), p.bias,                 \
       static_cast<T*>(p.y), static_cast<T*>(p.y2), p.o1, p.ep, p.tiles_n, p.tiles,              \
       p.partial, p.slabs_per_split, p.splits, bid)
@@ -796,7 +798,7 @@ __global__ __launch_bounds__(256, 3) void conv_igemm_mixed_kernel(IgemmGroup grp
   case V:                                                                                       \
     OGLE_MIXED_TILE(false, BM, BN, WM, WN, PW);                                                 \
     break;
-  if constexpr (kSplit) {
+  if constexpr (SPLIT) {
     bool done = false;
     switch (p.variant) {
       case 16: done = OGLE_MIXED_TILE(true, 64, 64, 2, 2, false); break;
@@ -1371,7 +1373,7 @@ int32_t launch_conv_batch(const OgleConvArgs* args, int count, hipStream_t s,
     IgemmGroup grp{};
     ReduceGroup red{};
     const Item& head = items[a0];
-    bool uniform = true;
+    bool uniform = true, pieces = false;
     for (size_t b0 = a0; b0 < items.size() && grp.count < kMaxGroup; ++b0) {
       const Item& it = items[b0];
       if (done[b0] || it.dtype != head.dtype) continue;
@@ -1379,6 +1381,7 @@ int32_t launch_conv_batch(const OgleConvArgs* args, int count, hipStream_t s,
       if (b0 != a0 && (it.cfg == CFG_128x256 || head.cfg == CFG_128x256)) continue;  // fills the chip alone
       if (!same && !(mixable(head) && mixable(it))) continue;
       uniform = uniform && same;
+      pieces = pieces || it.pieces;
       done[b0] = true;
       const Prepared& pr = it.pr;
       grp.first[grp.count + 1] = grp.first[grp.count] + (int)pr.grid;
@@ -1397,11 +1400,12 @@ int32_t launch_conv_batch(const OgleConvArgs* args, int count, hipStream_t s,
       OGLE_SPLIT_DISPATCH(conv_igemm_group_split_kernel, head.cfg, head.pw, grid, s, grp);
     } else if (uniform && !is_wave(head.cfg)) {
       OGLE_IGEMM_DISPATCH(conv_igemm_group_kernel, head.dtype, head.cfg, head.pw, grid, s, grp);
+    } else if (pieces) {
+      launch((conv_igemm_mixed_kernel<float, kRowBytesF32, true>), dim3(grid), dim3(256), 0, s, grp);
     } else if (head.dtype == OGLE_F16) {
-      launch((conv_igemm_mixed_kernel<__half, 128>), dim3(grid), dim3(256), 0, s, grp);
+      launch((conv_igemm_mixed_kernel<__half, 128, false>), dim3(grid), dim3(256), 0, s, grp);
     } else {
-      launch((conv_igemm_mixed_kernel<float, kRowBytesF32>), dim3(grid), dim3(256), 0,
-                         s, grp);
+      launch((conv_igemm_mixed_kernel<float, kRowBytesF32, false>), dim3(grid), dim3(256), 0, s, grp);
     }
     int32_t st = check_launch("conv_igemm_group");
     if (st != OGLE_OK) return st;

@@ -171,3 +171,10 @@ def test_large_fp32_tiles_are_pieces(probe):
             large += 1
             assert plan["pieces"], shape
     assert large > 300
+
+
+def test_heads_of_one_image_have_no_pieces(probe):
+    """So that their grouped launch is the kernel without the code, registers and LDS of pieces."""
+    for m, c, a in ((19, 512, 3), (10, 1024, 6), (5, 512, 6), (3, 256, 6), (2, 256, 6), (1, 128, 6)):
+        for o in (4 * a, 21 * a):
+            assert not igemm_plan(probe, 1, m, m, c, o, 3, 1, 1)["pieces"], (m, o)
