@@ -178,3 +178,16 @@ def test_heads_of_one_image_have_no_pieces(probe):
     for m, c, a in ((19, 512, 3), (10, 1024, 6), (5, 512, 6), (3, 256, 6), (2, 256, 6), (1, 128, 6)):
         for o in (4 * a, 21 * a):
             assert not igemm_plan(probe, 1, m, m, c, o, 3, 1, 1)["pieces"], (m, o)
+
+
+@pytest.mark.parametrize("dtype", [H.F32, H.F16])
+def test_patch_cases_run_what_they_name(probe, dtype):
+    direct = [probe.probe_direct(ctypes.byref(conv(*case, dtype=dtype))) for case in K.PATCH_CASES]
+    assert direct == [PATCH, PATCH, PATCH, -1, PATCH, PATCH, GENERAL, PATCH, GENERAL, GENERAL, PATCH, PATCH]
+    for case, want in K.PATCH_WIDE_CASES:
+        plan = patch_plan(probe, *case, dtype=dtype)
+        assert plan is not None, case
+        plan["several"] = plan["boxes"] > plan["box_blocks"]
+        assert {key: plan[key] for key in want} == want, (case, plan)
+        n, h, w, c, _, k, s, p, d, g = case   # not a stem kernel's
+        assert g > 1 or k * k * c > 32 or n * H.out_size(h, k, s, p, d) * H.out_size(w, k, s, p, d) < 4096

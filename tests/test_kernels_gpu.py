@@ -137,20 +137,43 @@ def test_conv_stem_kernel(case, dtype):
 
 
 PATCH_CASES = [
-    # n, h, w, c, o, k, s, p, d, g   what only the direct kernels take: the LDS patch kernel
+    # n, h, w, c, o, k, s, p, d, g   mostly the LDS patch kernel, 16 columns, one box per workgroup
     (4, 57, 43, 96, 144, 3, 1, 1, 1, 12),   # several groups per workgroup, vector staging, ragged box
     (2, 23, 19, 80, 80, 3, 1, 1, 1, 5),     # 16 channels per group: exactly one 16-wide block
     (2, 23, 19, 34, 34, 3, 1, 1, 1, 2),     # 17 per group: one past it, odd channel count (merged runs)
-    (1, 31, 33, 64, 99, 3, 2, 1, 1, 1),     # fp32 only the ragged N of the MFMA path; fp16: stays there
-    (1, 29, 31, 33, 64, 3, 2, 1, 1, 1),     # chunks of channels with a ragged last one, 64 columns
-    (1, 40, 41, 131, 65, 3, 1, 1, 1, 1),    # many chunks, one channel past a 64-wide block
-    (3, 21, 22, 77, 45, 1, 2, 0, 1, 1),     # one tap, stride 2: skipped pixels are not staged
+    (1, 31, 33, 64, 99, 3, 2, 1, 1, 1),     # ragged N of the implicit GEMM, next to the direct kernels
+    (1, 29, 31, 33, 64, 3, 2, 1, 1, 1),     # chunks of channels with a ragged last one, 4 column blocks
+    (1, 40, 41, 131, 65, 3, 1, 1, 1, 1),    # many chunks, a last column block of one channel
+    (3, 21, 22, 77, 45, 1, 2, 0, 1, 1),     # one tap, stride 2: one thread per output
     (2, 40, 38, 3, 64, 7, 2, 3, 1, 1),      # 7x7 RGB stem: whole filter rows as runs, 4 column blocks
-    (9, 2, 3, 30, 42, 3, 1, 1, 1, 3),       # maps smaller than a box: several images per workgroup
-    (2, 24, 20, 21, 24, 3, 1, 2, 2, 3),     # dilation 2, seven channels per group
+    (9, 2, 3, 30, 42, 3, 1, 1, 1, 3),       # tiny maps: one thread per output
+    (2, 24, 20, 21, 24, 3, 1, 2, 2, 3),     # dilation 2, seven channels per group: one thread per output
     (1, 50, 50, 25, 40, 5, 3, 2, 1, 5),     # 5x5, stride 3
     (1, 20, 20, 64, 64, 11, 1, 5, 1, 2),    # 11x11: a few channels at a time
 ]
+
+PATCH_WIDE_CASES = [
+    # n, h, w, c, o, k, s, p, d, g          and what its plan has to be (test_conv_plan_cpu.py)
+    # 64 columns, two of three groups per workgroup (the last block is narrower), several boxes
+    ((33, 55, 49, 48, 99, 1, 1, 0, 1, 3), dict(cols=64, gp=2, several=True, vec_x=1)),
+    # 64 columns and 35 more, whole filter rows as runs, several boxes
+    ((33, 35, 25, 49, 693, 3, 2, 1, 1, 7), dict(cols=64, gp=1, runs=1, several=True)),
+    # 48 of 64 columns, channels in chunks, vector staging, dilation 2, stride 2
+    ((33, 41, 35, 24, 96, 3, 2, 2, 2, 2), dict(cols=64, cc=8, several=False, vec_x=1)),
+    # 32 columns, a last block of one channel, several boxes
+    ((33, 34, 26, 66, 65, 1, 1, 0, 1, 1), dict(cols=32, cc=66, several=True)),
+    # 32 columns, two chunks of channels, boxes of several images
+    ((16, 12, 11, 112, 910, 3, 2, 2, 2, 7), dict(cols=32, cc=8, several=False)),
+    # one tap, stride 2: skipped pixels are not staged
+    ((4, 37, 25, 49, 910, 1, 2, 0, 1, 7), dict(cols=32, cc=7, several=False)),
+    # six of seven groups per workgroup, several boxes, dilation 2
+    ((8, 90, 111, 21, 35, 3, 1, 2, 2, 7), dict(cols=16, gp=6, several=True)),
+    # maps smaller than a box, 32 columns
+    ((33, 5, 5, 140, 693, 1, 1, 0, 1, 7), dict(cols=32, cc=20, several=False)),
+    # maps smaller than a box, 16 columns
+    ((8, 2, 2, 16, 10, 3, 1, 1, 1, 2), dict(cols=16, boxes=1)),
+]
+
 
 FULL_LDS_CASES = [
     # n, h, w, c, o, k, s, p, d, g   as much LDS as a launch may ask for
@@ -159,11 +182,11 @@ FULL_LDS_CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", PATCH_CASES + FULL_LDS_CASES)
+@pytest.mark.parametrize("case", PATCH_CASES + FULL_LDS_CASES + [case for case, _ in PATCH_WIDE_CASES])
 @pytest.mark.parametrize("dtype", [H.F32, H.F16])
 def test_conv_patch_kernel(case, dtype):
     n, h, w, c, o, k, s, p, d, g = case
-    r = rng(2900 + (PATCH_CASES + FULL_LDS_CASES).index(case))
+    r = rng(2900 + (PATCH_CASES + FULL_LDS_CASES + [case for case, _ in PATCH_WIDE_CASES]).index(case))
     x = r.uniform(-1, 1, (n, h, w, c)).astype(np.float32)
     wt = r.normal(0, 0.5, (o, c // g, k, k)).astype(np.float32)
     b = r.uniform(-0.1, 0.1, o).astype(np.float32)
