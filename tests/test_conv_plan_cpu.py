@@ -191,3 +191,21 @@ def test_patch_cases_run_what_they_name(probe, dtype):
         assert {key: plan[key] for key in want} == want, (case, plan)
         n, h, w, c, _, k, s, p, d, g = case   # not a stem kernel's
         assert g > 1 or k * k * c > 32 or n * H.out_size(h, k, s, p, d) * H.out_size(w, k, s, p, d) < 4096
+
+
+def test_pieces_cases_run_what_they_name(probe):
+    def tile(*shape, scratch=True):
+        plan = igemm_plan(probe, *shape, scratch=scratch)
+        return "%dx%d%s%s" % (plan["bm"], plan["bn"], " split" if plan["splits"] > 1 else "", " pieces" if plan["pieces"] else "")
+    assert [tile(*case) for case in K.PIECES_CASES] == [
+        "64x64", "64x64", "64x64 pieces", "128x128 pieces", "64x64 pieces", "32x32", "128x32 pieces", "64x64",
+        "64x64 split", "64x64 pieces", "64x64 pieces", "128x128 pieces", "64x64 split pieces"]
+    assert [tile(3, 75, 75, 512, 64, 3, 1, 1, scratch=False), tile(16, 19, 19, 512, 512, 1),
+            tile(1, 160, 160, 32, 256, 3, 1, 1)] == ["64x64 pieces", "64x64 pieces", "128x128 pieces"]
+    assert [tile(n, h, w, c, o, k, 1, p) for n, h, w, c, o, k, p in K.NOT_FINITE_CASES] == [
+        "64x64 pieces", "128x128 pieces", "64x64", "64x64 pieces", "64x64 split pieces", "128x32 pieces", "128x128 pieces"]
+    assert [tile(n, h, w, c, o, k, 1, p) for n, h, w, c, o, k, p in K.TINY_CASES] == [
+        "64x64 pieces", "128x128 pieces", "128x32 pieces"]
+    assert [[tile(*case) for case in batch] for batch in K.BATCHES_OF_PIECES] == [
+        ["64x64 pieces"] * 2, ["128x32 pieces"] * 2, ["128x128 pieces"] * 2,
+        ["64x64 split pieces", "128x16 split", "64x64", "128x32 pieces"]]

@@ -263,16 +263,20 @@ def test_fp16_tiles_by_filled_columns(o, c):
 
 
 PIECES_CASES = [
-    # n, h, w, c, o, k, s, p   fp32 as bf16 pieces: more workgroups than compute units
-    (1, 96, 174, 64, 40, 1, 1, 0),      # 64x64 tiles, pointwise, ragged N; 261 workgroups
-    (1, 96, 168, 64, 40, 1, 1, 0),      # 252 workgroups: the fp32 tile, next to the line
+    # n, h, w, c, o, k, s, p   fp32 as bf16 pieces, and next to them (test_conv_plan_cpu.py)
+    (1, 96, 174, 64, 40, 1, 1, 0),      # 64x64 tiles, 261 workgroups of four slabs: fp32
+    (1, 96, 168, 64, 40, 1, 1, 0),      # 252 workgroups: fp32
     (16, 19, 19, 512, 512, 1, 1, 0),    # 64x64 tiles, 728 workgroups
     (1, 223, 221, 256, 128, 1, 1, 0),   # 128x128 tiles, 386 of them, last one ragged
     (1, 217, 221, 260, 124, 1, 1, 0),   # 375 large tiles: 64x64; K tail inside a slab, ragged N
-    (2, 75, 73, 36, 32, 3, 1, 1),       # 128x32 tile, 3x3, 86 workgroups: fp32
+    (2, 75, 73, 36, 32, 3, 1, 1),       # 86 tiles of 128x32: the wave-split kernel, fp32
     (5, 84, 84, 36, 31, 3, 1, 1),       # 128x32 tile, 3x3, 276 workgroups, odd N
-    (3, 75, 73, 44, 70, 3, 2, 1),       # 64x64, stride 2: split-K partials or one tile column and a bit
-    (2, 19, 19, 512, 63, 3, 1, 1),      # split-K partials, odd N, K = 4608
+    (3, 75, 73, 44, 70, 3, 2, 1),       # 64x64, stride 2, 132 workgroups: fp32
+    (2, 19, 19, 512, 63, 3, 1, 1),      # ranges of six slabs, odd N, K = 4608: fp32
+    (1, 96, 174, 260, 40, 1, 1, 0),     # 64x64 tiles, 261 workgroups of 17 slabs, ragged N
+    (6, 75, 73, 44, 70, 3, 2, 1),       # 64x64, stride 2, 264 workgroups, one tile column and a bit
+    (1, 160, 160, 32, 256, 3, 1, 1),    # 128x128 tiles, 3x3
+    (8, 19, 19, 512, 63, 3, 1, 1),      # ranges of K, odd N, K = 4608; without scratch fp32
 ]
 
 
@@ -300,7 +304,36 @@ def test_conv_fp32_as_bf16_pieces(case):
         assert np.max(np.abs(got - ref) / scale) <= bound, (case, ws)
 
 
-@pytest.mark.parametrize("case", [(16, 19, 19, 512, 512, 1, 0), (1, 223, 221, 256, 128, 1, 0), (2, 75, 75, 64, 63, 3, 1)])
+@pytest.mark.parametrize("case", [
+    # n, h, w, c, o, k, s, p   K of 4608 without a split, 512, and 128x128 tiles of K = 288
+    (3, 75, 75, 512, 64, 3, 1, 1), (16, 19, 19, 512, 512, 1, 1, 0), (1, 160, 160, 32, 256, 3, 1, 1)])
+def test_conv_fp32_as_bf16_pieces_sums_in_two_norms(case):
+    """No product may be left out: any of h * l, l * h, m * m missing would show as about 2^-18.5 of the
+    result's 2-norm.  What is allowed are the roundings: one of at most half an ulp per 16 products of
+    a running sum that grows with their square root, together sqrt(K / 32) * 2^-25 at most, twice
+    that, and one more for the sums of the small products and the store."""
+    n, h, w, c, o, k, s, p = case
+    r = rng(3140 + o)
+    x = r.uniform(-1, 1, (n, h, w, c)).astype(np.float32)
+    wt = r.normal(0, 0.2, (o, c, k, k)).astype(np.float32)
+    ref = _pieces_reference(x, wt, k, s, p)
+    got = gpu_conv(x, wt, None, s, p, workspace=False, entry="ogle_hip_conv2d")
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert err <= (np.sqrt(k * k * c / 32) + 1) * 2.0 ** -24, err
+
+
+NOT_FINITE_CASES = [
+    # n, h, w, c, o, k, p
+    (16, 19, 19, 512, 512, 1, 0), (1, 223, 221, 256, 128, 1, 0),
+    (2, 75, 75, 64, 63, 3, 1),          # 176 workgroups: fp32
+    (4, 75, 75, 64, 63, 3, 1),          # 64x64 tiles, 3x3, odd N
+    (8, 19, 19, 512, 63, 3, 1),         # ranges of K
+    (5, 84, 84, 36, 31, 3, 1),          # 128x32 tiles
+    (1, 160, 160, 32, 256, 3, 1),       # 128x128 tiles, 3x3
+]
+
+
+@pytest.mark.parametrize("case", NOT_FINITE_CASES)
 def test_conv_fp32_as_bf16_pieces_not_finite(case):
     """Infinite, NaN and very large operands, whose pieces are no numbers, give what fp32 gives."""
     n, h, w, c, o, k, p = case
@@ -322,7 +355,10 @@ def test_conv_fp32_as_bf16_pieces_not_finite(case):
     np.testing.assert_allclose(got[ok], ref[ok], rtol=1e-4)
 
 
-@pytest.mark.parametrize("case", [(16, 19, 19, 512, 512, 1, 0), (1, 223, 221, 256, 128, 1, 0), (8, 75, 75, 64, 32, 3, 1)])
+TINY_CASES = [(16, 19, 19, 512, 512, 1, 0), (1, 223, 221, 256, 128, 1, 0), (8, 75, 75, 64, 32, 3, 1)]   # n, h, w, c, o, k, p
+
+
+@pytest.mark.parametrize("case", TINY_CASES)
 @pytest.mark.parametrize("low,high,wlow", [(-126, -123, 0), (-137, -130, 20), (-146, -140, 30), (-110, -100, 48)])
 def test_conv_fp32_as_bf16_pieces_of_tiny_operands(case, low, high, wlow):
     """Operands whose pieces fall below bf16's smallest subnormal (2^-133): their sums are contracted
@@ -553,6 +589,51 @@ def test_config3_pointwise_gemm(dtype):
     ora = O.conv2d(x[:1], w, b, act=O.ACT_RELU, variant=O.VARIANT_PW)
     assert_conv_close(got[:1], ora, scale[:361].reshape(1, 19, 19, 1024).astype(np.float32), rtol,
                       "C3 vs oracle")
+
+
+BATCHES_OF_PIECES = [
+    # n, h, w, c, o, k, s, p   one tile shape each: the grouped kernel of 64x64, 128x32, 128x128 tiles
+    [(8, 19, 19, 256, 512, 1, 1, 0), (7, 19, 19, 260, 500, 1, 1, 0)],
+    [(5, 84, 84, 36, 31, 3, 1, 1), (5, 84, 83, 32, 24, 3, 1, 1)],
+    [(1, 160, 160, 32, 256, 3, 1, 1), (1, 161, 160, 32, 250, 3, 1, 1)],
+    # 64x64 and 128x32, with and without pieces: the mixed kernel
+    [(8, 19, 19, 512, 63, 3, 1, 1), (8, 19, 19, 512, 12, 3, 1, 1), (2, 9, 9, 32, 40, 1, 1, 0), (5, 84, 84, 36, 31, 3, 1, 1)],
+]
+
+
+@pytest.mark.parametrize("cases", BATCHES_OF_PIECES)
+def test_conv_batch_of_pieces_equals_single_launches(cases):
+    """Grouped launches of fp32 tiles contracted as bf16 pieces, one problem with an infinite and a
+    large operand: exactly what one launch each gives."""
+    import ctypes
+    import torch
+    from util import pack_filter
+    r = rng(2600 + len(cases) + cases[0][3])
+    keep, single, args = [], [], (H.ConvArgs * len(cases))()
+    for i, (n, h, w, c, o, k, st, p) in enumerate(cases):
+        xh = r.uniform(-1, 1, (n, h, w, c)).astype(np.float32)
+        if i == 0:
+            xh[0, 1, 2, 3], xh[n - 1, 4, 5, 6] = np.inf, 3.4e38
+        x, wd = torch.from_numpy(xh).cuda(), pack_filter(r.normal(0, 0.2, (o, c, k, k)).astype(np.float32), H.FILTER_OHWI)
+        oh, ow = H.out_size(h, k, st, p), H.out_size(w, k, st, p)
+        y1, y2 = (torch.full((n, oh, ow, o), -7.0, device="cuda") for _ in range(2))
+        a = H.conv_args(x.data_ptr(), wd.data_ptr(), None, y1.data_ptr(), n, h, w, c, o, k, st, p, 1, 1, H.ACT_NONE)
+        need = H.lib().ogle_hip_conv_workspace_bytes(ctypes.byref(a))
+        ws = [torch.empty(max(need, 16), dtype=torch.uint8, device="cuda") for _ in range(2)]
+        if need:
+            a.workspace_dev, a.workspace_bytes = ws[0].data_ptr(), need
+        H.check(H.lib().ogle_hip_conv2d(ctypes.byref(a), 0))
+        a.output_dev = y2.data_ptr()
+        if need:
+            a.workspace_dev = ws[1].data_ptr()
+        args[i] = a
+        keep += [x, wd, ws]
+        single.append((y1, y2))
+    H.check(H.lib().ogle_hip_conv2d_batch(args, len(cases), 0))
+    torch.cuda.synchronize()
+    for i, (y1, y2) in enumerate(single):
+        assert bool(torch.isfinite(y1).all()) == (i != 0)
+        np.testing.assert_array_equal(y2.cpu().numpy(), y1.cpu().numpy(), err_msg=str(cases[i]))
 
 
 def test_conv_batch_equals_single_launches():
