@@ -153,7 +153,7 @@ def mobilenet_v1_ssd(batch, seed=20240005, num_classes=21, image=300, head_std=0
 
 
 def separable_block(batch, seed=20240002, size=38, cin=256, cout=512):
-    """depthwise 3x3 s1 p1 + BN + ReLU6, pointwise 1x1 + BN + ReLU6."""
+    """Depthwise 3x3 s1 p1 + BN + ReLU6, pointwise 1x1 + BN + ReLU6."""
     r = np.random.Generator(np.random.PCG64(seed))
     g = dlx.GraphBuilder()
     x = g.add_input("input", [batch, cin, size, size])
