@@ -367,7 +367,7 @@ __global__ __launch_bounds__(256) void conv_direct_general(
 // arithmetic, was 15 % slower on the stem and its extra code cost the other shapes 8 %.
 //
 // Taps outside the image are staged as zeros.  0 * w is 0 only for a finite w, so a workgroup
-// that meets an infinite or NaN filter value recomputes its outputs one by one, skipping taps.
+// that meets an infinite or NaN filter value computes its outputs one by one instead, skipping taps.
 
 __device__ __forceinline__ int div_fast(int n, const FastDiv& f) {
   return f.d == 1 ? n : (int)__umulhi((unsigned)n, f.mul);
@@ -435,8 +435,7 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
   }
 
   // `bad`: this thread has staged an infinite or NaN filter value; `repair`: some thread of the
-  // workgroup has, known to all of them before the first output is stored, so that every output
-  // is stored once, either contracted or, below, one by one (by whichever wave its index falls to)
+  // workgroup has
   bool bad = false, repair = false;
   if (tid == 0) filter_not_finite = 0;
   for (int tile = tblock; tile < tiles; tile += p.tile_blocks) {
@@ -449,7 +448,7 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
     // with gp > 1 all channels are staged at once: only one of the two loops below has more
     // than one turn, and one set of accumulators serves both
     Acc acc[FR][NB];
-    for (int c0 = repair ? cpg : 0; c0 < cpg; c0 += p.cc) {
+    for (int c0 = 0; c0 < cpg; c0 += p.cc) {
       const int cc = min(p.cc, cpg - c0);
       const int cs = p.gp > 1 ? groups_here * cpg : cc;   // channels per patch pixel this time
       // the last chunk and the last group block are narrower than the divisors the host prepared
@@ -531,10 +530,6 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
         if (bad) filter_not_finite = 1;
       }
       __syncthreads();
-      if (c0 + p.cc >= cpg && filter_not_finite != 0) {   // the whole filter has been seen
-        repair = true;
-        break;
-      }
 
       const int len = p.runs_x == 1 ? q.k * cc : cc;    // values per run
       for (int gi = 0; gi < groups_here; ++gi) {
@@ -625,7 +620,9 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
       }
     }
 
+    if (tile == tblock) repair = filter_not_finite != 0;   // (in chunks: one box per workgroup)
     if (repair) {
+      __syncthreads();   // outputs go by thread index: every wave's contracted ones are stored before
       const int per_pixel = groups_here * cols_here;
       for (int i = tid; i < kPatchPixels * per_pixel; i += 256) {
         const int pix = i / per_pixel, rest2 = i - pix * per_pixel;

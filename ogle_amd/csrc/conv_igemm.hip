@@ -12,16 +12,19 @@
 // Tiling.  A workgroup of 4 waves (256 threads) owns a BM x BN output tile and
 // walks K in slabs of ROWB bytes per row.  Slabs are staged global -> registers
 // -> LDS (double buffered, one barrier per slab) with the next slab's global
-// loads in flight while the current one is multiplied.  LDS rows are padded by
-// 16 bytes so the 16-byte-per-lane operand reads are bank-conflict free.
+// loads in flight while the current one is multiplied.  The 16-byte K groups of an
+// LDS row are permuted by a function of the row, so that staging writes and operand
+// reads are bank-conflict free.
 //
-// MFMA mapping (64-wide waves).  fp32 uses v_mfma_f32_32x32x2_f32: lane l
+// MFMA mapping (64-wide waves).  fp32 tiles that give a unit enough to do are split
+// into bf16 pieces on the way to LDS and contracted by v_mfma_f32_32x32x16_bf16
+// (split_bf16 below).  The others use v_mfma_f32_32x32x2_f32: lane l
 // supplies A[l%32][l/32] and B[l/32][l%32].  Since the contraction sums over k
 // in any order, a lane reads four consecutive k of its row with one 16-byte LDS
 // read (lanes 0-31 take k 0..3 of an 8-wide group, lanes 32-63 take k 4..7) and
 // issues four MFMAs, one per element.  fp16 storage uses
 // v_mfma_f32_32x32x16_f16: a lane's 16 bytes are the 8 halves the instruction
-// wants (k = 8*(l/32)..+7).  Accumulation is fp32 in both cases.
+// wants (k = 8*(l/32)..+7).  Accumulation is fp32 in all cases.
 //
 // Result layout of a 32x32 block: register r of lane l holds
 // row 8*(r/4) + 4*(l/32) + r%4, column l%32, so a store instruction writes two
