@@ -207,5 +207,5 @@ def test_pieces_cases_run_what_they_name(probe):
     assert [tile(n, h, w, c, o, k, 1, p) for n, h, w, c, o, k, p in K.TINY_CASES] == [
         "64x64 pieces", "128x128 pieces", "128x32 pieces"]
     assert [[tile(*case) for case in batch] for batch in K.BATCHES_OF_PIECES] == [
-        ["64x64 pieces"] * 2, ["128x32 pieces"] * 2, ["128x128 pieces"] * 2,
+        ["64x64 pieces"] * 2, ["128x32 pieces"] * 2, ["128x128 pieces"] * 2, ["64x64 pieces", "64x64"],
         ["64x64 split pieces", "128x16 split", "64x64", "128x32 pieces"]]

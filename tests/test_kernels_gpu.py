@@ -596,7 +596,9 @@ BATCHES_OF_PIECES = [
     [(8, 19, 19, 256, 512, 1, 1, 0), (7, 19, 19, 260, 500, 1, 1, 0)],
     [(5, 84, 84, 36, 31, 3, 1, 1), (5, 84, 83, 32, 24, 3, 1, 1)],
     [(1, 160, 160, 32, 256, 3, 1, 1), (1, 161, 160, 32, 250, 3, 1, 1)],
-    # 64x64 and 128x32, with and without pieces: the mixed kernel
+    # one tile shape, with and without pieces: the mixed kernel
+    [(16, 28, 28, 128, 128, 3, 1, 1), (16, 56, 56, 64, 128, 1, 2, 0)],
+    # 64x64 and 128x32, with and without pieces
     [(8, 19, 19, 512, 63, 3, 1, 1), (8, 19, 19, 512, 12, 3, 1, 1), (2, 9, 9, 32, 40, 1, 1, 0), (5, 84, 84, 36, 31, 3, 1, 1)],
 ]
 
