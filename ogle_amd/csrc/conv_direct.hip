@@ -622,7 +622,9 @@ __global__ __launch_bounds__(256, COLS == 16 ? 4 : 3) void conv_patch_mfma(const
 
     if (tile == tblock) repair = filter_not_finite != 0;   // (in chunks: one box per workgroup)
     if (repair) {
-      __syncthreads();   // outputs go by thread index: every wave's contracted ones are stored before
+      // outputs go by thread index: every wave's contracted ones have been stored before
+      __threadfence();
+      __syncthreads();
       const int per_pixel = groups_here * cols_here;
       for (int i = tid; i < kPatchPixels * per_pixel; i += 256) {
         const int pix = i / per_pixel, rest2 = i - pix * per_pixel;
