@@ -16,9 +16,8 @@
 // LDS row are permuted by a function of the row, so that staging writes and operand
 // reads are bank-conflict free.
 //
-// MFMA mapping (64-wide waves).  fp32 tiles that give a unit enough to do are split
-// into bf16 pieces on the way to LDS and contracted by v_mfma_f32_32x32x16_bf16
-// (split_bf16 below).  The others use v_mfma_f32_32x32x2_f32: lane l
+// MFMA mapping (64-wide waves).  Most fp32 problems are contracted as bf16 pieces by kernels of
+// their own (pieces_tile below).  The others use v_mfma_f32_32x32x2_f32: lane l
 // supplies A[l%32][l/32] and B[l/32][l%32].  Since the contraction sums over k
 // in any order, a lane reads four consecutive k of its row with one 16-byte LDS
 // read (lanes 0-31 take k 0..3 of an 8-wide group, lanes 32-63 take k 4..7) and
@@ -34,6 +33,7 @@
 // blocks instead: v_mfma_f32_16x16x4_f32 (lane l supplies A[l%16][l/16], four lane
 // groups take k 0..3, 4..7, 8..11, 12..15 of a 16-wide group and issue four MFMAs)
 // or v_mfma_f32_16x16x32_f16; register r of lane l is row 4*(l/16) + r, column l%16.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -128,59 +128,72 @@ struct WaveMma<__half, 16> {
   }
 };
 
-// fp32 operands as three bf16 pieces each: x = h + m + l (24 significand bits in three times 8;
-// each piece is the rounded rest of the one before, every rest is exact in fp32), so
-// x * w = hh + hm + mh + hl + lh + mm plus terms below 2^-26 of the product, and a 32x32x16 step
-// is six bf16 MFMAs of 32 cycles where fp32 takes eight of 64.
-// The three terms left out cost a product at most 0.43 ulp beside its rounding of half an ulp: a
-// sum that one product dominates may be 0.93 ulp off (fp32 MFMAs: 0.5), longer ones are nearer than
-// fp32 MFMAs bring them (figures below).
-// The pieces are exact for |x| from 2^-110 up to where h overflows.  Below, bf16's smallest
-// subnormal cuts them off at 2^-134, which shows in a sum only if its products are tiny too.  So a
-// tile with a sum that is not finite, or neither zero nor at least 2^-60, or (whole sums: a range of
-// K can lie in the padding) with none but zeros, is contracted by fp32 MFMAs.  What is left are
-// operands below 2^-110 that meet others above 2^50 in one sum, and sums of operands below 2^-134
-// in a tile with larger sums or in a range of K: these are zero.  (Splitting operands scaled by 2^24
-// would be exact for those as well and cost 4 % of every tile, 7 % with 3x3.)
-// Measured on MI355X, M = 11552, K = 512, N = 1024: 103 -> 72 us (168 TFLOP/s) with 128x128 tiles;
-// error against 64-bit sums 4.0e-7 -> 1.2e-7.  Bound by power: over long K the loop runs at 178
-// TFLOP/s (six times that in bf16) and 1.6 GHz, the library's bf16 GEMM of 8192 cubed reaches
-// 1145 / 6 = 191.  Hence nothing gained by residuals by v_dot2_f32_bf16, loads pinned to the top of a
-// slab, or MFMAs and splitting interleaved by hand (equal to 8 % behind).
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float floatx2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void split_bf16(const u32x4& v, uint2 (&piece)[3]) {
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    floatx2_t x = {__uint_as_float(v[2 * e]), __uint_as_float(v[2 * e + 1])};
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const bf16x2_t h = __builtin_convertvector(x, bf16x2_t);
-      (e == 0 ? piece[q].x : piece[q].y) = __builtin_bit_cast(unsigned, h);
-      if (q < 2) {
-        const unsigned b = __builtin_bit_cast(unsigned, h);
-        x[0] -= __uint_as_float(b << 16);
-        x[1] -= __uint_as_float(b & 0xffff0000u);
-      }
+// Work assignment.  Workgroups are dealt to the 8 XCDs by linear id modulo 8 and
+// every XCD has a private L2, so the (tile, split) pairs are laid out such that
+// tiles sharing a band of A rows run on one XCD and, when K is split, an XCD owns
+// a fixed subset of the K ranges: the filter and input slabs of one K range are
+// then fetched into one L2 only instead of all eight.
+// When K is split and the input is the larger operand (a 3x3 head on a big map), the
+// other layout is used instead (splits < 0 marks it): tile rows are dealt to the XCDs and
+// all K ranges of a tile row run on the same XCD, so each band of input rows (with the
+// halo its taps share) is fetched into one L2 only, and the filter into all eight.
+// `splits` says which layout (work_layout below).  Returns false for a workgroup beyond the last tile.
+__device__ __forceinline__ bool assign_work(int bid, int tiles_n, int tiles, int splits, int& pid, int& split) {
+  const int xcd = bid & 7, j = bid >> 3;
+  if (splits < 0) {
+    if (splits >= -kMaxSplits) {
+      splits = -splits;
+      const int per_row = tiles_n * splits;
+      const int r = (j / per_row) * 8 + xcd;
+      const int rem = j % per_row;
+      pid = r * tiles_n + rem / splits;
+      split = rem % splits;
+    } else {
+      splits = -splits - kMaxSplits;
+      const int per = (tiles * splits + 7) >> 3;
+      const int q = j < per ? xcd * per + j : tiles * splits;
+      pid = q / splits;
+      split = q - pid * splits;
     }
+    if (pid >= tiles) return false;
+  } else {
+    if (splits == 1) {
+      // tile row r (the tiles_n tiles that share one band of A rows) goes to XCD
+      // r % 8, so all XCDs advance through memory together
+      const int r = (j / tiles_n) * 8 + xcd;
+      pid = r * tiles_n + j % tiles_n;
+      split = 0;
+    } else if (splits == 0) {
+      const int per = (tiles + 7) >> 3;
+      pid = j < per ? xcd * per + j : tiles;
+      split = 0;
+    } else if (splits >= 8 && (splits & 7) == 0) {
+      const int zs = splits >> 3;
+      pid = j / zs;
+      split = xcd + 8 * (j - pid * zs);
+    } else if (splits == 2 || splits == 4) {
+      const int xpz = 8 / splits;
+      split = xcd % splits;
+      pid = j * xpz + xcd / splits;
+    } else {                       // any other count: the splits of a tile are neighbours
+      pid = bid / splits;
+      split = bid - pid * splits;
+    }
+    if (pid >= tiles) return false;
   }
+  return true;
 }
 
 // One workgroup's share of one convolution: output tile / K range number `bid` of
 // the problem.  Shared by the single-problem kernel and the grouped kernel.
 // LDS bytes of one workgroup: two K-slab buffers of BM + BN padded rows.
-template <int BM, int BN, int ROWB, bool SPLIT = false>
+template <int BM, int BN, int ROWB>
 constexpr int igemm_lds_bytes() {
-  return 2 * (BM + BN) * (SPLIT ? 96 : ROWB + 16);
+  return 2 * (BM + BN) * (ROWB + 16);
 }
 
-// SPLIT (fp32 only): the operands are contracted as bf16 pieces.  Returns false, before anything
-// is stored, if a sum is not finite (an operand was infinite, NaN or so large that a piece
-// overflowed) or so small that pieces may have been cut off, and the caller contracts the tile in
-// fp32 instead.
-template <typename T, int BM, int BN, int WM, int WN, int ROWB, bool PW, bool SPLIT = false>
-__device__ __forceinline__ bool igemm_tile(
+template <typename T, int BM, int BN, int WM, int WN, int ROWB, bool PW>
+__device__ __forceinline__ void igemm_tile(
     unsigned char* __restrict__ lds, const ConvGeom& g, const T* __restrict__ x, const T* __restrict__ w,
     const float* __restrict__ bias, T* __restrict__ y, T* __restrict__ y2, int o1,
     const Epilogue& ep, int tiles_n, int tiles, float* __restrict__ partial,
@@ -219,61 +232,15 @@ __device__ __forceinline__ bool igemm_tile(
   constexpr int CHUNKB = (64 / MB) * 16;  // bytes of a row one MFMA step consumes (64 / MB lane groups x 16)
   constexpr int CHUNKS = ROWB / CHUNKB;
   static_assert(CHUNKS >= 1, "a K slab holds at least one MFMA step");
-  constexpr int STAGE = igemm_lds_bytes<BM, BN, ROWB, SPLIT>() / 2;  // one buffer: A rows then B rows
-  // SPLIT: three planes (pieces) of rows of 16 bf16.  Eight rows fill a 256-byte window; in the
-  // windows of rows 16-31 of a block the two 16-byte groups of a row change places: the 16 rows
-  // an operand read serves in one cycle (0-3, 12-15, 20-23, 24-27 or the others) then fall into
-  // 16 different columns.
-  constexpr int PLANE = (BM + BN) * 32;
-  static_assert(!SPLIT || (sizeof(T) == 4 && ROWB == 64 && MB == 32), "split form");
-  auto window_perm = [](int row) { return (row >> 4) & 1; };
+  constexpr int STAGE = igemm_lds_bytes<BM, BN, ROWB>() / 2;  // one buffer: A rows then B rows
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wave_m = wave / WN, wave_n = wave % WN;
 
-  // Work assignment.  Workgroups are dealt to the 8 XCDs by linear id modulo 8 and
-  // every XCD has a private L2, so the (tile, split) pairs are laid out such that
-  // tiles sharing a band of A rows run on one XCD and, when K is split, an XCD owns
-  // a fixed subset of the K ranges: the filter and input slabs of one K range are
-  // then fetched into one L2 only instead of all eight.
-  // When K is split and the input is the larger operand (a 3x3 head on a big map), the
-  // other layout is used instead (splits < 0 marks it): tile rows are dealt to the XCDs and
-  // all K ranges of a tile row run on the same XCD, so each band of input rows (with the
-  // halo its taps share) is fetched into one L2 only, and the filter into all eight.
   int pid, split;
-  if (splits < 0) {
-    splits = -splits;
-    const int xcd = bid & 7, j = bid >> 3;
-    const int per_row = tiles_n * splits;
-    const int r = (j / per_row) * 8 + xcd;
-    const int rem = j % per_row;
-    pid = r * tiles_n + rem / splits;
-    split = rem % splits;
-    if (pid >= tiles) return true;
-  } else {
-    const int xcd = bid & 7, j = bid >> 3;
-    if (splits == 1) {
-      // tile row r (the tiles_n tiles that share one band of A rows) goes to XCD
-      // r % 8, so all XCDs advance through memory together
-      const int r = (j / tiles_n) * 8 + xcd;
-      pid = r * tiles_n + j % tiles_n;
-      split = 0;
-    } else if (splits >= 8 && (splits & 7) == 0) {
-      const int zs = splits >> 3;
-      pid = j / zs;
-      split = xcd + 8 * (j - pid * zs);
-    } else if (splits == 2 || splits == 4) {
-      const int xpz = 8 / splits;
-      split = xcd % splits;
-      pid = j * xpz + xcd / splits;
-    } else {                       // any other count: the splits of a tile are neighbours
-      pid = bid / splits;
-      split = bid - pid * splits;
-    }
-    if (pid >= tiles) return true;
-  }
+  if (!assign_work(bid, tiles_n, tiles, splits, pid, split)) return;
   const int tile_n = pid % tiles_n;
   const int tile_m = pid / tiles_n;
   const int m0 = tile_m * BM;
@@ -360,18 +327,6 @@ __device__ __forceinline__ bool igemm_tile(
   // Writes ra / rb into LDS buffer `buf`.
 #define OGLE_STORE_SLAB(buf, SET)                                                            \
   {                                                                                          \
-    if constexpr (SPLIT) {                                                                   \
-      unsigned char* base_ = lds + (buf) * STAGE + (vrow >> 3) * 256 + (vcol & 1) * 8 +      \
-                             ((((vrow & 7) * 2 + (vcol >> 1)) ^ window_perm(vrow)) * 16);    \
-      _Pragma("unroll") for (int p = 0; p < AP + BP; ++p) {                                  \
-        const int row_ = p < AP ? p * RPP : BM + (p - AP) * RPP;                             \
-        if (p < AP ? (A_PART && row_ + vrow >= BM) : (B_PART && row_ + vrow >= BM + BN)) continue; \
-        uint2 piece_[3];                                                                     \
-        split_bf16(p < AP ? ra[SET][p < AP ? p : 0] : rb[SET][p < AP ? 0 : p - AP], piece_); \
-        _Pragma("unroll") for (int q = 0; q < 3; ++q)                                        \
-          *reinterpret_cast<uint2*>(base_ + q * PLANE + row_ * 32) = piece_[q];              \
-      }                                                                                      \
-    } else {                                                                                 \
       unsigned char* base_ = lds + (buf) * STAGE + vrow * LROW +                             \
                              (SWZ ? (vcol ^ row_perm(vrow)) : vcol) * 16;                    \
       _Pragma("unroll") for (int p = 0; p < AP; ++p)                                         \
@@ -380,7 +335,6 @@ __device__ __forceinline__ bool igemm_tile(
       _Pragma("unroll") for (int p = 0; p < BP; ++p)                                         \
         if (!B_PART || p * RPP + vrow < BN)                                                  \
           *reinterpret_cast<u32x4*>(base_ + (BM + p * RPP) * LROW) = rb[SET][p];             \
-    }                                                                                        \
   }
 
   Acc acc[TM][TN];
@@ -390,19 +344,6 @@ __device__ __forceinline__ bool igemm_tile(
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < REGS; ++r) acc[i][j][r] = 0.f;
-
-  // SPLIT: the five products below h * h have sums of their own, a few hundredths of the main
-  // ones: their roundings vanish and the main sums are rounded once per 16 products (K = 4608:
-  // 5.3e-7 from the 64-bit sums with one set of accumulators; fp32 MFMAs 6.1e-7).
-  Acc rest[SPLIT ? TM : 1][SPLIT ? TN : 1];
-  if constexpr (SPLIT) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < REGS; ++r) rest[i][j][r] = 0.f;
-  }
 
   const int l32 = lane & 31;
   const int lh = lane >> 5;
@@ -414,30 +355,9 @@ __device__ __forceinline__ bool igemm_tile(
   const int kt_begin = split * slabs_per_split;
   const int kt_end = min(g.ktiles, kt_begin + slabs_per_split);
 
-#define OGLE_SPLIT_PRODUCT(ACC, QA, QB)                                                      \
-  _Pragma("unroll") for (int i = 0; i < TM; ++i)                                             \
-    _Pragma("unroll") for (int j = 0; j < TN; ++j)                                           \
-      ACC[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[QA][i], bv[QB][j], ACC[i][j], 0, 0, 0);
-
   // One K slab from LDS buffer `buf` into the accumulators.
 #define OGLE_COMPUTE_SLAB(buf)                                                               \
-  if constexpr (SPLIT) {                                                                     \
-    const unsigned char* pr_ = lds + (buf) * STAGE + (lrow >> 3) * 256 +                     \
-                               ((((lrow & 7) * 2 + lq) ^ window_perm(lrow)) * 16);           \
-    bf16x8_t av[3][TM], bv[3][TN];                                                           \
-    _Pragma("unroll") for (int q = 0; q < 3; ++q) {                                          \
-      _Pragma("unroll") for (int i = 0; i < TM; ++i)                                         \
-        av[q][i] = *reinterpret_cast<const bf16x8_t*>(pr_ + q * PLANE + (wave_m * WTM + i * 32) * 32); \
-      _Pragma("unroll") for (int j = 0; j < TN; ++j)                                         \
-        bv[q][j] = *reinterpret_cast<const bf16x8_t*>(pr_ + q * PLANE + (BM + wave_n * WTN + j * 32) * 32); \
-    }                                                                                        \
-    OGLE_SPLIT_PRODUCT(rest, 1, 1)                                                           \
-    OGLE_SPLIT_PRODUCT(acc, 0, 0)                                                            \
-    OGLE_SPLIT_PRODUCT(rest, 0, 2)                                                           \
-    OGLE_SPLIT_PRODUCT(rest, 2, 0)                                                           \
-    OGLE_SPLIT_PRODUCT(rest, 0, 1)                                                           \
-    OGLE_SPLIT_PRODUCT(rest, 1, 0)                                                           \
-  } else {                                                                                   \
+  {                                                                                          \
     const unsigned char* pa = lds + (buf) * STAGE + (wave_m * WTM + lrow) * LROW;            \
     const unsigned char* pb = lds + (buf) * STAGE + (BM + wave_n * WTN + lrow) * LROW;       \
     _Pragma("unroll") for (int ch = 0; ch < CHUNKS; ++ch) {                                  \
@@ -489,33 +409,8 @@ __device__ __forceinline__ bool igemm_tile(
     __syncthreads();
   }
 #undef OGLE_COMPUTE_SLAB
-#undef OGLE_SPLIT_PRODUCT
 #undef OGLE_LOAD_SLAB
 #undef OGLE_STORE_SLAB
-
-  if constexpr (SPLIT) {
-    float probe = 0.f;
-    unsigned low = 0xffffffffu;   // least magnitude of the sums that are not zero, as bits
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < REGS; ++r) {
-          acc[i][j][r] += rest[i][j][r];
-          probe = fmaf(acc[i][j][r], 0.f, probe);
-          low = min(low, (__float_as_uint(acc[i][j][r]) << 1) - 1u);
-        }
-    // bit 0: a sum that is not zero, bit 1: one that the pieces may have got wrong
-    constexpr unsigned kLeast = (127u - 60u) << 24;   // 2^-60
-    __shared__ int verdict[4];
-    const bool wrong = probe != 0.f || probe != probe || low < kLeast - 1u;
-    const int mine = (__any(low != 0xffffffffu) ? 1 : 0) | (__any(wrong) ? 2 : 0);
-    if (lane == 0) verdict[wave] = mine;
-    __syncthreads();
-    const int all = verdict[0] | verdict[1] | verdict[2] | verdict[3];
-    if ((all & 2) != 0 || (all == 0 && partial == nullptr)) return false;
-  }
 
   // Epilogue.  Destinations: split-K partial sums go to `partial` (rows of opitch floats,
   // the channel count rounded up to 4 so that rows stay 16-byte aligned); finished outputs
@@ -554,7 +449,7 @@ __device__ __forceinline__ bool igemm_tile(
         }
       }
     }
-    return true;
+    return;
   } else {
   // The staging region (reused K-loop LDS) takes JC 32-column blocks of a wave's tile at a
   // time: as many as fit, so that a row segment a wave stores is as long as possible.
@@ -605,7 +500,7 @@ __device__ __forceinline__ bool igemm_tile(
         }
       }
     }
-    return true;
+    return;
   }
   if constexpr (sizeof(T) == 2) {
     if ((g.o & 7) == 0 && y2 == nullptr && (g.oimg & 7) == 0) {
@@ -653,7 +548,7 @@ __device__ __forceinline__ bool igemm_tile(
           }
         }
       }
-      return true;
+      return;
     }
   }
 #pragma unroll
@@ -680,7 +575,6 @@ __device__ __forceinline__ bool igemm_tile(
     }
   }
   }  // MB == 32
-  return true;
 }
 
 // Everything one convolution's workgroups need, as plain data (a kernel argument).
@@ -699,21 +593,439 @@ struct IgemmProblem {
   int variant;  // mixed-group kernel only: 2 * (tile is 128x32) + (pointwise); 4..7: wave-split 32 / 16; 8, 9: 128x16 tile; + 16: as bf16 pieces
 };
 
-template <int BM, int BN, int WM, int WN, bool PW>
-__device__ __forceinline__ void igemm_tile_split(unsigned char* lds, const IgemmProblem& p, int bid) {
-#define OGLE_TILE(SPLIT)                                                                             \
-  igemm_tile<float, BM, BN, WM, WN, 64, PW, SPLIT>(                                                   \
-      lds, p.g, static_cast<const float*>(p.x), static_cast<const float*>(p.w), p.bias,               \
-      static_cast<float*>(p.y), static_cast<float*>(p.y2), p.o1, p.ep, p.tiles_n, p.tiles, p.partial, \
-      p.slabs_per_split, p.splits, bid)
-  if (!OGLE_TILE(true)) OGLE_TILE(false);
-#undef OGLE_TILE
+// fp32 operands as three bf16 pieces each: x = h + m + l (24 significand bits in three times 8;
+// each piece is the rounded rest of the one before, every rest is exact in fp32), so
+// x * w = hh + hm + mh + hl + lh + mm plus terms below 2^-26 of the product: six bf16 MFMAs of 16
+// cycles per 16x16x32 step where fp32 takes eight of 32.
+// The three terms left out cost a product at most 0.43 ulp beside its rounding of half an ulp: a
+// sum that one product dominates may be 0.93 ulp off (fp32 MFMAs: 0.5), longer ones are nearer than
+// fp32 MFMAs bring them (figures below).
+// The pieces are exact for |x| from 2^-110 up to where h overflows.  Below, bf16's smallest
+// subnormal cuts them off at 2^-134, which shows in a sum only if its products are tiny too.  So a
+// tile with a sum that is not finite, or neither zero nor at least 2^-60, or (whole sums: a range of
+// K can lie in the padding) with none but zeros, is contracted by fp32 MFMAs.  What is left are
+// operands below 2^-110 that meet others above 2^50 in one sum, and sums of operands below 2^-134
+// in a tile with larger sums or in a range of K: these are zero.  (Splitting operands scaled by 2^24
+// would be exact for those as well and cost 4 % of every tile, 7 % with 3x3.)
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float floatx2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split_bf16(const u32x4& v, uint2 (&piece)[3]) {
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    floatx2_t x = {__uint_as_float(v[2 * e]), __uint_as_float(v[2 * e + 1])};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const bf16x2_t h = __builtin_convertvector(x, bf16x2_t);
+      (e == 0 ? piece[q].x : piece[q].y) = __builtin_bit_cast(unsigned, h);
+      if (q < 2) {
+        const unsigned b = __builtin_bit_cast(unsigned, h);
+        x[0] -= __uint_as_float(b << 16);
+        x[1] -= __uint_as_float(b & 0xffff0000u);
+      }
+    }
+  }
 }
 
-template <int BM, int BN, int WM, int WN, bool PW>
-__global__ __launch_bounds__(256, 2) void conv_igemm_split_kernel(IgemmProblem p) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[igemm_lds_bytes<BM, BN, 64, true>()];
-  igemm_tile_split<BM, BN, WM, WN, PW>(lds, p, (int)blockIdx.x);
+// LDS of one workgroup of a pieces tile with NB blocks of 16 output channels: per K group two
+// stages of three planes of 64-byte rows.
+template <int NB, int KG>
+constexpr int pieces_lds_bytes() { return KG * 2 * 3 * NB * 1024; }
+
+// One workgroup's share of an fp32 convolution contracted as bf16 pieces.
+//
+// WM waves, each with its own 16 * WR output pixels and all 16 * NB channels of the tile.  An input
+// value is used by one wave only and goes from memory straight into that wave's registers, where it
+// is split; the filter, which all waves share, is split once per workgroup on its way to LDS.  So a
+// stage writes only the filter's planes to LDS (72 bytes per cycle and unit measured, against 228 for
+// reads) and no input value is split or gathered twice.  KG groups of WM waves take stages in turn and
+// add their sums at the end.
+//
+// A stage is two slabs of 16 channels (each of one tap); v_mfma_f32_16x16x32_bf16 takes it in one
+// step.  Lane l holds, of row l % 16 (a pixel, or a channel's filter), channels 4q .. 4q+3 of both
+// slabs, q = l / 16: its two 16-byte loads and its neighbours' in q are one 64-byte run.  The filter is
+// the first operand: register r of lane l of a result block is pixel l % 16, channel 4 * (l / 16) + r,
+// so four channels of a pixel are stored as 16 bytes without a trip through LDS.
+//
+// The five products below h * h have sums of their own, a few hundredths of the main ones: their
+// roundings vanish and the main sums are rounded once per 32 products.
+//
+// Measured on MI355X against both operands split on their way to LDS (32x32x16 MFMAs, 64 rows of each
+// operand per 64x64 tile and 16 channels), us: 19x19x512 -> 512 at batch 16 27.8 -> 24.4, 3x3 56x56x64 ->
+// 64 36.7 -> 29.1, 28x28x128 -> 128 38.0 -> 31.0, M = 11552, K = 512, N = 1024 74.5 -> 68.5 (177 TFLOP/s);
+// error against 64-bit sums at K = 512 1.24e-7 -> 1.20e-7 (fp32 MFMAs 4.1e-7).  Large problems are bound by
+// power: the library's bf16 GEMM of 8192 cubed reaches 1145 / 6 = 191.  Smaller ones share it among LDS
+// writes, splitting and MFMAs; loads further ahead, and splitting interleaved with MFMAs by hand, gained nothing.
+template <int WR, int NB, int WM, int KG, bool PW>
+__device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, const IgemmProblem& p, int bid) {
+  constexpr int BM = WM * WR * 16, BN = NB * 16;
+  constexpr int TG = WM * 64;                          // threads of a K group
+  constexpr int BP = (BN * 8 + TG - 1) / TG;           // 16-byte filter vectors a thread loads per stage
+  constexpr bool B_PART = BN * 8 % TG != 0;
+  constexpr int PLANE = BN * 64, STAGE = 3 * PLANE;
+  const ConvGeom& g = p.g;
+
+  int pid, split;
+  if (!assign_work(bid, p.tiles_n, p.tiles, p.splits, pid, split)) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int kgroup = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / TG);
+  const int tg = KG == 1 ? tid : tid % TG, wave = __builtin_amdgcn_readfirstlane(tg >> 6);
+  const int tile_n = pid % p.tiles_n, tile_m = pid / p.tiles_n;
+  const int m0 = tile_m * BM + wave * (WR * 16), n0 = tile_n * BN;
+  const int lr = lane & 15, kq = lane >> 4;
+  unsigned char* const planes = lds + kgroup * (2 * STAGE);
+
+  const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, g.x_bytes);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.w, g.w_bytes);
+
+  // this lane's pixels: their offset (PW), or that of their first tap, and its place
+  unsigned a_base[WR], a_tap[WR];
+  int a_iy[WR], a_ix[WR];
+#pragma unroll
+  for (int i = 0; i < WR; ++i) {
+    const int m = m0 + i * 16 + lr;
+    const bool ok = m < g.m_total;
+    if (PW) {
+      a_tap[i] = ok ? (unsigned)m * (unsigned)(g.c * 4) + kq * 16 : kOutOfRange;
+    } else {
+      const int ox = m % g.ow;
+      const int t = m / g.ow;
+      const int oy = t % g.oh;
+      const int b = t / g.oh;
+      a_iy[i] = ok ? oy * g.stride - g.pad : -0x40000000;   // fails every in-image test
+      a_ix[i] = ox * g.stride - g.pad;
+      a_base[i] = (unsigned)(((b * g.h + oy * g.stride - g.pad) * g.w + a_ix[i]) * g.c * 4) + kq * 16;
+    }
+  }
+  // this thread's filter rows and its place in the stage: vector bc of eight in a 128-byte row
+  const int bc = tg & 7, br = tg >> 3;
+  const unsigned krow_bytes = (unsigned)(g.k * g.k * g.c * 4);
+  unsigned b_row[BP];
+#pragma unroll
+  for (int i = 0; i < BP; ++i) {
+    const int row = i * (TG / 8) + br, o = n0 + row;
+    b_row[i] = o < g.o && (!B_PART || row < BN) ? (unsigned)o * krow_bytes + (bc & 3) * 16 : kOutOfRange;
+  }
+
+  const int kt_begin = split * p.slabs_per_split;
+  const int kt_end = min(g.ktiles, kt_begin + p.slabs_per_split);
+  const int stages = (kt_end - kt_begin + 1) >> 1;
+  __shared__ float bias[BN];
+  if (tid < BN) bias[tid] = p.bias != nullptr && n0 + tid < g.o ? p.bias[n0 + tid] : 0.f;
+
+  // Cursor over slabs: the tap's offsets, the slab within the tap.
+  int l_kt, l_cc, l_kx, l_dy, l_dx;
+  unsigned l_tapbyte;
+  auto enter_tap = [&]() {
+    const unsigned from = (unsigned)((l_dy * g.w + l_dx) * g.c * 4);
+#pragma unroll
+    for (int i = 0; i < WR; ++i) {
+      const bool in = (unsigned)(a_iy[i] + l_dy) < (unsigned)g.h && (unsigned)(a_ix[i] + l_dx) < (unsigned)g.w;
+      a_tap[i] = in ? a_base[i] + from : kOutOfRange;
+    }
+  };
+  auto seek = [&](int kt) {
+    l_kt = kt;
+    if (PW) {
+      l_cc = kt;
+      l_tapbyte = 0;
+    } else {
+      const int tap = kt / g.cchunks, ky = tap / g.k;
+      l_cc = kt - tap * g.cchunks;
+      l_kx = tap - ky * g.k;
+      l_dy = ky * g.dil;
+      l_dx = l_kx * g.dil;
+      l_tapbyte = (unsigned)(tap * g.c * 4);
+      enter_tap();
+    }
+  };
+  auto step = [&]() {
+    ++l_kt;
+    ++l_cc;
+    if (!PW && l_cc == g.cchunks) {
+      l_cc = 0;
+      l_tapbyte += (unsigned)(g.c * 4);
+      l_dx += g.dil;
+      if (++l_kx == g.k) {
+        l_kx = 0;
+        l_dx = 0;
+        l_dy += g.dil;
+      }
+      enter_tap();
+    }
+  };
+  // Requests the loads of the cursor's next stage.  Slabs past the end are zeros, and so are the filter's
+  // channels past the last; the input values that these meet are whatever comes next in memory (should
+  // that be infinite or NaN, the sums are found not finite and contracted again).
+  auto load = [&](u32x4 (&xa)[WR][2], u32x4 (&wb)[BP]) {
+    unsigned b_at[2];
+    int b_c[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const unsigned off = l_kt < kt_end ? 0u : kOutOfRange;
+      b_at[h] = l_tapbyte + (unsigned)l_cc * 64u;
+      b_c[h] = l_kt < kt_end ? g.c - l_cc * 16 : 0;   // channels left
+#pragma unroll
+      for (int i = 0; i < WR; ++i)
+        xa[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)((a_tap[i] | off) + (unsigned)l_cc * 64u), 0, 0);
+      step();
+    }
+    const unsigned at = bc & 4 ? b_at[1] : b_at[0];
+    const unsigned off = (bc & 3) * 4 < (bc & 4 ? b_c[1] : b_c[0]) ? 0u : kOutOfRange;
+#pragma unroll
+    for (int i = 0; i < BP; ++i)
+      wb[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)((b_row[i] | off) + at), 0, 0);
+    if (KG > 1) {
+#pragma unroll
+      for (int i = 0; i < 2 * (KG - 1); ++i) step();
+    }
+  };
+  // Splits filter values into the planes of buffer `buf`.  Row of 64 bytes: the 16 bytes of q = 0 .. 3; in
+  // rows 8 .. 15 of a block q and q ^ 2 change places, so that the 16 lanes an LDS cycle serves (same
+  // lane / 32, same parity of (lane >> 2) & 7) read 16 different columns of a 256-byte window.
+  auto store_b = [&](int buf, const u32x4 (&wb)[BP]) {
+#pragma unroll
+    for (int i = 0; i < BP; ++i) {
+      const int row = i * (TG / 8) + br;
+      if (B_PART && row >= BN) continue;
+      uint2 piece[3];
+      split_bf16(wb[i], piece);
+      unsigned char* at = planes + buf * STAGE + row * 64 + (((bc & 3) ^ ((row >> 2) & 2)) * 16) + (bc >> 2) * 8;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2*>(at + q * PLANE) = piece[q];
+    }
+  };
+
+  typedef floatx4v Acc;
+  Acc acc[WR][NB], rest[WR][NB];
+#pragma unroll
+  for (int i = 0; i < WR; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = rest[i][j] = Acc{0.f, 0.f, 0.f, 0.f};
+
+  // Splits a stage's input values and multiplies them with buffer `buf`.
+  auto multiply = [&](int buf, const bf16x8_t (&xp)[WR][3]) {
+    // blocks of channels whose operands are held at once (as registers allow)
+    constexpr int JB = NB % 2 == 0 && (PW || WR * NB < 16) ? 2 : 1;
+    const unsigned char* at = planes + buf * STAGE + lr * 64 + ((kq ^ ((lr >> 2) & 2)) * 16);
+#pragma unroll
+    for (int j0 = 0; j0 < NB; j0 += JB) {
+      bf16x8_t wp[JB][3];
+#pragma unroll
+      for (int j = 0; j < JB; ++j)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) wp[j][q] = *reinterpret_cast<const bf16x8_t*>(at + q * PLANE + (j0 + j) * 1024);
+      auto product = [&](Acc (&sum)[WR][NB], int qw, int qx) {
+#pragma unroll
+        for (int j = 0; j < JB; ++j)
+#pragma unroll
+          for (int i = 0; i < WR; ++i)
+            sum[i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wp[j][qw], xp[i][qx], sum[i][j0 + j], 0, 0, 0);
+      };
+      product(rest, 1, 1);
+      product(acc, 0, 0);
+      product(rest, 0, 2);
+      product(rest, 2, 0);
+      product(rest, 0, 1);
+      product(rest, 1, 0);
+    }
+  };
+  auto split_a = [&](const u32x4 (&xa)[WR][2], bf16x8_t (&xp)[WR][3]) {
+#pragma unroll
+    for (int i = 0; i < WR; ++i) {
+      uint2 lo[3], hi[3];
+      split_bf16(xa[i][0], lo);
+      split_bf16(xa[i][1], hi);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) xp[i][q] = __builtin_bit_cast(bf16x8_t, u32x4{lo[q].x, lo[q].y, hi[q].x, hi[q].y});
+    }
+  };
+
+  // Two register sets: the loads of stage s + 2 are requested when stage s has been split.  One barrier
+  // per stage: the planes of stage s + 1 are written while those of stage s are read.  Large tiles
+  // split the filter before they multiply, which frees its registers for the next loads (the other
+  // order spills: 11552 x 512 -> 1024 87 us instead of 68), small ones behind (19x19x512 -> 512, batch
+  // 16, 24.3 instead of 24.9; 3x3 56x56x64 -> 64 33.7 / 34.3).
+  {
+    constexpr bool SPLIT_FIRST = WR * NB >= 16;
+    u32x4 xa[2][WR][2], wb[2][BP];
+    bf16x8_t xp[WR][3];
+    // Pointwise ones, short as they can be, leave out what the last turns would do for nothing (75x75x64 ->
+    // 128 at batch 16 20.3 -> 18.7 us; the others lose by the branches, 3x3 28x28x128 -> 128 31.0 -> 34.7).
+    constexpr bool CUT = PW && KG == 1 && WM == 4 && WR == 1;
+    auto turn = [&](auto cur, int left) {
+      constexpr int C = decltype(cur)::value;
+      split_a(xa[C], xp);
+      if (SPLIT_FIRST) store_b(C ^ 1, wb[C ^ 1]);
+      if (!CUT || left > 2) load(xa[C], wb[C]);
+      if (SPLIT_FIRST) __builtin_amdgcn_sched_barrier(0);
+      multiply(C, xp);
+      if (!SPLIT_FIRST && (!CUT || left > 1)) store_b(C ^ 1, wb[C ^ 1]);
+      __syncthreads();
+    };
+    seek(kt_begin + 2 * kgroup);
+    load(xa[0], wb[0]);
+    load(xa[1], wb[1]);
+    store_b(0, wb[0]);
+    __syncthreads();
+    const int turns = (stages + KG - 1) / KG;
+    for (int t = 0; t + 1 < turns; t += 2) {
+      turn(std::integral_constant<int, 0>(), turns - t);
+      turn(std::integral_constant<int, 1>(), turns - t - 1);
+    }
+    if (turns & 1) turn(std::integral_constant<int, 0>(), 1);
+  }
+#pragma unroll
+  for (int i = 0; i < WR; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      asm volatile("" : "+v"(rest[i][j]));   // (the addition would be done in every turn of the loop)
+      acc[i][j] += rest[i][j];
+    }
+
+  // the K groups' sums, in order
+  auto add_groups = [&]() {
+    if constexpr (KG > 1) {
+      float4* const mine = reinterpret_cast<float4*>(lds) + tg;
+      for (int k = 1; k < KG; ++k) {
+        if (kgroup == k) {
+#pragma unroll
+          for (int i = 0; i < WR; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+              mine[(i * NB + j) * TG] = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+        }
+        __syncthreads();
+        if (kgroup == 0) {
+#pragma unroll
+          for (int i = 0; i < WR; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+              const float4 t = mine[(i * NB + j) * TG];
+              acc[i][j] += Acc{t.x, t.y, t.z, t.w};
+            }
+        }
+        __syncthreads();
+      }
+    }
+  };
+  add_groups();
+  if ((KG > 1 && kgroup != 0) || m0 >= g.m_total) return;
+
+  // A wave whose sums are not finite (an operand was infinite, NaN or so large that a piece overflowed)
+  // or so small that pieces may have been cut off contracts them again, in fp32.
+  {
+    float probe = 0.f;
+    unsigned low = 0xffffffffu;   // least magnitude of the sums that are not zero, as bits
+#pragma unroll
+    for (int i = 0; i < WR; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          probe = fmaf(acc[i][j][r], 0.f, probe);
+          low = min(low, (__float_as_uint(acc[i][j][r]) << 1) - 1u);
+        }
+    constexpr unsigned kLeast = (127u - 60u) << 24;   // 2^-60
+    const bool wrong = probe != 0.f || probe != probe || low < kLeast - 1u;
+    const bool again = __any(wrong);
+    if (again || (p.partial == nullptr && !__any(low != 0xffffffffu))) {
+      // v_mfma_f32_16x16x4_f32 four times per slab, both operands straight from memory
+#pragma unroll
+      for (int i = 0; i < WR; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = Acc{0.f, 0.f, 0.f, 0.f};
+      seek(kt_begin);
+#pragma unroll 1
+      while (l_kt < kt_end) {
+        const bool off = l_cc * 16 + kq * 4 >= g.c;
+        u32x4 xv[WR], wv[NB];
+#pragma unroll
+        for (int i = 0; i < WR; ++i)
+          xv[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, off ? (int)kOutOfRange : (int)(a_tap[i] + (unsigned)l_cc * 64u), 0, 0);
+        if (!again) {   // sums of nothing but zeros: most likely the input is zero here
+          unsigned bits = 0;
+#pragma unroll
+          for (int i = 0; i < WR; ++i) bits |= (xv[i][0] | xv[i][1] | xv[i][2] | xv[i][3]) & 0x7fffffffu;
+          if (!__any(bits != 0)) {
+            step();
+            continue;
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const int o = n0 + j * 16 + lr;
+          const unsigned at = (unsigned)o * krow_bytes + l_tapbyte + (unsigned)l_cc * 64u + kq * 16u;
+          wv[j] = __builtin_amdgcn_raw_buffer_load_b128(rw, off || o >= g.o ? (int)kOutOfRange : (int)at, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int i = 0; i < WR; ++i) WaveMma<float, 16>::run(wv[j], xv[i], acc[i][j]);
+        step();
+      }
+    }
+  }
+
+  // Results.  Split-K partial sums go to `partial` (rows of opitch floats, the channel count rounded up
+  // to 4); finished outputs to y or, with a second destination, channels [0, o1) to y and [o1, o) to y2.
+  // JC blocks of a wave's 16 pixels change places in LDS of its own, so that a store instruction writes
+  // whole runs of a pixel's channels (64 bytes of 16 pixels each, straight from the accumulators: 75x75x128
+  // -> 128 at batch 16 33.6 us instead of 31.9).
+  constexpr auto fits = [](int jc) { return NB % jc == 0 && WM * 16 * (jc * 16 + 4) * 4 <= pieces_lds_bytes<NB, KG>(); };
+  constexpr int JC = fits(4) ? 4 : fits(2) ? 2 : 1;
+  static_assert(fits(JC), "result staging exceeds the planes");
+  constexpr int PITCH = JC * 16 + 4, LPR = JC * 4, RPI = 64 / LPR;   // floats and lanes per row, rows per instruction
+  float* const mine = reinterpret_cast<float*>(lds) + wave * (16 * PITCH);
+  const int cv = lane % LPR, rsub = lane / LPR;
+  const int opitch = (g.o + 3) & ~3, o1 = p.o1, o2 = g.o - o1;
+  const bool whole = p.partial == nullptr;
+#pragma unroll
+  for (int i = 0; i < WR; ++i) {
+#pragma unroll
+    for (int j0 = 0; j0 < NB; j0 += JC) {
+#pragma unroll
+      for (int j = 0; j < JC; ++j) {
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          v[r] = acc[i][j0 + j][r];
+          if (whole) v[r] = apply_epilogue(v[r] + bias[(j0 + j) * 16 + kq * 4 + r], p.ep);
+        }
+        *reinterpret_cast<float4*>(mine + lr * PITCH + j * 16 + kq * 4) = make_float4(v[0], v[1], v[2], v[3]);
+      }
+      const int col = n0 + j0 * 16 + cv * 4;
+#pragma unroll
+      for (int it = 0; it < 16 / RPI; ++it) {
+        const float4 v = *reinterpret_cast<const float4*>(mine + (it * RPI + rsub) * PITCH + cv * 4);
+        const int row = m0 + i * 16 + it * RPI + rsub;
+        if (row >= g.m_total) continue;
+        if (!whole) {
+          if (col < opitch) store_result16(p.partial + ((long)split * g.m_total + row) * opitch + col, v);
+          continue;
+        }
+        // (a 16-byte store needs no more than 4-byte alignment)
+        float* const dst = static_cast<float*>(p.y) + out_row_offset(g, row, o1) + col;
+        float* const dst2 = static_cast<float*>(p.y2) + (long)row * o2 + (col - o1);
+        if (col + 4 <= o1) {
+          store_result16(dst, v);
+        } else if (col >= o1 && col + 4 <= g.o) {
+          store_result16(dst2, v);
+        } else {
+          const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (col + r < g.o) (col + r < o1 ? dst : dst2)[r] = e[r];
+        }
+      }
+    }
+  }
+}
+
+template <int WR, int NB, int WM, int KG, bool PW>
+__global__ __launch_bounds__(WM * KG * 64, 2) void conv_pieces_kernel(IgemmProblem p) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[pieces_lds_bytes<NB, KG>()];
+  pieces_tile<WR, NB, WM, KG, PW>(lds, p, (int)blockIdx.x);
 }
 
 template <typename T, int BM, int BN, int WM, int WN, int ROWB, bool PW>
@@ -749,12 +1061,12 @@ struct IgemmGroup {
   IgemmProblem p[kMaxGroup];
 };
 
-template <int BM, int BN, int WM, int WN, bool PW>
-__global__ __launch_bounds__(256, 2) void conv_igemm_group_split_kernel(IgemmGroup grp) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[igemm_lds_bytes<BM, BN, 64, true>()];
+template <int WR, int NB, int WM, int KG, bool PW>
+__global__ __launch_bounds__(WM * KG * 64, 2) void conv_pieces_group_kernel(IgemmGroup grp) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[pieces_lds_bytes<NB, KG>()];
   int i = 0;
   while (i + 1 < grp.count && (int)blockIdx.x >= grp.first[i + 1]) ++i;
-  igemm_tile_split<BM, BN, WM, WN, PW>(lds, grp.p[i], (int)blockIdx.x - grp.first[i]);
+  pieces_tile<WR, NB, WM, KG, PW>(lds, grp.p[i], (int)blockIdx.x - grp.first[i]);
 }
 
 template <typename T, int BM, int BN, int WM, int WN, int ROWB, bool PW>
@@ -784,32 +1096,33 @@ __device__ __forceinline__ void igemm_wave_tile(
 // and code than the others': a group without (the heads of one image) does without them as well.
 template <typename T, int ROWB, bool SPLIT>
 __global__ __launch_bounds__(256, SPLIT ? 3 : 1) void conv_igemm_mixed_kernel(IgemmGroup grp) {
-  constexpr int kLds = igemm_lds_bytes<128, 32, ROWB, SPLIT>();  // the largest of the tiles below
-  static_assert(kLds >= igemm_lds_bytes<128, 16, ROWB>() && kLds >= igemm_lds_bytes<64, 64, ROWB, SPLIT>(), "LDS size");
+  constexpr int kLds = SPLIT ? std::max(igemm_lds_bytes<128, 32, ROWB>(), pieces_lds_bytes<4, 2>())
+                             : igemm_lds_bytes<128, 32, ROWB>();  // the largest of the tiles below
+  static_assert(kLds >= igemm_lds_bytes<128, 16, ROWB>() && kLds >= igemm_lds_bytes<64, 64, ROWB>(), "LDS size");
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
   int i = 0;
   while (i + 1 < grp.count && (int)blockIdx.x >= grp.first[i + 1]) ++i;
   // a copy: with a use of the argument per path, the compiler keeps the whole group in scratch
   typename std::conditional<SPLIT, const IgemmProblem, const IgemmProblem&>::type p = grp.p[i];
   const int bid = (int)blockIdx.x - grp.first[i];
-#define OGLE_MIXED_TILE(PIECES, BM, BN, WM, WN, PW)                                             \
-  igemm_tile<T, BM, BN, WM, WN, ROWB, PW, PIECES>(                                              \
-      lds, p.g, static_cast<const T*>(p.x), static_cast<const T*>(p.w), p.bias,                 \
-      static_cast<T*>(p.y), static_cast<T*>(p.y2), p.o1, p.ep, p.tiles_n, p.tiles,              \
-      p.partial, p.slabs_per_split, p.splits, bid)
 #define OGLE_MIXED_CASE(V, BM, BN, WM, WN, PW)                                                  \
   case V:                                                                                       \
-    OGLE_MIXED_TILE(false, BM, BN, WM, WN, PW);                                                 \
+    igemm_tile<T, BM, BN, WM, WN, ROWB, PW>(                                                    \
+        lds, p.g, static_cast<const T*>(p.x), static_cast<const T*>(p.w), p.bias,               \
+        static_cast<T*>(p.y), static_cast<T*>(p.y2), p.o1, p.ep, p.tiles_n, p.tiles,            \
+        p.partial, p.slabs_per_split, p.splits, bid);                                           \
     break;
   if constexpr (SPLIT) {
-    bool done = false;
     switch (p.variant) {
-      case 16: done = OGLE_MIXED_TILE(true, 64, 64, 2, 2, false); break;
-      case 17: done = OGLE_MIXED_TILE(true, 64, 64, 2, 2, true); break;
-      case 18: done = OGLE_MIXED_TILE(true, 128, 32, 4, 1, false); break;
-      case 19: done = OGLE_MIXED_TILE(true, 128, 32, 4, 1, true); break;
+      case 16: pieces_tile<1, 4, 4, 1, false>(lds, p, bid); return;
+      case 17: pieces_tile<1, 4, 4, 1, true>(lds, p, bid); return;
+      case 18: pieces_tile<2, 2, 4, 1, false>(lds, p, bid); return;
+      case 19: pieces_tile<2, 2, 4, 1, true>(lds, p, bid); return;
+      case 20: pieces_tile<1, 4, 2, 2, false>(lds, p, bid); return;
+      case 21: pieces_tile<1, 4, 2, 2, true>(lds, p, bid); return;
+      case 22: pieces_tile<2, 1, 4, 1, false>(lds, p, bid); return;
+      case 23: pieces_tile<2, 1, 4, 1, true>(lds, p, bid); return;
     }
-    if (done) return;
   }
   switch (p.variant & 15) {
     OGLE_MIXED_CASE(0, 64, 64, 2, 2, false)
@@ -833,7 +1146,6 @@ __global__ __launch_bounds__(256, SPLIT ? 3 : 1) void conv_igemm_mixed_kernel(Ig
 #undef OGLE_MIXED_WAVE
   }
 #undef OGLE_MIXED_CASE
-#undef OGLE_MIXED_TILE
 }
 
 // ---------------------------------------------------------------------------
@@ -1132,11 +1444,22 @@ __global__ __launch_bounds__(256) void splitk_reduce_group_kernel(ReduceGroup gr
   }
 }
 
-// Grid size of one problem under the kernel's XCD-aware work layout.
+// Few tile rows spread unevenly over the XCDs: then each gets an eighth of the tiles, or of the (tile, K range)
+// pairs, in order.  17 rows of 12 128x64 tiles by rows give one XCD 36 for its 32 units (M = 2116, K = 864 ->
+// 768 channels 38.2 us, like this 26.5); 10x10x1024 -> 24, 3x3 at batch 64, with K ranges on XCDs 48.1 us, so 43.5.
+int work_layout(const IgemmPlan& p, int tiles_m) {
+  if (p.splits == 1) return rows_even(tiles_m) ? 1 : 0;
+  if (p.rows_on_xcd) return rows_even(tiles_m) ? -p.splits : -p.splits - kMaxSplits;
+  return p.splits;
+}
+
+// Grid size of one problem under that layout.
 unsigned grid_blocks(const IgemmPlan& p, int tiles_m, int tiles_n) {
   const int tiles = tiles_m * tiles_n;
-  if (p.splits == 1) return 8u * (unsigned)((tiles_m + 7) / 8) * (unsigned)tiles_n;
-  if (p.rows_on_xcd) return 8u * (unsigned)((tiles_m + 7) / 8) * (unsigned)tiles_n * (unsigned)p.splits;
+  if (p.splits == 1 || p.rows_on_xcd) {
+    if (rows_even(tiles_m)) return 8u * (unsigned)((tiles_m + 7) / 8) * (unsigned)tiles_n * (unsigned)p.splits;
+    return 8u * (unsigned)(((long)tiles * p.splits + 7) / 8);
+  }
   if (p.splits != 2 && p.splits != 4) return (unsigned)tiles * (unsigned)p.splits;
   const int xpz = 8 / p.splits;
   return 8u * (unsigned)((tiles + xpz - 1) / xpz);
@@ -1150,7 +1473,8 @@ struct Prepared {
   int reduce_lanes;
 };
 
-Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p) {
+// `form` in place of the plan's: what a problem runs as in a grouped launch.
+Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p, int form) {
   Prepared out{};
   ConvGeom& g = out.prob.g;
   g.n = a.n; g.h = a.in_h; g.w = a.in_w; g.c = a.in_c;
@@ -1163,8 +1487,10 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p) {
   g.x_bytes = (unsigned)((long)a.n * a.in_h * a.in_w * a.in_c * esz);
   g.w_bytes = (unsigned)((long)a.out_c * a.kernel_size * a.kernel_size * a.in_c * esz);
   g.oimg = a.out_image_stride == (long)a.out_h * a.out_w * a.out_c ? 0 : a.out_image_stride;
-  const int tiles_m = (g.m_total + tile_bm(p.cfg) - 1) / tile_bm(p.cfg);
-  const int tiles_n = (g.o + tile_bn(p.cfg) - 1) / tile_bn(p.cfg);
+  const int bm = form != FORM_NONE ? kFormBM[form] : tile_bm(p.cfg);
+  const int bn = form != FORM_NONE ? kFormBN[form] : tile_bn(p.cfg);
+  const int tiles_m = (g.m_total + bm - 1) / bm;
+  const int tiles_n = (g.o + bn - 1) / bn;
   out.prob.x = a.input_dev;
   out.prob.w = a.filter_dev;
   out.prob.bias = a.bias_dev;
@@ -1176,11 +1502,13 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p) {
   out.prob.tiles = tiles_m * tiles_n;
   out.prob.partial = p.splits > 1 ? static_cast<float*>(a.workspace_dev) : nullptr;
   out.prob.slabs_per_split = p.slabs_per_split;
-  out.prob.splits = p.rows_on_xcd ? -p.splits : p.splits;
-  out.prob.variant = (p.cfg == CFG_WAVE32 ? 4 : p.cfg == CFG_WAVE16 ? 6 : p.cfg == CFG_128x32 ? 2 :
+  out.prob.splits = work_layout(p, tiles_m);
+  out.prob.variant = (form == FORM_64x64 ? 16 : form == FORM_128x32 ? 18 : form == FORM_32x64_K2 ? 20 :
+                      form == FORM_128x16 ? 22 :
+                      p.cfg == CFG_WAVE32 ? 4 : p.cfg == CFG_WAVE16 ? 6 : p.cfg == CFG_128x32 ? 2 :
                       p.cfg == CFG_128x16 ? 8 : 0) +
-                     (is_pointwise(a) ? 1 : 0) + (p.pieces ? 16 : 0);
-  if (is_wave(p.cfg)) {
+                     (is_pointwise(a) ? 1 : 0);
+  if (is_wave(p.cfg) && form == FORM_NONE) {
     out.grid = (unsigned)(tiles_m * tiles_n);
     return out;
   }
@@ -1200,27 +1528,53 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p) {
   return out;
 }
 
-// Instantiates kernel `K<BM, BN, WM, WN, PW>` for a runtime (cfg, pw).
-#define OGLE_SPLIT_DISPATCH(K, cfg, pw, grid, s, arg)                                        \
-  do {                                                                                       \
-    if (pw) {                                                                                \
-      OGLE_SPLIT_DISPATCH_C(K, true, cfg, grid, s, arg)                                      \
-    } else {                                                                                 \
-      OGLE_SPLIT_DISPATCH_C(K, false, cfg, grid, s, arg)                                     \
-    }                                                                                        \
-  } while (0)
-#define OGLE_SPLIT_DISPATCH_C(K, PW, cfg, grid, s, arg)                                      \
-  switch (cfg) {                                                                             \
-    case CFG_128x128:                                                                        \
-      launch((K<128, 128, 2, 2, PW>), dim3(grid), dim3(256), 0, s, arg);                     \
-      break;                                                                                 \
-    case CFG_64x64:                                                                          \
-      launch((K<64, 64, 2, 2, PW>), dim3(grid), dim3(256), 0, s, arg);                       \
-      break;                                                                                 \
-    default:                                                                                 \
-      launch((K<128, 32, 4, 1, PW>), dim3(grid), dim3(256), 0, s, arg);                      \
-      break;                                                                                 \
+// The form a problem takes next to others in one launch: with 256 threads, adding in the same order.
+int grouped_form(int form) {
+  switch (form) {
+    case FORM_128x64:
+    case FORM_128x64_W8: return FORM_64x64;
+    case FORM_64x64_K2:
+    case FORM_64x32_K2: return FORM_32x64_K2;
+    default: return form;
   }
+}
+
+// Launches pieces kernel `K<WR, NB, WM, KG, PW>`.
+#define OGLE_PIECES_CASE(K, FORM, WR, NB, WM, KG)                                            \
+  case FORM:                                                                                 \
+    if (pw) launch((K<WR, NB, WM, KG, true>), dim3(grid), dim3(WM * KG * 64), 0, s, arg);    \
+    else launch((K<WR, NB, WM, KG, false>), dim3(grid), dim3(WM * KG * 64), 0, s, arg);      \
+    break;
+
+void launch_pieces(int form, bool pw, unsigned grid, hipStream_t s, const IgemmProblem& arg) {
+  switch (form) {
+    OGLE_PIECES_CASE(conv_pieces_kernel, FORM_64x64, 1, 4, 4, 1)
+    OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x32, 2, 2, 4, 1)
+    OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x16, 2, 1, 4, 1)
+    case FORM_128x128:   // pointwise only; the others have too many registers to keep
+      launch((conv_pieces_kernel<2, 8, 4, 1, true>), dim3(grid), dim3(256), 0, s, arg);
+      break;
+    OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x64_W8, 1, 4, 8, 1)
+    OGLE_PIECES_CASE(conv_pieces_kernel, FORM_64x64_K2, 1, 4, 4, 2)
+    OGLE_PIECES_CASE(conv_pieces_kernel, FORM_64x32_K2, 1, 2, 4, 2)
+    OGLE_PIECES_CASE(conv_pieces_kernel, FORM_32x64_K2, 1, 4, 2, 2)
+    OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x64, 2, 4, 4, 1)
+  }
+}
+
+// Several problems of one grouped form (and all pointwise or none).
+void launch_pieces_group(int form, bool pw, unsigned grid, hipStream_t s, const IgemmGroup& arg) {
+  switch (form) {
+    OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_64x64, 1, 4, 4, 1)
+    OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_128x32, 2, 2, 4, 1)
+    OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_128x16, 2, 1, 4, 1)
+    case FORM_128x128:
+      launch((conv_pieces_group_kernel<2, 8, 4, 1, true>), dim3(grid), dim3(256), 0, s, arg);
+      break;
+    OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_32x64_K2, 1, 4, 2, 2)
+  }
+}
+#undef OGLE_PIECES_CASE
 
 // Instantiates kernel `K<T, BM, BN, WM, WN, ROWB, PW>` for a runtime (dtype, cfg, pw).
 #define OGLE_IGEMM_DISPATCH(K, dtype, cfg, pw, grid, s, arg)                                 \
@@ -1259,14 +1613,10 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p) {
   }
 
 // One problem, one grid of the LDS-tiled kernel.
-void launch_single(int dtype, int cfg, bool pieces, bool pw, unsigned grid, hipStream_t s, const IgemmProblem& prob) {
+void launch_single(int dtype, int cfg, bool pw, unsigned grid, hipStream_t s, const IgemmProblem& prob) {
   if (cfg == CFG_128x256) {  // fp16 storage only (plan_igemm)
     if (pw) launch(conv_igemm_wide_f16_kernel<true>, dim3(grid), dim3(256), 0, s, prob);
     else launch(conv_igemm_wide_f16_kernel<false>, dim3(grid), dim3(256), 0, s, prob);
-    return;
-  }
-  if (pieces) {
-    OGLE_SPLIT_DISPATCH(conv_igemm_split_kernel, cfg, pw, grid, s, prob);
     return;
   }
   OGLE_IGEMM_DISPATCH(conv_igemm_kernel, dtype, cfg, pw, grid, s, prob);
@@ -1321,13 +1671,16 @@ int32_t launch_conv_igemm(const OgleConvArgs& a, hipStream_t s) {
   if (!igemm_eligible(a, &m)) return OGLE_ERR_UNSUPPORTED;
   if (f16_async_config(a) >= 0) return launch_pw_gemm_f16_async(a, s);
   const IgemmPlan p = final_plan(a, m);
-  const Prepared pr = prepare(a, m, p);
+  const Prepared pr = prepare(a, m, p, p.form);
   const bool pw = is_pointwise(a);
-  if (is_wave(p.cfg)) {
+  if (p.form != FORM_NONE) {
+    launch_pieces(p.form, pw, pr.grid, s, pr.prob);
+  } else if (is_wave(p.cfg)) {
     launch_wave(a.dtype, pw, p.cfg, pr, s);
     return check_launch("conv_igemm_wave");
+  } else {
+    launch_single(a.dtype, p.cfg, pw, pr.grid, s, pr.prob);
   }
-  launch_single(a.dtype, p.cfg, p.pieces, pw, pr.grid, s, pr.prob);
   int32_t st = check_launch("conv_igemm");
   if (st != OGLE_OK || p.splits == 1) return st;
   if (a.dtype == OGLE_F16) launch_reduce_single<__half>(pr, s);
@@ -1346,8 +1699,10 @@ int32_t launch_conv_batch(const OgleConvArgs* args, int count, hipStream_t s,
                           int32_t* reduce_pending) {
   struct Item {
     int dtype, cfg;
-    bool pieces, pw;
-    Prepared pr;
+    int own, form;        // alone, and next to others
+    bool pw;
+    Prepared alone, pr;
+    bool wave() const { return form == FORM_NONE && is_wave(cfg); }
   };
   std::vector<Item> items;
   for (int i = 0; i < count; ++i) {
@@ -1364,10 +1719,13 @@ int32_t launch_conv_batch(const OgleConvArgs* args, int count, hipStream_t s,
       continue;
     }
     const IgemmPlan p = final_plan(args[i], m);
-    items.push_back(Item{args[i].dtype, p.cfg, p.pieces, is_pointwise(args[i]), prepare(args[i], m, p)});
+    const int form = grouped_form(p.form);
+    items.push_back(Item{args[i].dtype, p.cfg, p.form, form, is_pointwise(args[i]), prepare(args[i], m, p, p.form),
+                         prepare(args[i], m, p, form)});
     if (reduce_pending != nullptr && p.splits > 1) reduce_pending[i] = 1;
   }
   auto mixable = [](const Item& it) {
+    if (it.form != FORM_NONE) return it.form != FORM_128x128;
     return it.cfg == CFG_64x64 || it.cfg == CFG_128x32 || it.cfg == CFG_128x16 || is_wave(it.cfg);
   };
   std::vector<bool> done(items.size(), false);
@@ -1380,11 +1738,12 @@ int32_t launch_conv_batch(const OgleConvArgs* args, int count, hipStream_t s,
     for (size_t b0 = a0; b0 < items.size() && grp.count < kMaxGroup; ++b0) {
       const Item& it = items[b0];
       if (done[b0] || it.dtype != head.dtype) continue;
-      const bool same = it.cfg == head.cfg && it.pw == head.pw && it.pieces == head.pieces && it.cfg != CFG_128x256;
+      const bool same = it.form == head.form && (it.form != FORM_NONE || it.cfg == head.cfg) && it.pw == head.pw &&
+                        it.cfg != CFG_128x256;
       if (b0 != a0 && (it.cfg == CFG_128x256 || head.cfg == CFG_128x256)) continue;  // fills the chip alone
       if (!same && !(mixable(head) && mixable(it))) continue;
       uniform = uniform && same;
-      pieces = pieces || it.pieces;
+      pieces = pieces || it.form != FORM_NONE;
       done[b0] = true;
       const Prepared& pr = it.pr;
       grp.first[grp.count + 1] = grp.first[grp.count] + (int)pr.grid;
@@ -1395,13 +1754,15 @@ int32_t launch_conv_batch(const OgleConvArgs* args, int count, hipStream_t s,
       }
     }
     const unsigned grid = (unsigned)grp.first[grp.count];
-    if (grp.count == 1 && is_wave(head.cfg)) {
+    if (grp.count == 1 && head.own != FORM_NONE) {
+      launch_pieces(head.own, head.pw, head.alone.grid, s, head.alone.prob);
+    } else if (grp.count == 1 && head.wave()) {
       launch_wave(head.dtype, head.pw, head.cfg, head.pr, s);
     } else if (grp.count == 1) {
-      launch_single(head.dtype, head.cfg, head.pieces, head.pw, grid, s, grp.p[0]);
-    } else if (uniform && head.pieces) {
-      OGLE_SPLIT_DISPATCH(conv_igemm_group_split_kernel, head.cfg, head.pw, grid, s, grp);
-    } else if (uniform && !is_wave(head.cfg)) {
+      launch_single(head.dtype, head.cfg, head.pw, grid, s, grp.p[0]);
+    } else if (uniform && head.form != FORM_NONE) {
+      launch_pieces_group(head.form, head.pw, grid, s, grp);
+    } else if (uniform && !head.wave()) {
       OGLE_IGEMM_DISPATCH(conv_igemm_group_kernel, head.dtype, head.cfg, head.pw, grid, s, grp);
     } else if (pieces) {
       launch((conv_igemm_mixed_kernel<float, kRowBytesF32, true>), dim3(grid), dim3(256), 0, s, grp);
@@ -1447,7 +1808,7 @@ int32_t launch_conv_reduce(const OgleConvArgs* args, int count, hipStream_t s) {
       if (p.splits <= 1) continue;
       if (dtype >= 0 && args[at].dtype != dtype) break;  // one storage type per grid
       dtype = args[at].dtype;
-      const Prepared pr = prepare(args[at], m, p);
+      const Prepared pr = prepare(args[at], m, p, p.form);
       red.first[red.count + 1] = red.first[red.count] + (int)pr.reduce_grid;
       red.p[red.count++] = pr.red;
     }

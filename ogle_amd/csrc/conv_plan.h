@@ -23,6 +23,19 @@ constexpr int kCfgBM[] = {128, 64, 128, 32, 16, 128, 128, 128, 128};
 constexpr int kCfgBN[] = {128, 64, 32, 32, 16, 96, 160, 256, 16};
 constexpr int kRowBytesF16Wide = 64;  // K bytes per tile row per slab of CFG_128x256
 
+// Workgroups that contract fp32 as bf16 pieces: rows x columns, four waves one above the other
+// unless named otherwise.  All but the K2 forms add an output's products in the same order.
+enum PiecesForm {
+  FORM_NONE = 0, FORM_64x64, FORM_128x32, FORM_128x128, FORM_128x64,
+  FORM_128x64_W8,    // eight waves of 16 rows
+  FORM_64x64_K2,     // two groups of four waves take K stages in turn
+  FORM_64x32_K2,
+  FORM_32x64_K2,     // two groups of two waves: the K2 forms in a grouped launch
+  FORM_128x16
+};
+constexpr int kFormBM[] = {0, 64, 128, 128, 128, 128, 64, 64, 32, 128};
+constexpr int kFormBN[] = {0, 64, 32, 128, 64, 64, 64, 32, 64, 16};
+
 struct IgemmPlan {
   int cfg;
   int splits;
@@ -31,12 +44,14 @@ struct IgemmPlan {
   int ktiles;
   int cchunks;
   size_t workspace_bytes;  // splits * M * N floats when splits > 1
-  bool pieces;             // fp32 contracted as bf16 pieces
+  bool pieces;             // fp32 contracted as bf16 pieces, in tiles of cfg
+  int form;                // the workgroup that runs such a tile, or one in place of cfg's (PiecesForm)
 };
 
 constexpr long kComputeUnits = 256;
 constexpr int kRowBytesF32 = 64;   // bytes of K per tile row per slab, fp32
 constexpr int kPiecesSlabs = 3;    // least slabs of a contraction as bf16 pieces
+constexpr int kMaxSplits = 64;     // most K ranges
 
 inline bool is_pointwise(const OgleConvArgs& a) {
   return a.kernel_size == 1 && a.stride == 1 && a.padding == 0;
@@ -45,6 +60,45 @@ inline bool is_pointwise(const OgleConvArgs& a) {
 inline bool is_wave(int cfg) { return cfg == CFG_WAVE32 || cfg == CFG_WAVE16; }
 inline int tile_bm(int cfg) { return kCfgBM[cfg]; }
 inline int tile_bn(int cfg) { return kCfgBN[cfg]; }
+
+// Whether whole tile rows spread evenly (within a tenth) over the eight XCDs.
+constexpr bool rows_even(long tiles_m) { return ((tiles_m + 7) / 8) * 8 * 10 <= tiles_m * 11; }
+
+// The form for `m` output rows: `large` a plan of 128x128 tiles, `pieces` whether 64x64 tiles would be
+// pieces.  What counts is how evenly the workgroups spread over 256 units, and that a unit has waves
+// enough to cover what each waits for.  Us of the form taken / of 64x64 tiles with four waves (and, with
+// at most 256 of those, of 64x64 fp32 tiles), 3x3 unless 1x1:
+//   64x32 K2, at most 256 of them: M = 6272, K = 576 -> 64 11.4 / 15.8 (13.4), 1x1 M = 400, 768 -> 200
+//     11.6 / 18.0 (14.5); where the last 64 columns are mostly padding: M = 8664, K = 432 -> 88 13.4 / 16.0
+//   64x64 K2: M = 3136, K = 1152 -> 256 21.9 / 26.1 (30.0), 1x1 M = 1444, 512 -> 512 11.1 / 14.1 (15.0),
+//     M = 22500, 1024 -> 40 30.4 / 36.3; K = 288 with at most 256 tiles 11.0 / 10.7 (11.2): the 64x64 ones
+//   128x64, eight waves: M = 50176, K = 576 -> 64 30.4 / 34.9, M = 12544, K = 1152 -> 128 31.8 / 34.6,
+//     M = 4704, K = 1872 -> 768 87.9 / 101.8, 1x1 M = 10000, 128 -> 384 10.9 / 11.9; between one and one
+//     and a half or above two workgroups per unit it is behind (M = 2400, K = 1024: 45.5 / 42.1)
+//   128x64: 1x1 M = 23104, 256 -> 256 24.8 / 27.5, 128 -> 256 15.7 / 17.4, M = 11552, 512 -> 512 41.7 / 45.6
+//   128x128: 1x1 M = 11552, 512 -> 1024 74.7 / 87.6 (128x64 78.2), but M = 12544, 512 -> 768, whose 588
+//     tiles leave two workgroups per unit a nearly empty second round, 71 (128x64 64)
+inline int pieces_form(const OgleConvArgs& a, long m, int ktiles, bool large, bool pieces) {
+  auto tiles = [&](int form) {
+    return ((m + kFormBM[form] - 1) / kFormBM[form]) * ((a.out_c + kFormBN[form] - 1) / kFormBN[form]);
+  };
+  const bool pw = is_pointwise(a);
+  const long n64 = tiles(FORM_64x64), n128 = tiles(FORM_128x64);
+  if (large) {
+    const long n = tiles(FORM_128x128), rounds = (n + 2 * kComputeUnits - 1) / (2 * kComputeUnits);
+    if (!pw) return FORM_128x64_W8;
+    return 20 * n >= 13 * rounds * 2 * kComputeUnits ? FORM_128x128 : FORM_128x64;
+  }
+  if (ktiles >= 12) {
+    const long n32 = tiles(FORM_64x32_K2);
+    if (n32 <= kComputeUnits || (2 * n32 <= 3 * n64 && n32 <= 2 * kComputeUnits)) return FORM_64x32_K2;
+    if (n64 <= kComputeUnits) return ktiles >= 24 ? FORM_64x64_K2 : ktiles >= 16 ? FORM_64x64 : FORM_NONE;
+    if (n128 <= kComputeUnits) return pw && ktiles >= 64 ? FORM_64x64_K2 : FORM_128x64_W8;
+  }
+  if (!pieces) return FORM_NONE;
+  if (pw && ktiles >= 8 && 2 * n128 >= 5 * kComputeUnits) return FORM_128x64;
+  return 2 * n128 >= 3 * kComputeUnits && n128 <= 2 * kComputeUnits ? FORM_128x64_W8 : FORM_64x64;
+}
 
 // Picks the output tile and the K split.  Problems with few output
 // tiles but a long contraction (the SSD heads, the small feature maps) are split
@@ -127,7 +181,7 @@ inline IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
     // take the s with the shortest estimated time, partial-sum traffic as the tie break.
     const double fixed = p.cfg == CFG_128x96 ? 6.0 : 4.0;
     double best = 1e30;
-    for (long s = 1; s <= 64 && p.ktiles / s >= 8; ++s) {
+    for (long s = 1; s <= kMaxSplits && p.ktiles / s >= 8; ++s) {
       const long rounds = (t * s + kComputeUnits - 1) / kComputeUnits;
       const double cost = (double)rounds * ((double)((p.ktiles + s - 1) / s) + fixed) + 0.25 * (double)s;
       if (cost < best - 1e-9) {
@@ -151,7 +205,7 @@ inline IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
     const long most = p.ktiles / 32;
     sp = want < most ? want : most;
   }
-  if (sp > 64) sp = 64;
+  if (sp > kMaxSplits) sp = kMaxSplits;
   // the kernel's XCD-aware work layout wants a divisor or a multiple of 8
   if (exact_split) {}
   else if (sp >= 8) sp -= sp % 8;
@@ -202,7 +256,8 @@ inline IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
   // are not built as such) where a compute unit has more than one workgroup and more than 16 slabs:
   // a lone workgroup has nothing to cover the splitting with, and a short sum is over before the faster
   // unit has made up for it.  Not for two slabs at all, nor for pointwise convolutions to at most 32
-  // channels: both are bound by their bytes.  Time with pieces over time with fp32 MFMAs, 64x64 tiles:
+  // channels: both are bound by their bytes.  Time with pieces (both operands split on their way to LDS; the
+  // present kernels are up to 15 % faster) over time with fp32 MFMAs, 64x64 tiles:
   //   slabs  workgroups to 384   512   768  1024  1536  2560  5000
   //     2         1.20  1.23  1.13  1.12  1.09  1.12  1.07
   //     3         1.12  1.13  1.07  1.03  0.99  0.98  0.90
@@ -219,6 +274,26 @@ inline IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
              workgroups > kComputeUnits && p.slabs_per_split >= kPiecesSlabs &&
              workgroups * p.slabs_per_split > 16 * kComputeUnits &&
              !(p.cfg == CFG_128x32 && is_pointwise(a));
+  if (a.dtype == OGLE_F32 && p.cfg == CFG_128x16 && p.splits == 1 && p.ktiles >= 12 && t <= kComputeUnits) {
+    // (75x75x64 -> 16 3x3 at batch 4 18.4 / 14.7, 19x19x512 -> 16 at batch 64 14.0 / 13.3; not with K ranges,
+    // which wait for the input, 19x19x512 -> 12 3x3 53 / 59, nor with more tiles, which do as well,
+    // 38x38x1024 -> 16 at batch 24 43.6 / 51.3)
+    p.form = FORM_128x16;
+  } else if (a.dtype != OGLE_F32 || p.splits > 1) {
+    p.form = !p.pieces ? FORM_NONE
+             : p.cfg == CFG_64x64 ? FORM_64x64
+             : p.cfg == CFG_128x32 ? FORM_128x32
+             : is_pointwise(a) ? FORM_128x128 : FORM_128x64_W8;
+  } else if (p.cfg == CFG_64x64 || p.cfg == CFG_128x128) {
+    p.form = pieces_form(a, m, p.ktiles, p.cfg == CFG_128x128, p.pieces);
+  } else if (p.cfg == CFG_128x32) {
+    p.form = p.pieces ? FORM_128x32 : FORM_NONE;
+  } else if (p.cfg == CFG_WAVE32 && is_pointwise(a) && p.ktiles >= 12) {
+    // two K groups against the wave-split kernel, where its 64x32 tiles are about one per unit: 1x1
+    // M = 1600, 1024 -> 256 14.9 / 16.4, M = 1444, 256 -> 256 6.1 / 6.8, M = 392, 208 -> 768 5.8 / 6.4
+    const long n32 = ((m + 63) / 64) * ((a.out_c + 31) / 32);
+    if (n32 <= kComputeUnits && 2 * n32 > kComputeUnits) p.form = FORM_64x32_K2;
+  }
   // Which operand an XCD's L2 should keep to itself: with K ranges pinned to XCDs the input is
   // fetched by all eight L2s and the filter by one, with tile rows pinned it is the other way
   // round (the rocprofv3 FETCH_SIZE of the 19x19x512 class head fell from 8.5x its input to
@@ -226,10 +301,7 @@ inline IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
   {
     const long x_bytes = (long)a.n * a.in_h * a.in_w * a.in_c * esz;
     const long w_bytes = (long)a.out_c * a.kernel_size * a.kernel_size * a.in_c * esz;
-    // whole tile rows per XCD: only when they spread evenly (within a tenth) over the eight
-    const long tiles_m = (m + kCfgBM[p.cfg] - 1) / kCfgBM[p.cfg];
-    const bool even = ((tiles_m + 7) / 8) * 8 * 10 <= tiles_m * 11;
-    p.rows_on_xcd = p.splits > 1 && !is_wave(p.cfg) && x_bytes > w_bytes && even;
+    p.rows_on_xcd = p.splits > 1 && !is_wave(p.cfg) && x_bytes > w_bytes;
   }
   return p;
 }

@@ -39,4 +39,10 @@ int probe_igemm(const OgleConvArgs* a, int scratch, int64_t* out) {
   for (int i = 0; i < 6; ++i) out[i] = v[i];
   return 1;
 }
+
+// How an fp32 convolution is contracted as bf16 pieces (PiecesForm); -1 if the implicit GEMM does not take it.
+int probe_form(const OgleConvArgs* a, int scratch) {
+  long m = 0;
+  return igemm_eligible(*a, &m) ? plan_igemm(*a, m, scratch != 0).form : -1;
+}
 }

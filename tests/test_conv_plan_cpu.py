@@ -209,3 +209,27 @@ def test_pieces_cases_run_what_they_name(probe):
     assert [[tile(*case) for case in batch] for batch in K.BATCHES_OF_PIECES] == [
         ["64x64 pieces"] * 2, ["128x32 pieces"] * 2, ["128x128 pieces"] * 2, ["64x64 pieces", "64x64"],
         ["64x64 split pieces", "128x16 split", "64x64", "128x32 pieces"]]
+
+
+def test_form_cases_run_what_they_name(probe):
+    """Every form of the pieces kernel is some case's (PiecesForm, conv_plan.h)."""
+    forms = [probe.probe_form(ctypes.byref(conv(*case)), 1) for case, _ in K.FORM_CASES]
+    assert forms == [form for _, form in K.FORM_CASES]
+    assert set(forms) == set(range(1, 10)) - {8}    # 8 is the K2 forms' in a grouped launch
+
+
+def test_forms_are_chosen_within_their_tiles(probe):
+    """128x128 workgroups are built for pointwise convolutions only; other types than fp32 have no form."""
+    r, seen = random.Random(11), set()
+    for _ in range(30000):
+        k = r.choice([1, 1, 3])
+        h = int(math.exp(r.uniform(1, 6)))
+        shape = (r.choice([1, 2, 16, 64]), h, h, 4 * r.choice([2, 3, 8, 9, 12, 16, 64, 128, 256]),
+                 r.choice([12, 31, 40, 65, 100, 128, 168, 256, 512, 1024]), k, r.choice([1, 2]), k // 2)
+        form = probe.probe_form(ctypes.byref(conv(*shape)), r.random() < 0.5)
+        seen.add(form)
+        if form == 3:
+            assert k == 1 and shape[6] == 1, shape
+        if shape[3] % 8 == 0:
+            assert probe.probe_form(ctypes.byref(conv(*shape, dtype=H.F16)), 1) <= 0
+    assert seen >= set(range(0, 10)) - {8}

@@ -374,6 +374,55 @@ def test_conv_fp32_as_bf16_pieces_of_tiny_operands(case, low, high, wlow):
     assert np.max(np.abs(got - ref) - kt * 2.0 ** -149 - (kt + 16) * 2.0 ** -24 * ref) <= 0
 
 
+FORM_CASES = [
+    # (n, h, w, c, o, k, s, p), PiecesForm   ragged rows and columns, odd stage counts, channels that end inside a slab
+    ((1, 97, 97, 32, 40, 3, 1, 1), 1),      # 64x64, at most one per unit, nine stages
+    ((16, 19, 19, 260, 500, 1, 1, 0), 1),   # 64x64, 17 slabs
+    ((5, 84, 84, 36, 31, 3, 1, 1), 2),      # 128x32
+    ((1, 223, 221, 260, 124, 1, 1, 0), 3),  # 128x128
+    ((1, 96, 97, 388, 520, 1, 1, 0), 4),    # 128x64
+    ((1, 119, 118, 36, 72, 3, 1, 1), 5),    # 128x64 of eight waves
+    ((1, 160, 160, 32, 255, 3, 1, 1), 5),   # the same in place of 128x128 tiles
+    ((1, 97, 97, 36, 40, 3, 1, 1), 6),      # 64x64, two K groups
+    ((4, 19, 19, 388, 512, 1, 1, 0), 6),    # the same, pointwise, 25 slabs
+    ((1, 66, 66, 44, 88, 3, 1, 1), 7),      # 64x32, two K groups
+    ((1, 133, 131, 44, 70, 3, 2, 1), 7),
+    ((2, 97, 98, 44, 12, 3, 1, 1), 9),      # 128x16
+    ((2, 97, 98, 200, 15, 1, 1, 0), 9),
+]
+
+
+@pytest.mark.parametrize("data", ["wide", "not finite", "zeros and tiny"])
+@pytest.mark.parametrize("case", [case for case, _ in FORM_CASES])
+def test_conv_fp32_pieces_forms(case, data):
+    """Each workgroup form of the pieces kernel, with finite operands of many magnitudes, with operands
+    whose pieces are no numbers, and with rows of zeros next to rows whose pieces are cut off.  Bound: a
+    rounding per 16 products (two allowed for) and a few at the end, relative to the sum of magnitudes;
+    half of 2^-149 per product and sum that are subnormal."""
+    n, h, w, c, o, k, s, p = case
+    r = rng(3190 + o + k)
+    x = (r.uniform(-1, 1, (n, h, w, c)) * 2.0 ** r.integers(-12, 12, (n, h, w, c))).astype(np.float32)
+    wt = (r.normal(0, 0.2, (o, c, k, k)) * 2.0 ** r.integers(-8, 8, (o, c, k, k))).astype(np.float32)
+    if data == "not finite":
+        x[0, 3, 4, 5], x[n - 1, h - 2, w - 3, c - 1], x[0, h // 2, 0, 0], x[0, 0, w - 1, 2] = np.inf, -np.inf, np.nan, 3.4e38
+    elif data == "zeros and tiny":
+        x[0, :h // 3] = 0
+        x[0, h // 3:2 * h // 3] *= np.float32(2.0 ** -118)
+    b = r.normal(0, 1, o).astype(np.float32) if data == "wide" else None
+    with np.errstate(over="ignore", invalid="ignore"):
+        ref, scale = _pieces_reference(x, wt, k, s, p), _pieces_reference(np.abs(x), np.abs(wt), k, s, p)
+    if b is not None:
+        ref, scale = ref + b, scale + np.abs(b)
+    for ws in (True, False):
+        got = gpu_conv(x, wt, b, s, p, workspace=ws, entry="ogle_hip_conv2d")
+        ok = np.isfinite(ref) & (scale < 1e38)
+        assert ok.mean() > 0.9 and (data != "not finite" or ok.mean() < 1)
+        over = np.abs(got[ok] - ref[ok]) - (k * k * c / 8 + 16) * 2.0 ** -24 * scale[ok] - k * k * c * 2.0 ** -149
+        assert np.max(over) <= 0, (case, ws)
+        bad = ~np.isfinite(ref)
+        np.testing.assert_array_equal(got[bad], ref[bad].astype(np.float32))
+
+
 WAVE_CASES = [
     # n, h, w, c, o, k, s, p, d   small problems with a long enough K: the wave-split kernel
     (1, 19, 19, 512, 512, 1, 1, 0, 1),    # 32x32 tiles, pointwise (a batch-1 MobileNet layer)
@@ -601,9 +650,15 @@ BATCHES_OF_PIECES = [
     # 64x64 and 128x32, with and without pieces
     [(8, 19, 19, 512, 63, 3, 1, 1), (8, 19, 19, 512, 12, 3, 1, 1), (2, 9, 9, 32, 40, 1, 1, 0), (5, 84, 84, 36, 31, 3, 1, 1)],
 ]
+# forms that another one stands in for in a group: two K groups alone, and all of them mixed
+BATCHES_OF_FORMS = [
+    [(1, 97, 97, 36, 40, 3, 1, 1), (1, 66, 66, 44, 88, 3, 1, 1)],
+    [(1, 119, 118, 36, 72, 3, 1, 1), (1, 66, 66, 44, 88, 3, 1, 1), (2, 97, 98, 44, 12, 3, 1, 1), (4, 19, 19, 388, 512, 1, 1, 0),
+     (1, 96, 97, 388, 520, 1, 1, 0), (1, 160, 160, 32, 255, 3, 1, 1), (3, 75, 73, 44, 70, 3, 2, 1)],
+]
 
 
-@pytest.mark.parametrize("cases", BATCHES_OF_PIECES)
+@pytest.mark.parametrize("cases", BATCHES_OF_PIECES + BATCHES_OF_FORMS)
 def test_conv_batch_of_pieces_equals_single_launches(cases):
     """Grouped launches of fp32 tiles contracted as bf16 pieces, one problem with an infinite and a
     large operand: exactly what one launch each gives."""
