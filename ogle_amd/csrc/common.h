@@ -131,6 +131,7 @@ __device__ __forceinline__ int xcd_swizzle(int pid, int grid) {
 // Launchers implemented in the .hip files (host side).
 int32_t launch_conv_igemm(const OgleConvArgs& a, hipStream_t s);   // returns OGLE_ERR_UNSUPPORTED if shape not eligible
 size_t conv_igemm_workspace_bytes(const OgleConvArgs& a);
+int32_t launch_conv_runs(const OgleConvArgs& a, hipStream_t s);    // the same: plan_runs
 bool conv_igemm_takes(const OgleConvArgs& a);  // launch_conv_igemm would not return OGLE_ERR_UNSUPPORTED
 int32_t launch_conv_igemm_static_scratch(const OgleConvArgs& a, hipStream_t s);
 // fp16-storage pointwise GEMM with operands streamed straight into LDS: the tile

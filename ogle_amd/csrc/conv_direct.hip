@@ -704,6 +704,10 @@ int32_t run_direct(const OgleConvArgs& a, hipStream_t s) {
 #undef OGLE_STEM_CASE
     return check_launch("conv_stem_mfma");
   }
+  if constexpr (sizeof(T) == 4) {
+    const int32_t st = launch_conv_runs(a, s);
+    if (st != OGLE_ERR_UNSUPPORTED) return st;
+  }
   PatchPlan plan;
   const DirectKernel kernel = plan_direct(a, &plan);
   if (kernel == DIRECT_PATCH) return launch_patch<T>(a, plan, ep, s);

@@ -58,6 +58,7 @@ struct ConvGeom {
   unsigned x_bytes;  // size of the input tensor (buffer-load range)
   unsigned w_bytes;  // size of the packed filter
   long oimg;         // elements between the outputs of consecutive images; 0: dense
+  int pixel;         // runs (pieces_tile): channels of a pixel, c being a run's values; else c
 };
 
 // Element offset of output row `row` (= (image, oy, ox) flattened) whose channels are
@@ -656,8 +657,17 @@ constexpr int pieces_lds_bytes() { return KG * 2 * 3 * NB * 1024; }
 // error against 64-bit sums at K = 512 1.24e-7 -> 1.20e-7 (fp32 MFMAs 4.1e-7).  Large problems are bound by
 // power: the library's bf16 GEMM of 8192 cubed reaches 1145 / 6 = 191.  Smaller ones share it among LDS
 // writes, splitting and MFMAs; loads further ahead, and splitting interleaved with MFMAs by hand, gained nothing.
-template <int WR, int NB, int WM, int KG, bool PW>
+//
+// MODE: KxK, whose slabs are channels of a tap; pointwise; or runs.  With no dilation the taps of a filter row
+// are one run of k * c values, in memory as in the filter, whatever the channel count: kRuns cuts that
+// run into slabs (g.c is its length, g.pixel the channels), so channel counts that fill no vector cost
+// one slab's rest per filter row.  Its 16-byte loads start on any value; waves with pixels whose run
+// reaches over the end of an image row clear what lies there, those at the tensor's ends load value by
+// value, and so does the filter, where the run's length is no multiple of four.
+enum PiecesMode { kKxK = 0, kPointwise = 1, kRuns = 2 };
+template <int WR, int NB, int WM, int KG, int MODE>
 __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, const IgemmProblem& p, int bid) {
+  constexpr bool PW = MODE == kPointwise, RUNS = MODE == kRuns;
   constexpr int BM = WM * WR * 16, BN = NB * 16;
   constexpr int TG = WM * 64;                          // threads of a K group
   constexpr int BP = (BN * 8 + TG - 1) / TG;           // 16-byte filter vectors a thread loads per stage
@@ -680,7 +690,8 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
 
   // this lane's pixels: their offset (PW), or that of their first tap, and its place
   unsigned a_base[WR], a_tap[WR];
-  int a_iy[WR], a_ix[WR];
+  int a_iy[WR], a_ix[WR];   // (runs: a_ix counts values, from the row's first)
+  bool edge = false, at_end = false;
 #pragma unroll
   for (int i = 0; i < WR; ++i) {
     const int m = m0 + i * 16 + lr;
@@ -694,12 +705,23 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
       const int b = t / g.oh;
       a_iy[i] = ok ? oy * g.stride - g.pad : -0x40000000;   // fails every in-image test
       a_ix[i] = ox * g.stride - g.pad;
-      a_base[i] = (unsigned)(((b * g.h + oy * g.stride - g.pad) * g.w + a_ix[i]) * g.c * 4) + kq * 16;
+      a_base[i] = (unsigned)(((b * g.h + oy * g.stride - g.pad) * g.w + a_ix[i]) * g.pixel * 4) + kq * 16;
+      if (RUNS) {
+        a_ix[i] *= g.pixel;
+        // (a 16-byte load with a value of the run must not begin before the tensor, nor end behind it)
+        const int low_row = min(g.h - 1, oy * g.stride - g.pad + g.k - 1);
+        const long end = (long)(b * g.h + low_row) * g.w * g.pixel + a_ix[i] + ((g.c + 3) & ~3);
+        edge = edge || (ok && (a_ix[i] < 0 || a_ix[i] + g.c > g.w * g.pixel));
+        at_end = at_end || (ok && (end * 4 > (long)g.x_bytes || (b == 0 && a_iy[i] <= 0 && a_ix[i] < 0)));
+        a_ix[i] += kq * 4;
+      }
     }
   }
   // this thread's filter rows and its place in the stage: vector bc of eight in a 128-byte row
   const int bc = tg & 7, br = tg >> 3;
-  const unsigned krow_bytes = (unsigned)(g.k * g.k * g.c * 4);
+  const unsigned krow_bytes = (unsigned)((RUNS ? g.k : g.k * g.k) * g.c * 4);
+  const int row_values = g.w * g.pixel;
+  const bool over_end = RUNS && __any(edge), by_value = RUNS && __any(at_end), b_by_value = RUNS && (g.c & 3) != 0;
   unsigned b_row[BP];
 #pragma unroll
   for (int i = 0; i < BP; ++i) {
@@ -717,10 +739,11 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
   int l_kt, l_cc, l_kx, l_dy, l_dx;
   unsigned l_tapbyte;
   auto enter_tap = [&]() {
-    const unsigned from = (unsigned)((l_dy * g.w + l_dx) * g.c * 4);
+    const unsigned from = (unsigned)((l_dy * g.w + (RUNS ? 0 : l_dx)) * g.pixel * 4);
 #pragma unroll
     for (int i = 0; i < WR; ++i) {
-      const bool in = (unsigned)(a_iy[i] + l_dy) < (unsigned)g.h && (unsigned)(a_ix[i] + l_dx) < (unsigned)g.w;
+      const bool in = (unsigned)(a_iy[i] + l_dy) < (unsigned)g.h &&
+                      (RUNS || (unsigned)(a_ix[i] + l_dx) < (unsigned)g.w);
       a_tap[i] = in ? a_base[i] + from : kOutOfRange;
     }
   };
@@ -730,9 +753,9 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
       l_cc = kt;
       l_tapbyte = 0;
     } else {
-      const int tap = kt / g.cchunks, ky = tap / g.k;
+      const int tap = kt / g.cchunks, ky = RUNS ? tap : tap / g.k;
       l_cc = kt - tap * g.cchunks;
-      l_kx = tap - ky * g.k;
+      l_kx = RUNS ? 0 : tap - ky * g.k;
       l_dy = ky * g.dil;
       l_dx = l_kx * g.dil;
       l_tapbyte = (unsigned)(tap * g.c * 4);
@@ -746,7 +769,7 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
       l_cc = 0;
       l_tapbyte += (unsigned)(g.c * 4);
       l_dx += g.dil;
-      if (++l_kx == g.k) {
+      if (RUNS || ++l_kx == g.k) {
         l_kx = 0;
         l_dx = 0;
         l_dy += g.dil;
@@ -765,16 +788,36 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
       const unsigned off = l_kt < kt_end ? 0u : kOutOfRange;
       b_at[h] = l_tapbyte + (unsigned)l_cc * 64u;
       b_c[h] = l_kt < kt_end ? g.c - l_cc * 16 : 0;   // channels left
+      if (by_value) {
 #pragma unroll
-      for (int i = 0; i < WR; ++i)
-        xa[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)((a_tap[i] | off) + (unsigned)l_cc * 64u), 0, 0);
+        for (int i = 0; i < WR; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            // (below zero before the tensor; as part of an instruction's offset it would not wrap around)
+            const int at = (int)((a_tap[i] | off) + (unsigned)l_cc * 64u + e * 4u);
+            xa[i][h][e] = __builtin_amdgcn_raw_buffer_load_b32(rx, at < 0 ? (int)kOutOfRange : at, 0, 0);
+          }
+      } else {
+#pragma unroll
+        for (int i = 0; i < WR; ++i)
+          xa[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)((a_tap[i] | off) + (unsigned)l_cc * 64u), 0, 0);
+      }
       step();
     }
     const unsigned at = bc & 4 ? b_at[1] : b_at[0];
-    const unsigned off = (bc & 3) * 4 < (bc & 4 ? b_c[1] : b_c[0]) ? 0u : kOutOfRange;
+    const int left = (bc & 4 ? b_c[1] : b_c[0]) - (bc & 3) * 4;
+    const unsigned off = left > 0 ? 0u : kOutOfRange;
+    if (b_by_value) {
 #pragma unroll
-    for (int i = 0; i < BP; ++i)
-      wb[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)((b_row[i] | off) + at), 0, 0);
+      for (int i = 0; i < BP; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          wb[i][e] = __builtin_amdgcn_raw_buffer_load_b32(rw, (int)(left > e ? b_row[i] + at + e * 4u : kOutOfRange), 0, 0);
+    } else {
+#pragma unroll
+      for (int i = 0; i < BP; ++i)
+        wb[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)((b_row[i] | off) + at), 0, 0);
+    }
     if (KG > 1) {
 #pragma unroll
       for (int i = 0; i < 2 * (KG - 1); ++i) step();
@@ -830,7 +873,24 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
       product(rest, 1, 0);
     }
   };
-  auto split_a = [&](const u32x4 (&xa)[WR][2], bf16x8_t (&xp)[WR][3]) {
+  int c_cc = 0;   // runs: the slab within the run that is split next
+  auto split_a = [&](u32x4 (&xa)[WR][2], bf16x8_t (&xp)[WR][3]) {
+    if (RUNS) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (over_end) {
+#pragma unroll
+          for (int i = 0; i < WR; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if ((unsigned)(a_ix[i] + c_cc * 16 + e) >= (unsigned)row_values) xa[i][h][e] = 0u;
+        }
+        if (++c_cc == g.cchunks) c_cc = 0;
+      }
+#pragma unroll
+      for (int q = 0; q < 2 * (KG - 1); ++q)
+        if (++c_cc == g.cchunks) c_cc = 0;
+    }
 #pragma unroll
     for (int i = 0; i < WR; ++i) {
       uint2 lo[3], hi[3];
@@ -864,6 +924,7 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
       __syncthreads();
     };
     seek(kt_begin + 2 * kgroup);
+    c_cc = l_cc;
     load(xa[0], wb[0]);
     load(xa[1], wb[1]);
     store_b(0, wb[0]);
@@ -929,7 +990,31 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
     constexpr unsigned kLeast = (127u - 60u) << 24;   // 2^-60
     const bool wrong = probe != 0.f || probe != probe || low < kLeast - 1u;
     const bool again = __any(wrong);
-    if (again || (p.partial == nullptr && !__any(low != 0xffffffffu))) {
+    if (RUNS && __any(probe != 0.f || probe != probe)) {
+      // taps outside the image contribute nothing, also where a filter value is infinite: value by value
+#pragma unroll
+      for (int i = 0; i < WR; ++i) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = Acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int ky = 0; ky < g.k; ++ky) {
+          if ((unsigned)(a_iy[i] + ky) >= (unsigned)g.h) continue;
+          const unsigned x_row = a_base[i] - kq * 16u + (unsigned)(ky * row_values * 4);
+#pragma unroll 1
+          for (int q = 0; q < g.c; ++q) {
+            if ((unsigned)(a_ix[i] - kq * 4 + q) >= (unsigned)row_values) continue;
+            const float xv = *reinterpret_cast<const float*>(static_cast<const char*>(p.x) + (x_row + q * 4u));
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const int o = n0 + j * 16 + kq * 4 + r;
+                if (o < g.o) acc[i][j][r] += xv * static_cast<const float*>(p.w)[((long)o * g.k + ky) * g.c + q];
+              }
+          }
+        }
+      }
+    } else if (again || (p.partial == nullptr && !__any(low != 0xffffffffu))) {
       // v_mfma_f32_16x16x4_f32 four times per slab, both operands straight from memory
 #pragma unroll
       for (int i = 0; i < WR; ++i)
@@ -941,8 +1026,18 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
         const bool off = l_cc * 16 + kq * 4 >= g.c;
         u32x4 xv[WR], wv[NB];
 #pragma unroll
-        for (int i = 0; i < WR; ++i)
-          xv[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, off ? (int)kOutOfRange : (int)(a_tap[i] + (unsigned)l_cc * 64u), 0, 0);
+        for (int i = 0; i < WR; ++i) {
+          if (!RUNS) {
+            xv[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, off ? (int)kOutOfRange : (int)(a_tap[i] + (unsigned)l_cc * 64u), 0, 0);
+            continue;
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const bool in = (unsigned)(a_ix[i] + l_cc * 16 + e) < (unsigned)row_values && l_cc * 16 + kq * 4 + e < g.c;
+            const int at = (int)(a_tap[i] + (unsigned)l_cc * 64u + e * 4u);
+            xv[i][e] = __builtin_amdgcn_raw_buffer_load_b32(rx, in && at >= 0 ? at : (int)kOutOfRange, 0, 0);
+          }
+        }
         if (!again) {   // sums of nothing but zeros: most likely the input is zero here
           unsigned bits = 0;
 #pragma unroll
@@ -956,7 +1051,14 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
         for (int j = 0; j < NB; ++j) {
           const int o = n0 + j * 16 + lr;
           const unsigned at = (unsigned)o * krow_bytes + l_tapbyte + (unsigned)l_cc * 64u + kq * 16u;
-          wv[j] = __builtin_amdgcn_raw_buffer_load_b128(rw, off || o >= g.o ? (int)kOutOfRange : (int)at, 0, 0);
+          if (!RUNS) {
+            wv[j] = __builtin_amdgcn_raw_buffer_load_b128(rw, off || o >= g.o ? (int)kOutOfRange : (int)at, 0, 0);
+            continue;
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            wv[j][e] = __builtin_amdgcn_raw_buffer_load_b32(
+                rw, l_cc * 16 + kq * 4 + e < g.c && o < g.o ? (int)(at + e * 4u) : (int)kOutOfRange, 0, 0);
         }
 #pragma unroll
         for (int j = 0; j < NB; ++j)
@@ -1022,10 +1124,10 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
   }
 }
 
-template <int WR, int NB, int WM, int KG, bool PW>
+template <int WR, int NB, int WM, int KG, int MODE>
 __global__ __launch_bounds__(WM * KG * 64, 2) void conv_pieces_kernel(IgemmProblem p) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[pieces_lds_bytes<NB, KG>()];
-  pieces_tile<WR, NB, WM, KG, PW>(lds, p, (int)blockIdx.x);
+  pieces_tile<WR, NB, WM, KG, MODE>(lds, p, (int)blockIdx.x);
 }
 
 template <typename T, int BM, int BN, int WM, int WN, int ROWB, bool PW>
@@ -1480,6 +1582,7 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p, int form) {
   g.n = a.n; g.h = a.in_h; g.w = a.in_w; g.c = a.in_c;
   g.oh = a.out_h; g.ow = a.out_w; g.o = a.out_c;
   g.k = a.kernel_size; g.stride = a.stride; g.pad = a.padding; g.dil = a.dilation;
+  g.pixel = g.c;
   g.m_total = (int)m;
   g.cchunks = p.cchunks;
   g.ktiles = p.ktiles;
@@ -1560,6 +1663,23 @@ void launch_pieces(int form, bool pw, unsigned grid, hipStream_t s, const IgemmP
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_32x64_K2, 1, 4, 2, 2)
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x64, 2, 4, 4, 1)
   }
+}
+
+// Launches the convolutions of plan_runs.
+void launch_runs(int form, unsigned grid, hipStream_t s, const IgemmProblem& arg) {
+#define OGLE_RUNS_CASE(FORM, WR, NB, WM, KG)                                                          \
+  case FORM:                                                                                          \
+    launch((conv_pieces_kernel<WR, NB, WM, KG, kRuns>), dim3(grid), dim3(WM * KG * 64), 0, s, arg);   \
+    break;
+  switch (form) {
+    OGLE_RUNS_CASE(FORM_64x64, 1, 4, 4, 1)
+    OGLE_RUNS_CASE(FORM_128x32, 2, 2, 4, 1)
+    OGLE_RUNS_CASE(FORM_128x16, 2, 1, 4, 1)
+    OGLE_RUNS_CASE(FORM_128x64_W8, 1, 4, 8, 1)
+    OGLE_RUNS_CASE(FORM_64x64_K2, 1, 4, 4, 2)
+    OGLE_RUNS_CASE(FORM_64x32_K2, 1, 2, 4, 2)
+  }
+#undef OGLE_RUNS_CASE
 }
 
 // Several problems of one grouped form (and all pointwise or none).
@@ -1686,6 +1806,16 @@ int32_t launch_conv_igemm(const OgleConvArgs& a, hipStream_t s) {
   if (a.dtype == OGLE_F16) launch_reduce_single<__half>(pr, s);
   else launch_reduce_single<float>(pr, s);
   return check_launch("splitk_reduce");
+}
+
+int32_t launch_conv_runs(const OgleConvArgs& a, hipStream_t s) {
+  IgemmPlan p{};
+  if (!plan_runs(a, &p)) return OGLE_ERR_UNSUPPORTED;
+  Prepared pr = prepare(a, (long)a.n * a.out_h * a.out_w, p, p.form);
+  ConvGeom& g = pr.prob.g;
+  g.c = a.in_c * a.kernel_size;
+  launch_runs(p.form, pr.grid, s, pr.prob);
+  return check_launch("conv_pieces_runs");
 }
 
 // Launches `count` mutually independent convolutions.  Those the implicit-GEMM

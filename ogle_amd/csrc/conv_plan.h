@@ -322,6 +322,41 @@ inline bool igemm_eligible(const OgleConvArgs& a, long* m_out) {
   return true;
 }
 
+// Ungrouped fp32 convolutions whose channels fill no vector, contracted as bf16 pieces out of the runs of
+// values that their filter rows are (pieces_tile).
+inline bool plan_runs(const OgleConvArgs& a, IgemmPlan* out) {
+  const int k = a.kernel_size;
+  if (a.dtype != OGLE_F32 || a.group != 1 || (a.dilation != 1 && k > 1)) return false;
+  const long m = (long)a.n * a.out_h * a.out_w, run = (long)k * a.in_c, lim = 0x7fffffffL;
+  if (m <= 0 || m > lim || run > lim / 64) return false;
+  if ((long)a.n * a.in_h * a.in_w * a.in_c * 4 > lim || (long)a.out_c * k * run * 4 > lim) return false;
+  // a pixel's first value, in the padding or not, is counted in 32 bits too
+  if (((long)a.in_w + 2L * a.padding + k) * a.in_c > lim / 4 || (long)a.padding * a.in_w * a.in_c * 4 > lim / 4) return false;
+  IgemmPlan p{};
+  p.cfg = CFG_64x64;
+  p.splits = 1;
+  p.cchunks = (int)((run + 15) / 16);
+  p.ktiles = p.slabs_per_split = k * p.cchunks;
+  // Against the direct kernels: a fit of 700 shapes (1x1, 3x3, 5x5, 5 to 181 channels); a chain of products
+  // takes them 0.08 us each, many products their rate.  Narrow outputs leave little of the work that gathering a
+  // pixel's values is worth.  Us with the direct kernels / like this, 3x3 unless noted: 4 x 56 x 56, 99 -> 99
+  // 95 / 45; 16 x 40 x 40, 1x1 131 -> 77 45 / 18; 16 x 224 x 224, 7x7 stride 2 3 -> 64 99 / 58; 4 x 4 x 4, 21 ->
+  // 16 16.5 / 9.5, but 22 x 49 x 47, 149 -> 5 71 / 103, 8 x 7 x 7, 1x1 39 -> 37 5.5 / 7.1.  (The faster each time
+  // would be 0.711 of the direct kernels' time in the mean, the rule 0.753.)
+  const double products = (double)m * a.out_c * k * run;
+  const double chain = (double)a.in_c * std::min(k, a.in_h) * std::min(k, a.in_w);
+  if (k * run < 24 || 0.07 * chain + 0.2e-6 * products <= 3 + 0.15 * p.ktiles) return false;
+  if (a.out_c <= 32 && k > 1 && (a.out_c <= 16 || products < 3e7)) return false;
+  if (a.out_c <= 32) p.form = a.out_c <= 16 ? FORM_128x16 : FORM_128x32;
+  else p.form = pieces_form(a, m, p.ktiles, false, true);
+  if (p.form == FORM_NONE || p.form == FORM_128x64) p.form = FORM_64x64;
+  // with many tiles the filter, gathered value by value, counts: half as often per pixel (the 7x7 stem 62.6 / 58.4,
+  // 13 x 78 x 98, 33 -> 64 3x3 54.1 / 50.1)
+  if (p.form == FORM_64x64 && m * a.out_c > 64L * 64 * 5 * kComputeUnits) p.form = FORM_128x64_W8;
+  *out = p;
+  return true;
+}
+
 // The plan the launch will use: split-K only with a workspace that is large enough.
 inline IgemmPlan final_plan(const OgleConvArgs& a, long m) {
   IgemmPlan p = plan_igemm(a, m, a.workspace_dev != nullptr);

@@ -45,4 +45,11 @@ int probe_form(const OgleConvArgs* a, int scratch) {
   long m = 0;
   return igemm_eligible(*a, &m) ? plan_igemm(*a, m, scratch != 0).form : -1;
 }
+
+// The form that contracts the runs of an ungrouped fp32 convolution of the direct kernels; -1: one of those does.
+int probe_runs(const OgleConvArgs* a) {
+  long m = 0;
+  IgemmPlan p;
+  return !igemm_eligible(*a, &m) && plan_runs(*a, &p) ? p.form : -1;
+}
 }

@@ -233,3 +233,22 @@ def test_forms_are_chosen_within_their_tiles(probe):
         if shape[3] % 8 == 0:
             assert probe.probe_form(ctypes.byref(conv(*shape, dtype=H.F16)), 1) <= 0
     assert seen >= set(range(0, 10)) - {8}
+
+
+def test_runs_cases_run_what_they_name(probe):
+    forms = [probe.probe_runs(ctypes.byref(conv(*case))) for case, _ in K.RUNS_CASES]
+    assert forms == [form for _, form in K.RUNS_CASES]
+    assert set(forms) == {1, 2, 5, 6, 7, 9}
+
+
+@pytest.mark.parametrize("shape,kw", [
+    ((16, 19, 19, 99, 99, 3, 1, 2, 2), {}),              # dilated
+    ((4, 48, 48, 99, 99, 3, 1, 1, 1, 3), {}),            # grouped
+    ((4, 56, 56, 99, 99, 3, 1, 1), dict(dtype=H.F16)),
+    ((8, 7, 7, 39, 37, 1), {}),                          # short sums of a small output
+    ((22, 49, 47, 149, 5, 3, 1, 1), {}),                 # five channels out
+    ((1, 1000, 1000, 511, 40, 1, 1, 2000), {}),          # an output beyond 2^31 bytes is fine, padding that long is not
+    ((3, 16000, 16000, 3, 64, 7, 2, 3), {}),             # an input beyond 2^31 bytes
+])
+def test_runs_leave_to_the_direct_kernels(probe, shape, kw):
+    assert probe.probe_runs(ctypes.byref(conv(*shape, **kw))) == -1

@@ -423,6 +423,63 @@ def test_conv_fp32_pieces_forms(case, data):
         np.testing.assert_array_equal(got[bad], ref[bad].astype(np.float32))
 
 
+RUNS_CASES = [
+    # (n, h, w, c, o, k, s, p), PiecesForm   channels that fill no vector, filter rows as runs of values
+    ((2, 70, 75, 3, 70, 7, 2, 3), 7),       # a run of 21; rows that begin and end in the padding
+    ((9, 70, 75, 3, 70, 7, 1, 3), 1),
+    ((1, 100, 101, 45, 64, 3, 1, 1), 6),    # a run of 135, 27 slabs
+    ((1, 119, 118, 37, 72, 3, 1, 1), 5),
+    ((16, 90, 90, 5, 70, 3, 1, 1), 5),      # many tiles
+    ((4, 12, 2, 37, 100, 3, 1, 1), 7),      # a run longer than an image row
+    ((2, 9, 1, 181, 40, 3, 1, 1), 7),       # one column: two of three taps in the padding
+    ((8, 37, 39, 33, 66, 1, 1, 0), 1),      # 1x1: the tensor ends inside a slab
+    ((3, 33, 35, 131, 77, 1, 2, 0), 1),
+    ((2, 40, 41, 67, 31, 3, 1, 1), 2),
+    ((7, 40, 41, 130, 15, 1, 1, 0), 9),     # two values past a vector
+    ((1, 64, 66, 1, 96, 9, 1, 4), 1),       # one channel
+    ((2, 31, 30, 22, 90, 3, 2, 0), 7),      # no padding, a run of 66
+]
+
+
+@pytest.mark.parametrize("data", ["wide", "not finite", "infinite filter", "zeros and tiny"])
+@pytest.mark.parametrize("case", [case for case, _ in RUNS_CASES])
+def test_conv_fp32_runs(case, data):
+    """Bounds as in test_conv_fp32_pieces_forms.  A filter value that is infinite shows only where its tap lies
+    inside the image."""
+    n, h, w, c, o, k, s, p = case
+    r = rng(3230 + o + k)
+    x = (r.uniform(-1, 1, (n, h, w, c)) * 2.0 ** r.integers(-12, 12, (n, h, w, c))).astype(np.float32)
+    wt = (r.normal(0, 0.2, (o, c, k, k)) * 2.0 ** r.integers(-8, 8, (o, c, k, k))).astype(np.float32)
+    inf = np.zeros((o, c, k, k), bool)
+    if data == "not finite":
+        x[0, 1, 0, 0], x[n - 1, h - 2, w - 1, c - 1], x[0, h // 2, 0, 0], x[0, 0, w - 1, 0] = np.inf, -np.inf, np.nan, 3.4e38
+    elif data == "infinite filter":
+        inf[o - 1, 0, 0, 0] = inf[3, c - 1, k - 1, k - 1] = inf[o // 2, 0, k // 2, k - 1] = True
+    elif data == "zeros and tiny":
+        x[0, :h // 3] = 0
+        x[0, h // 3:2 * h // 3] *= np.float32(2.0 ** -118)
+    b = r.normal(0, 1, o).astype(np.float32) if data == "wide" else None
+    with np.errstate(over="ignore", invalid="ignore"):
+        ref, scale = _pieces_reference(x, wt, k, s, p), _pieces_reference(np.abs(x), np.abs(wt), k, s, p)
+    if b is not None:
+        ref, scale = ref + b, scale + np.abs(b)
+    ok = np.isfinite(ref) & (scale < 1e38)
+    if data == "infinite filter":   # which outputs have such a tap inside the image
+        hit = _pieces_reference(np.ones_like(x), inf.astype(np.float32), k, s, p) > 0
+        ok &= ~hit
+        wt[inf] = np.inf
+    got = gpu_conv(x, wt, b, s, p, entry="ogle_hip_conv2d")
+    assert ok.any() and (ok.all() or data in ("not finite", "infinite filter"))
+    over = np.abs(got[ok] - ref[ok]) - (k * k * c / 8 + 16) * 2.0 ** -24 * scale[ok] - k * k * c * 2.0 ** -149
+    assert np.max(over) <= 0, case
+    if data == "infinite filter":
+        assert not np.isfinite(got[hit]).any()
+    else:
+        # (next to an infinite product, one of 3.4e38 and up that overflows fp32 makes NaN of it: not compared)
+        bad = ~np.isfinite(ref) & (_pieces_reference(np.where(np.isfinite(x), np.abs(x), 0), np.abs(wt), k, s, p) < 1e38)
+        np.testing.assert_array_equal(got[bad], ref[bad].astype(np.float32))
+
+
 WAVE_CASES = [
     # n, h, w, c, o, k, s, p, d   small problems with a long enough K: the wave-split kernel
     (1, 19, 19, 512, 512, 1, 1, 0, 1),    # 32x32 tiles, pointwise (a batch-1 MobileNet layer)
