@@ -973,99 +973,134 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
   add_groups();
   if ((KG > 1 && kgroup != 0) || m0 >= g.m_total) return;
 
-  // A wave whose sums are not finite (an operand was infinite, NaN or so large that a piece overflowed)
-  // or so small that pieces may have been cut off contracts them again, in fp32.
+  // Sums that are not finite (an operand was infinite, NaN or so large that a piece overflowed) or so small
+  // that pieces may have been cut off are contracted again, in fp32: 16 pixels x 32 channels at a time, so
+  // that an output does not depend on the form that computed it.
   {
-    float probe = 0.f;
-    unsigned low = 0xffffffffu;   // least magnitude of the sums that are not zero, as bits
+    constexpr int UJ = NB % 2 == 0 ? 2 : 1;
+    constexpr unsigned kLeast = (127u - 60u) << 24;   // 2^-60
+    // `low`: least magnitude of the sums that are not zero, as bits
+    auto look = [&](int i, int j0, float& probe, unsigned& low) {
 #pragma unroll
-    for (int i = 0; i < WR; ++i)
-#pragma unroll
-      for (int j = 0; j < NB; ++j)
+      for (int j = j0; j < j0 + UJ; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           probe = fmaf(acc[i][j][r], 0.f, probe);
           low = min(low, (__float_as_uint(acc[i][j][r]) << 1) - 1u);
         }
-    constexpr unsigned kLeast = (127u - 60u) << 24;   // 2^-60
-    const bool wrong = probe != 0.f || probe != probe || low < kLeast - 1u;
-    const bool again = __any(wrong);
-    if (RUNS && __any(probe != 0.f || probe != probe)) {
-      // taps outside the image contribute nothing, also where a filter value is infinite: value by value
+    };
+    float probe_all = 0.f;
+    unsigned low_all = 0xffffffffu, low_most = 0;   // over all units, and of the unit where it is largest
 #pragma unroll
-      for (int i = 0; i < WR; ++i) {
+    for (int i = 0; i < WR; ++i)
 #pragma unroll
-        for (int j = 0; j < NB; ++j) acc[i][j] = Acc{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-        for (int ky = 0; ky < g.k; ++ky) {
-          if ((unsigned)(a_iy[i] + ky) >= (unsigned)g.h) continue;
-          const unsigned x_row = a_base[i] - kq * 16u + (unsigned)(ky * row_values * 4);
-#pragma unroll 1
-          for (int q = 0; q < g.c; ++q) {
-            if ((unsigned)(a_ix[i] - kq * 4 + q) >= (unsigned)row_values) continue;
-            const float xv = *reinterpret_cast<const float*>(static_cast<const char*>(p.x) + (x_row + q * 4u));
-#pragma unroll
-            for (int j = 0; j < NB; ++j)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                const int o = n0 + j * 16 + kq * 4 + r;
-                if (o < g.o) acc[i][j][r] += xv * static_cast<const float*>(p.w)[((long)o * g.k + ky) * g.c + q];
-              }
-          }
-        }
+      for (int j0 = 0; j0 < NB; j0 += UJ) {
+        unsigned low = 0xffffffffu;
+        look(i, j0, probe_all, low);
+        low_all = min(low_all, low);
+        low_most = max(low_most, low);
       }
-    } else if (again || (p.partial == nullptr && !__any(low != 0xffffffffu))) {
-      // v_mfma_f32_16x16x4_f32 four times per slab, both operands straight from memory
+    // (no unit is all zeros if some lane has a sum that is not in each)
+    const bool seems_right = !__any(probe_all != 0.f || probe_all != probe_all || low_all < kLeast - 1u) &&
+                             (p.partial != nullptr || __any(low_most != 0xffffffffu));
+    if (!seems_right) {
+      unsigned redo = 0;         // units to replace, bit i * NB + j
+      bool again = false, no_number = false;
 #pragma unroll
       for (int i = 0; i < WR; ++i)
 #pragma unroll
-        for (int j = 0; j < NB; ++j) acc[i][j] = Acc{0.f, 0.f, 0.f, 0.f};
-      seek(kt_begin);
-#pragma unroll 1
-      while (l_kt < kt_end) {
-        const bool off = l_cc * 16 + kq * 4 >= g.c;
-        u32x4 xv[WR], wv[NB];
+        for (int j0 = 0; j0 < NB; j0 += UJ) {
+          float probe = 0.f;
+          unsigned low = 0xffffffffu;
+          look(i, j0, probe, low);
+          const bool inf = __any(probe != 0.f || probe != probe), wrong = inf || __any(low < kLeast - 1u);
+          const bool zeros = p.partial == nullptr && !__any(low != 0xffffffffu);
+          if ((wrong || zeros) && m0 + i * 16 < g.m_total && n0 + j0 * 16 < g.o) {
+            redo |= 1u << (i * NB + j0);
+            again = again || wrong;
+            no_number = no_number || inf;
+          }
+        }
+#pragma unroll
+      for (int i = 0; i < WR; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) rest[i][j] = Acc{0.f, 0.f, 0.f, 0.f};
+      if (RUNS && no_number) {
+        // taps outside the image contribute nothing, also where a filter value is infinite: value by value
 #pragma unroll
         for (int i = 0; i < WR; ++i) {
-          if (!RUNS) {
-            xv[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, off ? (int)kOutOfRange : (int)(a_tap[i] + (unsigned)l_cc * 64u), 0, 0);
-            continue;
-          }
+#pragma unroll 1
+          for (int ky = 0; ky < g.k; ++ky) {
+            if ((unsigned)(a_iy[i] + ky) >= (unsigned)g.h) continue;
+            const unsigned x_row = a_base[i] - kq * 16u + (unsigned)(ky * row_values * 4);
+#pragma unroll 1
+            for (int q = 0; q < g.c; ++q) {
+              if ((unsigned)(a_ix[i] - kq * 4 + q) >= (unsigned)row_values) continue;
+              const float xv = *reinterpret_cast<const float*>(static_cast<const char*>(p.x) + (x_row + q * 4u));
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const bool in = (unsigned)(a_ix[i] + l_cc * 16 + e) < (unsigned)row_values && l_cc * 16 + kq * 4 + e < g.c;
-            const int at = (int)(a_tap[i] + (unsigned)l_cc * 64u + e * 4u);
-            xv[i][e] = __builtin_amdgcn_raw_buffer_load_b32(rx, in && at >= 0 ? at : (int)kOutOfRange, 0, 0);
-          }
-        }
-        if (!again) {   // sums of nothing but zeros: most likely the input is zero here
-          unsigned bits = 0;
+              for (int j = 0; j < NB; ++j)
 #pragma unroll
-          for (int i = 0; i < WR; ++i) bits |= (xv[i][0] | xv[i][1] | xv[i][2] | xv[i][3]) & 0x7fffffffu;
-          if (!__any(bits != 0)) {
-            step();
-            continue;
+                for (int r = 0; r < 4; ++r) {
+                  const int o = n0 + j * 16 + kq * 4 + r;
+                  if (o < g.o) rest[i][j][r] += xv * static_cast<const float*>(p.w)[((long)o * g.k + ky) * g.c + q];
+                }
+            }
           }
         }
+      } else if (redo != 0) {
+        // v_mfma_f32_16x16x4_f32 four times per slab, both operands straight from memory
+        seek(kt_begin);
+#pragma unroll 1
+        while (l_kt < kt_end) {
+          const bool off = l_cc * 16 + kq * 4 >= g.c;
+          u32x4 xv[WR], wv[NB];
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-          const int o = n0 + j * 16 + lr;
-          const unsigned at = (unsigned)o * krow_bytes + l_tapbyte + (unsigned)l_cc * 64u + kq * 16u;
-          if (!RUNS) {
-            wv[j] = __builtin_amdgcn_raw_buffer_load_b128(rw, off || o >= g.o ? (int)kOutOfRange : (int)at, 0, 0);
-            continue;
+          for (int i = 0; i < WR; ++i) {
+            if (!RUNS) {
+              xv[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, off ? (int)kOutOfRange : (int)(a_tap[i] + (unsigned)l_cc * 64u), 0, 0);
+              continue;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const bool in = (unsigned)(a_ix[i] + l_cc * 16 + e) < (unsigned)row_values && l_cc * 16 + kq * 4 + e < g.c;
+              const int at = (int)(a_tap[i] + (unsigned)l_cc * 64u + e * 4u);
+              xv[i][e] = __builtin_amdgcn_raw_buffer_load_b32(rx, in && at >= 0 ? at : (int)kOutOfRange, 0, 0);
+            }
+          }
+          if (!again) {   // sums of nothing but zeros: most likely the input is zero here
+            unsigned bits = 0;
+#pragma unroll
+            for (int i = 0; i < WR; ++i) bits |= (xv[i][0] | xv[i][1] | xv[i][2] | xv[i][3]) & 0x7fffffffu;
+            if (!__any(bits != 0)) {
+              step();
+              continue;
+            }
           }
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            wv[j][e] = __builtin_amdgcn_raw_buffer_load_b32(
-                rw, l_cc * 16 + kq * 4 + e < g.c && o < g.o ? (int)(at + e * 4u) : (int)kOutOfRange, 0, 0);
+          for (int j = 0; j < NB; ++j) {
+            const int o = n0 + j * 16 + lr;
+            const unsigned at = (unsigned)o * krow_bytes + l_tapbyte + (unsigned)l_cc * 64u + kq * 16u;
+            if (!RUNS) {
+              wv[j] = __builtin_amdgcn_raw_buffer_load_b128(rw, off || o >= g.o ? (int)kOutOfRange : (int)at, 0, 0);
+              continue;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              wv[j][e] = __builtin_amdgcn_raw_buffer_load_b32(
+                  rw, l_cc * 16 + kq * 4 + e < g.c && o < g.o ? (int)(at + e * 4u) : (int)kOutOfRange, 0, 0);
+          }
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int i = 0; i < WR; ++i) WaveMma<float, 16>::run(wv[j], xv[i], rest[i][j]);
+          step();
         }
+      }
+#pragma unroll
+      for (int i = 0; i < WR; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j)
-#pragma unroll
-          for (int i = 0; i < WR; ++i) WaveMma<float, 16>::run(wv[j], xv[i], acc[i][j]);
-        step();
-      }
+          if (redo >> (i * NB + j / UJ * UJ) & 1) acc[i][j] = rest[i][j];
     }
   }
 
@@ -1195,10 +1230,12 @@ __device__ __forceinline__ void igemm_wave_tile(
 // uniform over the workgroup; all four paths keep 16 accumulator registers per
 // lane, so the register budget is that of the largest one.
 // SPLIT: some problem of the group is contracted as bf16 pieces.  Its tiles need more registers, LDS
-// and code than the others': a group without (the heads of one image) does without them as well.
+// and code than the others': a group without (the heads of one image) does without them as well.  Forms of
+// 128 rows and of two times four waves are replaced (grouped_form) so that four workgroups fit a unit: the heads
+// of 64 images 320 -> 311 us, of 16 97 -> 91 (before, 160 registers and 48 KB: three).
 template <typename T, int ROWB, bool SPLIT>
-__global__ __launch_bounds__(256, SPLIT ? 3 : 1) void conv_igemm_mixed_kernel(IgemmGroup grp) {
-  constexpr int kLds = SPLIT ? std::max(igemm_lds_bytes<128, 32, ROWB>(), pieces_lds_bytes<4, 2>())
+__global__ __launch_bounds__(256, SPLIT ? 4 : 1) void conv_igemm_mixed_kernel(IgemmGroup grp) {
+  constexpr int kLds = SPLIT ? std::max(igemm_lds_bytes<128, 32, ROWB>(), std::max(pieces_lds_bytes<4, 1>(), pieces_lds_bytes<2, 2>()))
                              : igemm_lds_bytes<128, 32, ROWB>();  // the largest of the tiles below
   static_assert(kLds >= igemm_lds_bytes<128, 16, ROWB>() && kLds >= igemm_lds_bytes<64, 64, ROWB>(), "LDS size");
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
@@ -1218,12 +1255,12 @@ __global__ __launch_bounds__(256, SPLIT ? 3 : 1) void conv_igemm_mixed_kernel(Ig
     switch (p.variant) {
       case 16: pieces_tile<1, 4, 4, 1, false>(lds, p, bid); return;
       case 17: pieces_tile<1, 4, 4, 1, true>(lds, p, bid); return;
-      case 18: pieces_tile<2, 2, 4, 1, false>(lds, p, bid); return;
-      case 19: pieces_tile<2, 2, 4, 1, true>(lds, p, bid); return;
-      case 20: pieces_tile<1, 4, 2, 2, false>(lds, p, bid); return;
-      case 21: pieces_tile<1, 4, 2, 2, true>(lds, p, bid); return;
-      case 22: pieces_tile<2, 1, 4, 1, false>(lds, p, bid); return;
-      case 23: pieces_tile<2, 1, 4, 1, true>(lds, p, bid); return;
+      case 18: pieces_tile<1, 2, 4, 1, false>(lds, p, bid); return;
+      case 19: pieces_tile<1, 2, 4, 1, true>(lds, p, bid); return;
+      case 20: pieces_tile<1, 2, 2, 2, false>(lds, p, bid); return;
+      case 21: pieces_tile<1, 2, 2, 2, true>(lds, p, bid); return;
+      case 22: pieces_tile<1, 1, 4, 1, false>(lds, p, bid); return;
+      case 23: pieces_tile<1, 1, 4, 1, true>(lds, p, bid); return;
     }
   }
   switch (p.variant & 15) {
@@ -1606,8 +1643,8 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p, int form) {
   out.prob.partial = p.splits > 1 ? static_cast<float*>(a.workspace_dev) : nullptr;
   out.prob.slabs_per_split = p.slabs_per_split;
   out.prob.splits = work_layout(p, tiles_m);
-  out.prob.variant = (form == FORM_64x64 ? 16 : form == FORM_128x32 ? 18 : form == FORM_32x64_K2 ? 20 :
-                      form == FORM_128x16 ? 22 :
+  out.prob.variant = (form == FORM_64x64 ? 16 : form == FORM_64x32 ? 18 : form == FORM_32x32_K2 ? 20 :
+                      form == FORM_64x16 ? 22 :
                       p.cfg == CFG_WAVE32 ? 4 : p.cfg == CFG_WAVE16 ? 6 : p.cfg == CFG_128x32 ? 2 :
                       p.cfg == CFG_128x16 ? 8 : 0) +
                      (is_pointwise(a) ? 1 : 0);
@@ -1637,7 +1674,9 @@ int grouped_form(int form) {
     case FORM_128x64:
     case FORM_128x64_W8: return FORM_64x64;
     case FORM_64x64_K2:
-    case FORM_64x32_K2: return FORM_32x64_K2;
+    case FORM_64x32_K2: return FORM_32x32_K2;
+    case FORM_128x32: return FORM_64x32;
+    case FORM_128x16: return FORM_64x16;
     default: return form;
   }
 }
@@ -1660,7 +1699,6 @@ void launch_pieces(int form, bool pw, unsigned grid, hipStream_t s, const IgemmP
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x64_W8, 1, 4, 8, 1)
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_64x64_K2, 1, 4, 4, 2)
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_64x32_K2, 1, 2, 4, 2)
-    OGLE_PIECES_CASE(conv_pieces_kernel, FORM_32x64_K2, 1, 4, 2, 2)
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x64, 2, 4, 4, 1)
   }
 }
@@ -1686,12 +1724,12 @@ void launch_runs(int form, unsigned grid, hipStream_t s, const IgemmProblem& arg
 void launch_pieces_group(int form, bool pw, unsigned grid, hipStream_t s, const IgemmGroup& arg) {
   switch (form) {
     OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_64x64, 1, 4, 4, 1)
-    OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_128x32, 2, 2, 4, 1)
-    OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_128x16, 2, 1, 4, 1)
+    OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_64x32, 1, 2, 4, 1)
+    OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_64x16, 1, 1, 4, 1)
     case FORM_128x128:
       launch((conv_pieces_group_kernel<2, 8, 4, 1, true>), dim3(grid), dim3(256), 0, s, arg);
       break;
-    OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_32x64_K2, 1, 4, 2, 2)
+    OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_32x32_K2, 1, 2, 2, 2)
   }
 }
 #undef OGLE_PIECES_CASE

@@ -30,11 +30,12 @@ enum PiecesForm {
   FORM_128x64_W8,    // eight waves of 16 rows
   FORM_64x64_K2,     // two groups of four waves take K stages in turn
   FORM_64x32_K2,
-  FORM_32x64_K2,     // two groups of two waves: the K2 forms in a grouped launch
-  FORM_128x16
+  FORM_32x32_K2,     // two groups of two waves: the K2 forms in a grouped launch
+  FORM_128x16,
+  FORM_64x32, FORM_64x16   // in a grouped launch for the two of 128 rows, which need more registers
 };
-constexpr int kFormBM[] = {0, 64, 128, 128, 128, 128, 64, 64, 32, 128};
-constexpr int kFormBN[] = {0, 64, 32, 128, 64, 64, 64, 32, 64, 16};
+constexpr int kFormBM[] = {0, 64, 128, 128, 128, 128, 64, 64, 32, 128, 64, 64};
+constexpr int kFormBN[] = {0, 64, 32, 128, 64, 64, 64, 32, 32, 16, 32, 16};
 
 struct IgemmPlan {
   int cfg;

@@ -712,6 +712,9 @@ BATCHES_OF_FORMS = [
     [(1, 97, 97, 36, 40, 3, 1, 1), (1, 66, 66, 44, 88, 3, 1, 1)],
     [(1, 119, 118, 36, 72, 3, 1, 1), (1, 66, 66, 44, 88, 3, 1, 1), (2, 97, 98, 44, 12, 3, 1, 1), (4, 19, 19, 388, 512, 1, 1, 0),
      (1, 96, 97, 388, 520, 1, 1, 0), (1, 160, 160, 32, 255, 3, 1, 1), (3, 75, 73, 44, 70, 3, 2, 1)],
+    # the first holds the operands that are no numbers: sums contracted again are the same ones in every form
+    [(1, 96, 97, 388, 520, 1, 1, 0), (2, 97, 98, 44, 12, 3, 1, 1)],
+    [(2, 97, 98, 44, 12, 3, 1, 1), (5, 84, 84, 36, 31, 3, 1, 1)],
 ]
 
 
