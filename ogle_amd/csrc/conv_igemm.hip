@@ -708,11 +708,8 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
       a_base[i] = (unsigned)(((b * g.h + oy * g.stride - g.pad) * g.w + a_ix[i]) * g.pixel * 4) + kq * 16;
       if (RUNS) {
         a_ix[i] *= g.pixel;
-        // (a 16-byte load with a value of the run must not begin before the tensor, nor end behind it)
-        const int low_row = min(g.h - 1, oy * g.stride - g.pad + g.k - 1);
-        const long end = (long)(b * g.h + low_row) * g.w * g.pixel + a_ix[i] + ((g.c + 3) & ~3);
         edge = edge || (ok && (a_ix[i] < 0 || a_ix[i] + g.c > g.w * g.pixel));
-        at_end = at_end || (ok && (end * 4 > (long)g.x_bytes || (b == 0 && a_iy[i] <= 0 && a_ix[i] < 0)));
+        at_end = at_end || (ok && runs_leave_tensor(g.n, g.h, g.w * g.pixel, g.k, g.c, b, a_iy[i], a_ix[i]));
         a_ix[i] += kq * 4;
       }
     }

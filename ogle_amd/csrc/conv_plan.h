@@ -358,6 +358,17 @@ inline bool plan_runs(const OgleConvArgs& a, IgemmPlan* out) {
   return true;
 }
 
+// Whether a 16-byte load with a value of a pixel's runs begins before the tensor or ends behind it: such a load
+// returns zeros for all four.  `iy`: the row of the first filter row, `start`: the runs' first value, counted from
+// their rows' first; both may lie in the padding.  (The first row counts wherever it lies: a row of one or two
+// values that is not the tensor's first can still share its first vector with what is before the tensor.)
+constexpr bool runs_leave_tensor(int images, int h, int row_values, int k, int run, int image, int iy, int start) {
+  const long first = (long)image * h + (iy < 0 ? 0 : iy);
+  const long last = (long)image * h + (iy + k - 1 < h - 1 ? iy + k - 1 : h - 1);
+  return first * row_values + start < 0 ||
+         last * row_values + start + ((run + 3) & ~3) > (long)images * h * row_values;
+}
+
 // The plan the launch will use: split-K only with a workspace that is large enough.
 inline IgemmPlan final_plan(const OgleConvArgs& a, long m) {
   IgemmPlan p = plan_igemm(a, m, a.workspace_dev != nullptr);

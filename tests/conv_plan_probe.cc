@@ -52,4 +52,26 @@ int probe_runs(const OgleConvArgs* a) {
   IgemmPlan p;
   return !igemm_eligible(*a, &m) && plan_runs(*a, &p) ? p.form : -1;
 }
+
+// Loads of four values as pieces_tile requests them for runs: the pixels of which some vector holds a value of
+// the image, does not lie inside the tensor and is not foretold by runs_leave_tensor.
+int probe_runs_lost(const OgleConvArgs* a) {
+  const int row_values = a->in_w * a->in_c, run = a->kernel_size * a->in_c;
+  const long values = (long)a->n * a->in_h * row_values;
+  int lost = 0;
+  for (int b = 0; b < a->n; ++b)
+    for (int oy = 0; oy < a->out_h; ++oy)
+      for (int ox = 0; ox < a->out_w; ++ox) {
+        const int iy = oy * a->stride - a->padding, start = (ox * a->stride - a->padding) * a->in_c;
+        bool loses = false;
+        for (int y = std::max(iy, 0); y < std::min(iy + a->kernel_size, a->in_h); ++y)
+          for (int q = 0; q < run; ++q) {   // the vector of each value of the image
+            if (start + q < 0 || start + q >= row_values) continue;
+            const long at = ((long)b * a->in_h + y) * row_values + start + q / 4 * 4;
+            loses = loses || at < 0 || at + 4 > values;
+          }
+        lost += loses && !runs_leave_tensor(a->n, a->in_h, row_values, a->kernel_size, run, b, iy, start);
+      }
+  return lost;
+}
 }

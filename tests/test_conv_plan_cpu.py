@@ -252,3 +252,15 @@ def test_runs_cases_run_what_they_name(probe):
 ])
 def test_runs_leave_to_the_direct_kernels(probe, shape, kw):
     assert probe.probe_runs(ctypes.byref(conv(*shape, **kw))) == -1
+
+
+def test_runs_lose_no_value_at_the_tensors_ends(probe):
+    """A vector that begins before the tensor or ends behind it is read value by value if it holds a value of
+    the image, in whatever row: all small maps, also those a padding is wider than."""
+    shapes = [case for case, _ in K.RUNS_CASES] + [
+        (n, h, w, c, 64, k, s, p) for n in (1, 3) for h in (1, 2, 5, 17) for w in (1, 2, 3, 5) for c in (1, 2, 3, 5)
+        for k in (1, 2, 3, 5, 7, 15) for s in (1, 2, 3) for p in (0, 1, 3, 7)
+        if h + 2 * p >= k and w + 2 * p >= k]
+    assert len(shapes) > 3000
+    lost = [shape for shape in shapes if probe.probe_runs_lost(ctypes.byref(conv(*shape)))]
+    assert not lost, (len(lost), lost[:5])

@@ -438,6 +438,9 @@ RUNS_CASES = [
     ((7, 40, 41, 130, 15, 1, 1, 0), 9),     # two values past a vector
     ((1, 64, 66, 1, 96, 9, 1, 4), 1),       # one channel
     ((2, 31, 30, 22, 90, 3, 2, 0), 7),      # no padding, a run of 66
+    ((2, 64, 2, 1, 512, 15, 1, 7), 7),      # rows of two values: runs of row 1 begin before the tensor
+    ((2, 33, 1, 1, 512, 7, 1, 7), 1),       # of one value: runs of rows 1 and 2
+    ((64, 2, 1, 1, 512, 7, 1, 7), 1),       # of the second image as well
 ]
 
 
