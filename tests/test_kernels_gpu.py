@@ -531,6 +531,8 @@ IMAGE_STRIDE_CASES = [
     (2, 38, 38, 128, 64, 1, 1, 0, 64, 128),      # pointwise, no split: the tile kernel's row stores
     (64, 10, 10, 256, 24, 3, 1, 1, 5064, 0),     # batch 64: tile kernel without a split
     (5, 7, 9, 32, 40, 3, 2, 1, 0, 0),            # stride equal to the image: the dense case
+    (8, 38, 38, 256, 53, 1, 1, 0, 3, 5),         # bf16 pieces: rows and images that are no multiple of 16 bytes
+    (8, 38, 38, 256, 56, 1, 1, 0, 2, 3),         # the same, images only
 ]
 
 
@@ -1521,6 +1523,8 @@ SPLIT_CASES = [
     (1, 3, 3, 128, 24, 126, 3, 1, 1, H.F32),       # tiny map: the wave-split kernel
     (1, 1, 1, 128, 24, 126, 3, 1, 1, H.F32),       # one pixel
     (2, 9, 9, 64, 16, 48, 3, 1, 1, H.F16),         # fp16 storage
+    (16, 38, 38, 256, 9, 47, 1, 1, 0, H.F32),      # bf16 pieces: parts that are no multiple of 4 next to each other
+    (16, 38, 38, 256, 8, 45, 1, 1, 0, H.F32),      # the first one is
 ]
 
 
