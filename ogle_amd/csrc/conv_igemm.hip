@@ -987,7 +987,9 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
         }
     };
     float probe_all = 0.f;
-    unsigned low_all = 0xffffffffu, low_most = 0;   // over all units, and of the unit where it is largest
+    // `low` over all units, and of the unit of this problem where it is largest (those past the last row or
+    // channel are zeros)
+    unsigned low_all = 0xffffffffu, low_most = 0;
 #pragma unroll
     for (int i = 0; i < WR; ++i)
 #pragma unroll
@@ -995,7 +997,7 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
         unsigned low = 0xffffffffu;
         look(i, j0, probe_all, low);
         low_all = min(low_all, low);
-        low_most = max(low_most, low);
+        if (m0 + i * 16 < g.m_total && n0 + j0 * 16 < g.o) low_most = max(low_most, low);
       }
     // (no unit is all zeros if some lane has a sum that is not in each)
     const bool seems_right = !__any(probe_all != 0.f || probe_all != probe_all || low_all < kLeast - 1u) &&
