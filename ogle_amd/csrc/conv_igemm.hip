@@ -1594,17 +1594,23 @@ __global__ __launch_bounds__(256) void splitk_reduce_group_kernel(ReduceGroup gr
 // Few tile rows spread unevenly over the XCDs: then each gets an eighth of the tiles, or of the (tile, K range)
 // pairs, in order.  17 rows of 12 128x64 tiles by rows give one XCD 36 for its 32 units (M = 2116, K = 864 ->
 // 768 channels 38.2 us, like this 26.5); 10x10x1024 -> 24, 3x3 at batch 64, with K ranges on XCDs 48.1 us, so 43.5.
-int work_layout(const IgemmPlan& p, int tiles_m) {
-  if (p.splits == 1) return rows_even(tiles_m) ? 1 : 0;
-  if (p.rows_on_xcd) return rows_even(tiles_m) ? -p.splits : -p.splits - kMaxSplits;
+// `form` in place of the plan's, as for prepare below.
+bool rows_dealt(const IgemmPlan& p, int form, int tiles_m, int tiles_n) {
+  return form == FORM_NONE ? rows_even(tiles_m) : pieces_rows_even(tiles_m, (long)tiles_n * p.splits);
+}
+int work_layout(const IgemmPlan& p, int form, int tiles_m, int tiles_n) {
+  const bool rows = rows_dealt(p, form, tiles_m, tiles_n);
+  if (p.splits == 1) return rows ? 1 : 0;
+  if (p.rows_on_xcd) return rows ? -p.splits : -p.splits - kMaxSplits;
   return p.splits;
 }
 
 // Grid size of one problem under that layout.
-unsigned grid_blocks(const IgemmPlan& p, int tiles_m, int tiles_n) {
+unsigned grid_blocks(const IgemmPlan& p, int form, int tiles_m, int tiles_n) {
   const int tiles = tiles_m * tiles_n;
   if (p.splits == 1 || p.rows_on_xcd) {
-    if (rows_even(tiles_m)) return 8u * (unsigned)((tiles_m + 7) / 8) * (unsigned)tiles_n * (unsigned)p.splits;
+    if (rows_dealt(p, form, tiles_m, tiles_n))
+      return 8u * (unsigned)((tiles_m + 7) / 8) * (unsigned)tiles_n * (unsigned)p.splits;
     return 8u * (unsigned)(((long)tiles * p.splits + 7) / 8);
   }
   if (p.splits != 2 && p.splits != 4) return (unsigned)tiles * (unsigned)p.splits;
@@ -1650,7 +1656,7 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p, int form) {
   out.prob.tiles = tiles_m * tiles_n;
   out.prob.partial = p.splits > 1 ? static_cast<float*>(a.workspace_dev) : nullptr;
   out.prob.slabs_per_split = p.slabs_per_split;
-  out.prob.splits = work_layout(p, tiles_m);
+  out.prob.splits = work_layout(p, form, tiles_m, tiles_n);
   out.prob.variant = (form == FORM_64x64 ? 16 : form == FORM_64x32 ? 18 : form == FORM_32x32_K2 ? 20 :
                       form == FORM_64x16 ? 22 :
                       p.cfg == CFG_WAVE32 ? 4 : p.cfg == CFG_WAVE16 ? 6 : p.cfg == CFG_128x32 ? 2 :
@@ -1660,7 +1666,7 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p, int form) {
     out.grid = (unsigned)(tiles_m * tiles_n);
     return out;
   }
-  out.grid = grid_blocks(p, tiles_m, tiles_n);
+  out.grid = grid_blocks(p, form, tiles_m, tiles_n);
   if (p.splits > 1) {
     const long mn = (long)g.m_total * g.o;
     // enough lanes per output that the grid still has about a thousand waves

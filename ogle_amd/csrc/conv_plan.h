@@ -65,6 +65,16 @@ inline int tile_bn(int cfg) { return kCfgBN[cfg]; }
 // Whether whole tile rows spread evenly (within a tenth) over the eight XCDs.
 constexpr bool rows_even(long tiles_m) { return ((tiles_m + 7) / 8) * 8 * 10 <= tiles_m * 11; }
 
+// The same for the workgroups that contract bf16 pieces, `per_row` to a tile row, of which a unit runs two at
+// a time: the fullest XCD must not need another round of its 32 units for them, nor be the only one to double up.
+// 100 rows of 5 leave one XCD 65 workgroups and a nearly empty second round (us by rows / in equal shares, 128x64
+// of eight waves: M = 12760, K = 288 -> 320 25.0 / 18.9; 128x128: 1x1 M = 10506, 392 -> 768 61.1 / 41.3).
+constexpr bool pieces_rows_even(long tiles_m, long per_row) {
+  const long most = (tiles_m + 7) / 8 * per_row, least = (tiles_m * per_row + 7) / 8, slots = 64;
+  return rows_even(tiles_m) && (most > slots / 2) == (least > slots / 2) &&
+         (most > 8 * slots || (most + slots - 1) / slots == (least + slots - 1) / slots);
+}
+
 // The form for `m` output rows: `large` a plan of 128x128 tiles, `pieces` whether 64x64 tiles would be
 // pieces.  What counts is how evenly the workgroups spread over 256 units, and that a unit has waves
 // enough to cover what each waits for.  Us of the form taken / of 64x64 tiles with four waves (and, with

@@ -74,4 +74,6 @@ int probe_runs_lost(const OgleConvArgs* a) {
       }
   return lost;
 }
+
+int probe_rows_even(int tiles_m, int per_row) { return pieces_rows_even(tiles_m, per_row); }
 }

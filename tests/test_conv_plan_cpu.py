@@ -218,6 +218,18 @@ def test_form_cases_run_what_they_name(probe):
     assert set(forms) == set(range(1, 10)) - {8}    # 8 is the K2 forms' in a grouped launch
 
 
+def test_rows_are_dealt_whole_where_no_unit_gets_another_round(probe):
+    """Two workgroups a unit and 32 units an XCD: the fullest XCD has as many rounds as equal shares would give."""
+    assert [probe.probe_rows_even(*a) for a in ((100, 5), (83, 6), (169, 3), (65, 4), (96, 5), (64, 4), (163, 3), (1000, 1))] == \
+        [0, 0, 0, 0, 1, 1, 1, 1]
+    for tiles_m in range(1, 300):
+        for per_row in (1, 2, 3, 5, 8):
+            if probe.probe_rows_even(tiles_m, per_row):
+                most = -(-tiles_m // 8) * per_row
+                assert 10 * 8 * -(-tiles_m // 8) <= 11 * tiles_m
+                assert most > 512 or -(-most // 64) == -(-(-(-tiles_m * per_row // 8)) // 64)
+
+
 def test_forms_are_chosen_within_their_tiles(probe):
     """128x128 workgroups are built for pointwise convolutions only; other types than fp32 have no form."""
     r, seen = random.Random(11), set()

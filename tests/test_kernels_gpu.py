@@ -383,6 +383,7 @@ FORM_CASES = [
     ((1, 96, 97, 388, 520, 1, 1, 0), 4),    # 128x64
     ((1, 119, 118, 36, 72, 3, 1, 1), 5),    # 128x64 of eight waves
     ((1, 160, 160, 32, 255, 3, 1, 1), 5),   # the same in place of 128x128 tiles
+    ((2, 77, 83, 16, 260, 3, 1, 1), 5),     # in equal shares: 100 tile rows of five, the last one ragged
     ((1, 97, 97, 36, 40, 3, 1, 1), 6),      # 64x64, two K groups
     ((4, 19, 19, 388, 512, 1, 1, 0), 6),    # the same, pointwise, 25 slabs
     ((1, 66, 66, 44, 88, 3, 1, 1), 7),      # 64x32, two K groups
