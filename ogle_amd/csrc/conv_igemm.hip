@@ -1685,7 +1685,6 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p, int form) {
 // The form a problem takes next to others in one launch: with 256 threads, adding in the same order.
 int grouped_form(int form) {
   switch (form) {
-    case FORM_128x64:
     case FORM_128x64_W8: return FORM_64x64;
     case FORM_64x64_K2:
     case FORM_64x32_K2: return FORM_32x32_K2;
@@ -1713,7 +1712,6 @@ void launch_pieces(int form, bool pw, unsigned grid, hipStream_t s, const IgemmP
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x64_W8, 1, 4, 8, 1)
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_64x64_K2, 1, 4, 4, 2)
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_64x32_K2, 1, 2, 4, 2)
-    OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x64, 2, 4, 4, 1)
   }
 }
 

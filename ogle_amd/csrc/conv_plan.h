@@ -26,16 +26,16 @@ constexpr int kRowBytesF16Wide = 64;  // K bytes per tile row per slab of CFG_12
 // Workgroups that contract fp32 as bf16 pieces: rows x columns, four waves one above the other
 // unless named otherwise.  All but the K2 forms add an output's products in the same order.
 enum PiecesForm {
-  FORM_NONE = 0, FORM_64x64, FORM_128x32, FORM_128x128, FORM_128x64,
-  FORM_128x64_W8,    // eight waves of 16 rows
-  FORM_64x64_K2,     // two groups of four waves take K stages in turn
+  FORM_NONE = 0, FORM_64x64, FORM_128x32, FORM_128x128,
+  FORM_128x64_W8 = 5,   // eight waves of 16 rows
+  FORM_64x64_K2,        // two groups of four waves take K stages in turn
   FORM_64x32_K2,
-  FORM_32x32_K2,     // two groups of two waves: the K2 forms in a grouped launch
+  FORM_32x32_K2,        // two groups of two waves: the K2 forms in a grouped launch
   FORM_128x16,
   FORM_64x32, FORM_64x16   // in a grouped launch for the two of 128 rows, which need more registers
 };
-constexpr int kFormBM[] = {0, 64, 128, 128, 128, 128, 64, 64, 32, 128, 64, 64};
-constexpr int kFormBN[] = {0, 64, 32, 128, 64, 64, 64, 32, 32, 16, 32, 16};
+constexpr int kFormBM[] = {0, 64, 128, 128, 0, 128, 64, 64, 32, 128, 64, 64};
+constexpr int kFormBN[] = {0, 64, 32, 128, 0, 64, 64, 32, 32, 16, 32, 16};
 
 struct IgemmPlan {
   int cfg;
@@ -77,38 +77,39 @@ constexpr bool pieces_rows_even(long tiles_m, long per_row) {
 
 // The form for `m` output rows: `large` a plan of 128x128 tiles, `pieces` whether 64x64 tiles would be
 // pieces.  What counts is how evenly the workgroups spread over 256 units, and that a unit has waves
-// enough to cover what each waits for.  Us of the form taken / of 64x64 tiles with four waves (and, with
-// at most 256 of those, of 64x64 fp32 tiles), 3x3 unless 1x1:
-//   64x32 K2, at most 256 of them: M = 6272, K = 576 -> 64 11.4 / 15.8 (13.4), 1x1 M = 400, 768 -> 200
-//     11.6 / 18.0 (14.5); where the last 64 columns are mostly padding: M = 8664, K = 432 -> 88 13.4 / 16.0
-//   64x64 K2: M = 3136, K = 1152 -> 256 21.9 / 26.1 (30.0), 1x1 M = 1444, 512 -> 512 11.1 / 14.1 (15.0),
+// enough to cover what each waits for.  Us of the form taken / of another one, 3x3 unless 1x1:
+//   64x32 K2, at most 256 of them: M = 6272, K = 576 -> 64 11.4 / 15.8 with 64x64 (13.4 as fp32), 1x1 M = 400,
+//     768 -> 200 11.6 / 18.0 (14.5); where the last 64 columns are mostly padding: M = 8664, K = 432 -> 88 13.4 / 16.0
+//   64x64 K2: M = 3136, K = 1152 -> 256 21.9 / 26.1 with 64x64 (30.0), 1x1 M = 1444, 512 -> 512 11.1 / 14.1 (15.0),
 //     M = 22500, 1024 -> 40 30.4 / 36.3; K = 288 with at most 256 tiles 11.0 / 10.7 (11.2): the 64x64 ones
-//   128x64, eight waves: M = 50176, K = 576 -> 64 30.4 / 34.9, M = 12544, K = 1152 -> 128 31.8 / 34.6,
-//     M = 4704, K = 1872 -> 768 87.9 / 101.8, 1x1 M = 10000, 128 -> 384 10.9 / 11.9; between one and one
-//     and a half or above two workgroups per unit it is behind (M = 2400, K = 1024: 45.5 / 42.1)
-//   128x64: 1x1 M = 23104, 256 -> 256 24.8 / 27.5, 128 -> 256 15.7 / 17.4, M = 11552, 512 -> 512 41.7 / 45.6
-//   128x128: 1x1 M = 11552, 512 -> 1024 74.7 / 87.6 (128x64 78.2), but M = 12544, 512 -> 768, whose 588
-//     tiles leave two workgroups per unit a nearly empty second round, 71 (128x64 64)
+//   128x128, pointwise: where they give a unit no more to do than 128x64 ones, in pairs (two run at a time) unless
+//     long or many: 1x1 M = 92416, 512 -> 512 183.6 / 209.9, M = 360000, 128 -> 128 111.6 / 120.0, M = 6400, 1024 ->
+//     1024 79.7 / 89.8, but M = 12544, 512 -> 768 71.7 / 62.2, M = 23104, 256 -> 512 46.3 / 44.1 (three a unit), M =
+//     73600, 40 -> 512 58.0 / 51.6, 96 channels of 128 M = 177480, 260 -> 96 86.8 / 81.3
+//   128x64, eight waves, against 64x64, mean ratio over 2000 shapes by number of workgroups: 257 to 383 1.06,
+//     384 to 512 0.93, 513 to 640 1.03, more 0.95; those many pointwise ones of up to 7 slabs 1.03 (3 slabs 1.06)
 inline int pieces_form(const OgleConvArgs& a, long m, int ktiles, bool large, bool pieces) {
   auto tiles = [&](int form) {
     return ((m + kFormBM[form] - 1) / kFormBM[form]) * ((a.out_c + kFormBN[form] - 1) / kFormBN[form]);
   };
   const bool pw = is_pointwise(a);
-  const long n64 = tiles(FORM_64x64), n128 = tiles(FORM_128x64);
+  const long n64 = tiles(FORM_64x64), n128 = tiles(FORM_128x64_W8);
   if (large) {
-    const long n = tiles(FORM_128x128), rounds = (n + 2 * kComputeUnits - 1) / (2 * kComputeUnits);
-    if (!pw) return FORM_128x64_W8;
-    return 20 * n >= 13 * rounds * 2 * kComputeUnits ? FORM_128x128 : FORM_128x64;
-  }
-  if (ktiles >= 12) {
+    auto per_unit = [&](int form) { return (tiles(form) + kComputeUnits - 1) / kComputeUnits; };
+    const long n = per_unit(FORM_128x128);
+    if (pw && ktiles >= 8 && (a.out_c + 127) / 128 * 128 * 10 <= a.out_c * 11 &&
+        2 * n <= per_unit(FORM_128x64_W8) && (ktiles >= 32 || n >= 8 || n % 2 == 0))
+      return FORM_128x128;
+  } else if (ktiles >= 12) {
     const long n32 = tiles(FORM_64x32_K2);
     if (n32 <= kComputeUnits || (2 * n32 <= 3 * n64 && n32 <= 2 * kComputeUnits)) return FORM_64x32_K2;
     if (n64 <= kComputeUnits) return ktiles >= 24 ? FORM_64x64_K2 : ktiles >= 16 ? FORM_64x64 : FORM_NONE;
     if (n128 <= kComputeUnits) return pw && ktiles >= 64 ? FORM_64x64_K2 : FORM_128x64_W8;
   }
-  if (!pieces) return FORM_NONE;
-  if (pw && ktiles >= 8 && 2 * n128 >= 5 * kComputeUnits) return FORM_128x64;
-  return 2 * n128 >= 3 * kComputeUnits && n128 <= 2 * kComputeUnits ? FORM_128x64_W8 : FORM_64x64;
+  if (!large && !pieces) return FORM_NONE;
+  if (2 * n128 <= 5 * kComputeUnits)
+    return 2 * n128 >= 3 * kComputeUnits && n128 <= 2 * kComputeUnits ? FORM_128x64_W8 : FORM_64x64;
+  return pw && ktiles < 8 ? FORM_64x64 : FORM_128x64_W8;
 }
 
 // Picks the output tile and the K split.  Problems with few output
@@ -360,9 +361,9 @@ inline bool plan_runs(const OgleConvArgs& a, IgemmPlan* out) {
   if (a.out_c <= 32 && k > 1 && (a.out_c <= 16 || products < 3e7)) return false;
   if (a.out_c <= 32) p.form = a.out_c <= 16 ? FORM_128x16 : FORM_128x32;
   else p.form = pieces_form(a, m, p.ktiles, false, true);
-  if (p.form == FORM_NONE || p.form == FORM_128x64) p.form = FORM_64x64;
-  // with many tiles the filter, gathered value by value, counts: half as often per pixel (the 7x7 stem 62.6 / 58.4,
-  // 13 x 78 x 98, 33 -> 64 3x3 54.1 / 50.1)
+  if (p.form == FORM_NONE) p.form = FORM_64x64;
+  // with many tiles the filter, gathered value by value, counts: half as often per pixel, pointwise too (4 x 100 x
+  // 140, 98 -> 127 28.2 / 27.0; the 7x7 stem 55.3 / 51.4)
   if (p.form == FORM_64x64 && m * a.out_c > 64L * 64 * 5 * kComputeUnits) p.form = FORM_128x64_W8;
   *out = p;
   return true;

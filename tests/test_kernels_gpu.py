@@ -380,7 +380,9 @@ FORM_CASES = [
     ((16, 19, 19, 260, 500, 1, 1, 0), 1),   # 64x64, 17 slabs
     ((5, 84, 84, 36, 31, 3, 1, 1), 2),      # 128x32
     ((1, 223, 221, 260, 124, 1, 1, 0), 3),  # 128x128
-    ((1, 96, 97, 388, 520, 1, 1, 0), 4),    # 128x64
+    ((1, 96, 97, 388, 520, 1, 1, 0), 5),    # 128x64, pointwise
+    ((1, 223, 221, 100, 130, 1, 1, 0), 1),  # many 64x64, seven slabs
+    ((1, 224, 224, 96, 384, 1, 1, 0), 1),   # the same in place of 128x128 tiles
     ((1, 119, 118, 36, 72, 3, 1, 1), 5),    # 128x64 of eight waves
     ((1, 160, 160, 32, 255, 3, 1, 1), 5),   # the same in place of 128x128 tiles
     ((2, 77, 83, 16, 260, 3, 1, 1), 5),     # in equal shares: 100 tile rows of five, the last one ragged
@@ -427,7 +429,7 @@ def test_conv_fp32_pieces_forms(case, data):
 RUNS_CASES = [
     # (n, h, w, c, o, k, s, p), PiecesForm   channels that fill no vector, filter rows as runs of values
     ((2, 70, 75, 3, 70, 7, 2, 3), 7),       # a run of 21; rows that begin and end in the padding
-    ((9, 70, 75, 3, 70, 7, 1, 3), 1),
+    ((9, 70, 75, 3, 70, 7, 1, 3), 5),
     ((1, 100, 101, 45, 64, 3, 1, 1), 6),    # a run of 135, 27 slabs
     ((1, 119, 118, 37, 72, 3, 1, 1), 5),
     ((16, 90, 90, 5, 70, 3, 1, 1), 5),      # many tiles
