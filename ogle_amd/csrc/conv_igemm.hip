@@ -1264,7 +1264,6 @@ __global__ __launch_bounds__(256, SPLIT ? 4 : 1) void conv_igemm_mixed_kernel(Ig
       case 16: pieces_tile<1, 4, 4, 1, false>(lds, p, bid); return;
       case 17: pieces_tile<1, 4, 4, 1, true>(lds, p, bid); return;
       case 18: pieces_tile<1, 2, 4, 1, false>(lds, p, bid); return;
-      case 19: pieces_tile<1, 2, 4, 1, true>(lds, p, bid); return;
       case 20: pieces_tile<1, 2, 2, 2, false>(lds, p, bid); return;
       case 21: pieces_tile<1, 2, 2, 2, true>(lds, p, bid); return;
       case 22: pieces_tile<1, 1, 4, 1, false>(lds, p, bid); return;
@@ -1704,7 +1703,9 @@ int grouped_form(int form) {
 void launch_pieces(int form, bool pw, unsigned grid, hipStream_t s, const IgemmProblem& arg) {
   switch (form) {
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_64x64, 1, 4, 4, 1)
-    OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x32, 2, 2, 4, 1)
+    case FORM_128x32:    // no pointwise one is (plan_igemm)
+      launch((conv_pieces_kernel<2, 2, 4, 1, false>), dim3(grid), dim3(256), 0, s, arg);
+      break;
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x16, 2, 1, 4, 1)
     case FORM_128x128:   // pointwise only; the others have too many registers to keep
       launch((conv_pieces_kernel<2, 8, 4, 1, true>), dim3(grid), dim3(256), 0, s, arg);
@@ -1736,7 +1737,9 @@ void launch_runs(int form, unsigned grid, hipStream_t s, const IgemmProblem& arg
 void launch_pieces_group(int form, bool pw, unsigned grid, hipStream_t s, const IgemmGroup& arg) {
   switch (form) {
     OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_64x64, 1, 4, 4, 1)
-    OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_64x32, 1, 2, 4, 1)
+    case FORM_64x32:
+      launch((conv_pieces_group_kernel<1, 2, 4, 1, false>), dim3(grid), dim3(256), 0, s, arg);
+      break;
     OGLE_PIECES_CASE(conv_pieces_group_kernel, FORM_64x16, 1, 1, 4, 1)
     case FORM_128x128:
       launch((conv_pieces_group_kernel<2, 8, 4, 1, true>), dim3(grid), dim3(256), 0, s, arg);

@@ -231,7 +231,8 @@ def test_rows_are_dealt_whole_where_no_unit_gets_another_round(probe):
 
 
 def test_forms_are_chosen_within_their_tiles(probe):
-    """128x128 workgroups are built for pointwise convolutions only; other types than fp32 have no form."""
+    """128x128 workgroups are built for pointwise convolutions only, 128x32 ones for others; other types than fp32
+    have no form."""
     r, seen = random.Random(11), set()
     for _ in range(30000):
         k = r.choice([1, 1, 3])
@@ -242,6 +243,8 @@ def test_forms_are_chosen_within_their_tiles(probe):
         seen.add(form)
         if form == 3:
             assert k == 1 and shape[6] == 1, shape
+        if form == 2:
+            assert k == 3 or shape[6] == 2, shape
         if shape[3] % 8 == 0:
             assert probe.probe_form(ctypes.byref(conv(*shape, dtype=H.F16)), 1) <= 0
     assert seen - {-1} == set(range(0, 10)) - {4, 8}
