@@ -301,10 +301,11 @@ inline IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
   } else if (p.cfg == CFG_128x32) {
     p.form = p.pieces ? FORM_128x32 : FORM_NONE;
   } else if (p.cfg == CFG_WAVE32 && is_pointwise(a) && p.ktiles >= 12) {
-    // two K groups against the wave-split kernel, where its 64x32 tiles are about one per unit: 1x1
-    // M = 1600, 1024 -> 256 14.9 / 16.4, M = 1444, 256 -> 256 6.1 / 6.8, M = 392, 208 -> 768 5.8 / 6.4
+    // two K groups against the wave-split kernel, where that one's 32x32 tiles need a second round of the units
+    // and 64x32 tiles do not: 1x1 M = 1600, 1024 -> 256 14.9 / 16.4, M = 1444, 256 -> 256 6.1 / 6.8, M = 392, 208 ->
+    // 768 5.8 / 6.4, M = 961, 312 -> 96 6.4 / 9.6, but M = 1624, 256 -> 154, 255 tiles of 32x32, 6.7 / 5.3
     const long n32 = ((m + 63) / 64) * ((a.out_c + 31) / 32);
-    if (n32 <= kComputeUnits && 2 * n32 > kComputeUnits) p.form = FORM_64x32_K2;
+    if (n32 <= kComputeUnits && tiles(CFG_WAVE32) > kComputeUnits) p.form = FORM_64x32_K2;
   }
   // Which operand an XCD's L2 should keep to itself: with K ranges pinned to XCDs the input is
   // fetched by all eight L2s and the filter by one, with tile rows pinned it is the other way

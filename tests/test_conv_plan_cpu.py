@@ -230,6 +230,13 @@ def test_rows_are_dealt_whole_where_no_unit_gets_another_round(probe):
                 assert most > 512 or -(-most // 64) == -(-(-(-tiles_m * per_row // 8)) // 64)
 
 
+def test_two_k_groups_where_the_wave_split_kernel_needs_a_second_round(probe):
+    """255 and 256 tiles of 32x32: one round; 257 and more: 64x32 tiles in two K groups."""
+    forms = [probe.probe_form(ctypes.byref(conv(*shape, 1)), 1)
+             for shape in ((2, 28, 29, 256, 154), (1, 32, 32, 256, 256), (1, 33, 32, 256, 256), (3, 31, 31, 312, 96))]
+    assert forms == [0, 0, 7, 7]
+
+
 def test_forms_are_chosen_within_their_tiles(probe):
     """128x128 workgroups are built for pointwise convolutions only, 128x32 ones for others; other types than fp32
     have no form."""
