@@ -360,7 +360,11 @@ inline bool plan_runs(const OgleConvArgs& a, IgemmPlan* out) {
   const double chain = (double)a.in_c * std::min(k, a.in_h) * std::min(k, a.in_w);
   if (k * run < 24 || 0.07 * chain + 0.2e-6 * products <= 3 + 0.15 * p.ktiles) return false;
   if (a.out_c <= 32 && k > 1 && (a.out_c <= 16 || products < 3e7)) return false;
-  if (a.out_c <= 32) p.form = a.out_c <= 16 ? FORM_128x16 : FORM_128x32;
+  // (two K groups where a unit has one workgroup or none: 3 x 3 x 2, 11 -> 256 3x3 stride 2 7.0 / 9.0 as 64x64, 1 x
+  // 86 x 119, 1x1 34 -> 32 5.1 / 7.0 as 128x32, 2 x 64 x 64, 9x9 1 -> 64 7.5 / 9.5, 14 x 4 x 5, 1x1 139 -> 9 7.0 /
+  // 8.3 as 128x16)
+  if (((m + 63) / 64) * ((a.out_c + 31) / 32) <= kComputeUnits) p.form = FORM_64x32_K2;
+  else if (a.out_c <= 32) p.form = a.out_c <= 16 ? FORM_128x16 : FORM_128x32;
   else p.form = pieces_form(a, m, p.ktiles, false, true);
   if (p.form == FORM_NONE) p.form = FORM_64x64;
   // with many tiles the filter, gathered value by value, counts: half as often per pixel, pointwise too (4 x 100 x

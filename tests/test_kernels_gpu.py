@@ -436,13 +436,16 @@ RUNS_CASES = [
     ((4, 12, 2, 37, 100, 3, 1, 1), 7),      # a run longer than an image row
     ((2, 9, 1, 181, 40, 3, 1, 1), 7),       # one column: two of three taps in the padding
     ((8, 37, 39, 33, 66, 1, 1, 0), 1),      # 1x1: the tensor ends inside a slab
-    ((3, 33, 35, 131, 77, 1, 2, 0), 1),
-    ((2, 40, 41, 67, 31, 3, 1, 1), 2),
-    ((7, 40, 41, 130, 15, 1, 1, 0), 9),     # two values past a vector
-    ((1, 64, 66, 1, 96, 9, 1, 4), 1),       # one channel
+    ((3, 33, 35, 131, 77, 1, 2, 0), 7),
+    ((2, 40, 41, 67, 31, 3, 1, 1), 7),
+    ((5, 60, 61, 67, 31, 3, 1, 1), 2),
+    ((7, 40, 41, 130, 15, 1, 1, 0), 7),     # two values past a vector
+    ((11, 40, 41, 130, 15, 1, 1, 0), 9),
+    ((1, 64, 66, 1, 96, 9, 1, 4), 7),       # one channel
+    ((2, 64, 66, 1, 96, 9, 1, 4), 1),
     ((2, 31, 30, 22, 90, 3, 2, 0), 7),      # no padding, a run of 66
     ((2, 64, 2, 1, 512, 15, 1, 7), 7),      # rows of two values: runs of row 1 begin before the tensor
-    ((2, 33, 1, 1, 512, 7, 1, 7), 1),       # of one value: runs of rows 1 and 2
+    ((2, 33, 1, 1, 512, 7, 1, 7), 7),       # of one value: runs of rows 1 and 2
     ((64, 2, 1, 1, 512, 7, 1, 7), 1),       # of the second image as well
 ]
 
