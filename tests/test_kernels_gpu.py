@@ -473,8 +473,11 @@ def test_conv_fp32_runs(case, data):
     if b is not None:
         ref, scale = ref + b, scale + np.abs(b)
     ok = np.isfinite(ref) & (scale < 1e38)
-    if data == "infinite filter":   # which outputs have such a tap inside the image
-        hit = _pieces_reference(np.ones_like(x), inf.astype(np.float32), k, s, p) > 0
+    if data == "infinite filter":   # such taps of an output that lie inside the image, by their input's sign
+        plus, minus, zero = (_pieces_reference(t.astype(np.float32), inf.astype(np.float32), k, s, p) > 0
+                             for t in (x > 0, x < 0, x == 0))
+        hit = plus | minus | zero
+        want = np.where(zero | (plus & minus), np.nan, np.where(plus, np.inf, -np.inf)).astype(np.float32)
         ok &= ~hit
         wt[inf] = np.inf
     got = gpu_conv(x, wt, b, s, p, entry="ogle_hip_conv2d")
@@ -482,7 +485,7 @@ def test_conv_fp32_runs(case, data):
     over = np.abs(got[ok] - ref[ok]) - (k * k * c / 8 + 16) * 2.0 ** -24 * scale[ok] - k * k * c * 2.0 ** -149
     assert np.max(over) <= 0, case
     if data == "infinite filter":
-        assert not np.isfinite(got[hit]).any()
+        np.testing.assert_array_equal(got[hit], want[hit])
     else:
         # (next to an infinite product, one of 3.4e38 and up that overflows fp32 makes NaN of it: not compared)
         bad = ~np.isfinite(ref) & (_pieces_reference(np.where(np.isfinite(x), np.abs(x), 0), np.abs(wt), k, s, p) < 1e38)
