@@ -972,7 +972,10 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
 
   // Sums that are not finite (an operand was infinite, NaN or so large that a piece overflowed) or so small
   // that pieces may have been cut off are contracted again, in fp32: 16 pixels x 32 channels at a time, so
-  // that an output does not depend on the form that computed it.
+  // that an output does not depend on the form that computed it.  What that costs (us with finite operands / a
+  // quarter of the rows zero above and below / all zeros / one NaN an image / all NaN): 16 x 224 x 224, 7x7 stem
+  // 54 / 59 / 64 / 63 / 195, 4 x 56 x 56, 3x3 99 -> 99 40 / 53 / 53 / 110 / 186, 16 x 56 x 56, 3x3 64 -> 64
+  // 32 / 37 / 40 / 58 / 103, 32 x 19 x 19, 1x1 512 -> 1024 79 / 92 / 87 / 111 / 176, 4 x 19 x 19, 512 -> 512 12 / 16 / 16 / 27 / 30.
   {
     constexpr int UJ = NB % 2 == 0 ? 2 : 1;
     constexpr unsigned kLeast = (127u - 60u) << 24;   // 2^-60
@@ -1004,7 +1007,7 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
                              (p.partial != nullptr || __any(low_most != 0xffffffffu));
     if (!seems_right) {
       unsigned redo = 0;         // units to replace, bit i * NB + j
-      bool again = false, no_number = false;
+      bool again = false;
 #pragma unroll
       for (int i = 0; i < WR; ++i)
 #pragma unroll
@@ -1012,22 +1015,105 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
           float probe = 0.f;
           unsigned low = 0xffffffffu;
           look(i, j0, probe, low);
-          const bool inf = __any(probe != 0.f || probe != probe), wrong = inf || __any(low < kLeast - 1u);
+          const bool wrong = __any(probe != 0.f || probe != probe || low < kLeast - 1u);
           const bool zeros = p.partial == nullptr && !__any(low != 0xffffffffu);
           if ((wrong || zeros) && m0 + i * 16 < g.m_total && n0 + j0 * 16 < g.o) {
             redo |= 1u << (i * NB + j0);
             again = again || wrong;
-            no_number = no_number || inf;
           }
         }
 #pragma unroll
       for (int i = 0; i < WR; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j) rest[i][j] = Acc{0.f, 0.f, 0.f, 0.f};
-      if (RUNS && no_number) {
+      auto wanted = [&](int i, int j) { return (redo >> (i * NB + j / UJ * UJ) & 1) != 0; };
+      // input values of the cursor's slab, zeros where they are not the run's or the image's
+      auto input = [&](int i) {
+        const bool off = l_kt >= kt_end || (redo >> (i * NB) & ((1u << NB) - 1)) == 0 || l_cc * 16 + kq * 4 >= g.c;
+        const unsigned at = a_tap[i] + (unsigned)l_cc * 64u;
+        u32x4 v;
+        if (RUNS && by_value) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            v[e] = __builtin_amdgcn_raw_buffer_load_b32(rx, off || (int)(at + e * 4u) < 0 ? (int)kOutOfRange : (int)(at + e * 4u), 0, 0);
+        } else {
+          v = __builtin_amdgcn_raw_buffer_load_b128(rx, off ? (int)kOutOfRange : (int)at, 0, 0);
+        }
+        if (RUNS) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if ((unsigned)(a_ix[i] + l_cc * 16 + e) >= (unsigned)row_values || l_cc * 16 + kq * 4 + e >= g.c) v[e] = 0u;
+        }
+        return v;
+      };
+      if (redo != 0 && !again) {
+        // sums of nothing but zeros: most likely the input is zero here.  Four slabs' loads at a time
+        seek(kt_begin);
+        bool zeros = true;
+#pragma unroll 1
+        while (zeros && l_kt < kt_end) {
+          u32x4 v[4][WR];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+#pragma unroll
+            for (int i = 0; i < WR; ++i) v[u][i] = input(i);
+            step();
+          }
+          unsigned bits = 0;
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int i = 0; i < WR; ++i) bits |= (v[u][i][0] | v[u][i][1] | v[u][i][2] | v[u][i][3]) & 0x7fffffffu;
+          zeros = !__any(bits != 0);
+        }
+        if (zeros) redo = 0;   // as they are
+      }
+      bool w_no_number = false;
+      if (redo != 0) {
+        // v_mfma_f32_16x16x4_f32 four times per slab, both operands straight from memory
+        seek(kt_begin);
+#pragma unroll 1
+        while (l_kt < kt_end) {
+          u32x4 xv[WR];
+#pragma unroll
+          for (int i = 0; i < WR; ++i) xv[i] = input(i);
+          u32x4 wv[NB];
+#pragma unroll
+          for (int j = 0; j < NB; ++j) {
+            bool none = true;
+#pragma unroll
+            for (int i = 0; i < WR; ++i) none = none && !wanted(i, j);
+            const int o = n0 + j * 16 + lr;
+            const unsigned at = (unsigned)o * krow_bytes + l_tapbyte + (unsigned)l_cc * 64u + kq * 16u;
+            const bool off = none || o >= g.o || l_cc * 16 + kq * 4 >= g.c;
+            if (b_by_value) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                wv[j][e] = __builtin_amdgcn_raw_buffer_load_b32(
+                    rw, off || l_cc * 16 + kq * 4 + e >= g.c ? (int)kOutOfRange : (int)(at + e * 4u), 0, 0);
+            } else {
+              wv[j] = __builtin_amdgcn_raw_buffer_load_b128(rw, off ? (int)kOutOfRange : (int)at, 0, 0);
+            }
+          }
+#pragma unroll
+          for (int j = 0; j < NB; ++j) {
+            if (RUNS) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) w_no_number = w_no_number || (wv[j][e] & 0x7f800000u) == 0x7f800000u;
+            }
+#pragma unroll
+            for (int i = 0; i < WR; ++i)
+              if (wanted(i, j)) WaveMma<float, 16>::run(wv[j], xv[i], rest[i][j]);
+          }
+          step();
+        }
+      }
+      if (RUNS && __any(w_no_number)) {
         // taps outside the image contribute nothing, also where a filter value is infinite: value by value
 #pragma unroll
         for (int i = 0; i < WR; ++i) {
+#pragma unroll
+          for (int j = 0; j < NB; ++j) rest[i][j] = Acc{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
           for (int ky = 0; ky < g.k; ++ky) {
             if ((unsigned)(a_iy[i] + ky) >= (unsigned)g.h) continue;
@@ -1045,54 +1131,6 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
                 }
             }
           }
-        }
-      } else if (redo != 0) {
-        // v_mfma_f32_16x16x4_f32 four times per slab, both operands straight from memory
-        seek(kt_begin);
-#pragma unroll 1
-        while (l_kt < kt_end) {
-          const bool off = l_cc * 16 + kq * 4 >= g.c;
-          u32x4 xv[WR], wv[NB];
-#pragma unroll
-          for (int i = 0; i < WR; ++i) {
-            if (!RUNS) {
-              xv[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, off ? (int)kOutOfRange : (int)(a_tap[i] + (unsigned)l_cc * 64u), 0, 0);
-              continue;
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const bool in = (unsigned)(a_ix[i] + l_cc * 16 + e) < (unsigned)row_values && l_cc * 16 + kq * 4 + e < g.c;
-              const int at = (int)(a_tap[i] + (unsigned)l_cc * 64u + e * 4u);
-              xv[i][e] = __builtin_amdgcn_raw_buffer_load_b32(rx, in && at >= 0 ? at : (int)kOutOfRange, 0, 0);
-            }
-          }
-          if (!again) {   // sums of nothing but zeros: most likely the input is zero here
-            unsigned bits = 0;
-#pragma unroll
-            for (int i = 0; i < WR; ++i) bits |= (xv[i][0] | xv[i][1] | xv[i][2] | xv[i][3]) & 0x7fffffffu;
-            if (!__any(bits != 0)) {
-              step();
-              continue;
-            }
-          }
-#pragma unroll
-          for (int j = 0; j < NB; ++j) {
-            const int o = n0 + j * 16 + lr;
-            const unsigned at = (unsigned)o * krow_bytes + l_tapbyte + (unsigned)l_cc * 64u + kq * 16u;
-            if (!RUNS) {
-              wv[j] = __builtin_amdgcn_raw_buffer_load_b128(rw, off || o >= g.o ? (int)kOutOfRange : (int)at, 0, 0);
-              continue;
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              wv[j][e] = __builtin_amdgcn_raw_buffer_load_b32(
-                  rw, l_cc * 16 + kq * 4 + e < g.c && o < g.o ? (int)(at + e * 4u) : (int)kOutOfRange, 0, 0);
-          }
-#pragma unroll
-          for (int j = 0; j < NB; ++j)
-#pragma unroll
-            for (int i = 0; i < WR; ++i) WaveMma<float, 16>::run(wv[j], xv[i], rest[i][j]);
-          step();
         }
       }
 #pragma unroll
