@@ -705,7 +705,7 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
       const int b = t / g.oh;
       a_iy[i] = ok ? oy * g.stride - g.pad : -0x40000000;   // fails every in-image test
       a_ix[i] = ox * g.stride - g.pad;
-      a_base[i] = (unsigned)(((b * g.h + oy * g.stride - g.pad) * g.w + a_ix[i]) * g.pixel * 4) + kq * 16;
+      a_base[i] = first_tap_offset(g.h, g.w, g.pixel, b, oy * g.stride - g.pad, a_ix[i]) + kq * 16;
       if (RUNS) {
         a_ix[i] *= g.pixel;
         edge = edge || (ok && (a_ix[i] < 0 || a_ix[i] + g.c > g.w * g.pixel));

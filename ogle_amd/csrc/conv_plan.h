@@ -374,6 +374,12 @@ inline bool plan_runs(const OgleConvArgs& a, IgemmPlan* out) {
   return true;
 }
 
+// Byte offset of a pixel's first tap, which may lie in the padding: modulo 2^32, so that a tap inside the image comes
+// out exact whatever the padding and however near to 2 GiB the tensor.
+constexpr unsigned first_tap_offset(int h, int w, int pixel, int image, int iy, int ix) {
+  return (((unsigned)image * (unsigned)h + (unsigned)iy) * (unsigned)w + (unsigned)ix) * (unsigned)pixel * 4u;
+}
+
 // Whether a 16-byte load with a value of a pixel's runs begins before the tensor or ends behind it: such a load
 // returns zeros for all four.  `iy`: the row of the first filter row, `start`: the runs' first value, counted from
 // their rows' first; both may lie in the padding.  (The first row counts wherever it lies: a row of one or two

@@ -4,6 +4,15 @@
 
 using namespace ogle;
 
+// First taps of pixels near the end of a tensor of almost 2 GiB and in a wide padding above it: no signed
+// arithmetic that overflows (which a constant expression may not), the 64-bit offset modulo 2^32.
+constexpr unsigned offset64(long h, long w, long pixel, long image, long iy, long ix) {
+  return (unsigned)((((image * h + iy) * w + ix) * pixel * 4) & 0xffffffffL);
+}
+static_assert(first_tap_offset(11000, 12000, 4, 0, 11003, 12001) == offset64(11000, 12000, 4, 0, 11003, 12001), "");
+static_assert(first_tap_offset(8000, 1000, 4, 16, 7999, 1200) == offset64(8000, 1000, 4, 16, 7999, 1200), "");
+static_assert(first_tap_offset(100, 2000, 1000, 1, -40000, -40000) == offset64(100, 2000, 1000, 1, -40000, -40000), "");
+
 extern "C" {
 
 // 1 if the patch kernel takes the convolution (once the implicit GEMM and the stem kernels have
