@@ -45,8 +45,7 @@ struct IgemmPlan {
   int ktiles;
   int cchunks;
   size_t workspace_bytes;  // splits * M * N floats when splits > 1
-  bool pieces;             // fp32 contracted as bf16 pieces, in tiles of cfg
-  int form;                // the workgroup that runs such a tile, or one in place of cfg's (PiecesForm)
+  int form;                // the workgroup that contracts fp32 as bf16 pieces in place of cfg's (PiecesForm)
 };
 
 constexpr long kComputeUnits = 256;
@@ -282,7 +281,7 @@ inline IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
   // 128x32 tiles 0.83 to 0.98 from 9 slabs on with 3x3, 0.97 to 1.04 pointwise.  150x150x32 -> 64 at batch
   // 16 26.4 us instead of 27.5, at batch 1 4.8 instead of 5.8.
   const long workgroups = tiles(p.cfg) * p.splits;
-  p.pieces = a.dtype == OGLE_F32 && (p.cfg == CFG_128x128 || p.cfg == CFG_64x64 || p.cfg == CFG_128x32) &&
+  const bool pieces = a.dtype == OGLE_F32 && (p.cfg == CFG_128x128 || p.cfg == CFG_64x64 || p.cfg == CFG_128x32) &&
              workgroups > kComputeUnits && p.slabs_per_split >= kPiecesSlabs &&
              workgroups * p.slabs_per_split > 16 * kComputeUnits &&
              !(p.cfg == CFG_128x32 && is_pointwise(a));
@@ -292,14 +291,14 @@ inline IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
     // 38x38x1024 -> 16 at batch 24 43.6 / 51.3)
     p.form = FORM_128x16;
   } else if (a.dtype != OGLE_F32 || p.splits > 1) {
-    p.form = !p.pieces ? FORM_NONE
+    p.form = !pieces ? FORM_NONE
              : p.cfg == CFG_64x64 ? FORM_64x64
              : p.cfg == CFG_128x32 ? FORM_128x32
              : is_pointwise(a) ? FORM_128x128 : FORM_128x64_W8;
   } else if (p.cfg == CFG_64x64 || p.cfg == CFG_128x128) {
-    p.form = pieces_form(a, m, p.ktiles, p.cfg == CFG_128x128, p.pieces);
+    p.form = pieces_form(a, m, p.ktiles, p.cfg == CFG_128x128, pieces);
   } else if (p.cfg == CFG_128x32) {
-    p.form = p.pieces ? FORM_128x32 : FORM_NONE;
+    p.form = pieces ? FORM_128x32 : FORM_NONE;
   } else if (p.cfg == CFG_WAVE32 && is_pointwise(a) && p.ktiles >= 12) {
     // two K groups against the wave-split kernel, where that one's 32x32 tiles need a second round of the units
     // and 64x32 tiles do not: 1x1 M = 1600, 1024 -> 256 14.9 / 16.4, M = 1444, 256 -> 256 6.1 / 6.8, M = 392, 208 ->

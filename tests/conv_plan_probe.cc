@@ -15,13 +15,14 @@ static_assert(first_tap_offset(100, 2000, 1000, 1, -40000, -40000) == offset64(1
 
 extern "C" {
 
-// 1 if the patch kernel takes the convolution (once the implicit GEMM and the stem kernels have
+// 1 if the patch kernel takes the convolution (once the implicit GEMM, the stem kernels and runs have
 // not), then out = columns, groups and channels staged at once, K runs per filter row, boxes,
 // workgroups along the boxes, workgroups in all, vector staging of patch and filter, LDS floats.
 int probe_patch(const OgleConvArgs* a, int64_t* out) {
   PatchPlan p;
+  IgemmPlan runs;
   long m = 0;
-  if (igemm_eligible(*a, &m) || plan_direct(*a, &p) != DIRECT_PATCH) return 0;
+  if (igemm_eligible(*a, &m) || plan_runs(*a, &runs) || plan_direct(*a, &p) != DIRECT_PATCH) return 0;
   const int64_t boxes = (int64_t)p.tiles_b * p.tiles_y * p.tiles_x;
   const int64_t v[] = {p.cols, p.gp, p.cc, p.runs_x, boxes, p.tile_blocks,
                        (int64_t)p.tile_blocks * p.gblocks * p.col_blocks, p.vec_x, p.vec_w, p.lds_floats};
@@ -29,23 +30,26 @@ int probe_patch(const OgleConvArgs* a, int64_t* out) {
   return 1;
 }
 
-// Which of the direct kernels takes the convolution (DirectKernel); -1 if the implicit GEMM does.
+// Which of the direct kernels takes the convolution (DirectKernel); -1 if the implicit GEMM does, -2 if it
+// is contracted as runs.
 int probe_direct(const OgleConvArgs* a) {
   PatchPlan p;
+  IgemmPlan runs;
   long m = 0;
-  return igemm_eligible(*a, &m) ? -1 : (int)plan_direct(*a, &p);
+  return igemm_eligible(*a, &m) ? -1 : plan_runs(*a, &runs) ? -2 : (int)plan_direct(*a, &p);
 }
 
-// 1 if the implicit GEMM takes the convolution, then out = rows and columns of the tile, tiles,
-// K ranges, whether fp32 is contracted as bf16 pieces, workspace bytes.
+// 1 if the implicit GEMM takes the convolution, then out = rows and columns of the planned tile, tiles,
+// K ranges, workspace bytes, whether fp32 is contracted as bf16 pieces and the rows and columns that a
+// workgroup then has.
 int probe_igemm(const OgleConvArgs* a, int scratch, int64_t* out) {
   long m = 0;
   if (!igemm_eligible(*a, &m)) return 0;
   const IgemmPlan p = plan_igemm(*a, m, scratch != 0);
   const int bm = tile_bm(p.cfg), bn = tile_bn(p.cfg);
   const int64_t v[] = {bm, bn, (int64_t)((m + bm - 1) / bm) * ((a->out_c + bn - 1) / bn),
-                       p.splits, p.pieces, (int64_t)p.workspace_bytes};
-  for (int i = 0; i < 6; ++i) out[i] = v[i];
+                       p.splits, (int64_t)p.workspace_bytes, p.form != FORM_NONE, kFormBM[p.form], kFormBN[p.form]};
+  for (int i = 0; i < 8; ++i) out[i] = v[i];
   return 1;
 }
 

@@ -43,7 +43,9 @@ def patch_plan(probe, *shape, **kw):
 def test_infinite_filter_cases_walk_several_boxes(probe):
     """Of the cases with infinite filter values some give a workgroup one box, some several, one
     stages its channels in chunks."""
-    plans = [patch_plan(probe, n, h, w, c, o, k, s, p, 1, g) for n, h, w, c, o, k, s, p, g in K.INFINITE_FILTER_CASES]
+    args = [(n, h, w, c, o, k, s, p, 1, g) for n, h, w, c, o, k, s, p, g in K.INFINITE_FILTER_CASES]
+    assert [probe.probe_direct(ctypes.byref(conv(*a))) for a in args] == [PATCH, PATCH, PATCH, RUNS, PATCH]
+    plans = [patch_plan(probe, *a) for a in args[:3] + args[4:]]
     assert [p["boxes"] > p["box_blocks"] for p in plans] == [False, False, True, True]
     assert plans[1]["cc"] < 130
     assert plans[2]["gp"] > 1
@@ -86,23 +88,31 @@ def test_patch_plan_stays_within_a_launch(probe):
     assert plan["cc"] < 511 and plan["boxes"] == plan["blocks"] and plan["blocks"] * 256 < 2 ** 32
 
 
-@pytest.mark.parametrize("shape,patch", [
-    # n, h, w, c, o, k, s, p, d, g: next to the line on both sides, as measured (conv_plan.h)
-    ((1, 1, 1, 17, 33, 3, 1, 1), False),            # eight of nine taps lie in the padding
-    ((1, 4, 4, 192, 192, 3, 1, 1, 1, 12), True),
-    ((1, 14, 14, 7, 33, 3, 1, 1), False),
-    ((1, 14, 14, 17, 33, 3, 1, 1), True),
-    ((1, 56, 56, 35, 33, 1), False),
-    ((1, 56, 56, 35, 75, 1), True),
-    ((1, 28, 28, 131, 33, 1), False),
-    ((4, 56, 56, 32, 48, 1, 1, 0, 1, 4), True),
-    ((4, 57, 43, 96, 144, 3, 1, 1, 1, 12), True),
-])
-def test_patch_kernel_where_it_is_faster(probe, shape, patch):
-    assert (patch_plan(probe, *shape) is not None) == patch
-
-
 GENERAL, PATCH, SMALL_K = 0, 1, 2   # DirectKernel
+RUNS = -2                           # none of them: contracted as runs of values
+
+
+@pytest.mark.parametrize("shape,dtype,kernel", [
+    # n, h, w, c, o, k, s, p, d, g: next to the line on both sides, as measured (conv_plan.h); in fp32 most ungrouped,
+    # undilated ones are runs by now
+    ((1, 1, 1, 17, 33, 3, 1, 1), H.F32, GENERAL),         # eight of nine taps lie in the padding
+    ((1, 4, 4, 192, 192, 3, 1, 1, 1, 12), H.F32, PATCH),
+    ((1, 14, 14, 7, 33, 3, 1, 1), H.F32, RUNS),
+    ((1, 14, 14, 7, 33, 3, 1, 1), H.F16, GENERAL),
+    ((1, 14, 14, 17, 33, 3, 1, 1), H.F32, RUNS),
+    ((1, 14, 14, 17, 33, 3, 1, 1), H.F16, PATCH),
+    ((1, 14, 14, 17, 33, 3, 1, 2, 2), H.F32, PATCH),
+    ((1, 56, 56, 35, 33, 1), H.F32, GENERAL),
+    ((1, 56, 56, 35, 75, 1), H.F32, RUNS),
+    ((1, 56, 56, 35, 75, 1), H.F16, PATCH),
+    ((1, 28, 28, 131, 33, 1), H.F32, RUNS),
+    ((1, 28, 28, 131, 33, 1), H.F16, GENERAL),
+    ((4, 56, 56, 32, 48, 1, 1, 0, 1, 4), H.F32, PATCH),
+    ((4, 57, 43, 96, 144, 3, 1, 1, 1, 12), H.F32, PATCH),
+])
+def test_patch_kernel_where_it_is_faster(probe, shape, dtype, kernel):
+    assert probe.probe_direct(ctypes.byref(conv(*shape, dtype=dtype))) == kernel
+    assert (patch_plan(probe, *shape, dtype=dtype) is not None) == (kernel == PATCH)
 
 
 @pytest.mark.parametrize("shape,dtype,kernel", [
@@ -110,13 +120,18 @@ GENERAL, PATCH, SMALL_K = 0, 1, 2   # DirectKernel
     ((1, 14, 14, 7, 16, 3, 1, 1), H.F32, SMALL_K),
     ((1, 14, 14, 17, 16, 3, 1, 1), H.F32, PATCH),
     ((1, 28, 28, 33, 16, 3, 2, 1), H.F16, SMALL_K),     # stride 2: three chunks of channels to stage
-    ((1, 56, 56, 35, 64, 1), H.F32, SMALL_K),
+    ((1, 56, 56, 35, 64, 1), H.F32, RUNS),
+    ((1, 56, 56, 35, 64, 1), H.F16, SMALL_K),
     ((1, 56, 56, 36, 64, 1), H.F16, SMALL_K),
-    ((4, 56, 56, 35, 256, 1), H.F32, PATCH),            # many products
-    ((8, 112, 112, 131, 16, 1), H.F32, PATCH),          # an input of 53 MB
-    ((8, 112, 112, 3, 64, 7, 2, 3), H.F32, PATCH),
+    ((4, 56, 56, 35, 256, 1), H.F32, RUNS),
+    ((4, 56, 56, 35, 256, 1), H.F16, PATCH),            # many products
+    ((8, 112, 112, 131, 16, 1), H.F32, RUNS),
+    ((8, 112, 112, 131, 16, 1), H.F16, PATCH),          # an input of 26 MB
+    ((8, 112, 112, 3, 64, 7, 2, 3), H.F32, RUNS),
+    ((8, 112, 112, 3, 64, 7, 2, 3), H.F16, PATCH),
     ((1, 14, 14, 28, 256, 1), H.F32, GENERAL),          # short sums of a small output
-    ((1, 28, 28, 131, 64, 1), H.F32, SMALL_K),
+    ((1, 28, 28, 131, 64, 1), H.F32, RUNS),
+    ((1, 28, 28, 131, 64, 1), H.F16, SMALL_K),
     ((1, 28, 28, 12, 16, 3, 1, 1), H.F16, PATCH),
 ])
 def test_direct_kernel_with_the_filter_in_lds(probe, shape, dtype, kernel):
@@ -125,13 +140,13 @@ def test_direct_kernel_with_the_filter_in_lds(probe, shape, dtype, kernel):
 
 @pytest.mark.parametrize("dtype", [H.F32, H.F16])
 def test_small_k_cases_run_that_kernel(probe, dtype):
-    for case in K.SMALL_K_CASES:
-        assert probe.probe_direct(ctypes.byref(conv(*case, dtype=dtype))) == SMALL_K, case
-    n, h, w, _, o = K.SMALL_K_CASES[-1][:5]
-    assert n * h * w * (o // 16) >= 256 * 256 * 4 > max(a[0] * a[1] * a[2] * (a[4] // 16) for a in K.SMALL_K_CASES[:-1])
+    kernels = [probe.probe_direct(ctypes.byref(conv(*case, dtype=dtype))) for case in K.SMALL_K_CASES]
+    assert kernels == [SMALL_K] * 3 + [RUNS if dtype == H.F32 else SMALL_K] * 2 + [SMALL_K]
+    threads = [a[0] * a[1] * a[2] * (a[4] // 16) for a in K.SMALL_K_CASES]
+    assert min(threads[-2:]) >= 256 * 256 * 4 > max(threads[:-2])
 
 
-IGEMM_FIELDS = ("bm", "bn", "tiles", "splits", "pieces", "workspace")
+IGEMM_FIELDS = ("bm", "bn", "tiles", "splits", "workspace", "pieces", "rows", "cols")
 
 
 def igemm_plan(probe, *shape, scratch=True, **kw):
@@ -159,7 +174,7 @@ def test_pieces_where_they_are_faster(probe, shape, pieces):
 
 
 def test_large_fp32_tiles_are_pieces(probe):
-    """128x128 tiles of fp32 are built as pieces only."""
+    """128x128 tiles of fp32 are not built: workgroups of pieces run their plans."""
     r, large = random.Random(7), 0
     for _ in range(40000):
         k = r.choice([1, 1, 3])
@@ -183,9 +198,14 @@ def test_heads_of_one_image_have_no_pieces(probe):
 @pytest.mark.parametrize("dtype", [H.F32, H.F16])
 def test_patch_cases_run_what_they_name(probe, dtype):
     direct = [probe.probe_direct(ctypes.byref(conv(*case, dtype=dtype))) for case in K.PATCH_CASES]
-    assert direct == [PATCH, PATCH, PATCH, -1, PATCH, PATCH, GENERAL, PATCH, GENERAL, GENERAL, PATCH, PATCH]
-    for case, want in K.PATCH_WIDE_CASES:
+    runs = dtype == H.F32
+    assert direct == [PATCH, PATCH, PATCH, -1] + ([RUNS] * 4 if runs else [PATCH, PATCH, GENERAL, PATCH]) + \
+        [GENERAL, GENERAL, PATCH, PATCH]
+    for case, want in K.PATCH_WIDE_CASES + K.PATCH_NOT_RUNS_CASES:
         plan = patch_plan(probe, *case, dtype=dtype)
+        if runs and case == (33, 34, 26, 66, 65, 1, 1, 0, 1, 1):
+            assert plan is None and probe.probe_direct(ctypes.byref(conv(*case))) == RUNS
+            continue
         assert plan is not None, case
         plan["several"] = plan["boxes"] > plan["box_blocks"]
         assert {key: plan[key] for key in want} == want, (case, plan)
@@ -196,19 +216,34 @@ def test_patch_cases_run_what_they_name(probe, dtype):
 def test_pieces_cases_run_what_they_name(probe):
     def tile(*shape, scratch=True):
         plan = igemm_plan(probe, *shape, scratch=scratch)
-        return "%dx%d%s%s" % (plan["bm"], plan["bn"], " split" if plan["splits"] > 1 else "", " pieces" if plan["pieces"] else "")
+        name = "%dx%d pieces" % (plan["rows"], plan["cols"]) if plan["pieces"] else "%dx%d" % (plan["bm"], plan["bn"])
+        return name + (" split" if plan["splits"] > 1 else "")
     assert [tile(*case) for case in K.PIECES_CASES] == [
-        "64x64", "64x64", "64x64 pieces", "128x128 pieces", "64x64 pieces", "32x32", "128x32 pieces", "64x64",
-        "64x64 split", "64x64 pieces", "64x64 pieces", "128x128 pieces", "64x64 split pieces"]
+        "64x64", "64x64", "64x64 pieces", "128x128 pieces", "128x64 pieces", "32x32", "128x32 pieces", "64x32 pieces",
+        "64x64 split", "128x64 pieces", "64x32 pieces", "128x64 pieces", "64x64 pieces split", "64x64"]
+    assert [tile(*case, scratch=False) for case in K.PIECES_CASES if tile(*case).endswith("split")] == ["64x32 pieces"] * 2
     assert [tile(3, 75, 75, 512, 64, 3, 1, 1, scratch=False), tile(16, 19, 19, 512, 512, 1),
-            tile(1, 160, 160, 32, 256, 3, 1, 1)] == ["64x64 pieces", "64x64 pieces", "128x128 pieces"]
+            tile(1, 160, 160, 32, 256, 3, 1, 1)] == ["128x64 pieces", "64x64 pieces", "128x64 pieces"]
     assert [tile(n, h, w, c, o, k, 1, p) for n, h, w, c, o, k, p in K.NOT_FINITE_CASES] == [
-        "64x64 pieces", "128x128 pieces", "64x64", "64x64 pieces", "64x64 split pieces", "128x32 pieces", "128x128 pieces"]
+        "64x64 pieces", "128x128 pieces", "64x64 pieces", "128x64 pieces", "64x64 pieces split", "128x32 pieces",
+        "128x64 pieces", "64x64"]
     assert [tile(n, h, w, c, o, k, 1, p) for n, h, w, c, o, k, p in K.TINY_CASES] == [
         "64x64 pieces", "128x128 pieces", "128x32 pieces"]
-    assert [[tile(*case) for case in batch] for batch in K.BATCHES_OF_PIECES] == [
-        ["64x64 pieces"] * 2, ["128x32 pieces"] * 2, ["128x128 pieces"] * 2, ["64x64 pieces", "64x64"],
-        ["64x64 split pieces", "128x16 split", "64x64", "128x32 pieces"]]
+    assert [[tile(*case) for case in batch] for batch in K.BATCHES_OF_PIECES] == [   # each alone
+        ["128x64 pieces"] * 2, ["128x32 pieces"] * 2, ["128x64 pieces"] * 2, ["128x64 pieces", "64x64"],
+        ["64x64 pieces split", "128x16 split", "64x64", "128x32 pieces"]]
+
+
+def test_batches_of_one_form(probe):
+    """Every form that a grouped launch of one kind has a kernel for is the form of some batch's members."""
+    grouped = {5: 1, 6: 8, 7: 8, 2: 10, 9: 11}     # what stands in for a form in a group
+    kinds = set()
+    for batch in K.BATCHES_OF_PIECES + K.BATCHES_OF_FORMS:
+        forms = [probe.probe_form(ctypes.byref(conv(*case)), 1) for case in batch]
+        of = {(grouped.get(f, f), case[5] == 1 and case[6] == 1) for f, case in zip(forms, batch)}
+        if len(of) == 1 and len(batch) > 1:
+            kinds |= of
+    assert kinds == {(1, True), (1, False), (3, True), (8, True), (8, False), (10, False), (11, True), (11, False)}
 
 
 def test_form_cases_run_what_they_name(probe):

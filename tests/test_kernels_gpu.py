@@ -137,7 +137,7 @@ def test_conv_stem_kernel(case, dtype):
 
 
 PATCH_CASES = [
-    # n, h, w, c, o, k, s, p, d, g   mostly the LDS patch kernel, 16 columns, one box per workgroup
+    # n, h, w, c, o, k, s, p, d, g   mostly the LDS patch kernel (in fp16), 16 columns, one box per workgroup
     (4, 57, 43, 96, 144, 3, 1, 1, 1, 12),   # several groups per workgroup, vector staging, ragged box
     (2, 23, 19, 80, 80, 3, 1, 1, 1, 5),     # 16 channels per group: exactly one 16-wide block
     (2, 23, 19, 34, 34, 3, 1, 1, 1, 2),     # 17 per group: one past it, odd channel count (merged runs)
@@ -182,11 +182,26 @@ FULL_LDS_CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", PATCH_CASES + FULL_LDS_CASES + [case for case, _ in PATCH_WIDE_CASES])
+# of those above, fp32 takes as runs of values what is ungrouped and not dilated; these are the patch kernel's
+PATCH_NOT_RUNS_CASES = [
+    # n, h, w, c, o, k, s, p, d, g          and what its plan has to be
+    # chunks of channels with a ragged last one, 4 column blocks
+    ((2, 29, 31, 33, 64, 3, 2, 2, 2, 1), dict(cols=16, cc=16, several=False)),
+    # many chunks, a last column block of one channel
+    ((1, 40, 41, 131, 65, 3, 1, 2, 2, 1), dict(cols=16, cc=32, several=False)),
+    # 32 columns, a last block of one channel, several boxes
+    ((66, 34, 26, 66, 130, 1, 1, 0, 1, 2), dict(cols=32, cc=33, several=True)),
+    # whole filter rows as runs, 4 column blocks
+    ((2, 40, 38, 6, 128, 7, 2, 3, 1, 2), dict(cols=16, runs=1, cc=3)),
+]
+PATCH_ALL_CASES = PATCH_CASES + FULL_LDS_CASES + [case for case, _ in PATCH_WIDE_CASES + PATCH_NOT_RUNS_CASES]
+
+
+@pytest.mark.parametrize("case", PATCH_ALL_CASES)
 @pytest.mark.parametrize("dtype", [H.F32, H.F16])
 def test_conv_patch_kernel(case, dtype):
     n, h, w, c, o, k, s, p, d, g = case
-    r = rng(2900 + (PATCH_CASES + FULL_LDS_CASES + [case for case, _ in PATCH_WIDE_CASES]).index(case))
+    r = rng(2900 + PATCH_ALL_CASES.index(case))
     x = r.uniform(-1, 1, (n, h, w, c)).astype(np.float32)
     wt = r.normal(0, 0.5, (o, c // g, k, k)).astype(np.float32)
     b = r.uniform(-0.1, 0.1, o).astype(np.float32)
@@ -203,7 +218,8 @@ SMALL_K_CASES = [
     (2, 1, 1, 33, 12, 3, 1, 1, 1),       # a map of one pixel: all taps but one in the padding
     (3, 9, 7, 11, 20, 3, 2, 2, 2),       # stride 2, dilation 2
     (1, 56, 55, 35, 64, 1, 1, 0, 1),     # pointwise, odd channel count
-    (8, 111, 112, 35, 64, 1, 1, 0, 1),   # sixteen channels per thread
+    (8, 111, 112, 35, 64, 1, 1, 0, 1),   # sixteen channels per thread (fp16; fp32 ones, like the last, run as runs)
+    (24, 110, 112, 5, 16, 3, 1, 2, 2),   # sixteen in fp32 too
 ]
 
 
@@ -226,7 +242,8 @@ INFINITE_FILTER_CASES = [
     (2, 20, 18, 24, 36, 3, 1, 1, 3),        # one box per workgroup, all channels staged at once
     (1, 17, 16, 130, 20, 3, 1, 1, 1),       # channels in chunks
     (16, 57, 43, 96, 144, 3, 1, 1, 12),     # several groups and several boxes per workgroup
-    (8, 224, 222, 3, 64, 7, 2, 3, 1),       # several boxes, merged runs, 64 columns
+    (8, 224, 222, 3, 64, 7, 2, 3, 1),       # ungrouped, undilated fp32: runs of values
+    (33, 35, 25, 49, 693, 3, 2, 1, 7),      # several boxes, merged runs, 64 columns
 ]
 
 
@@ -268,15 +285,16 @@ PIECES_CASES = [
     (1, 96, 168, 64, 40, 1, 1, 0),      # 252 workgroups: fp32
     (16, 19, 19, 512, 512, 1, 1, 0),    # 64x64 tiles, 728 workgroups
     (1, 223, 221, 256, 128, 1, 1, 0),   # 128x128 tiles, 386 of them, last one ragged
-    (1, 217, 221, 260, 124, 1, 1, 0),   # 375 large tiles: 64x64; K tail inside a slab, ragged N
+    (1, 217, 221, 260, 124, 1, 1, 0),   # 375 large tiles: 128x64; K tail inside a slab, ragged N
     (2, 75, 73, 36, 32, 3, 1, 1),       # 86 tiles of 128x32: the wave-split kernel, fp32
     (5, 84, 84, 36, 31, 3, 1, 1),       # 128x32 tile, 3x3, 276 workgroups, odd N
-    (3, 75, 73, 44, 70, 3, 2, 1),       # 64x64, stride 2, 132 workgroups: fp32
-    (2, 19, 19, 512, 63, 3, 1, 1),      # ranges of six slabs, odd N, K = 4608: fp32
-    (1, 96, 174, 260, 40, 1, 1, 0),     # 64x64 tiles, 261 workgroups of 17 slabs, ragged N
-    (6, 75, 73, 44, 70, 3, 2, 1),       # 64x64, stride 2, 264 workgroups, one tile column and a bit
-    (1, 160, 160, 32, 256, 3, 1, 1),    # 128x128 tiles, 3x3
-    (8, 19, 19, 512, 63, 3, 1, 1),      # ranges of K, odd N, K = 4608; without scratch fp32
+    (3, 75, 73, 44, 70, 3, 2, 1),       # 64x32, two K groups, stride 2
+    (2, 19, 19, 512, 63, 3, 1, 1),      # ranges of six slabs, odd N, K = 4608: fp32; without scratch 64x32
+    (1, 96, 174, 260, 40, 1, 1, 0),     # 128x64, 131 workgroups of 17 slabs, ragged N
+    (6, 75, 73, 44, 70, 3, 2, 1),       # 64x32, stride 2, one tile column and a bit
+    (1, 160, 160, 32, 256, 3, 1, 1),    # 128x64 in place of 128x128 tiles, 3x3
+    (8, 19, 19, 512, 63, 3, 1, 1),      # ranges of K, odd N, K = 4608; without scratch 64x32
+    (3, 75, 73, 12, 70, 3, 2, 1),       # 64x64, stride 2, 132 workgroups of nine slabs: fp32
 ]
 
 
@@ -325,11 +343,12 @@ def test_conv_fp32_as_bf16_pieces_sums_in_two_norms(case):
 NOT_FINITE_CASES = [
     # n, h, w, c, o, k, p
     (16, 19, 19, 512, 512, 1, 0), (1, 223, 221, 256, 128, 1, 0),
-    (2, 75, 75, 64, 63, 3, 1),          # 176 workgroups: fp32
-    (4, 75, 75, 64, 63, 3, 1),          # 64x64 tiles, 3x3, odd N
+    (2, 75, 75, 64, 63, 3, 1),          # 64x64 tiles, two K groups
+    (4, 75, 75, 64, 63, 3, 1),          # 128x64, 3x3, odd N
     (8, 19, 19, 512, 63, 3, 1),         # ranges of K
     (5, 84, 84, 36, 31, 3, 1),          # 128x32 tiles
-    (1, 160, 160, 32, 256, 3, 1),       # 128x128 tiles, 3x3
+    (1, 160, 160, 32, 256, 3, 1),       # 128x64 in place of 128x128 tiles, 3x3
+    (2, 75, 75, 16, 63, 3, 1),          # 176 workgroups of nine slabs: fp32
 ]
 
 
@@ -712,11 +731,11 @@ def test_config3_pointwise_gemm(dtype):
 
 
 BATCHES_OF_PIECES = [
-    # n, h, w, c, o, k, s, p   one tile shape each: the grouped kernel of 64x64, 128x32, 128x128 tiles
+    # n, h, w, c, o, k, s, p   one form each: the grouped kernel of 64x64 workgroups, pointwise and 3x3, and of 64x32 ones
     [(8, 19, 19, 256, 512, 1, 1, 0), (7, 19, 19, 260, 500, 1, 1, 0)],
     [(5, 84, 84, 36, 31, 3, 1, 1), (5, 84, 83, 32, 24, 3, 1, 1)],
     [(1, 160, 160, 32, 256, 3, 1, 1), (1, 161, 160, 32, 250, 3, 1, 1)],
-    # one tile shape, with and without pieces: the mixed kernel
+    # 64x64, with and without pieces: the mixed kernel
     [(16, 28, 28, 128, 128, 3, 1, 1), (16, 56, 56, 64, 128, 1, 2, 0)],
     # 64x64 and 128x32, with and without pieces
     [(8, 19, 19, 512, 63, 3, 1, 1), (8, 19, 19, 512, 12, 3, 1, 1), (2, 9, 9, 32, 40, 1, 1, 0), (5, 84, 84, 36, 31, 3, 1, 1)],
@@ -726,6 +745,11 @@ BATCHES_OF_FORMS = [
     [(1, 97, 97, 36, 40, 3, 1, 1), (1, 66, 66, 44, 88, 3, 1, 1)],
     [(1, 119, 118, 36, 72, 3, 1, 1), (1, 66, 66, 44, 88, 3, 1, 1), (2, 97, 98, 44, 12, 3, 1, 1), (4, 19, 19, 388, 512, 1, 1, 0),
      (1, 96, 97, 388, 520, 1, 1, 0), (1, 160, 160, 32, 255, 3, 1, 1), (3, 75, 73, 44, 70, 3, 2, 1)],
+    # the other kernels of one form: 128x128, 64x16 3x3 and pointwise, 32x32 in two K groups, pointwise
+    [(1, 223, 221, 256, 128, 1, 1, 0), (1, 223, 221, 260, 124, 1, 1, 0)],
+    [(2, 97, 98, 44, 12, 3, 1, 1), (2, 97, 95, 48, 15, 3, 1, 1)],
+    [(2, 97, 98, 200, 15, 1, 1, 0), (2, 97, 97, 204, 16, 1, 1, 0)],
+    [(4, 19, 19, 388, 512, 1, 1, 0), (4, 19, 19, 392, 500, 1, 1, 0)],
     # the first holds the operands that are no numbers: sums contracted again are the same ones in every form
     [(1, 96, 97, 388, 520, 1, 1, 0), (2, 97, 98, 44, 12, 3, 1, 1)],
     [(2, 97, 98, 44, 12, 3, 1, 1), (5, 84, 84, 36, 31, 3, 1, 1)],
