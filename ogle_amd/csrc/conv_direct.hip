@@ -3,8 +3,9 @@
 // conv_stem_* (K = k*k*C <= 32, group 1), conv_patch_mfma (input patch and filter staged in
 // LDS, contracted on the MFMA units), conv_direct_small_k (group 1, the filter in LDS, one thread
 // per 4 or 16 channels of a pixel) and conv_direct_general (one thread per output).  plan_direct
-// chooses among the last three, for what plan_runs leaves: ungrouped fp32 convolutions of any size
-// run as bf16 pieces (conv_igemm.hip).
+// chooses among the last three, for what plan_runs leaves: ungrouped fp32 convolutions without dilation run
+// as bf16 pieces (conv_igemm.hip), unless their sums are short, their outputs small, with more than one tap at
+// most 16 channels, or an operand reaches 2 GiB.
 //
 // Semantics follow conv2d.glsl:29-92 / conv2d_grp.glsl:30-123: bias, taps outside the image
 // contribute nothing, then the fused activation.

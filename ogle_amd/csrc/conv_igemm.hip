@@ -591,7 +591,9 @@ struct IgemmProblem {
   int tiles_n, tiles;
   float* partial;
   int slabs_per_split, splits;
-  int variant;  // mixed-group kernel only: 2 * (tile is 128x32) + (pointwise); 4..7: wave-split 32 / 16; 8, 9: 128x16 tile; + 16: as bf16 pieces
+  // mixed-group kernel only, + 1 if pointwise: tiles of 64x64 0, 128x32 2, 128x16 8, wave-split 32x32 4, 16x16 6; as
+  // bf16 pieces 64x64 16, 64x32 18 (never pointwise), 32x32 in two K groups 20, 64x16 22
+  int variant;
 };
 
 // fp32 operands as three bf16 pieces each: x = h + m + l (24 significand bits in three times 8;
@@ -652,8 +654,8 @@ constexpr int pieces_lds_bytes() { return KG * 2 * 3 * NB * 1024; }
 // roundings vanish and the main sums are rounded once per 32 products.
 //
 // Measured on MI355X against both operands split on their way to LDS (32x32x16 MFMAs, 64 rows of each
-// operand per 64x64 tile and 16 channels), us: 19x19x512 -> 512 at batch 16 27.8 -> 24.4, 3x3 56x56x64 ->
-// 64 36.7 -> 29.1, 28x28x128 -> 128 38.0 -> 31.0, M = 11552, K = 512, N = 1024 74.5 -> 68.5 (177 TFLOP/s);
+// operand per 64x64 tile and 16 channels), us: 19x19x512 -> 512 at batch 16 25.4 -> 23.8, 3x3 56x56x64 ->
+// 64 35.6 -> 28.7, 28x28x128 -> 128 38.1 -> 31.3, M = 11552, K = 512, N = 1024 73.1 -> 73.3 (165 TFLOP/s);
 // error against 64-bit sums at K = 512 1.24e-7 -> 1.20e-7 (fp32 MFMAs 4.1e-7).  Large problems are bound by
 // power: the library's bf16 GEMM of 8192 cubed reaches 1145 / 6 = 191.  Smaller ones share it among LDS
 // writes, splitting and MFMAs; loads further ahead, and splitting interleaved with MFMAs by hand, gained nothing.
@@ -901,7 +903,7 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
   // Two register sets: the loads of stage s + 2 are requested when stage s has been split.  One barrier
   // per stage: the planes of stage s + 1 are written while those of stage s are read.  Large tiles
   // split the filter before they multiply, which frees its registers for the next loads (the other
-  // order spills: 11552 x 512 -> 1024 87 us instead of 68), small ones behind (19x19x512 -> 512, batch
+  // order spills: a quarter slower), small ones behind (19x19x512 -> 512, batch
   // 16, 24.3 instead of 24.9; 3x3 56x56x64 -> 64 33.7 / 34.3).
   {
     constexpr bool SPLIT_FIRST = WR * NB >= 16;
@@ -1271,10 +1273,10 @@ __device__ __forceinline__ void igemm_wave_tile(
     const float* __restrict__ bias, T* __restrict__ y, T* __restrict__ y2, int o1, const Epilogue& ep,
     int tiles_n, int bid);
 
-// A group whose members differ in tile shape (64x64 or 128x32) or in being
-// pointwise: each workgroup takes the code path of its own problem.  The branch is
-// uniform over the workgroup; all four paths keep 16 accumulator registers per
-// lane, so the register budget is that of the largest one.
+// A group whose members differ in tile shape or in being pointwise: each workgroup
+// takes the code path of its own problem.  The branch is uniform over the workgroup;
+// the paths without pieces keep up to 16 accumulator registers per lane, those with
+// them two sets of 16, so the register budget is that of the largest one.
 // SPLIT: some problem of the group is contracted as bf16 pieces.  Its tiles need more registers, LDS
 // and code than the others': a group without (the heads of one image) does without them as well.  Forms of
 // 128 rows and of two times four waves are replaced (grouped_form) so that four workgroups fit a unit: the heads
@@ -1308,7 +1310,7 @@ __global__ __launch_bounds__(256, SPLIT ? 4 : 1) void conv_igemm_mixed_kernel(Ig
       case 23: pieces_tile<1, 1, 4, 1, true>(lds, p, bid); return;
     }
   }
-  switch (p.variant & 15) {
+  switch (p.variant) {
     OGLE_MIXED_CASE(0, 64, 64, 2, 2, false)
     OGLE_MIXED_CASE(1, 64, 64, 2, 2, true)
     OGLE_MIXED_CASE(2, 128, 32, 4, 1, false)

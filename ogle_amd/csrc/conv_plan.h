@@ -265,21 +265,21 @@ inline IgemmPlan plan_igemm(const OgleConvArgs& a, long m, bool allow_split) {
       p.splits > 1 ? (size_t)p.splits * (size_t)m * ((a.out_c + 3) & ~3) * sizeof(float) : 0;
   // fp32 tiles of 32x32 MFMA blocks are contracted as bf16 pieces (the 96 and 160 columns wide ones
   // are not built as such) where a compute unit has more than one workgroup and more than 16 slabs:
-  // a lone workgroup has nothing to cover the splitting with, and a short sum is over before the faster
+  // a lone workgroup has little to cover the splitting with, and a short sum is over before the faster
   // unit has made up for it.  Not for two slabs at all, nor for pointwise convolutions to at most 32
-  // channels: both are bound by their bytes.  Time with pieces (both operands split on their way to LDS; the
-  // present kernels are up to 15 % faster) over time with fp32 MFMAs, 64x64 tiles:
+  // channels: both are bound by their bytes.  Time with pieces in the form of pieces_form over time with fp32 MFMAs,
+  // plans of 64x64 tiles, means of 950 shapes:
   //   slabs  workgroups to 384   512   768  1024  1536  2560  5000
-  //     2         1.20  1.23  1.13  1.12  1.09  1.12  1.07
-  //     3         1.12  1.13  1.07  1.03  0.99  0.98  0.90
-  //     4         1.12  1.15  1.07  1.03  0.98  0.99  0.91
-  //     6         1.02  1.05  0.99  0.95  0.93  0.95  0.87
-  //     9         0.97  0.96  0.92  0.87  0.84  0.86  0.84
-  //    16         0.97  0.98  0.90  0.93  0.88  0.89
-  //    36         0.87  0.90  0.88  0.90  0.85  0.89
-  //    72         0.84  0.90  0.88  0.89  0.86  0.86
-  // 128x32 tiles 0.83 to 0.98 from 9 slabs on with 3x3, 0.97 to 1.04 pointwise.  150x150x32 -> 64 at batch
-  // 16 26.4 us instead of 27.5, at batch 1 4.8 instead of 5.8.
+  //     2         1.06        0.96  0.91  1.09  1.11  1.13
+  //     3         0.91  0.94  0.92  0.97  0.95  0.95  0.93
+  //     4         0.98  0.99  0.90  0.96  0.96  0.94  0.93
+  //     6         0.94  0.92  0.85  0.89  0.90  0.90  0.87
+  //     9         0.91  0.88  0.85  0.87  0.85  0.84  0.83
+  //    16         0.77  0.80  0.76  0.80  0.77  0.75  0.75
+  //    36         0.73  0.77  0.76  0.77  0.74  0.73  0.70
+  //    72         0.71  0.75  0.70  0.77  0.69
+  // The line was drawn for kernels 5 to 15 % behind these; below it the full products stay although pieces would be up
+  // to a tenth faster by now.  128x32 tiles 0.83 to 0.98 from 9 slabs on with 3x3, 0.97 to 1.04 pointwise.
   const long workgroups = tiles(p.cfg) * p.splits;
   const bool pieces = a.dtype == OGLE_F32 && (p.cfg == CFG_128x128 || p.cfg == CFG_64x64 || p.cfg == CFG_128x32) &&
              workgroups > kComputeUnits && p.slabs_per_split >= kPiecesSlabs &&
