@@ -738,7 +738,7 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
   int l_kt, l_cc, l_kx, l_dy, l_dx;
   unsigned l_tapbyte;
   auto enter_tap = [&]() {
-    const unsigned from = (unsigned)((l_dy * g.w + (RUNS ? 0 : l_dx)) * g.pixel * 4);
+    const unsigned from = tap_offset(g.w, g.pixel, l_dy, RUNS ? 0 : l_dx);
 #pragma unroll
     for (int i = 0; i < WR; ++i) {
       const bool in = (unsigned)(a_iy[i] + l_dy) < (unsigned)g.h &&

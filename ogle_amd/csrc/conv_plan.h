@@ -379,6 +379,12 @@ constexpr unsigned first_tap_offset(int h, int w, int pixel, int image, int iy, 
   return (((unsigned)image * (unsigned)h + (unsigned)iy) * (unsigned)w + (unsigned)ix) * (unsigned)pixel * 4u;
 }
 
+// How far behind a pixel's first tap another lies, modulo 2^32 as well: a first tap high up in the padding is farther
+// from the image's last rows than a signed offset reaches.
+constexpr unsigned tap_offset(int w, int pixel, int dy, int dx) {
+  return ((unsigned)dy * (unsigned)w + (unsigned)dx) * (unsigned)pixel * 4u;
+}
+
 // Whether a 16-byte load with a value of a pixel's runs begins before the tensor or ends behind it: such a load
 // returns zeros for all four.  `iy`: the row of the first filter row, `start`: the runs' first value, counted from
 // their rows' first; both may lie in the padding.  (The first row counts wherever it lies: a row of one or two

@@ -12,6 +12,10 @@ constexpr unsigned offset64(long h, long w, long pixel, long image, long iy, lon
 static_assert(first_tap_offset(11000, 12000, 4, 0, 11003, 12001) == offset64(11000, 12000, 4, 0, 11003, 12001), "");
 static_assert(first_tap_offset(8000, 1000, 4, 16, 7999, 1200) == offset64(8000, 1000, 4, 16, 7999, 1200), "");
 static_assert(first_tap_offset(100, 2000, 1000, 1, -40000, -40000) == offset64(100, 2000, 1000, 1, -40000, -40000), "");
+// A dilation as large as the map: the last tap, inside the image, from a first one above it.
+static_assert(tap_offset(100, 4, 2000000, 50) == offset64(1, 100, 4, 0, 2000000, 50), "");
+static_assert(first_tap_offset(1200000, 100, 4, 0, -1100000, 0) + tap_offset(100, 4, 2200000, 0) ==
+                  offset64(1200000, 100, 4, 0, 1100000, 0), "");
 
 extern "C" {
 
