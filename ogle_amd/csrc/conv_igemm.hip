@@ -655,7 +655,7 @@ constexpr int pieces_lds_bytes() { return KG * 2 * 3 * NB * 1024; }
 //
 // Measured on MI355X against both operands split on their way to LDS (32x32x16 MFMAs, 64 rows of each
 // operand per 64x64 tile and 16 channels), us: 19x19x512 -> 512 at batch 16 25.4 -> 23.8, 3x3 56x56x64 ->
-// 64 35.6 -> 28.7, 28x28x128 -> 128 38.1 -> 31.3, M = 11552, K = 512, N = 1024 73.1 -> 73.3 (165 TFLOP/s);
+// 64 35.6 -> 28.7, 28x28x128 -> 128 38.1 -> 31.3, M = 11552, K = 512, N = 1024 73.1 -> 68.0 (178 TFLOP/s);
 // error against 64-bit sums at K = 512 1.24e-7 -> 1.20e-7 (fp32 MFMAs 4.1e-7).  Large problems are bound by
 // power: the library's bf16 GEMM of 8192 cubed reaches 1145 / 6 = 191.  Smaller ones share it among LDS
 // writes, splitting and MFMAs; loads further ahead, and splitting interleaved with MFMAs by hand, gained nothing.
@@ -1002,7 +1002,7 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
         unsigned low = 0xffffffffu;
         look(i, j0, probe_all, low);
         low_all = min(low_all, low);
-        if (m0 + i * 16 < g.m_total && n0 + j0 * 16 < g.o) low_most = max(low_most, low);
+        low_most = max(low_most, m0 + i * 16 < g.m_total && n0 + j0 * 16 < g.o ? low : 0u);
       }
     // (no unit is all zeros if some lane has a sum that is not in each)
     const bool seems_right = !__any(probe_all != 0.f || probe_all != probe_all || low_all < kLeast - 1u) &&
@@ -1165,46 +1165,57 @@ __device__ __forceinline__ void pieces_tile(unsigned char* __restrict__ lds, con
     if (through) store_result16(at, v);
     else *reinterpret_cast<floatx4u*>(at) = floatx4u{v.x, v.y, v.z, v.w};
   };
+  // ONE: finished outputs to dense rows of whole vectors in one destination: nothing else is asked per store (M = 11552,
+  // K = 512, N = 1024 73.8 -> 68.0 us, 112 x 112 x 32, 3x3 -> 64 10.2 -> 9.8)
+  auto store_all = [&](auto one) {
+    constexpr bool ONE = decltype(one)::value;
 #pragma unroll
-  for (int i = 0; i < WR; ++i) {
+    for (int i = 0; i < WR; ++i) {
 #pragma unroll
-    for (int j0 = 0; j0 < NB; j0 += JC) {
+      for (int j0 = 0; j0 < NB; j0 += JC) {
 #pragma unroll
-      for (int j = 0; j < JC; ++j) {
-        float v[4];
+        for (int j = 0; j < JC; ++j) {
+          float v[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          v[r] = acc[i][j0 + j][r];
-          if (whole) v[r] = apply_epilogue(v[r] + bias[(j0 + j) * 16 + kq * 4 + r], p.ep);
+          for (int r = 0; r < 4; ++r) {
+            v[r] = acc[i][j0 + j][r];
+            if (ONE || whole) v[r] = apply_epilogue(v[r] + bias[(j0 + j) * 16 + kq * 4 + r], p.ep);
+          }
+          *reinterpret_cast<float4*>(mine + lr * PITCH + j * 16 + kq * 4) = make_float4(v[0], v[1], v[2], v[3]);
         }
-        *reinterpret_cast<float4*>(mine + lr * PITCH + j * 16 + kq * 4) = make_float4(v[0], v[1], v[2], v[3]);
-      }
-      const int col = n0 + j0 * 16 + cv * 4;
+        const int col = n0 + j0 * 16 + cv * 4;
 #pragma unroll
-      for (int it = 0; it < 16 / RPI; ++it) {
-        const float4 v = *reinterpret_cast<const float4*>(mine + (it * RPI + rsub) * PITCH + cv * 4);
-        const int row = m0 + i * 16 + it * RPI + rsub;
-        if (row >= g.m_total) continue;
-        if (!whole) {
-          if (col < opitch) store_result16(p.partial + ((long)split * g.m_total + row) * opitch + col, v);
-          continue;
-        }
-        // (a 16-byte store needs no more than 4-byte alignment)
-        float* const dst = static_cast<float*>(p.y) + out_row_offset(g, row, o1) + col;
-        float* const dst2 = static_cast<float*>(p.y2) + (long)row * o2 + (col - o1);
-        if (col + 4 <= o1) {
-          put(dst, v);
-        } else if (col >= o1 && col + 4 <= g.o) {
-          put(dst2, v);
-        } else {
-          const float e[4] = {v.x, v.y, v.z, v.w};
+        for (int it = 0; it < 16 / RPI; ++it) {
+          const float4 v = *reinterpret_cast<const float4*>(mine + (it * RPI + rsub) * PITCH + cv * 4);
+          const int row = m0 + i * 16 + it * RPI + rsub;
+          if (ONE) {
+            if (row < g.m_total && col < g.o) store_result16(static_cast<float*>(p.y) + (long)row * g.o + col, v);
+            continue;
+          }
+          if (row >= g.m_total) continue;
+          if (!whole) {
+            if (col < opitch) store_result16(p.partial + ((long)split * g.m_total + row) * opitch + col, v);
+            continue;
+          }
+          // (a 16-byte store needs no more than 4-byte alignment)
+          float* const dst = static_cast<float*>(p.y) + out_row_offset(g, row, o1) + col;
+          float* const dst2 = static_cast<float*>(p.y2) + (long)row * o2 + (col - o1);
+          if (col + 4 <= o1) {
+            put(dst, v);
+          } else if (col >= o1 && col + 4 <= g.o) {
+            put(dst2, v);
+          } else {
+            const float e[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (col + r < g.o) (col + r < o1 ? dst : dst2)[r] = e[r];
+            for (int r = 0; r < 4; ++r)
+              if (col + r < g.o) (col + r < o1 ? dst : dst2)[r] = e[r];
+          }
         }
       }
     }
-  }
+  };
+  if (whole && through && o2 == 0 && g.oimg == 0) store_all(std::true_type());
+  else store_all(std::false_type());
 }
 
 template <int WR, int NB, int WM, int KG, int MODE>
