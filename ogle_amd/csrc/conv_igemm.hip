@@ -1735,6 +1735,7 @@ Prepared prepare(const OgleConvArgs& a, long m, const IgemmPlan& p, int form) {
 // The form a problem takes next to others in one launch: with 256 threads, adding in the same order.
 int grouped_form(int form) {
   switch (form) {
+    case FORM_128x64:
     case FORM_128x64_W8: return FORM_64x64;
     case FORM_64x64_K2:
     case FORM_64x32_K2: return FORM_32x32_K2;
@@ -1760,6 +1761,9 @@ void launch_pieces(int form, bool pw, unsigned grid, hipStream_t s, const IgemmP
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x16, 2, 1, 4, 1)
     case FORM_128x128:   // pointwise only; the others have too many registers to keep
       launch((conv_pieces_kernel<2, 8, 4, 1, true>), dim3(grid), dim3(256), 0, s, arg);
+      break;
+    case FORM_128x64:    // the same
+      launch((conv_pieces_kernel<2, 4, 4, 1, true>), dim3(grid), dim3(256), 0, s, arg);
       break;
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_128x64_W8, 1, 4, 8, 1)
     OGLE_PIECES_CASE(conv_pieces_kernel, FORM_64x64_K2, 1, 4, 4, 2)

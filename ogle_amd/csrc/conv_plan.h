@@ -26,16 +26,16 @@ constexpr int kRowBytesF16Wide = 64;  // K bytes per tile row per slab of CFG_12
 // Workgroups that contract fp32 as bf16 pieces: rows x columns, four waves one above the other
 // unless named otherwise.  All but the K2 forms add an output's products in the same order.
 enum PiecesForm {
-  FORM_NONE = 0, FORM_64x64, FORM_128x32, FORM_128x128,
-  FORM_128x64_W8 = 5,   // eight waves of 16 rows
+  FORM_NONE = 0, FORM_64x64, FORM_128x32, FORM_128x128, FORM_128x64,
+  FORM_128x64_W8,       // eight waves of 16 rows
   FORM_64x64_K2,        // two groups of four waves take K stages in turn
   FORM_64x32_K2,
   FORM_32x32_K2,        // two groups of two waves: the K2 forms in a grouped launch
   FORM_128x16,
   FORM_64x32, FORM_64x16   // in a grouped launch for the two of 128 rows, which need more registers
 };
-constexpr int kFormBM[] = {0, 64, 128, 128, 0, 128, 64, 64, 32, 128, 64, 64};
-constexpr int kFormBN[] = {0, 64, 32, 128, 0, 64, 64, 32, 32, 16, 32, 16};
+constexpr int kFormBM[] = {0, 64, 128, 128, 128, 128, 64, 64, 32, 128, 64, 64};
+constexpr int kFormBN[] = {0, 64, 32, 128, 64, 64, 64, 32, 32, 16, 32, 16};
 
 struct IgemmPlan {
   int cfg;
@@ -74,6 +74,12 @@ constexpr bool pieces_rows_even(long tiles_m, long per_row) {
          (most > 8 * slots || (most + slots - 1) / slots == (least + slots - 1) / slots);
 }
 
+// 128x64 workgroups on the XCD that gets most of them.
+constexpr long most_on_xcd(long m, long out_c) {
+  const long rows = (m + 127) / 128, per_row = (out_c + 63) / 64;
+  return pieces_rows_even(rows, per_row) ? (rows + 7) / 8 * per_row : (rows * per_row + 7) / 8;
+}
+
 // The form for `m` output rows: `large` a plan of 128x128 tiles, `pieces` whether 64x64 tiles would be
 // pieces.  What counts is how evenly the workgroups spread over 256 units, and that a unit has waves
 // enough to cover what each waits for.  Us of the form taken / of another one, 3x3 unless 1x1:
@@ -87,6 +93,10 @@ constexpr bool pieces_rows_even(long tiles_m, long per_row) {
 //     73600, 40 -> 512 58.0 / 51.6, 96 channels of 128 M = 177480, 260 -> 96 86.8 / 81.3
 //   128x64, eight waves, against 64x64, mean ratio over 2000 shapes by number of workgroups: 257 to 383 1.06,
 //     384 to 512 0.93, 513 to 640 1.03, more 0.95; those many pointwise ones of up to 7 slabs 1.03 (3 slabs 1.06)
+//   128x64, four waves, against eight, pointwise from 8 slabs on, where a unit has more than two and a half: 641 to 1024
+//     1.05 over 90 shapes, 1025 to 1536 1.00, to 2560 0.99, more 0.95.  Three fit a unit at once; where no XCD has more,
+//     as 11552 x 256 -> 512, they are taken too: 28.1 / 28.0 alone (inputs half zeros 26.0 / 26.7), 21.5 / 22.4 behind its
+//     depthwise convolution, in the mean of 17 shapes alone 1.01
 inline int pieces_form(const OgleConvArgs& a, long m, int ktiles, bool large, bool pieces) {
   auto tiles = [&](int form) {
     return ((m + kFormBM[form] - 1) / kFormBM[form]) * ((a.out_c + kFormBN[form] - 1) / kFormBN[form]);
@@ -108,7 +118,9 @@ inline int pieces_form(const OgleConvArgs& a, long m, int ktiles, bool large, bo
   if (!large && !pieces) return FORM_NONE;
   if (2 * n128 <= 5 * kComputeUnits)
     return 2 * n128 >= 3 * kComputeUnits && n128 <= 2 * kComputeUnits ? FORM_128x64_W8 : FORM_64x64;
-  return pw && ktiles < 8 ? FORM_64x64 : FORM_128x64_W8;
+  if (!pw) return FORM_128x64_W8;
+  if (ktiles < 8) return FORM_64x64;
+  return n128 > 4 * kComputeUnits || most_on_xcd(m, a.out_c) <= 3 * kComputeUnits / 8 ? FORM_128x64 : FORM_128x64_W8;
 }
 
 // Picks the output tile and the K split.  Problems with few output
@@ -365,7 +377,7 @@ inline bool plan_runs(const OgleConvArgs& a, IgemmPlan* out) {
   if (((m + 63) / 64) * ((a.out_c + 31) / 32) <= kComputeUnits) p.form = FORM_64x32_K2;
   else if (a.out_c <= 32) p.form = a.out_c <= 16 ? FORM_128x16 : FORM_128x32;
   else p.form = pieces_form(a, m, p.ktiles, false, true);
-  if (p.form == FORM_NONE) p.form = FORM_64x64;
+  if (p.form == FORM_NONE || p.form == FORM_128x64) p.form = FORM_64x64;
   // with many tiles the filter, gathered value by value, counts: half as often per pixel, pointwise too (4 x 100 x
   // 140, 98 -> 127 28.2 / 27.0; the 7x7 stem 55.3 / 51.4)
   if (p.form == FORM_64x64 && m * a.out_c > 64L * 64 * 5 * kComputeUnits) p.form = FORM_128x64_W8;

@@ -236,7 +236,7 @@ def test_pieces_cases_run_what_they_name(probe):
 
 def test_batches_of_one_form(probe):
     """Every form that a grouped launch of one kind has a kernel for is the form of some batch's members."""
-    grouped = {5: 1, 6: 8, 7: 8, 2: 10, 9: 11}     # what stands in for a form in a group
+    grouped = {4: 1, 5: 1, 6: 8, 7: 8, 2: 10, 9: 11}     # what stands in for a form in a group
     kinds = set()
     for batch in K.BATCHES_OF_PIECES + K.BATCHES_OF_FORMS:
         forms = [probe.probe_form(ctypes.byref(conv(*case)), 1) for case in batch]
@@ -250,7 +250,7 @@ def test_form_cases_run_what_they_name(probe):
     """Every form of the pieces kernel is some case's (PiecesForm, conv_plan.h)."""
     forms = [probe.probe_form(ctypes.byref(conv(*case)), 1) for case, _ in K.FORM_CASES]
     assert forms == [form for _, form in K.FORM_CASES]
-    assert set(forms) == set(range(1, 10)) - {4, 8}   # 8 is the K2 forms' in a grouped launch, 4 no form
+    assert set(forms) == set(range(1, 10)) - {8}   # 8 is the K2 forms' in a grouped launch
 
 
 def test_rows_are_dealt_whole_where_no_unit_gets_another_round(probe):
@@ -273,7 +273,7 @@ def test_two_k_groups_where_the_wave_split_kernel_needs_a_second_round(probe):
 
 
 def test_forms_are_chosen_within_their_tiles(probe):
-    """128x128 workgroups are built for pointwise convolutions only, 128x32 ones for others; other types than fp32
+    """128x128 workgroups and 128x64 ones of four waves are built for pointwise convolutions only, 128x32 ones for others; other types than fp32
     have no form."""
     r, seen = random.Random(11), set()
     for _ in range(30000):
@@ -283,13 +283,13 @@ def test_forms_are_chosen_within_their_tiles(probe):
                  r.choice([12, 31, 40, 65, 100, 128, 168, 256, 512, 1024]), k, r.choice([1, 2]), k // 2)
         form = probe.probe_form(ctypes.byref(conv(*shape)), r.random() < 0.5)
         seen.add(form)
-        if form == 3:
+        if form in (3, 4):
             assert k == 1 and shape[6] == 1, shape
         if form == 2:
             assert k == 3 or shape[6] == 2, shape
         if shape[3] % 8 == 0:
             assert probe.probe_form(ctypes.byref(conv(*shape, dtype=H.F16)), 1) <= 0
-    assert seen - {-1} == set(range(0, 10)) - {4, 8}
+    assert seen - {-1} == set(range(0, 10)) - {8}
 
 
 def test_runs_cases_run_what_they_name(probe):

@@ -399,7 +399,9 @@ FORM_CASES = [
     ((16, 19, 19, 260, 500, 1, 1, 0), 1),   # 64x64, 17 slabs
     ((5, 84, 84, 36, 31, 3, 1, 1), 2),      # 128x32
     ((1, 223, 221, 260, 124, 1, 1, 0), 3),  # 128x128
-    ((1, 96, 97, 388, 520, 1, 1, 0), 5),    # 128x64, pointwise
+    ((1, 96, 97, 388, 520, 1, 1, 0), 4),    # 128x64 of four waves, all of them at once
+    ((1, 101, 103, 132, 864, 1, 1, 0), 4),  # the same, more than four a unit
+    ((1, 100, 102, 388, 650, 1, 1, 0), 5),  # 128x64 of eight waves, pointwise
     ((1, 223, 221, 100, 130, 1, 1, 0), 1),  # many 64x64, seven slabs
     ((1, 224, 224, 96, 384, 1, 1, 0), 1),   # the same in place of 128x128 tiles
     ((1, 119, 118, 36, 72, 3, 1, 1), 5),    # 128x64 of eight waves
